@@ -2,6 +2,7 @@
 // tiled MFMA kernel: an order-exact generic kernel for shapes/layouts the tiled kernel does not take, the B-operand
 // transpose (Layout::ND -> the K-contiguous form the MFMA path reads) and the MX scale re-layout.
 #include "common_host.hpp"
+#include "gemm_ring.hpp"
 #include "gemm_tile.hpp"
 
 #include <stdlib.h>
@@ -32,6 +33,21 @@ hipError_t launch_gemm_tile(int tile, int op, const TileGemmParams& p, hipStream
         case TOP_FP8_E4E5: return launch_gemm_tile_fp8_e4e5(tile, p, stream);
         case TOP_FP8_E5E4: return launch_gemm_tile_fp8_e5e4(tile, p, stream);
         case TOP_FP4: return launch_gemm_tile_fp4(tile, p, stream);
+        default: return hipErrorInvalidValue;
+    }
+}
+
+static hipError_t launch_gemm_ring(int shape, int op, const TileGemmParams& p, hipStream_t stream)
+{
+    switch (op) {
+        case TOP_BF16: return launch_gemm_ring_bf16(shape, p, stream);
+        case TOP_F16: return launch_gemm_ring_f16(shape, p, stream);
+        case TOP_I8: return launch_gemm_ring_i8(shape, p, stream);
+        case TOP_FP8_E4E4: return launch_gemm_ring_fp8_e4e4(shape, p, stream);
+        case TOP_FP8_E5E5: return launch_gemm_ring_fp8_e5e5(shape, p, stream);
+        case TOP_FP8_E4E5: return launch_gemm_ring_fp8_e4e5(shape, p, stream);
+        case TOP_FP8_E5E4: return launch_gemm_ring_fp8_e5e4(shape, p, stream);
+        case TOP_FP4: return launch_gemm_ring_fp4(shape, p, stream);
         default: return hipErrorInvalidValue;
     }
 }
@@ -267,7 +283,8 @@ static bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 
 static long ws_row_bytes(long k_bytes) { return (k_bytes + 15) / 16 * 16; }  // row pitch of a transposed B in a workspace
 static bool aligned4(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 3u) == 0; }
 
-// Which tile shape to run: the largest whose grid still fills most of the 256 CUs.  PTOAMD_TILE=0|1|2 overrides,
+// Which tile shape to run where the operands are not the DMA kernels' (pick_dma_tile, below, chooses among those): the largest
+// whose grid still fills most of the 256 CUs.  PTOAMD_TILE=0..7 overrides (both choices),
 // PTOAMD_FORCE_GENERIC=1 sends everything to the order-exact kernel (used by the parity tests).
 // Tiles 0-2 stage slabs through registers (any K); tiles 3-7 DMA slabs straight into LDS and need K to be a whole
 // number of 128-byte slabs (7: the 256 x 128 tile with a ring of three slabs, block-scaled types only -- for the other
@@ -317,6 +334,82 @@ static int pick_tile(int m, int n, long k_bytes, bool scaled, bool fp4 = false, 
     if (t128 >= 3 * cus / 8)
         return dtl_ok ? 5 : 1;
     return 2;
+}
+
+// ---- which DMA kernel: a shape of the deep-ring kernel or one of the two- and three-slab tiles above -------------------
+// A launch is estimated, in microseconds, as 3 for the launch plus, per round of workgroups over the CUs, a fixed part
+// (first copies, store) and a time per 128-byte slab of K -- what a round costs hardly depends on how full it is, each CU
+// waits for its own copies -- and no less than its slabs at the rate a full chip sustains (power, and the copies from the
+// L2s).  The numbers are fits to the times of every kernel on 110 sizes per operand type (m 1 .. 4096, n 256 .. 14336, k
+// 256 .. 8192).  Summed over those sizes, the fitted estimate's choices take 3.22, 2.74, 2.54 and 1.81 ms (bf16, int8, MXFP8,
+// MXFP4) where the best kernel for each takes 3.12, 2.64, 2.42 and 1.73 and the two- and three-slab tiles chosen by grid size
+// alone 4.74, 3.51, 3.23 and 2.10.
+struct TileCost {
+    float round, slab;  // us per round; us per round and slab
+    float rate;         // million elements of C times slabs per us
+};
+enum { COST_TILE4 = RING_SHAPES, COST_TILE5, COST_TILE7, COST_COUNT };
+static const TileCost tile_costs[3][COST_COUNT] = {
+    // plain types: 32x16, 32x32, 64x32, 64x64, 96x64, 128x64, 128x128, 192x128, 256x128; 256x256, 128x128 (two a CU), -
+    {{2.2f, 0.0625f, 8.0f}, {2.0f, 0.086f, 8.0f}, {2.6f, 0.125f, 8.0f}, {2.9f, 0.165f, 7.0f}, {3.2f, 0.19f, 7.0f}, {3.6f, 0.20f, 6.3f},
+     {4.7f, 0.29f, 8.0f}, {5.5f, 0.385f, 8.1f}, {6.0f, 0.49f, 7.8f}, {11.0f, 1.1f, 12.0f}, {2.9f, 0.545f, 6.6f}, {}},
+    // fp8: the first seven; 256x256, 128x128 (two a CU), 256x128 with three slabs
+    {{2.25f, 0.08f, 8.0f}, {2.0f, 0.12f, 8.0f}, {2.4f, 0.15f, 8.0f}, {3.0f, 0.19f, 5.0f}, {3.6f, 0.25f, 5.5f}, {3.75f, 0.24f, 5.0f},
+     {4.2f, 0.42f, 5.9f}, {}, {}, {7.1f, 1.1f, 11.0f}, {3.2f, 0.59f, 7.3f}, {4.7f, 0.55f, 8.5f}},
+    // fp4
+    {{2.5f, 0.09f, 8.0f}, {2.1f, 0.15f, 8.0f}, {2.4f, 0.20f, 8.0f}, {3.1f, 0.235f, 5.0f}, {3.8f, 0.265f, 5.0f}, {4.5f, 0.25f, 5.3f},
+     {5.0f, 0.40f, 5.5f}, {}, {}, {6.9f, 1.11f, 9.5f}, {4.2f, 0.56f, 6.7f}, {5.2f, 0.57f, 7.5f}},
+};
+constexpr int TILE_RING = 16;  // tile ids from here on: the deep-ring kernel's shapes
+
+// Block-scaled products of more than 64 rows keep away from the shapes that split K over groups of waves (0 .. 2): their sums
+// then run in k order and equal, bit for bit, those of the same product written in the tile ISA.
+// dtl_ok: tiles 4, 5 and 7 take this operand as well (K and, for block-scaled types, rows of scales they can stream)
+static int pick_dma_tile(int m, int n, long k_bytes, int op, bool dtl_ok)
+{
+    const bool scaled = op >= TOP_FP8_E4E4;
+    const int shapes = scaled ? RING_SHAPES_SCALED : RING_SHAPES;
+    if (options().ring >= 0 && options().ring < shapes)
+        return TILE_RING + options().ring;
+    // A round or more of 256 x 256 tiles: those (with the split of a part-filled last round below) are ahead from K = 1024 on
+    // -- bf16 4096 x 8192 x 2048: 105 us against 129 on 256 x 128 -- and within a tenth of the best where a sixteenth of a round
+    // is left over (4096 x 4312: 192 x 128 tiles 79 against 87 us at K = 2048).
+    if (dtl_ok && (long)((m + 255) / 256) * ((n + 255) / 256) >= device_compute_units())
+        return 4;
+    const TileCost* cost = tile_costs[op == TOP_FP4 ? 2 : (scaled ? 1 : 0)];
+    const int cus = device_compute_units();
+    const float slabs = (float)((k_bytes + 127) / 128);
+    // (a K that is no whole number of slabs costs the two-slab tiles half as much again: bf16 1280 x 4096, K 2048: 24.8 us,
+    // K 2056: 38.4 us)
+    const float ragged = (k_bytes % 128) != 0 ? 1.5f : 1.0f;
+    int best = TILE_RING;
+    float best_us = 1e30f;
+    for (int c = 0; c < COST_COUNT; ++c) {
+        if (c < RING_SHAPES ? c >= shapes : (!dtl_ok || (c == COST_TILE7 && !scaled)))
+            continue;
+        if (scaled && c <= 2 && m > 64)
+            continue;
+        static const int ids[3] = {4, 5, 7};
+        const int id = c < RING_SHAPES ? TILE_RING + c : ids[c - RING_SHAPES];
+        int bm, bn;
+        if (c < RING_SHAPES)
+            ring_shape(c, &bm, &bn);
+        else
+            tile_shape(id, &bm, &bn);
+        const long tiles = (long)((m + bm - 1) / bm) * ((n + bn - 1) / bn);
+        float rounds = (float)((tiles + cus - 1) / cus);
+        if (c == COST_TILE5) {  // two workgroups share a CU: the second adds 0.45 of the first one's time
+            const long whole = tiles / (2 * cus), rest = tiles % (2 * cus);
+            rounds = 1.45f * (float)whole + (rest == 0 ? 0.0f : rest <= cus ? 1.0f : 1.0f + 0.45f * (float)(rest - cus) / (float)cus);
+        }
+        const float full = (float)tiles * (float)(bm * bn) * 1e-6f / cost[c].rate;
+        const float us = 3.0f + rounds * cost[c].round + slabs * std::max(rounds * cost[c].slab, full) * (c < RING_SHAPES ? 1.0f : ragged);
+        if (us < best_us) {
+            best_us = us;
+            best = id;
+        }
+    }
+    return best;
 }
 
 // Launch on the chosen tile.  When the 256x256 grid is some (nearly) whole rounds of the CUs plus at most half a round,
@@ -379,6 +472,15 @@ static hipError_t launch_tiles_as(int tile, int op, const TileGemmParams& p, hip
 
 static hipError_t launch_tiles(int tile, int op, const TileGemmParams& p, hipStream_t stream)
 {
+    if (tile >= TILE_RING) {
+        int bm, bn;
+        ring_shape(tile - TILE_RING, &bm, &bn);
+        TileGemmParams r = p;
+        // a contiguous run of tiles shares an XCD's L2: whole columns of up to eight tiles, so that a panel of B is read once
+        const int tiles_m = (p.m + bm - 1) / bm;
+        r.group_m = tiles_m <= 8 ? tiles_m : 4;
+        return launch_gemm_ring(tile - TILE_RING, op, r, stream);
+    }
     // tile id 3: the 16x16x128 form of the block-scaled fp8 types' large tile (the other types have one form, under both
     // ids).  Same results bit for bit and, on MXFP8 4096 x 14336 x 4096, the same time: 2 718 clocks per slab at 1.71 GHz
     // against 2 500 at 1.58 GHz on one box -- what the part sustains under this kernel is a rate of matrix work, not a
@@ -407,6 +509,12 @@ static const char* tile_kernel_name(int tile, int op)
     static const char* tiles[8] = {"tile256x256", "tile128x128", "tile64x64", "tile256x256w8x16_dtl", "tile256x256w8_dtl",
                                    "tile128x128_dtl", "tile256x128_dtl", "tile256x128r3_dtl"};
     static thread_local char buf[64];
+    if (tile >= TILE_RING) {
+        int bm, bn;
+        ring_shape(tile - TILE_RING, &bm, &bn);
+        snprintf(buf, sizeof buf, "tile%dx%d_dtl_%s", bm, bn, ops[op]);
+        return buf;
+    }
     snprintf(buf, sizeof buf, "%s_%s", tiles[tile], ops[op]);
     return buf;
 }
@@ -450,8 +558,10 @@ static int static_scratch(uint8_t** ptr)
 
 int prepare_gemm_kernels()
 {
-    for (int op : {TOP_BF16, TOP_F16, TOP_I8, TOP_FP8_E4E4, TOP_FP8_E5E5, TOP_FP8_E4E5, TOP_FP8_E5E4, TOP_FP4})
+    for (int op : {TOP_BF16, TOP_F16, TOP_I8, TOP_FP8_E4E4, TOP_FP8_E5E5, TOP_FP8_E4E5, TOP_FP8_E5E4, TOP_FP4}) {
         PTOAMD_HIP_CHECK(launch_gemm_tile(TILE_PREPARE_ALL, op, TileGemmParams{}, nullptr));
+        PTOAMD_HIP_CHECK(launch_gemm_ring(TILE_PREPARE_ALL, op, TileGemmParams{}, nullptr));
+    }
     uint8_t* unused = nullptr;
     return static_scratch(&unused);
 }
@@ -646,7 +756,12 @@ static int gemm_common(void* c, int c_type, const void* a, const void* b, int ab
     // (LDS-DMA needs dword-aligned global addresses, no more: rows at 4-byte alignment run 114 against 100 us on bf16 4096^3)
     const bool dma_ok = !b_in_kernel && aligned4(a) && aligned4(b_kmajor) && (lda_b % 4) == 0 && (ldb_kmajor % 4) == 0 &&
                         dma_offsets_fit(m, n, lda_b, ldb_kmajor, k_bytes);
-    const int tile = pick_tile(m, n, k_bytes, false, false, dma_ok, op == TOP_BF16 || op == TOP_F16 || op == TOP_I8);
+    // (the deep-ring kernel reads a chunk that K ends in as the 16 bytes ending there, which must start on a dword)
+    // (the deep-ring kernel reads a chunk that K ends in as the 16 bytes ending there, which must start on a dword)
+    const bool ragged_k_form = op == TOP_BF16 || op == TOP_F16 || op == TOP_I8, whole_slabs = (k_bytes % 128) == 0;
+    const int tile = options().tile < 0 && dma_ok && (k_bytes % 4) == 0
+                         ? pick_dma_tile(m, n, k_bytes, op, whole_slabs || (ragged_k_form && k_bytes > 128))
+                         : pick_tile(m, n, k_bytes, false, false, dma_ok, ragged_k_form);
     PTOAMD_HIP_CHECK(launch_tiles(tile, op, p, stream));
     set_last_kernel(tile_kernel_name(tile_as_launched(tile, op, m, n), op));
     return PTOAMD_OK;
@@ -684,7 +799,8 @@ int ptoamd_gemm_w8a8(void* out_bf16, int32_t* acc_out, const int8_t* a, const in
     p.out_kind = OUT_W8A8_BF16; p.group_m = 4;
     p.b_nd = b_in_kernel; p.b_esz = 1;
     const bool dma_ok = !b_in_kernel && aligned4(a) && aligned4(b) && (lda % 4) == 0 && (ldb % 4) == 0 && dma_offsets_fit(m, n, lda, ldb, k);
-    const int tile = pick_tile(m, n, k, false, false, dma_ok, true);
+    const int tile = options().tile < 0 && dma_ok && (k % 4) == 0 ? pick_dma_tile(m, n, k, TOP_I8, (k % 128) == 0 || k > 128)
+                                                                  : pick_tile(m, n, k, false, false, dma_ok, true);
     PTOAMD_HIP_CHECK(launch_tiles(tile, TOP_I8, p, stream));
     set_last_kernel(tile_kernel_name(tile, TOP_I8));
     return PTOAMD_OK;
@@ -826,8 +942,11 @@ static int gemm_mx_common(const char* who, void* c, int c_type, const void* a, c
     const long k_slabs = k_bytes / 128;
     const bool scale_dma_ok = plain_scales && !b_in_kernel && (kg % 16) == 0 && aligned16(sa_nd) && aligned16(sb_dn) &&
                               (k_slabs % (a4 ? 2 : 4)) == 0;
+    // (the deep-ring kernel fetches them as dwords: any K that is a multiple of 128, which the row-length check above asks for)
+    const bool dma_ok = !e1m2 && plain_scales && !b_in_kernel && dma_offsets_fit(m, n, lda_b, ldb_b, k_bytes);
     const int tile = e1m2 ? pick_tile(m, n, k, true, false, false)
-                          : pick_tile(m, n, k_bytes, true, a4, scale_dma_ok && dma_offsets_fit(m, n, lda_b, ldb_b, k_bytes));
+                     : options().tile < 0 && dma_ok && (kg % 4) == 0 ? pick_dma_tile(m, n, k_bytes, op, scale_dma_ok)
+                                                                    : pick_tile(m, n, k_bytes, true, a4, dma_ok && scale_dma_ok);
     PTOAMD_HIP_CHECK(launch_tiles(tile, op, p, stream));
     set_last_kernel(tile_kernel_name(tile_as_launched(tile, op, m, n), op));
     return PTOAMD_OK;

@@ -1,0 +1,52 @@
+// The tile shapes of the deep-ring kernel (gemm_tile_ring.hpp) and its launchers, one per operand type.
+#pragma once
+#include <hip/hip_runtime.h>
+
+namespace ptoamd {
+
+struct TileGemmParams;
+
+// id, BM, BN, then waves along M, N, K, stage bytes per row and stages in the ring -- of the plain types and of the
+// block-scaled ones, whose matrix instruction takes 128 bytes (fp8) of K --, then waves that only copy, pipelined form.
+// Stage widths: 1 KiB where K is split over eight waves of a narrow tile (a copy is then one contiguous KiB of a weight
+// row), 256 bytes where it is split over two or the tile is small, one 128-byte slab otherwise.  Block-scaled types split K in
+// the first three shapes only.  Ring depth: what 160 KiB hold.  The narrow
+// tiles wait for memory whoever copies, so all their waves do; in the others four extra waves only copy, because a wave
+// that issues copies stands still while the CU's memory queue is full (128 x 128, bf16 2048 x 2048 x 4096: 50 us with every
+// wave copying and multiplying, 33 us with the roles split).
+#define PTOAMD_RING_SHAPES_ALL(X)                                 \
+    X(0, 32, 16, 1, 1, 8, 1024, 3, 1, 1, 8, 1024, 3, 0, false)    \
+    X(1, 32, 32, 1, 1, 8, 512, 4, 1, 2, 4, 512, 4, 0, false)      \
+    X(2, 64, 32, 1, 1, 8, 512, 3, 2, 1, 4, 512, 3, 0, false)      \
+    X(3, 64, 64, 2, 2, 2, 256, 4, 2, 4, 1, 256, 4, 4, true)       \
+    X(4, 96, 64, 2, 2, 2, 256, 4, 2, 4, 1, 256, 3, 4, true)       \
+    X(5, 128, 64, 2, 2, 2, 256, 3, 4, 2, 1, 256, 3, 4, true)      \
+    X(6, 128, 128, 2, 4, 1, 128, 4, 2, 4, 1, 128, 4, 4, true)
+// the plain types only: a block-scaled wave tile of this size does not fit the 168 registers of twelve waves
+#define PTOAMD_RING_SHAPES_PLAIN(X)                               \
+    X(7, 192, 128, 4, 2, 1, 128, 4, 4, 2, 1, 128, 3, 4, true)     \
+    X(8, 256, 128, 4, 2, 1, 128, 3, 4, 2, 1, 128, 3, 4, true)
+constexpr int RING_SHAPES = 9, RING_SHAPES_SCALED = 7;
+
+inline void ring_shape(int shape, int* bm, int* bn)
+{
+    static const int dims[RING_SHAPES][2] = {
+#define PTOAMD_RING_DIM(id, bm, bn, ...) {bm, bn},
+        PTOAMD_RING_SHAPES_ALL(PTOAMD_RING_DIM) PTOAMD_RING_SHAPES_PLAIN(PTOAMD_RING_DIM)
+#undef PTOAMD_RING_DIM
+    };
+    *bm = dims[shape][0];
+    *bn = dims[shape][1];
+}
+
+// shape: 0 .. RING_SHAPES - 1, or TILE_PREPARE_ALL
+hipError_t launch_gemm_ring_bf16(int shape, const TileGemmParams& p, hipStream_t stream);
+hipError_t launch_gemm_ring_f16(int shape, const TileGemmParams& p, hipStream_t stream);
+hipError_t launch_gemm_ring_i8(int shape, const TileGemmParams& p, hipStream_t stream);
+hipError_t launch_gemm_ring_fp8_e4e4(int shape, const TileGemmParams& p, hipStream_t stream);
+hipError_t launch_gemm_ring_fp8_e4e5(int shape, const TileGemmParams& p, hipStream_t stream);
+hipError_t launch_gemm_ring_fp8_e5e4(int shape, const TileGemmParams& p, hipStream_t stream);
+hipError_t launch_gemm_ring_fp8_e5e5(int shape, const TileGemmParams& p, hipStream_t stream);
+hipError_t launch_gemm_ring_fp4(int shape, const TileGemmParams& p, hipStream_t stream);
+
+}  // namespace ptoamd

@@ -1,0 +1,59 @@
+// Instantiates gemm_tile_ring_kernel for one operand type at the shapes of gemm_ring.hpp.  Included by
+// gemm_ring_<op>.hip with PTOAMD_RING_OP (the traits type) and PTOAMD_RING_FN (the launcher's name) defined.
+#include "common_host.hpp"
+#include "gemm_ring.hpp"
+#include "gemm_tile_ring.hpp"
+
+namespace ptoamd {
+
+template <class Cfg>
+static hipError_t launch_ring(const TileGemmParams& p, hipStream_t stream)
+{
+    const hipError_t e = ensure_dynamic_lds(reinterpret_cast<const void*>(&gemm_tile_ring_kernel<Cfg>), Cfg::LDS_BYTES);
+    if (e != hipSuccess || p.m <= 0)  // m = 0: only make the kernel ready to launch on the current device
+        return e;
+    const int tiles = ((p.m + Cfg::BM - 1) / Cfg::BM) * ((p.n + Cfg::BN - 1) / Cfg::BN);
+    hipLaunchKernelGGL((gemm_tile_ring_kernel<Cfg>), dim3(tiles), dim3(Cfg::THREADS), Cfg::LDS_BYTES, stream, p);
+    return hipGetLastError();
+}
+
+template <class Op>
+static hipError_t launch_ring_shape(int shape, const TileGemmParams& p, hipStream_t stream)
+{
+    switch (shape) {
+#define PTOAMD_RING_CASE(id, bm, bn, wm, wn, wk, sb, r, swm, swn, swk, ssb, sr, lw, pipe)                            \
+    case id:                                                                                                        \
+        if constexpr (Op::SCALED)                                                                                   \
+            return launch_ring<RingCfg<bm, bn, swm, swn, swk, ssb, sr, lw, pipe, Op>>(p, stream);                   \
+        else                                                                                                        \
+            return launch_ring<RingCfg<bm, bn, wm, wn, wk, sb, r, lw, pipe, Op>>(p, stream);
+        PTOAMD_RING_SHAPES_ALL(PTOAMD_RING_CASE)
+#undef PTOAMD_RING_CASE
+        default: break;
+    }
+    if constexpr (!Op::SCALED) {
+        switch (shape) {
+#define PTOAMD_RING_CASE(id, bm, bn, wm, wn, wk, sb, r, swm, swn, swk, ssb, sr, lw, pipe) \
+    case id: return launch_ring<RingCfg<bm, bn, wm, wn, wk, sb, r, lw, pipe, Op>>(p, stream);
+            PTOAMD_RING_SHAPES_PLAIN(PTOAMD_RING_CASE)
+#undef PTOAMD_RING_CASE
+            default: break;
+        }
+    }
+    return hipErrorInvalidValue;
+}
+
+hipError_t PTOAMD_RING_FN(int shape, const TileGemmParams& p, hipStream_t stream)
+{
+    if (shape != TILE_PREPARE_ALL)
+        return launch_ring_shape<PTOAMD_RING_OP>(shape, p, stream);
+    const TileGemmParams none{};
+    for (int s = 0; s < (PTOAMD_RING_OP::SCALED ? RING_SHAPES_SCALED : RING_SHAPES); ++s) {
+        const hipError_t e = launch_ring_shape<PTOAMD_RING_OP>(s, none, stream);
+        if (e != hipSuccess)
+            return e;
+    }
+    return hipSuccess;
+}
+
+}  // namespace ptoamd

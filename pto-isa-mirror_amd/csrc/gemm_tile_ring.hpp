@@ -1,0 +1,517 @@
+// Tiled MFMA GEMM, deep-ring form: for grids that leave CUs idle or have one workgroup per CU, and for few rows of A.
+//
+// What bounds such a grid is the latency of the copy-in, not the matrix cores and not a bandwidth: the 128 x 128 DMA
+// tile takes 0.6 us per 128-byte slab whether 128 or 256 of them run, because only one slab is in flight while one is
+// multiplied.  Here a CU's LDS holds a ring of R stages, R - 1 of them in flight, a tile's shape is chosen so that one
+// round of workgroups covers the matrix, and a stage of a narrow tile is up to 1 KiB of every row, split over groups of
+// waves along K (each group multiplies its own part of the stage; the partial sums meet in LDS when K is done).  With
+// 16 columns of B per workgroup a decode step of 4096 columns reads its weights through 256 CUs.
+//
+//   TLOAD      global_load_lds_dwordx4, lane-linear in LDS, 16-byte chunks swizzled on the global-address side; every wave
+//              issues the same number of copies per stage, so a stage is waited for by count (vmcnt)
+//   TEXTRACT   ds_read_b128 fragments; the swizzle makes the 16 rows of a lane group fall into different banks
+//   TMATMUL    the 16x16 matrix instructions of every operand type (block-scaled types: one dword of E8M0 per 128 K)
+//   sync       one workgroup barrier per stage: behind it the stage has landed and the previous one may be overwritten
+//   K tail     copies never read past a row: a chunk that would is read as the 16 bytes that END at the row's end, and the
+//              last stage's fragments are masked in registers -- the same bytes of A and B, so k positions still agree
+#pragma once
+#include "gemm_tile_dtl.hpp"
+
+namespace ptoamd {
+
+// fp4 E2M1 on the 16x16x128 scaled instruction: a lane holds 16 bytes of one of 16 rows = one MX block, and its scale
+struct OpFP4x16 {
+    static constexpr int BLK = 16, ACC_REGS = 4;
+    using Acc = f32x4;
+    using Elem = float;
+    static constexpr int FRAG_BYTES = 16;
+    static constexpr bool SCALED = true;
+    static constexpr int GROUPS_PER_SLAB = 8;
+    __device__ static __forceinline__ void mma(Acc& c, const uint4* a, const uint4* b, uint32_t sa, uint32_t sb)
+    {
+        i32x8 av = {0, 0, 0, 0, 0, 0, 0, 0}, bv = {0, 0, 0, 0, 0, 0, 0, 0};
+        av.s0 = a[0].x; av.s1 = a[0].y; av.s2 = a[0].z; av.s3 = a[0].w;
+        bv.s0 = b[0].x; bv.s1 = b[0].y; bv.s2 = b[0].z; bv.s3 = b[0].w;
+        c = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(bv, av, c, 4, 4, 0, (int)sb, 0, (int)sa);
+    }
+};
+
+// WM x WN x WK waves: WK groups share the tile and split every stage of SB bytes per row along K; R stages in the ring
+template <int BM_, int BN_, int WM_, int WN_, int WK_, int SB_, int R_, int LW_, bool PIPE_, class Op_>
+struct RingCfg {
+    static constexpr int BM = BM_, BN = BN_, WM = WM_, WN = WN_, WK = WK_, SB = SB_, R = R_;
+    static constexpr bool PIPE = PIPE_;
+    using Op = Op_;
+    static constexpr int CW = WM * WN * WK, LW = LW_, THREADS = (CW + LW) * 64;
+    static constexpr int NW = LW > 0 ? LW : CW;  // waves that copy
+    static constexpr int WTM = BM / WM, WTN = BN / WN, MB = WTM / 16, NB = WTN / 16;
+    static constexpr int FR = Op::FRAG_BYTES / 16, KB = 4 * Op::FRAG_BYTES;  // bytes of K one matrix instruction takes
+    static constexpr int KW = SB / WK, KSTEPS = KW / KB;
+    static constexpr int ROWS = BM + BN, CPR = SB / 16, RPP = 1024 / SB;  // chunks per row, rows per 1 KiB piece
+    static constexpr int PIECES = ROWS * SB / 1024, A_PIECES = BM * SB / 1024, NPW = PIECES / NW;
+    static constexpr int SC = Op::SCALED ? SB / KB : 0;                   // scale dwords (four groups each) per row and stage
+    static constexpr int SPC = ROWS * SC / 64, NSW = (SPC + NW - 1) / NW; // 64-dword scale pieces; per wave
+    static constexpr int NV = NPW + NSW;                                  // copies a wave issues per stage
+    static constexpr int STAGE = ROWS * SB + ROWS * SC * 4;
+    static constexpr int RED_PITCH = BN + 4;                              // elements
+    static constexpr int RED_BYTES = WK * BM * RED_PITCH * 4;
+    static constexpr int LDS_BYTES = (R * STAGE > RED_BYTES ? R * STAGE : RED_BYTES);
+    static_assert(BM % (16 * WM) == 0 && BN % (16 * WN) == 0, "wave tiles are made of 16x16 blocks");
+    static_assert(KW % KB == 0 && SB <= 1024 && 1024 % SB == 0, "a k-group's part of a stage is whole k-steps");
+    static_assert(PIECES % NW == 0 && (BM * SB) % 1024 == 0, "every wave issues the same number of 1 KiB copies, each of one operand");
+    static_assert((ROWS * SC) % 64 == 0, "scale pieces are whole");
+    static_assert(LDS_BYTES <= 160 * 1024 && R >= 2 && (R - 1) * NV < 64, "LDS capacity; vmcnt is a 6-bit count");
+};
+
+// position of a row's 16-byte chunk is chunk ^ ring_swizzle(row)
+template <int SB>
+__device__ __forceinline__ int ring_swizzle(int row)
+{
+    return SB == 128 ? swizzle_chunk(row, 0) : (row & 15);
+}
+
+template <int N>
+__device__ __forceinline__ void ring_wait_and_barrier()
+{
+    // own copies up to the stage have landed, own fragment reads of the previous stage have returned; then everybody's
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" : : "n"(N) : "memory");
+}
+
+// the K tail: of the 16 bytes of a fragment chunk only `valid` belong to the row, the last ones (valid >= 16: all)
+__device__ __forceinline__ uint4 ring_mask_chunk(uint4 v, int valid)
+{
+    const int drop = 16 - valid;  // low bytes to clear
+    uint32_t w[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const int n = drop - 4 * i;
+        w[i] = n <= 0 ? w[i] : (n >= 4 ? 0u : w[i] & (0xFFFFFFFFu << (8 * n)));
+    }
+    return make_uint4(w[0], w[1], w[2], w[3]);
+}
+
+// Consecutive columns of an output row that one thread drains: 16 bytes of 16- and 32-bit outputs.
+template <int KIND>
+constexpr int ring_cols = out_bytes<KIND> == 2 ? 8 : 4;
+// What depends on the column only.  A thread drains the same columns of several rows and fetches these once (fetched with
+// every row they cost bf16 1237 x 4100 x 2056 with a bias row 8 us).
+template <int KIND, int NE, class Elem>
+struct RingColumns {
+    Elem bias[NE];
+    float scale[NE];
+    uint64_t qw[NE];
+    __device__ __forceinline__ void load(const TileGemmParams& p, int gj)
+    {
+#pragma unroll
+        for (int e = 0; e < NE; ++e) {
+            const int c = min(gj + e, p.n - 1);
+            bias[e] = p.bias != nullptr ? reinterpret_cast<const Elem*>(p.bias)[c] : 0;
+            scale[e] = KIND == OUT_W8A8_BF16 ? p.col_scale[c] : 1.0f;
+            qw[e] = out_quant<KIND> ? p.qwords[p.q_per_column ? c : 0] : 0;
+        }
+    }
+};
+template <int KIND, int NE, class Elem>
+__device__ __forceinline__ void ring_store(const TileGemmParams& p, Elem (&v)[NE], const RingColumns<KIND, NE, Elem>& cols, float rs, int gi, int gj)
+{
+    const long o = (long)gi * p.ldc + gj;
+    const int live = min(NE, p.n - gj);
+    const bool raw = KIND == OUT_W8A8_BF16 && p.acc_out != nullptr;
+    if (p.c_in != nullptr) {
+#pragma unroll
+        for (int e = 0; e < NE; ++e)
+            v[e] += reinterpret_cast<const Elem*>(p.c_in)[o + (e < live ? e : 0)];
+    }
+    if (p.bias != nullptr) {
+#pragma unroll
+        for (int e = 0; e < NE; ++e)
+            v[e] += cols.bias[e];
+    }
+    if (!out_quant<KIND> && (p.relu & 1)) {
+#pragma unroll
+        for (int e = 0; e < NE; ++e)
+            v[e] = v[e] > 0 ? v[e] : 0;
+    }
+    if (raw) {
+#pragma unroll
+        for (int e = 0; e < NE; ++e)
+            if (e < live)
+                p.acc_out[o + e] = (int32_t)v[e];
+    }
+    uint32_t bits[NE];
+#pragma unroll
+    for (int e = 0; e < NE; ++e)
+        bits[e] = tstore_bits<KIND>(v[e], rs, cols.scale[e], cols.qw[e], p.q_per_column != 0, p.relu, p.out_kind);
+    if ((KIND == OUT_F32 || KIND == OUT_I32) && p.atomic_add) {
+#pragma unroll
+        for (int e = 0; e < NE; ++e)
+            if (e < live) {
+                if (KIND == OUT_F32)
+                    atomicAdd(reinterpret_cast<float*>(p.c) + o + e, __builtin_bit_cast(float, bits[e]));
+                else
+                    atomicAdd(reinterpret_cast<int*>(p.c) + o + e, (int)bits[e]);
+            }
+        return;
+    }
+    uint8_t* dst = reinterpret_cast<uint8_t*>(p.c) + o * out_bytes<KIND>;
+    if (live == NE) {
+        // Vector stores go to any address.  Non-temporal: C is not read again here, and written back from the L2s it slows the
+        // next launch (2048 x 4096 x 4096 to f32: 82 us with plain stores, 67 with these).
+        if constexpr (out_bytes<KIND> == 1) {
+            const uint32_t w = bits[0] | (bits[1] << 8) | (bits[2] << 16) | (bits[3] << 24);
+            __builtin_memcpy(dst, &w, 4);
+        } else {
+            typedef uint32_t nt4 __attribute__((ext_vector_type(4), aligned(1)));
+            nt4 w;
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                w[i] = out_bytes<KIND> == 2 ? bits[(2 * i) % NE] | (bits[(2 * i + 1) % NE] << 16) : bits[i];
+            __builtin_nontemporal_store(w, reinterpret_cast<nt4*>(dst));
+        }
+    } else {
+#pragma unroll
+        for (int e = 0; e < NE - 1; ++e)
+            if (e < live) {
+                if (out_bytes<KIND> == 4)
+                    reinterpret_cast<uint32_t*>(dst)[e] = bits[e];
+                else if (out_bytes<KIND> == 2)
+                    reinterpret_cast<uint16_t*>(dst)[e] = (uint16_t)bits[e];
+                else
+                    dst[e] = (uint8_t)bits[e];
+            }
+    }
+}
+
+template <class Cfg>
+__global__ void __launch_bounds__(Cfg::THREADS) gemm_tile_ring_kernel(const TileGemmParams p)
+{
+    using Op = typename Cfg::Op;
+    using Acc = typename Op::Acc;
+    using Elem = typename Op::Elem;
+    constexpr int BM = Cfg::BM, BN = Cfg::BN, MB = Cfg::MB, NB = Cfg::NB, FR = Cfg::FR, SB = Cfg::SB, R = Cfg::R, NW = Cfg::NW;
+    constexpr int NPW = Cfg::NPW, NSW = Cfg::NSW, NV = Cfg::NV, SC = Cfg::SC, CPR = Cfg::CPR;
+    extern __shared__ __align__(16) uint8_t smem[];
+
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const bool loads = Cfg::LW == 0 || wave >= Cfg::CW, computes = Cfg::LW == 0 || wave < Cfg::CW;
+    const int lw = Cfg::LW == 0 ? wave : wave - Cfg::CW;  // number among the waves that copy
+    const int wk = wave / (Cfg::WM * Cfg::WN), wmn = wave % (Cfg::WM * Cfg::WN), wm = wmn % Cfg::WM, wn = wmn / Cfg::WM;
+    const int l16 = lane & 15, lg = lane >> 4;
+
+    // ---- workgroup -> tile.  Workgroup ids go round-robin to the 8 XCDs; XCD x takes a contiguous run of tiles, walked in
+    // groups of group_m tile rows, so that what an L2 holds is a few panels of A and of B.
+    const int tiles_m = (p.m + BM - 1) / BM, tiles_n = (p.n + BN - 1) / BN, grid = tiles_m * tiles_n;
+    const int xcd = blockIdx.x & 7;
+    const int lid = xcd * (grid >> 3) + min(xcd, grid & 7) + (blockIdx.x >> 3);
+    const int per_group = p.group_m * tiles_n;
+    const int first_m = (lid / per_group) * p.group_m;
+    const int gsize = min(tiles_m - first_m, p.group_m);
+    const int m0 = (first_m + (lid % per_group) % gsize) * BM, n0 = ((lid % per_group) / gsize) * BN;
+
+    // ---- TLOAD addressing: piece w + q * NW of a stage, lane -> (row, position) linear, fetching chunk position ^ swizzle
+    const int nst = (p.k_bytes + SB - 1) / SB;
+    const bool k_tail = p.k_bytes % SB != 0;
+    const uint32_t lds0 = lds_address(smem);
+    auto piece_row = [&](int q) { return (lw + q * NW) * Cfg::RPP + lane / CPR; };
+    auto piece_chunk = [&](int q) { return (lane % CPR) ^ ring_swizzle<SB>(piece_row(q)); };
+    auto row_offset = [&](int q) -> uint32_t {
+        const int r = piece_row(q);
+        return lw + q * NW < Cfg::A_PIECES ? (uint32_t)(min(m0 + r, p.m - 1) * p.lda_bytes) : (uint32_t)(min(n0 + r - BM, p.n - 1) * p.ldb_bytes);
+    };
+    uint32_t goff[NPW];
+#pragma unroll
+    for (int q = 0; q < NPW; ++q)
+        goff[q] = row_offset(q) + piece_chunk(q) * 16;
+    // scales: dword e = row * SC + d of a stage's scale area; without scale arrays the copies fetch bytes of A that are not used
+    const bool has_scales = Op::SCALED && p.sa != nullptr;
+    const uint8_t* sc_row[NSW > 0 ? NSW : 1];
+    int sc_d[NSW > 0 ? NSW : 1];
+    const int sc_last = has_scales ? p.scale_ld / 4 - 1 : 0;  // last scale dword of a row
+    if constexpr (NSW > 0) {
+#pragma unroll
+        for (int q = 0; q < NSW; ++q) {
+            const int e = ((lw + q * NW) % Cfg::SPC) * 64 + lane, r = e / SC;
+            sc_d[q] = e % SC;
+            sc_row[q] = !has_scales ? p.a : r < BM ? p.sa + (long)min(m0 + r, p.m - 1) * p.scale_ld : p.sb + (long)min(n0 + r - BM, p.n - 1) * p.scale_ld;
+        }
+    }
+    auto issue = [&](int st, int buf) __attribute__((always_inline)) {
+        const uint32_t dst = __builtin_amdgcn_readfirstlane(lds0 + buf * Cfg::STAGE);
+        const long kb = (long)st * SB;
+        if (k_tail && st == nst - 1) {
+#pragma unroll
+            for (int q = 0; q < NPW; ++q) {
+                const int piece = lw + q * NW;
+                const uint32_t off = row_offset(q) + (uint32_t)min(st * SB + piece_chunk(q) * 16, p.k_bytes - 16);
+                lds_dma16_off(piece < Cfg::A_PIECES ? p.a : p.b, off, dst + piece * 1024);
+            }
+        } else {
+#pragma unroll
+            for (int q = 0; q < NPW; ++q) {
+                const int piece = lw + q * NW;
+                lds_dma16_off((piece < Cfg::A_PIECES ? p.a : p.b) + kb, goff[q], dst + piece * 1024);
+            }
+        }
+        if constexpr (NSW > 0) {
+#pragma unroll
+            for (int q = 0; q < NSW; ++q)
+                lds_dma4(sc_row[q] + 4 * min(st * SC + sc_d[q], sc_last), dst + Cfg::ROWS * SB + ((lw + q * NW) % Cfg::SPC) * 256);
+        }
+    };
+
+    Acc acc[MB][NB];
+#pragma unroll
+    for (int i = 0; i < MB; ++i)
+#pragma unroll
+        for (int j = 0; j < NB; ++j)
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+                acc[i][j][r] = 0;
+
+    // ---- fragments: chunk c0 + lg of row l16 of a block, c0 a multiple of 4, sits at position c0 ^ (lg ^ swizzle(l16))
+    const uint32_t lane_x = (uint32_t)((lg ^ ring_swizzle<SB>(l16)) ^ (wk * (Cfg::KW / 16))) << 4;
+    const uint32_t fa_row = (wm * Cfg::WTM + l16) * SB, fb_row = (BM + wn * Cfg::WTN + l16) * SB;
+    const uint32_t sa_at = Cfg::ROWS * SB + (wm * Cfg::WTM + l16) * (SC * 4) + lg, sb_at = Cfg::ROWS * SB + (BM + wn * Cfg::WTN + l16) * (SC * 4) + lg;
+    // Fragment registers.  PIPE: B's fragments and A's last row block have two sets, alternating per k-step; the other row
+    // blocks of A are refilled in place right after their last matrix instruction, several of them before the next k-step
+    // reads them.
+    constexpr int SETS = Cfg::PIPE ? 2 : 1, NMMA = MB * NB;
+    uint4 fa[SETS][MB][FR], fb[SETS][NB][FR];
+    uint32_t xa[SETS][MB], xb[SETS][NB];
+    auto aset = [](int set, int i) constexpr { return i == MB - 1 ? set : 0; };
+    auto read_a = [&](int set, int i, int s, int b) __attribute__((always_inline)) {
+        const uint8_t* base = smem + b * Cfg::STAGE;
+#pragma unroll
+        for (int f = 0; f < FR; ++f)
+            fa[set][i][f] = *reinterpret_cast<const uint4*>(base + fa_row + i * (16 * SB) + (lane_x ^ ((s * 4 * FR + 4 * f) << 4)));
+        if constexpr (Op::SCALED)
+            xa[set][i] = base[sa_at + (wk * Cfg::KSTEPS + s) * 4 + i * (16 * SC * 4)];
+    };
+    auto read_b = [&](int set, int j, int s, int b) __attribute__((always_inline)) {
+        const uint8_t* base = smem + b * Cfg::STAGE;
+#pragma unroll
+        for (int f = 0; f < FR; ++f)
+            fb[set][j][f] = *reinterpret_cast<const uint4*>(base + fb_row + j * (16 * SB) + (lane_x ^ ((s * 4 * FR + 4 * f) << 4)));
+        if constexpr (Op::SCALED)
+            xb[set][j] = base[sb_at + (wk * Cfg::KSTEPS + s) * 4 + j * (16 * SC * 4)];
+    };
+    auto read_all = [&](int set, int s, int b) __attribute__((always_inline)) {
+#pragma unroll
+        for (int j = 0; j < NB; ++j)
+            read_b(set, j, s, b);
+#pragma unroll
+        for (int i = 0; i < MB; ++i)
+            read_a(Cfg::PIPE ? aset(set, i) : 0, i, s, b);
+    };
+    auto mma = [&](int set, int i, int j) __attribute__((always_inline)) {
+        const int as = Cfg::PIPE ? aset(set, i) : 0;
+        Op::mma(acc[i][j], fa[as][i], fb[set][j], Op::SCALED ? (has_scales ? xa[as][i] : 127u) : 0u, Op::SCALED ? (has_scales ? xb[set][j] : 127u) : 0u);
+    };
+    // k-step s of the last stage, which may reach past K
+    auto tail_step = [&](int set, int s) __attribute__((always_inline)) {
+        const int k0 = (nst - 1) * SB + wk * Cfg::KW + s * Cfg::KB;  // first K byte of the step
+        if (k0 >= p.k_bytes)
+            return;
+#pragma unroll
+        for (int f = 0; f < FR; ++f) {
+            const int valid = p.k_bytes - (k0 + (4 * f + lg) * 16);
+#pragma unroll
+            for (int i = 0; i < MB; ++i)
+                fa[Cfg::PIPE ? aset(set, i) : 0][i][f] = ring_mask_chunk(fa[Cfg::PIPE ? aset(set, i) : 0][i][f], valid);
+#pragma unroll
+            for (int j = 0; j < NB; ++j)
+                fb[set][j][f] = ring_mask_chunk(fb[set][j][f], valid);
+        }
+#pragma unroll
+        for (int i = 0; i < MB; ++i)
+#pragma unroll
+            for (int j = 0; j < NB; ++j)
+                mma(set, i, j);
+    };
+
+    // ---- the K loop
+    using std::integral_constant;
+    // the copying side of a barrier: `behind` later stages may still be in flight
+    auto loader_barrier = [&](int behind) __attribute__((always_inline)) {
+        static_for<R>([&](auto ac) {
+            constexpr int a = decltype(ac)::value;
+            if (behind == a)
+                ring_wait_and_barrier<a * NV>();
+        });
+    };
+    if constexpr (!Cfg::PIPE) {
+        // Barrier st: stage st has landed and no wave reads stage st - 1 any more, whose buffer is refilled.
+        if (loads) {
+#pragma unroll
+            for (int s = 0; s < R - 1; ++s)
+                if (s < nst)
+                    issue(s, s);
+        }
+        int buf = 0;
+        auto step = [&](int st) __attribute__((always_inline)) {
+            if (!loads)
+                ring_wait_and_barrier<63>();
+            else {
+                loader_barrier(min(R - 2, nst - 1 - st));
+                if (st + R - 1 < nst)
+                    issue(st + R - 1, buf == 0 ? R - 1 : buf - 1);
+            }
+        };
+        for (int st = 0; st < nst - 1; ++st) {
+            step(st);
+            if (computes)
+                static_for<Cfg::KSTEPS>([&](auto sc) {
+                    read_all(0, decltype(sc)::value, buf);
+#pragma unroll
+                    for (int i = 0; i < MB; ++i)
+#pragma unroll
+                        for (int j = 0; j < NB; ++j)
+                            mma(0, i, j);
+                });
+            buf = buf + 1 == R ? 0 : buf + 1;
+        }
+        step(nst - 1);
+        if (computes)
+            static_for<Cfg::KSTEPS>([&](auto sc) {
+                read_all(0, decltype(sc)::value, buf);
+                tail_step(0, decltype(sc)::value);
+            });
+    } else {
+        // Barrier st stands before the last k-step of stage st: every wave holds that k-step's fragments, so the stage's
+        // buffer is refilled with stage st + R, and stage st + 1 has landed, whose first fragments are read under that
+        // k-step's matrix instructions.
+        static_assert(Cfg::LW > 0, "the pipelined form has waves that only copy");
+        if (!computes) {
+#pragma unroll
+            for (int s = 0; s < R; ++s)
+                if (s < nst)
+                    issue(s, s);
+            loader_barrier(min(R - 1, nst - 1));
+            int buf = 0;
+            for (int st = 0; st < nst - 1; ++st) {
+                loader_barrier(min(R - 2, nst - 2 - st));
+                if (st + R < nst)
+                    issue(st + R, buf);
+                buf = buf + 1 == R ? 0 : buf + 1;
+            }
+        } else {
+            ring_wait_and_barrier<63>();
+            read_all(0, 0, 0);
+            int buf = 0;
+            auto body = [&](auto parc) __attribute__((always_inline)) {
+                constexpr int PAR = decltype(parc)::value;
+                const int nbuf = buf + 1 == R ? 0 : buf + 1;
+                static_for<Cfg::KSTEPS>([&](auto sc) {
+                    constexpr int s = decltype(sc)::value, SET = (PAR + s) & 1;
+                    constexpr bool LASTSTEP = s + 1 == Cfg::KSTEPS;
+                    constexpr int rs = LASTSTEP ? 0 : s + 1;
+                    const int rb = LASTSTEP ? nbuf : buf;
+                    if constexpr (LASTSTEP)
+                        ring_wait_and_barrier<63>();
+                    // (reads pinned behind the instruction that frees their registers; B first, each next k-step needs all of it)
+                    static_for<NMMA>([&](auto xc) {
+                        constexpr int x = decltype(xc)::value, i = x / NB, j = x % NB;
+                        mma(SET, i, j);
+                        constexpr int AL = NB < NMMA ? NB : NMMA - 1;
+                        if constexpr (x < NB || x == AL || (j == NB - 1 && i < MB - 1)) {
+                            __builtin_amdgcn_sched_barrier(0);
+                            if constexpr (x < NB)
+                                read_b(SET ^ 1, x, rs, rb);
+                            if constexpr (x == AL)
+                                read_a(SET ^ 1, MB - 1, rs, rb);
+                            if constexpr (j == NB - 1 && i < MB - 1)
+                                read_a(0, i, rs, rb);
+                            __builtin_amdgcn_sched_barrier(0);
+                        }
+                    });
+                });
+                buf = nbuf;
+            };
+            auto last = [&](auto parc) __attribute__((always_inline)) {
+                static_for<Cfg::KSTEPS>([&](auto sc) {
+                    constexpr int s = decltype(sc)::value, SET = (decltype(parc)::value + s) & 1;
+                    if constexpr (s > 0)
+                        read_all(SET, s, buf);
+                    tail_step(SET, s);
+                });
+            };
+            if constexpr (Cfg::KSTEPS % 2 == 0) {
+                for (int st = 0; st < nst - 1; ++st)
+                    body(integral_constant<int, 0>{});
+                last(integral_constant<int, 0>{});
+            } else {  // the register sets change places from stage to stage
+                int st = 0;
+                for (; st + 2 < nst; st += 2) {
+                    body(integral_constant<int, 0>{});
+                    body(integral_constant<int, 1>{});
+                }
+                if (st + 1 < nst) {
+                    body(integral_constant<int, 0>{});
+                    last(integral_constant<int, 1>{});
+                } else {
+                    last(integral_constant<int, 0>{});
+                }
+            }
+        }
+    }
+
+    // ---- TSTORE: the k-groups' partial sums meet in LDS (the ring is free), are added in group order and leave as 16
+    // bytes per thread.  A block is transposed in its lanes: lane (l16, lg) holds row l16, columns 4 lg .. + 3.
+    __syncthreads();
+    Elem* red = reinterpret_cast<Elem*>(smem) + wk * (BM * Cfg::RED_PITCH);
+    if (computes) {
+#pragma unroll
+        for (int i = 0; i < MB; ++i)
+#pragma unroll
+            for (int j = 0; j < NB; ++j)
+                *reinterpret_cast<Acc*>(red + (wm * Cfg::WTM + i * 16 + l16) * Cfg::RED_PITCH + wn * Cfg::WTN + j * 16 + 4 * lg) = acc[i][j];
+    }
+    __syncthreads();
+    auto drain = [&](auto kc) __attribute__((always_inline)) {
+        constexpr int KIND = decltype(kc)::value, NE = ring_cols<KIND>, CT = BN / NE, RSTEP = Cfg::THREADS / CT;
+        static_assert(Cfg::THREADS % CT == 0, "a thread keeps its columns from row to row");
+        const int c = (tid % CT) * NE, gj = n0 + c;
+        if (gj >= p.n)
+            return;
+        RingColumns<KIND, NE, Elem> cols;
+        cols.load(p, gj);
+#pragma unroll 1
+        for (int r = tid / CT; r < BM && m0 + r < p.m; r += RSTEP) {
+            const float rs = KIND == OUT_W8A8_BF16 ? p.row_scale[m0 + r] : 1.0f;
+            Elem v[NE];
+#pragma unroll
+            for (int e = 0; e < NE; ++e)
+                v[e] = 0;
+#pragma unroll
+            for (int g = 0; g < Cfg::WK; ++g)
+#pragma unroll
+                for (int q = 0; q < NE / 4; ++q) {
+                    const Acc x = *reinterpret_cast<const Acc*>(reinterpret_cast<const Elem*>(smem) + (g * BM + r) * Cfg::RED_PITCH + c + 4 * q);
+#pragma unroll
+                    for (int e = 0; e < 4; ++e)
+                        v[4 * q + e] += x[e];
+                }
+            ring_store<KIND>(p, v, cols, rs, m0 + r, gj);
+        }
+    };
+    if (p.out_kind == OUT_Q8)
+        drain(std::integral_constant<int, OUT_Q8>{});
+    else if (p.out_kind >= OUT_QF16)
+        drain(std::integral_constant<int, OUT_QF16>{});
+    else if constexpr (std::is_same<Elem, int32_t>::value) {
+        if (p.out_kind == OUT_I32)
+            drain(std::integral_constant<int, OUT_I32>{});
+        else
+            drain(std::integral_constant<int, OUT_W8A8_BF16>{});
+    } else {
+        if (p.out_kind == OUT_F32)
+            drain(std::integral_constant<int, OUT_F32>{});
+        else if (p.out_kind == OUT_F16)
+            drain(std::integral_constant<int, OUT_F16>{});
+        else
+            drain(std::integral_constant<int, OUT_BF16>{});
+    }
+}
+
+}  // namespace ptoamd

@@ -46,6 +46,9 @@ void read_options()
     const char* t = getenv("PTOAMD_TILE");
     if (t != nullptr && t[0] >= '0' && t[0] <= '7')
         o.tile = t[0] - '0';
+    const char* rg = getenv("PTOAMD_RING");
+    if (rg != nullptr && rg[0] >= '0' && rg[0] <= '8')
+        o.ring = rg[0] - '0';
     o.no_tail_split = getenv("PTOAMD_NO_TAIL_SPLIT") != nullptr;
     o.mx_16x16 = getenv("PTOAMD_MX_16X16") != nullptr;
     const char* tt = getenv("PTOAMD_TAIL_TILE");

@@ -1,0 +1,99 @@
+"""The deep-ring kernel's tile shapes at the sizes where they can go wrong: one row less and a few columns more than a tile,
+one chunk of K, a stage and four bytes, fewer stages than the ring holds and more, against the CPU oracle."""
+import numpy as np
+import pytest
+import torch
+
+from oracle import binding as ob
+from test_gpu_parity import (PA_T, _mx_inputs, _mx_unpack, _w8a8_reference, bf16_bits, bf16_to_f32, check_f32_drain, dev, host, pa,  # noqa: F401
+                             relerr, tile_env)
+
+pytestmark = pytest.mark.gpu
+
+# rows, columns, bytes of K per stage (plain types, block-scaled types)
+SHAPES = [(32, 16, 1024, 1024), (32, 32, 512, 512), (64, 32, 512, 512), (64, 64, 256, 256), (96, 64, 256, 256), (128, 64, 256, 256),
+          (128, 128, 128, 128), (192, 128, 128, None), (256, 128, 128, None)]
+
+
+def _sizes(shape, scaled):
+    bm, bn, stage = SHAPES[shape][0], SHAPES[shape][1], SHAPES[shape][3 if scaled else 2]
+    ks = (128, stage + 128, 6 * stage + 256) if scaled else (16, stage + 4, 2 * stage, 6 * stage + 36)
+    return [(m, n, kb) for kb, (m, n) in zip(ks, ((bm - 1, bn + 3), (1, bn), (bm + 1, 2 * bn + 1), (bm, bn - 1)))]
+
+
+@pytest.mark.parametrize("shape", range(9))
+@pytest.mark.parametrize("kind", ["bf16", "f16", "i8"])
+def test_plain_types(pa, oracle, kind, shape):  # noqa: F811
+    r = np.random.default_rng(shape)
+    for m, n, kb in _sizes(shape, False):
+        k = kb if kind == "i8" else kb // 2
+        if kind == "i8":
+            a, b = (r.integers(-128, 128, (x, k)).astype(np.int8) for x in (m, n))
+            da, db, ta, tc, ref = dev(a), dev(b), pa.I8, pa.I32, oracle.matmul_i8(a, b, b_dn=True)
+        else:
+            conv = (lambda x: x.astype(np.float16).view(np.uint16)) if kind == "f16" else bf16_bits
+            a, b = (conv(r.uniform(-1, 1, (x, k)).astype(np.float32)) for x in (m, n))
+            tdt = torch.float16 if kind == "f16" else torch.bfloat16
+            da, db, ta, tc = dev(a).view(tdt), dev(b).view(tdt), pa.F16 if kind == "f16" else pa.BF16, pa.F32
+            ref = (oracle.matmul_f16 if kind == "f16" else oracle.matmul_bf16)(a, b, b_dn=True)
+        with tile_env(PTOAMD_RING=shape):
+            got = host(pa.gemm(da, db, ta, tc, pa.B_DN))
+            assert pa.last_kernel().startswith(f"tile{SHAPES[shape][0]}x{SHAPES[shape][1]}_dtl"), pa.last_kernel()
+        if kind == "i8":
+            assert np.array_equal(got, ref), (m, n, k)
+        else:
+            fa, fb = (x.view(np.float16).astype(np.float64) if kind == "f16" else bf16_to_f32(x).astype(np.float64) for x in (a, b))
+            check_f32_drain(got, ref, np.abs(fa) @ np.abs(fb).T, k, f"{kind} {m}x{n}x{k} shape {shape}")
+
+
+@pytest.mark.parametrize("shape", range(7))
+@pytest.mark.parametrize("ta,tb", [(ob.E4M3, ob.E4M3), (ob.E5M2, ob.E4M3), (ob.E4M3, ob.E5M2), (ob.E5M2, ob.E5M2), (ob.E2M1, ob.E2M1)])
+def test_block_scaled_types(pa, oracle, ta, tb, shape):  # noqa: F811
+    r = np.random.default_rng(shape + 16 * ta + tb)
+    fp4 = ta == ob.E2M1
+    for m, n, kb in _sizes(shape, True):
+        k = 2 * kb if fp4 else kb
+        a, _, sa, sb = _mx_inputs(r, ta, m, n, k)
+        _, b, _, _ = _mx_inputs(r, tb, m, n, k)
+        ref = oracle.matmul_mx(a, b, sa, sb, m, k, n, ta, tb)
+        with tile_env(PTOAMD_RING=shape):
+            got = host(pa.gemm_mx(dev(a), dev(b), dev(sa), dev(sb), m, n, k, PA_T[ta], PA_T[tb], pa.F32))
+            assert pa.last_kernel().startswith(f"tile{SHAPES[shape][0]}x{SHAPES[shape][1]}_dtl"), pa.last_kernel()
+        ua = _mx_unpack(oracle, a, ta) * np.repeat(2.0 ** (sa.astype(np.float64) - 127), 32, 1)
+        ub = _mx_unpack(oracle, b, tb) * np.repeat(2.0 ** (sb.astype(np.float64) - 127), 32, 1)
+        # (the fp8 form of the scaled instruction keeps about 13 bits below the largest of a block's products: 2^-11 of sum|a||b|)
+        check_f32_drain(got, ref, np.abs(ua) @ np.abs(ub).T, k, f"MX {ta}x{tb} {m}x{n}x{k} shape {shape}",
+                        max_rel=1e-4 if fp4 else 1e-3, eps=None if fp4 else 2.0 ** -11)
+
+
+@pytest.mark.parametrize("shape", [0, 3, 7])
+def test_store_forms(pa, oracle, shape):  # noqa: F811
+    """Accumulator input, bias, relu, 16-bit rows at an odd pitch, W8A8 with raw accumulators, per-column requantisation and
+    atomic adds: integer and rounding steps are the oracle's, bit for bit."""
+    r = np.random.default_rng(50 + shape)
+    m, n, k = SHAPES[shape][0] + 5, SHAPES[shape][1] + 13, 324
+    a, b = (r.integers(-128, 128, (x, k)).astype(np.int8) for x in (m, n))
+    cin, bias = r.integers(-2 ** 30, 2 ** 30, (m, n)).astype(np.int32), r.integers(-1000, 1000, n).astype(np.int32)
+    acc = oracle.matmul_i8(a, b, b_dn=True)
+    sa, sb = r.uniform(0.001, 0.02, m).astype(np.float32), r.uniform(0.001, 0.02, n).astype(np.float32)
+    words = np.array([(int(np.float32(r.uniform(1e-4, 1e-3)).view(np.uint32)) & 0xFFFFE000) | (int(r.integers(0, 16)) << 37) | (1 << 46)
+                      for _ in range(n)], np.uint64)
+    x, y = bf16_bits(r.uniform(-1, 1, (m, k)).astype(np.float32)), bf16_bits(r.uniform(-1, 1, (n, k)).astype(np.float32))
+    with tile_env(PTOAMD_RING=shape):
+        got = host(pa.gemm(dev(a), dev(b), pa.I8, pa.I32, pa.B_DN, c_in=dev(cin), bias=dev(bias), relu=True))
+        out, raw = pa.gemm_w8a8(dev(a), dev(b), dev(sa), dev(sb), want_acc=True)
+        q8 = host(pa.gemm_requant(dev(a), dev(b), pa.I8, pa.I8, dev(words.view(np.int64)), per_column=True))
+        summed = dev(cin)
+        pa.gemm_atomic_add(summed, dev(a), dev(b), pa.I8)
+        wide = torch.full((m, n + 3), 7.0, dtype=torch.bfloat16, device="cuda:0")
+        dx, dy = dev(x).view(torch.bfloat16), dev(y).view(torch.bfloat16)
+        f32 = host(pa.gemm(dx, dy, pa.BF16, pa.F32, pa.B_DN))
+        pa.gemm(dx, dy, pa.BF16, pa.BF16, pa.B_DN, out=wide[:, :n])
+        assert "_dtl_" in pa.last_kernel()
+    assert np.array_equal(got, np.maximum((acc.astype(np.int64) + cin + bias).astype(np.int32), 0))
+    ref_acc, ref_out = _w8a8_reference(oracle, a, b, sa, sb)
+    assert np.array_equal(host(raw), ref_acc) and np.array_equal(host(out), ref_out)
+    assert np.array_equal(q8.view(np.uint8).ravel(), np.asarray(oracle.store_quant(acc, ob.ST_I8, words, True)).view(np.uint8).ravel())
+    assert np.array_equal(host(summed), (acc.astype(np.int64) + cin).astype(np.int32))
+    assert np.array_equal(host(wide)[:, :n], oracle.store_f32(f32, ob.ST_BF16))
+    assert bool((wide[:, n:] == 7.0).all())
