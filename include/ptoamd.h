@@ -144,10 +144,12 @@ int ptoamd_gemm_bias(void* c, int c_type, const void* a, const void* b, int ab_t
                      int m, int n, int k, int lda, int ldb, int ldc, int b_layout, int relu, void* stream);
 
 /*
- * ptoamd_gemm_bias with a caller-owned workspace for a row-major B (PTOAMD_B_ND): B is re-ordered into the workspace once
- * ([N][K] with rows padded to 16 bytes, ptoamd_gemm_workspace_bytes(n, k, ab_type, b_layout) bytes, 256-byte aligned) and the product then runs on the
- * fastest tiles, where ptoamd_gemm transposes B inside the loader of the register-staged tiles for every tile row of C --
- * the better choice for small M, the slower one for large M.  workspace == NULL is ptoamd_gemm_bias.  No counterpart in
+ * ptoamd_gemm_bias with a caller-owned workspace for a row-major B (PTOAMD_B_ND): where the fastest tiles need a column-major
+ * B, it is re-ordered into the workspace ([N][K] with rows padded to 16 bytes, ptoamd_gemm_workspace_bytes(n, k, ab_type,
+ * b_layout) bytes, 256-byte aligned) first.  The deep-ring tiles read a row-major B of 16-bit elements in place, with or
+ * without a workspace, where n is a multiple of 8, k and both pitches are even and the operands lie on 4-byte addresses;
+ * otherwise ptoamd_gemm transposes B inside the loader of the register-staged tiles, for every tile row of C.
+ * workspace == NULL is ptoamd_gemm_bias.  No counterpart in
  * the reference (its TLOAD re-orders an ND panel into L1 per tile, cpu/TLoad.hpp:287-321).
  */
 size_t ptoamd_gemm_workspace_bytes(int n, int k, int ab_type, int b_layout);

@@ -111,7 +111,7 @@ def gemm(a, b, ab_type, c_type=F32, b_layout=B_DN, c_in=None, relu=False, m=None
          bias=None, workspace=None):
     """TLOAD -> TMATMUL / TMATMUL_ACC / TMATMUL_BIAS -> TSTORE.  a: [m, k]; b: [n, k] (B_DN) or [k, n] (B_ND), raw-typed
     tensors; bias: [n] of the accumulator type; workspace: a uint8 device tensor of gemm_workspace_bytes(...) bytes into
-    which a row-major b is re-ordered (without one it is transposed inside the loader)."""
+    which a row-major b is re-ordered where the fastest kernel for the size cannot read it in place."""
     m = a.shape[0] if m is None else m
     k = a.shape[1] if k is None else k
     n = (b.shape[0] if b_layout == B_DN else b.shape[1]) if n is None else n

@@ -502,7 +502,7 @@ static int tile_as_launched(int tile, int op, int m, int n)
     return tile == 3 ? 4 : tile;
 }
 
-static const char* tile_kernel_name(int tile, int op)
+static const char* tile_kernel_name(int tile, int op, bool row_major_b = false)
 {
     static const char* ops[TOP_COUNT] = {"bf16", "f16", "i8", "fp8_e4m3_e4m3", "fp8_e5m2_e5m2", "fp8_e4m3_e5m2",
                                          "fp8_e5m2_e4m3", "fp4_e2m1"};
@@ -512,7 +512,7 @@ static const char* tile_kernel_name(int tile, int op)
     if (tile >= TILE_RING) {
         int bm, bn;
         ring_shape(tile - TILE_RING, &bm, &bn);
-        snprintf(buf, sizeof buf, "tile%dx%d_dtl_%s", bm, bn, ops[op]);
+        snprintf(buf, sizeof buf, row_major_b ? "tile%dx%d_bnd_%s" : "tile%dx%d_dtl_%s", bm, bn, ops[op]);
         return buf;
     }
     snprintf(buf, sizeof buf, "%s_%s", tiles[tile], ops[op]);
@@ -727,9 +727,25 @@ static int gemm_common(void* c, int c_type, const void* a, const void* b, int ab
         g.qwords = qwords; g.q_per_column = q_per_column; g.atomic_add = atomic_add;
         return launch_generic(g, stream);
     }
+    const int op = ab_type == PTOAMD_BF16 ? TOP_BF16
+                   : ab_type == PTOAMD_F16 ? TOP_F16
+                   : ab_type == PTOAMD_I8 ? TOP_I8
+                   : ab_type == PTOAMD_E4M3 ? (b_type == PTOAMD_E4M3 ? TOP_FP8_E4E4 : TOP_FP8_E4E5)
+                                            : (b_type == PTOAMD_E5M2 ? TOP_FP8_E5E5 : TOP_FP8_E5E4);
+    const bool ragged_k_form = op == TOP_BF16 || op == TOP_F16 || op == TOP_I8, whole_slabs = (k_bytes % 128) == 0;
+    const bool dtl_k_ok = whole_slabs || (ragged_k_form && k_bytes > 128);
+    // A row-major B of 16-bit elements is read by the deep-ring kernel as it is, transposed on its way out of LDS (its rows have
+    // to be whole 16-byte chunks; a column chunk past N is fetched from the row's last one).  With a workspace the shape is the
+    // one that the same product takes with a column-major B, so that both have the same bits; where that is one of the two-
+    // and three-slab tiles, B is re-ordered for it.
+    const bool nd_ok = b_layout == PTOAMD_B_ND && ebytes == 2 && !options().b_nd_in_loader && options().tile < 0 && (n % 8) == 0 &&
+                       aligned4(a) && aligned4(b) && (lda_b % 4) == 0 && (ldb_b % 4) == 0 && (k_bytes % 4) == 0 &&
+                       dma_offsets_fit(m, RING_MAX_STAGE_BYTES / 2 + 8, lda_b, ldb_b, std::max(k_bytes, 2 * (long)n));
+    const int nd_tile = nd_ok ? pick_dma_tile(m, n, k_bytes, op, b_via_ws && dtl_k_ok) : -1;
+    const bool nd_direct = nd_tile >= TILE_RING;
     const uint8_t* b_kmajor = reinterpret_cast<const uint8_t*>(b);
     long ldb_kmajor = ldb_b;
-    if (b_via_ws) {  // TLOAD of an ND B panel: re-order once so the MFMA path reads K-contiguous rows
+    if (b_via_ws && !nd_direct) {  // TLOAD of an ND B panel: re-order once so the MFMA path reads K-contiguous rows
         // rows of the re-ordered copy start on 16-byte boundaries whatever K is
         const long pitch = ws_row_bytes(k_bytes);
         const int rc = ebytes == 2 ? transpose_b<uint16_t>(ws, b, k, n, ldb, pitch / 2, stream)
@@ -747,23 +763,16 @@ static int gemm_common(void* c, int c_type, const void* a, const void* b, int ab
     p.lda_bytes = lda_b; p.ldb_bytes = ldb_kmajor; p.ldc = ldc;
     p.relu = relu; p.out_kind = out_kind; p.group_m = 4;
     p.qwords = qwords; p.q_per_column = q_per_column; p.atomic_add = atomic_add;
-    const int op = ab_type == PTOAMD_BF16 ? TOP_BF16
-                   : ab_type == PTOAMD_F16 ? TOP_F16
-                   : ab_type == PTOAMD_I8 ? TOP_I8
-                   : ab_type == PTOAMD_E4M3 ? (b_type == PTOAMD_E4M3 ? TOP_FP8_E4E4 : TOP_FP8_E4E5)
-                                            : (b_type == PTOAMD_E5M2 ? TOP_FP8_E5E5 : TOP_FP8_E5E4);
-    p.b_nd = b_in_kernel; p.b_esz = ebytes;
+    p.b_nd = b_in_kernel || nd_direct; p.b_esz = ebytes;
     // (LDS-DMA needs dword-aligned global addresses, no more: rows at 4-byte alignment run 114 against 100 us on bf16 4096^3)
     const bool dma_ok = !b_in_kernel && aligned4(a) && aligned4(b_kmajor) && (lda_b % 4) == 0 && (ldb_kmajor % 4) == 0 &&
                         dma_offsets_fit(m, n, lda_b, ldb_kmajor, k_bytes);
     // (the deep-ring kernel reads a chunk that K ends in as the 16 bytes ending there, which must start on a dword)
-    // (the deep-ring kernel reads a chunk that K ends in as the 16 bytes ending there, which must start on a dword)
-    const bool ragged_k_form = op == TOP_BF16 || op == TOP_F16 || op == TOP_I8, whole_slabs = (k_bytes % 128) == 0;
-    const int tile = options().tile < 0 && dma_ok && (k_bytes % 4) == 0
-                         ? pick_dma_tile(m, n, k_bytes, op, whole_slabs || (ragged_k_form && k_bytes > 128))
-                         : pick_tile(m, n, k_bytes, false, false, dma_ok, ragged_k_form);
+    const int tile = nd_direct ? nd_tile
+                     : options().tile < 0 && dma_ok && (k_bytes % 4) == 0 ? pick_dma_tile(m, n, k_bytes, op, dtl_k_ok)
+                                                                          : pick_tile(m, n, k_bytes, false, false, dma_ok, ragged_k_form);
     PTOAMD_HIP_CHECK(launch_tiles(tile, op, p, stream));
-    set_last_kernel(tile_kernel_name(tile_as_launched(tile, op, m, n), op));
+    set_last_kernel(tile_kernel_name(tile_as_launched(tile, op, m, n), op, nd_direct));
     return PTOAMD_OK;
 }
 

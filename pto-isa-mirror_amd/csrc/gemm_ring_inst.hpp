@@ -17,7 +17,7 @@ static hipError_t launch_ring(const TileGemmParams& p, hipStream_t stream)
     return hipGetLastError();
 }
 
-template <class Op>
+template <class Op, bool BND = false>
 static hipError_t launch_ring_shape(int shape, const TileGemmParams& p, hipStream_t stream)
 {
     switch (shape) {
@@ -26,7 +26,7 @@ static hipError_t launch_ring_shape(int shape, const TileGemmParams& p, hipStrea
         if constexpr (Op::SCALED)                                                                                   \
             return launch_ring<RingCfg<bm, bn, swm, swn, swk, ssb, sr, lw, pipe, Op>>(p, stream);                   \
         else                                                                                                        \
-            return launch_ring<RingCfg<bm, bn, wm, wn, wk, sb, r, lw, pipe, Op>>(p, stream);
+            return launch_ring<RingCfg<bm, bn, wm, wn, wk, sb, r, lw, pipe, Op, BND>>(p, stream);
         PTOAMD_RING_SHAPES_ALL(PTOAMD_RING_CASE)
 #undef PTOAMD_RING_CASE
         default: break;
@@ -34,7 +34,7 @@ static hipError_t launch_ring_shape(int shape, const TileGemmParams& p, hipStrea
     if constexpr (!Op::SCALED) {
         switch (shape) {
 #define PTOAMD_RING_CASE(id, bm, bn, wm, wn, wk, sb, r, swm, swn, swk, ssb, sr, lw, pipe) \
-    case id: return launch_ring<RingCfg<bm, bn, wm, wn, wk, sb, r, lw, pipe, Op>>(p, stream);
+    case id: return launch_ring<RingCfg<bm, bn, wm, wn, wk, sb, r, lw, pipe, Op, BND>>(p, stream);
             PTOAMD_RING_SHAPES_PLAIN(PTOAMD_RING_CASE)
 #undef PTOAMD_RING_CASE
             default: break;
@@ -45,11 +45,25 @@ static hipError_t launch_ring_shape(int shape, const TileGemmParams& p, hipStrea
 
 hipError_t PTOAMD_RING_FN(int shape, const TileGemmParams& p, hipStream_t stream)
 {
-    if (shape != TILE_PREPARE_ALL)
-        return launch_ring_shape<PTOAMD_RING_OP>(shape, p, stream);
+#ifdef PTOAMD_RING_BND  // the 16-bit types also take a row-major B
+    constexpr bool has_bnd = true;
+#else
+    constexpr bool has_bnd = false;
+#endif
+    if (shape != TILE_PREPARE_ALL) {
+        if (!p.b_nd)
+            return launch_ring_shape<PTOAMD_RING_OP>(shape, p, stream);
+        if constexpr (has_bnd)
+            return launch_ring_shape<PTOAMD_RING_OP, true>(shape, p, stream);
+        return hipErrorInvalidValue;
+    }
     const TileGemmParams none{};
     for (int s = 0; s < (PTOAMD_RING_OP::SCALED ? RING_SHAPES_SCALED : RING_SHAPES); ++s) {
-        const hipError_t e = launch_ring_shape<PTOAMD_RING_OP>(s, none, stream);
+        hipError_t e = launch_ring_shape<PTOAMD_RING_OP>(s, none, stream);
+        if constexpr (has_bnd) {
+            if (e == hipSuccess)
+                e = launch_ring_shape<PTOAMD_RING_OP, true>(s, none, stream);
+        }
         if (e != hipSuccess)
             return e;
     }

@@ -12,6 +12,10 @@
 //   TEXTRACT   ds_read_b128 fragments; the swizzle makes the 16 rows of a lane group fall into different banks
 //   TMATMUL    the 16x16 matrix instructions of every operand type (block-scaled types: one dword of E8M0 per 128 K)
 //   sync       one workgroup barrier per stage: behind it the stage has landed and the previous one may be overwritten
+//   B row-major (BND, 16-bit types): a stage holds its k rows as they lie in memory and ds_read_b64_tr_b16 turns four of them at a
+//              time into fragments, so no copy of B is made and no thread moves elements.  Measured, bf16: 2048 x 4096 x 4096
+//              57 us (column-major B 56; re-ordered through a workspace first 80; scattered by the register-staged loader
+//              101), 24 x 4096 x 4096 14.2 us (column-major 9.6: here a copy takes 32 bytes of each row; loader 58)
 //   K tail     copies never read past a row: a chunk that would is read as the 16 bytes that END at the row's end, and the
 //              last stage's fragments are masked in registers -- the same bytes of A and B, so k positions still agree
 #pragma once
@@ -37,10 +41,10 @@ struct OpFP4x16 {
 };
 
 // WM x WN x WK waves: WK groups share the tile and split every stage of SB bytes per row along K; R stages in the ring
-template <int BM_, int BN_, int WM_, int WN_, int WK_, int SB_, int R_, int LW_, bool PIPE_, class Op_>
+template <int BM_, int BN_, int WM_, int WN_, int WK_, int SB_, int R_, int LW_, bool PIPE_, class Op_, bool BND_ = false>
 struct RingCfg {
     static constexpr int BM = BM_, BN = BN_, WM = WM_, WN = WN_, WK = WK_, SB = SB_, R = R_;
-    static constexpr bool PIPE = PIPE_;
+    static constexpr bool PIPE = PIPE_, BND = BND_;  // BND: B is row-major [K][N]
     using Op = Op_;
     static constexpr int CW = WM * WN * WK, LW = LW_, THREADS = (CW + LW) * 64;
     static constexpr int NW = LW > 0 ? LW : CW;  // waves that copy
@@ -53,12 +57,14 @@ struct RingCfg {
     static constexpr int SPC = ROWS * SC / 64, NSW = (SPC + NW - 1) / NW; // 64-dword scale pieces; per wave
     static constexpr int NV = NPW + NSW;                                  // copies a wave issues per stage
     static constexpr int STAGE = ROWS * SB + ROWS * SC * 4;
+    static constexpr int KR = SB / 2, RB = BN * 2, CB = RB / 16;          // BND: k rows of a stage, bytes and chunks per row
     static constexpr int RED_PITCH = BN + 4;                              // elements
     static constexpr int RED_BYTES = WK * BM * RED_PITCH * 4;
     static constexpr int LDS_BYTES = (R * STAGE > RED_BYTES ? R * STAGE : RED_BYTES);
     static_assert(BM % (16 * WM) == 0 && BN % (16 * WN) == 0, "wave tiles are made of 16x16 blocks");
     static_assert(KW % KB == 0 && SB <= 1024 && 1024 % SB == 0, "a k-group's part of a stage is whole k-steps");
     static_assert(PIECES % NW == 0 && (BM * SB) % 1024 == 0, "every wave issues the same number of 1 KiB copies, each of one operand");
+    static_assert(!BND || (!Op::SCALED && FR == 1 && (NB & (NB - 1)) == 0), "the row-major form is for the 16-bit types");
     static_assert((ROWS * SC) % 64 == 0, "scale pieces are whole");
     static_assert(LDS_BYTES <= 160 * 1024 && R >= 2 && (R - 1) * NV < 64, "LDS capacity; vmcnt is a 6-bit count");
 };
@@ -68,6 +74,24 @@ template <int SB>
 __device__ __forceinline__ int ring_swizzle(int row)
 {
     return SB == 128 ? swizzle_chunk(row, 0) : (row & 15);
+}
+
+// BND: which of a k row's 32-byte pieces (16 columns) stands where: piece ^ ring_swizzle_nd(row).  A half wave of the
+// transposing read takes one piece of rows 0 .. 3 and 8 .. 11 (of a multiple of 4): they go to different banks from 32 columns on.
+template <int BN>
+__device__ __forceinline__ int ring_swizzle_nd(int row)
+{
+    const int b3 = (row >> 3) & 1;
+    return BN == 128 ? (row & 3) | (b3 << 2) : BN == 64 ? ((row >> 1) & 1) | (b3 << 1) : BN == 32 ? b3 : 0;
+}
+
+// Four k rows of 16 columns, transposed on their way out of LDS: every lane of a group of 16 names 8 bytes -- row l16 / 4,
+// columns 4 (l16 % 4) .. + 3 -- and receives column l16 of the four rows.
+__device__ __forceinline__ uint2 ring_read_transposed(const uint8_t* at)
+{
+    typedef short s16x4 __attribute__((ext_vector_type(4)));
+    typedef __attribute__((address_space(3))) s16x4* lds_s16x4_ptr;
+    return __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_ptr)(at)));
 }
 
 template <int N>
@@ -219,10 +243,16 @@ __global__ void __launch_bounds__(Cfg::THREADS) gemm_tile_ring_kernel(const Tile
         const int r = piece_row(q);
         return lw + q * NW < Cfg::A_PIECES ? (uint32_t)(min(m0 + r, p.m - 1) * p.lda_bytes) : (uint32_t)(min(n0 + r - BM, p.n - 1) * p.ldb_bytes);
     };
+    // BND: a stage's B is KR rows of BN columns; row and byte offset (columns past N repeat the row's last chunk)
+    auto nd_row = [&](int q) { return ((lw + q * NW - Cfg::A_PIECES) * 64 + lane) / Cfg::CB; };
+    auto nd_col = [&](int q) -> uint32_t {
+        const int chunk = (lane % Cfg::CB) ^ (ring_swizzle_nd<BN>(nd_row(q)) << 1);
+        return (uint32_t)min(n0 * 2 + chunk * 16, p.n * 2 - 16);
+    };
     uint32_t goff[NPW];
 #pragma unroll
     for (int q = 0; q < NPW; ++q)
-        goff[q] = row_offset(q) + piece_chunk(q) * 16;
+        goff[q] = Cfg::BND && lw + q * NW >= Cfg::A_PIECES ? (uint32_t)(nd_row(q) * p.ldb_bytes) + nd_col(q) : row_offset(q) + piece_chunk(q) * 16;
     // scales: dword e = row * SC + d of a stage's scale area; without scale arrays the copies fetch bytes of A that are not used
     const bool has_scales = Op::SCALED && p.sa != nullptr;
     const uint8_t* sc_row[NSW > 0 ? NSW : 1];
@@ -238,11 +268,18 @@ __global__ void __launch_bounds__(Cfg::THREADS) gemm_tile_ring_kernel(const Tile
     }
     auto issue = [&](int st, int buf) __attribute__((always_inline)) {
         const uint32_t dst = __builtin_amdgcn_readfirstlane(lds0 + buf * Cfg::STAGE);
-        const long kb = (long)st * SB;
+        const long kb = (long)st * SB, kb_b = Cfg::BND ? (long)st * Cfg::KR * p.ldb_bytes : kb;
         if (k_tail && st == nst - 1) {
 #pragma unroll
             for (int q = 0; q < NPW; ++q) {
                 const int piece = lw + q * NW;
+                if (Cfg::BND && piece >= Cfg::A_PIECES) {
+                    // eight rows that K ends in are the eight that end there, as in A's chunk of the same k
+                    const int k = p.k_bytes / 2, row = st * Cfg::KR + nd_row(q), base_row = max(st * Cfg::KR - 8, 0);
+                    const int src = (row | 7) < k ? row : k - 8 + (row & 7);
+                    lds_dma16_off(p.b + (long)base_row * p.ldb_bytes, (uint32_t)((src - base_row) * p.ldb_bytes) + nd_col(q), dst + piece * 1024);
+                    continue;
+                }
                 const uint32_t off = row_offset(q) + (uint32_t)min(st * SB + piece_chunk(q) * 16, p.k_bytes - 16);
                 lds_dma16_off(piece < Cfg::A_PIECES ? p.a : p.b, off, dst + piece * 1024);
             }
@@ -250,7 +287,7 @@ __global__ void __launch_bounds__(Cfg::THREADS) gemm_tile_ring_kernel(const Tile
 #pragma unroll
             for (int q = 0; q < NPW; ++q) {
                 const int piece = lw + q * NW;
-                lds_dma16_off((piece < Cfg::A_PIECES ? p.a : p.b) + kb, goff[q], dst + piece * 1024);
+                lds_dma16_off(piece < Cfg::A_PIECES ? p.a + kb : p.b + kb_b, goff[q], dst + piece * 1024);
             }
         }
         if constexpr (NSW > 0) {
@@ -273,6 +310,9 @@ __global__ void __launch_bounds__(Cfg::THREADS) gemm_tile_ring_kernel(const Tile
     const uint32_t lane_x = (uint32_t)((lg ^ ring_swizzle<SB>(l16)) ^ (wk * (Cfg::KW / 16))) << 4;
     const uint32_t fa_row = (wm * Cfg::WTM + l16) * SB, fb_row = (BM + wn * Cfg::WTN + l16) * SB;
     const uint32_t sa_at = Cfg::ROWS * SB + (wm * Cfg::WTM + l16) * (SC * 4) + lg, sb_at = Cfg::ROWS * SB + (BM + wn * Cfg::WTN + l16) * (SC * 4) + lg;
+    // BND: this lane's 8 bytes of a k-step's first block, k rows 8 lg .. + 3
+    const int nd_l = lg * 8 + (l16 >> 2);
+    const uint32_t nd_at = BM * SB + (wk * (Cfg::KW / 2) + nd_l) * Cfg::RB + ((wn * (Cfg::WTN / 16) ^ ring_swizzle_nd<BN>(nd_l)) << 5) + (l16 & 3) * 8;
     // Fragment registers.  PIPE: B's fragments and A's last row block have two sets, alternating per k-step; the other row
     // blocks of A are refilled in place right after their last matrix instruction, several of them before the next k-step
     // reads them.
@@ -290,6 +330,12 @@ __global__ void __launch_bounds__(Cfg::THREADS) gemm_tile_ring_kernel(const Tile
     };
     auto read_b = [&](int set, int j, int s, int b) __attribute__((always_inline)) {
         const uint8_t* base = smem + b * Cfg::STAGE;
+        if constexpr (Cfg::BND) {
+            const uint8_t* at = base + (nd_at ^ (j << 5)) + s * 32 * Cfg::RB;
+            const uint2 lo = ring_read_transposed(at), hi = ring_read_transposed(at + 4 * Cfg::RB);
+            fb[set][j][0] = make_uint4(lo.x, lo.y, hi.x, hi.y);
+            return;
+        }
 #pragma unroll
         for (int f = 0; f < FR; ++f)
             fb[set][j][f] = *reinterpret_cast<const uint4*>(base + fb_row + j * (16 * SB) + (lane_x ^ ((s * 4 * FR + 4 * f) << 4)));

@@ -46,6 +46,29 @@ def test_plain_types(pa, oracle, kind, shape):  # noqa: F811
             check_f32_drain(got, ref, np.abs(fa) @ np.abs(fb).T, k, f"{kind} {m}x{n}x{k} shape {shape}")
 
 
+@pytest.mark.parametrize("shape", range(9))
+@pytest.mark.parametrize("kind", ["bf16", "f16"])
+def test_row_major_b(pa, oracle, kind, shape):  # noqa: F811
+    """B as [K][N] with columns that end in part of a tile and rows at a wider pitch (the columns past N hold NaN), K ending
+    inside a stage and inside a chunk of eight rows: bit for bit the product with the same B given column-major."""
+    r = np.random.default_rng(100 + shape)
+    tdt, t = (torch.float16, pa.F16) if kind == "f16" else (torch.bfloat16, pa.BF16)
+    for m, n, kb in _sizes(shape, False):
+        n, k = (n + 7) // 8 * 8, kb // 2
+        a, b = (torch.from_numpy(r.uniform(-1, 1, x).astype(np.float32)).to(tdt).cuda() for x in ((m, k), (k, n)))
+        wide = torch.full((k, n + 10), float("nan"), dtype=tdt, device="cuda")
+        wide[:, :n] = b
+        with tile_env(PTOAMD_RING=shape):
+            same = pa.gemm(a, b.t().contiguous(), t, pa.F32, pa.B_DN)
+            got = pa.gemm(a, b, t, pa.F32, pa.B_ND)
+            pitched = pa.gemm(a, wide, t, pa.F32, pa.B_ND, n=n)
+            assert pa.last_kernel() == f"tile{SHAPES[shape][0]}x{SHAPES[shape][1]}_bnd_{kind}", pa.last_kernel()
+        assert torch.equal(got, same) and torch.equal(pitched, same), (m, n, k)
+        ref = a.double() @ b.double()  # (f32 sums of k products, each of them exact)
+        bound = k * 2.0 ** -23 * (a.double().abs() @ b.double().abs()) + 1e-30
+        assert bool(((got.double() - ref).abs() <= bound).all()), (m, n, k)
+
+
 @pytest.mark.parametrize("shape", range(7))
 @pytest.mark.parametrize("ta,tb", [(ob.E4M3, ob.E4M3), (ob.E5M2, ob.E4M3), (ob.E4M3, ob.E5M2), (ob.E5M2, ob.E5M2), (ob.E2M1, ob.E2M1)])
 def test_block_scaled_types(pa, oracle, ta, tb, shape):  # noqa: F811
