@@ -364,8 +364,10 @@ constexpr int TILE_RING = 16;  // tile ids from here on: the deep-ring kernel's 
 
 // Block-scaled products of more than 64 rows keep away from the shapes that split K over groups of waves (0 .. 2): their sums
 // then run in k order and equal, bit for bit, those of the same product written in the tile ISA.
-// dtl_ok: tiles 4, 5 and 7 take this operand as well (K and, for block-scaled types, rows of scales they can stream)
-static int pick_dma_tile(int m, int n, long k_bytes, int op, bool dtl_ok)
+// dtl: which of the two- and three-slab tiles take this operand as well (K and, for block-scaled types, rows of scales they can
+// stream; a row-major B)
+enum DtlTiles { DTL_NONE, DTL_256_ONLY, DTL_ALL };
+static int pick_dma_tile(int m, int n, long k_bytes, int op, DtlTiles dtl)
 {
     const bool scaled = op >= TOP_FP8_E4E4;
     const int shapes = scaled ? RING_SHAPES_SCALED : RING_SHAPES;
@@ -374,7 +376,7 @@ static int pick_dma_tile(int m, int n, long k_bytes, int op, bool dtl_ok)
     // A round or more of 256 x 256 tiles: those (with the split of a part-filled last round below) are ahead from K = 1024 on
     // -- bf16 4096 x 8192 x 2048: 105 us against 129 on 256 x 128 -- and within a tenth of the best where a sixteenth of a round
     // is left over (4096 x 4312: 192 x 128 tiles 79 against 87 us at K = 2048).
-    if (dtl_ok && (long)((m + 255) / 256) * ((n + 255) / 256) >= device_compute_units())
+    if (dtl != DTL_NONE && (long)((m + 255) / 256) * ((n + 255) / 256) >= device_compute_units())
         return 4;
     const TileCost* cost = tile_costs[op == TOP_FP4 ? 2 : (scaled ? 1 : 0)];
     const int cus = device_compute_units();
@@ -385,7 +387,7 @@ static int pick_dma_tile(int m, int n, long k_bytes, int op, bool dtl_ok)
     int best = TILE_RING;
     float best_us = 1e30f;
     for (int c = 0; c < COST_COUNT; ++c) {
-        if (c < RING_SHAPES ? c >= shapes : (!dtl_ok || (c == COST_TILE7 && !scaled)))
+        if (c < RING_SHAPES ? c >= shapes : (dtl == DTL_NONE || (dtl == DTL_256_ONLY && c != COST_TILE4) || (c == COST_TILE7 && !scaled)))
             continue;
         if (scaled && c <= 2 && m > 64)
             continue;
@@ -417,7 +419,7 @@ static int pick_dma_tile(int m, int n, long k_bytes, int op, bool dtl_ok)
 // one workgroup per CU, same wave tile as the large form) or 128x128 tiles (two workgroups per CU); a tile of the tail
 // then costs a half or a quarter of a 256x256 tile's time instead of a whole round (MXFP8 4096 x 14336 x 4096, 3.5
 // rounds of 256 CUs).  PTOAMD_TILE (an explicit tile) and PTOAMD_NO_TAIL_SPLIT=1 switch the split off;
-// PTOAMD_TAIL_TILE=5|6|7 picks the tail's tile (default: 7 for the block-scaled types, 5 otherwise).
+// PTOAMD_TAIL_TILE=5|6|7 picks the tail's tile (default: 7 for the block-scaled types, the deep-ring 128 x 128 one otherwise).
 static hipError_t launch_tiles_as(int tile, int op, const TileGemmParams& p, hipStream_t stream)
 {
     if ((tile == 4 || tile == 3) && options().tile < 0 && !options().no_tail_split) {
@@ -448,7 +450,7 @@ static hipError_t launch_tiles_as(int tile, int op, const TileGemmParams& p, hip
             TileGemmParams tail = p;
             const size_t esz = (p.out_kind == OUT_F32 || p.out_kind == OUT_I32) ? 4 : (p.out_kind == OUT_Q8 ? 1 : 2);
             tail.n = p.n - n1;
-            tail.b = p.b + (long)n1 * p.ldb_bytes;
+            tail.b = p.b + (p.b_nd ? (long)n1 * p.b_esz : (long)n1 * p.ldb_bytes);
             tail.c = static_cast<uint8_t*>(p.c) + (size_t)n1 * esz;
             if (p.c_in)
                 tail.c_in = static_cast<const uint8_t*>(p.c_in) + (size_t)n1 * 4;
@@ -463,7 +465,11 @@ static hipError_t launch_tiles_as(int tile, int op, const TileGemmParams& p, hip
             if (p.qwords && p.q_per_column)
                 tail.qwords = p.qwords + n1;
             // block-scaled types: the 256 x 128 tile with the three-slab ring unless a tail tile was asked for
+            // plain types: the deep-ring kernel's 128 x 128 shape, which also reads a row-major B (bf16 4096 x 4312 x 2048: 76.8
+            // us, with tile 5 84.4); its last chunk of K starts on a dword
             const bool scaled_op = op >= TOP_FP8_E4E4;
+            if (p.b_nd || (!scaled_op && options().tail_tile == 0 && (p.k_bytes % 4) == 0))
+                return launch_gemm_ring(RING_SHAPE_128X128, op, tail, stream);
             return launch_gemm_tile(options().tail_tile > 0 ? options().tail_tile : (scaled_op ? 7 : 5), op, tail, stream);
         }
     }
@@ -515,7 +521,10 @@ static const char* tile_kernel_name(int tile, int op, bool row_major_b = false)
         snprintf(buf, sizeof buf, row_major_b ? "tile%dx%d_bnd_%s" : "tile%dx%d_dtl_%s", bm, bn, ops[op]);
         return buf;
     }
-    snprintf(buf, sizeof buf, "%s_%s", tiles[tile], ops[op]);
+    if (row_major_b)
+        snprintf(buf, sizeof buf, "tile256x256w8_bnd_%s", ops[op]);
+    else
+        snprintf(buf, sizeof buf, "%s_%s", tiles[tile], ops[op]);
     return buf;
 }
 
@@ -733,16 +742,16 @@ static int gemm_common(void* c, int c_type, const void* a, const void* b, int ab
                    : ab_type == PTOAMD_E4M3 ? (b_type == PTOAMD_E4M3 ? TOP_FP8_E4E4 : TOP_FP8_E4E5)
                                             : (b_type == PTOAMD_E5M2 ? TOP_FP8_E5E5 : TOP_FP8_E5E4);
     const bool ragged_k_form = op == TOP_BF16 || op == TOP_F16 || op == TOP_I8, whole_slabs = (k_bytes % 128) == 0;
-    const bool dtl_k_ok = whole_slabs || (ragged_k_form && k_bytes > 128);
-    // A row-major B of 16-bit elements is read by the deep-ring kernel as it is, transposed on its way out of LDS (its rows have
-    // to be whole 16-byte chunks; a column chunk past N is fetched from the row's last one).  With a workspace the shape is the
-    // one that the same product takes with a column-major B, so that both have the same bits; where that is one of the two-
-    // and three-slab tiles, B is re-ordered for it.
+    const DtlTiles dtl_k = whole_slabs || (ragged_k_form && k_bytes > 128) ? DTL_ALL : DTL_NONE;
+    // A row-major B of 16-bit elements is read as it is by the deep-ring kernel and, over whole slabs, by the 256 x 256 tile,
+    // transposed on its way out of LDS (its rows have to be whole 16-byte chunks; a column chunk past N is fetched from the
+    // row's last one).  With a workspace the tile is the one that the same product takes with a column-major B, so that both
+    // have the same bits; where that tile has no row-major form, B is re-ordered for it.
     const bool nd_ok = b_layout == PTOAMD_B_ND && ebytes == 2 && !options().b_nd_in_loader && options().tile < 0 && (n % 8) == 0 &&
                        aligned4(a) && aligned4(b) && (lda_b % 4) == 0 && (ldb_b % 4) == 0 && (k_bytes % 4) == 0 &&
                        dma_offsets_fit(m, RING_MAX_STAGE_BYTES / 2 + 8, lda_b, ldb_b, std::max(k_bytes, 2 * (long)n));
-    const int nd_tile = nd_ok ? pick_dma_tile(m, n, k_bytes, op, b_via_ws && dtl_k_ok) : -1;
-    const bool nd_direct = nd_tile >= TILE_RING;
+    const int nd_tile = nd_ok ? pick_dma_tile(m, n, k_bytes, op, b_via_ws ? dtl_k : whole_slabs ? DTL_256_ONLY : DTL_NONE) : -1;
+    const bool nd_direct = nd_tile >= TILE_RING || (nd_tile == 4 && whole_slabs);
     const uint8_t* b_kmajor = reinterpret_cast<const uint8_t*>(b);
     long ldb_kmajor = ldb_b;
     if (b_via_ws && !nd_direct) {  // TLOAD of an ND B panel: re-order once so the MFMA path reads K-contiguous rows
@@ -769,7 +778,7 @@ static int gemm_common(void* c, int c_type, const void* a, const void* b, int ab
                         dma_offsets_fit(m, n, lda_b, ldb_kmajor, k_bytes);
     // (the deep-ring kernel reads a chunk that K ends in as the 16 bytes ending there, which must start on a dword)
     const int tile = nd_direct ? nd_tile
-                     : options().tile < 0 && dma_ok && (k_bytes % 4) == 0 ? pick_dma_tile(m, n, k_bytes, op, dtl_k_ok)
+                     : options().tile < 0 && dma_ok && (k_bytes % 4) == 0 ? pick_dma_tile(m, n, k_bytes, op, dtl_k)
                                                                           : pick_tile(m, n, k_bytes, false, false, dma_ok, ragged_k_form);
     PTOAMD_HIP_CHECK(launch_tiles(tile, op, p, stream));
     set_last_kernel(tile_kernel_name(tile_as_launched(tile, op, m, n), op, nd_direct));
@@ -808,7 +817,7 @@ int ptoamd_gemm_w8a8(void* out_bf16, int32_t* acc_out, const int8_t* a, const in
     p.out_kind = OUT_W8A8_BF16; p.group_m = 4;
     p.b_nd = b_in_kernel; p.b_esz = 1;
     const bool dma_ok = !b_in_kernel && aligned4(a) && aligned4(b) && (lda % 4) == 0 && (ldb % 4) == 0 && dma_offsets_fit(m, n, lda, ldb, k);
-    const int tile = options().tile < 0 && dma_ok && (k % 4) == 0 ? pick_dma_tile(m, n, k, TOP_I8, (k % 128) == 0 || k > 128)
+    const int tile = options().tile < 0 && dma_ok && (k % 4) == 0 ? pick_dma_tile(m, n, k, TOP_I8, (k % 128) == 0 || k > 128 ? DTL_ALL : DTL_NONE)
                                                                   : pick_tile(m, n, k, false, false, dma_ok, true);
     PTOAMD_HIP_CHECK(launch_tiles(tile, TOP_I8, p, stream));
     set_last_kernel(tile_kernel_name(tile, TOP_I8));
@@ -954,7 +963,7 @@ static int gemm_mx_common(const char* who, void* c, int c_type, const void* a, c
     // (the deep-ring kernel fetches them as dwords: any K that is a multiple of 128, which the row-length check above asks for)
     const bool dma_ok = !e1m2 && plain_scales && !b_in_kernel && dma_offsets_fit(m, n, lda_b, ldb_b, k_bytes);
     const int tile = e1m2 ? pick_tile(m, n, k, true, false, false)
-                     : options().tile < 0 && dma_ok && (kg % 4) == 0 ? pick_dma_tile(m, n, k_bytes, op, scale_dma_ok)
+                     : options().tile < 0 && dma_ok && (kg % 4) == 0 ? pick_dma_tile(m, n, k_bytes, op, scale_dma_ok ? DTL_ALL : DTL_NONE)
                                                                     : pick_tile(m, n, k_bytes, true, a4, dma_ok && scale_dma_ok);
     PTOAMD_HIP_CHECK(launch_tiles(tile, op, p, stream));
     set_last_kernel(tile_kernel_name(tile_as_launched(tile, op, m, n), op));

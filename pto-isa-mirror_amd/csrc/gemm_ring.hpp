@@ -26,7 +26,7 @@ struct TileGemmParams;
 #define PTOAMD_RING_SHAPES_PLAIN(X)                               \
     X(7, 192, 128, 4, 2, 1, 128, 4, 4, 2, 1, 128, 3, 4, true)     \
     X(8, 256, 128, 4, 2, 1, 128, 3, 4, 2, 1, 128, 3, 4, true)
-constexpr int RING_SHAPES = 9, RING_SHAPES_SCALED = 7, RING_MAX_STAGE_BYTES = 1024;
+constexpr int RING_SHAPES = 9, RING_SHAPES_SCALED = 7, RING_MAX_STAGE_BYTES = 1024, RING_SHAPE_128X128 = 6;
 
 inline void ring_shape(int shape, int* bm, int* bn)
 {

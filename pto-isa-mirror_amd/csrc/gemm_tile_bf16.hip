@@ -2,5 +2,6 @@
 #define PTOAMD_TILE_OP OpBF16
 #define PTOAMD_TILE_OP16 OpBF16x16
 #define PTOAMD_TILE_RAGGED_K
+#define PTOAMD_TILE_ROW_MAJOR_B
 #define PTOAMD_TILE_FN launch_gemm_tile_bf16
 #include "gemm_tile_inst.hpp"

@@ -86,10 +86,15 @@ __host__ __device__ constexpr int dma_phase_begin(int phase)
 // bytes past K zero, and chunks past K are written as zeros -- so the MFMAs run over a whole slab and the products
 // beyond K vanish.  A compile-time form: the kernel for whole slabs carries none of it.  Its slabs go out in one DMA
 // phase, so that a slab is requested in exactly one place.
-template <class Cfg, bool RAGGED = false>
+// BND: B is row-major [K][N] of 16-bit elements (a whole number of slabs of K).  A slab of B is then 64 k rows as they lie in
+// memory, and the fragment reads transpose them (read_transposed_16, lds_dma.hpp); products, order and results are those
+// of a column-major B.  bf16 4096^3: 95 us (column-major 94, re-ordered through a workspace first 131).
+template <class Cfg, bool RAGGED = false, bool BND = false>
 __global__ void __launch_bounds__(Cfg::THREADS) gemm_tile_dtl_kernel(const TileGemmParams p)
 {
     static_assert(!RAGGED || (Cfg::RING == 2 && !Cfg::Op::SCALED), "the ragged-K form exists for the two-slab ring of the plain types");
+    static_assert(!BND || (!RAGGED && !Cfg::Op::SCALED && Cfg::BLK == 16 && Cfg::NB == 4 && Cfg::BN % 128 == 0 && Cfg::THREADS % (Cfg::BN * 2) == 0),
+                  "the row-major form exists for whole slabs of the 16-bit types on the 16x16 instructions");
     using Op = typename Cfg::Op;
     using Acc = typename Op::Acc;
     constexpr int BM = Cfg::BM, BN = Cfg::BN, MB = Cfg::MB, NB = Cfg::NB, LA = Cfg::LA, LB = Cfg::LB;
@@ -128,6 +133,15 @@ __global__ void __launch_bounds__(Cfg::THREADS) gemm_tile_dtl_kernel(const TileG
 #pragma unroll
     for (int i = 0; i < LB; ++i)
         goff_b[i] = (uint32_t)((long)min(n0 + ld_row + i * (NT / 8), p.n - 1) * p.ldb_bytes + ld_chunk * 16);
+    // BND: piece i is k rows i * NT / (BN / 8) .. of the slab; columns past N repeat the row's last chunk
+    constexpr int ND_CPR = BN / 8, ND_ROWS = NT / ND_CPR;
+    if constexpr (BND) {
+        const int chunk = (tid % ND_CPR) ^ (swizzle_row_major<128>(tid / ND_CPR) << 1);
+#pragma unroll
+        for (int i = 0; i < LB; ++i)
+            goff_b[i] = (uint32_t)((tid / ND_CPR + i * ND_ROWS) * p.ldb_bytes) + (uint32_t)min(n0 * 2 + chunk * 16, p.n * 2 - 16);
+    }
+    const long b_slab = BND ? 64 * p.ldb_bytes : 128;
     const int k_slabs = RAGGED ? (p.k_bytes + 127) / 128 : p.k_bytes / 128;
 
     const uint32_t lds_wave_base = __builtin_amdgcn_readfirstlane(lds_address(smem) + wave * 1024);
@@ -137,7 +151,7 @@ __global__ void __launch_bounds__(Cfg::THREADS) gemm_tile_dtl_kernel(const TileG
         if (q < LA)
             lds_dma16_off(p.a + (long)kt * 128, goff_a[q], dst + q * (NT * 16));
         else
-            lds_dma16_off(p.b + (long)kt * 128, goff_b[q - LA], dst + Cfg::A_BYTES + (q - LA) * (NT * 16));
+            lds_dma16_off(p.b + kt * b_slab, goff_b[q - LA], dst + Cfg::A_BYTES + (q - LA) * (NT * 16));
     };
     // the same for the last slab of a ragged K (see RAGGED above)
     auto tload_piece_last = [&](int buf, int q) __attribute__((always_inline)) {
@@ -250,6 +264,9 @@ __global__ void __launch_bounds__(Cfg::THREADS) gemm_tile_dtl_kernel(const TileG
     static_assert(Cfg::WTM % 32 == 0 && Cfg::WTN % 32 == 0, "wave tiles start on 32-row boundaries");
     const uint32_t fa_lane = (wm * Cfg::WTM + l32) * 128 + ((lhi ^ swizzle_chunk(l32, 0)) << 4);
     const uint32_t fb_lane = Cfg::A_BYTES + (wn * Cfg::WTN + l32) * 128 + ((lhi ^ swizzle_chunk(l32, 0)) << 4);
+    // BND: this lane's 8 bytes of a k-step's first block, k rows 8 lhi .. + 3
+    const int nd_row = lhi * 8 + (l32 >> 2);
+    const uint32_t nd_at = Cfg::A_BYTES + nd_row * (BN * 2) + ((wn * NB ^ swizzle_row_major<128>(nd_row)) << 5) + (l32 & 3) * 8;
     // Two fragment register sets (next k-step's reads overlap this k-step's MFMAs).  Where 32-byte fragments of a large
     // wave tile would not fit the register file twice next to the accumulators (HYBRID), only the fragments that stay
     // live until the end of a k-step get a second copy -- all of B and A's last row block; the other A row blocks are
@@ -268,6 +285,11 @@ __global__ void __launch_bounds__(Cfg::THREADS) gemm_tile_dtl_kernel(const TileG
         const uint8_t* base = smem + buf * Cfg::STAGE_BYTES;
         if (q < NB * FR) {
             const int j = q / FR, f = q % FR;
+            if constexpr (BND) {
+                const uint8_t* at = base + (nd_at ^ (j << 5)) + s * (32 * BN * 2);
+                fb[set][j][f] = read_transposed_16(at, at + 4 * BN * 2);
+                return;
+            }
             fb[set][j][f] = *reinterpret_cast<const uint4*>(base + (fb_lane ^ (frag_chunk<FR, LG>(s, 0, f) << 4)) + j * (BLK * 128));
         } else {
             const int i = (q - NB * FR) / FR, f = (q - NB * FR) % FR;
@@ -332,7 +354,7 @@ __global__ void __launch_bounds__(Cfg::THREADS) gemm_tile_dtl_kernel(const TileG
             }
         });
         if constexpr (SETS == 2 && !HYBRID)
-            sched_kstep<NMMA, NREAD, 0>();
+            sched_kstep<NMMA, BND ? NREAD + NB : NREAD, 0>();  // (a transposed fragment is two reads)
     };
 
     // ---- prologue: slabs 0 and 1 in flight, first fragments in registers

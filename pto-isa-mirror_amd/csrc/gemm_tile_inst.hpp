@@ -27,7 +27,8 @@ static hipError_t launch_cfg(const TileGemmParams& p, hipStream_t stream)
 
 // RAGGED_K: this tile also exists in the form that takes a K extent of any length (the plain types' 256 x 256 and
 // 128 x 128 tiles); the launcher picks it when K is not a whole number of 128-byte slabs.
-template <class Cfg, bool RAGGED_K = false>
+// ROW_MAJOR_B: likewise the form that reads a row-major B in place (the 16-bit types' 256 x 256 tile), for p.b_nd.
+template <class Cfg, bool RAGGED_K = false, bool ROW_MAJOR_B = false>
 static hipError_t launch_dtl(const TileGemmParams& p, hipStream_t stream)
 {
     hipError_t e = ensure_dynamic_lds(reinterpret_cast<const void*>(&gemm_tile_dtl_kernel<Cfg, false>), Cfg::LDS_BYTES);
@@ -35,9 +36,22 @@ static hipError_t launch_dtl(const TileGemmParams& p, hipStream_t stream)
         if (e == hipSuccess)
             e = ensure_dynamic_lds(reinterpret_cast<const void*>(&gemm_tile_dtl_kernel<Cfg, true>), Cfg::LDS_BYTES);
     }
+    if constexpr (ROW_MAJOR_B) {
+        if (e == hipSuccess)
+            e = ensure_dynamic_lds(reinterpret_cast<const void*>(&gemm_tile_dtl_kernel<Cfg, false, true>), Cfg::LDS_BYTES);
+    }
     if (e != hipSuccess || p.m <= 0)
         return e;
     const int tiles = ((p.m + Cfg::BM - 1) / Cfg::BM) * ((p.n + Cfg::BN - 1) / Cfg::BN);
+    if (p.b_nd) {
+        if constexpr (ROW_MAJOR_B) {
+            if (p.k_bytes % 128 == 0) {
+                hipLaunchKernelGGL((gemm_tile_dtl_kernel<Cfg, false, true>), dim3(tiles), dim3(Cfg::THREADS), Cfg::LDS_BYTES, stream, p);
+                return hipGetLastError();
+            }
+        }
+        return hipErrorInvalidValue;  // (as below)
+    }
     if (p.k_bytes % 128 != 0) {
         if constexpr (RAGGED_K) {
             hipLaunchKernelGGL((gemm_tile_dtl_kernel<Cfg, true>), dim3(tiles), dim3(Cfg::THREADS), Cfg::LDS_BYTES, stream, p);
@@ -69,6 +83,12 @@ static hipError_t launch_mx16(const TileGemmParams& p, hipStream_t stream)
 #define PTOAMD_RK false
 #endif
 
+#ifdef PTOAMD_TILE_ROW_MAJOR_B
+#define PTOAMD_ND true
+#else
+#define PTOAMD_ND false
+#endif
+
 hipError_t PTOAMD_TILE_FN(int tile, const TileGemmParams& p, hipStream_t stream)
 {
     if (tile == TILE_PREPARE_ALL) {  // every kernel of this unit gets its launch attributes on the current device
@@ -85,7 +105,7 @@ hipError_t PTOAMD_TILE_FN(int tile, const TileGemmParams& p, hipStream_t stream)
         // and a third of this translation unit's compile time; the id now selects tile 4)
 #ifdef PTOAMD_TILE_OP16  // the large eight-wave tile runs on the 16x16 instructions where the operand type has them
         case 3:
-        case 4: return launch_dtl<TileCfg<256, 256, 2, 4, PTOAMD_TILE_OP16>, PTOAMD_RK>(p, stream);
+        case 4: return launch_dtl<TileCfg<256, 256, 2, 4, PTOAMD_TILE_OP16>, PTOAMD_RK, PTOAMD_ND>(p, stream);
 #elif defined(PTOAMD_TILE_MX16)  // block-scaled fp8: id 3 is the large tile on the 16x16x128 instruction
         case 3:  // (tiles that lie inside the matrix; a ragged edge takes the 32x32x64 form, whose loader clamps its rows)
             if (p.m % 256 == 0 && p.n % 256 == 0)

@@ -76,24 +76,6 @@ __device__ __forceinline__ int ring_swizzle(int row)
     return SB == 128 ? swizzle_chunk(row, 0) : (row & 15);
 }
 
-// BND: which of a k row's 32-byte pieces (16 columns) stands where: piece ^ ring_swizzle_nd(row).  A half wave of the
-// transposing read takes one piece of rows 0 .. 3 and 8 .. 11 (of a multiple of 4): they go to different banks from 32 columns on.
-template <int BN>
-__device__ __forceinline__ int ring_swizzle_nd(int row)
-{
-    const int b3 = (row >> 3) & 1;
-    return BN == 128 ? (row & 3) | (b3 << 2) : BN == 64 ? ((row >> 1) & 1) | (b3 << 1) : BN == 32 ? b3 : 0;
-}
-
-// Four k rows of 16 columns, transposed on their way out of LDS: every lane of a group of 16 names 8 bytes -- row l16 / 4,
-// columns 4 (l16 % 4) .. + 3 -- and receives column l16 of the four rows.
-__device__ __forceinline__ uint2 ring_read_transposed(const uint8_t* at)
-{
-    typedef short s16x4 __attribute__((ext_vector_type(4)));
-    typedef __attribute__((address_space(3))) s16x4* lds_s16x4_ptr;
-    return __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_ptr)(at)));
-}
-
 template <int N>
 __device__ __forceinline__ void ring_wait_and_barrier()
 {
@@ -246,7 +228,7 @@ __global__ void __launch_bounds__(Cfg::THREADS) gemm_tile_ring_kernel(const Tile
     // BND: a stage's B is KR rows of BN columns; row and byte offset (columns past N repeat the row's last chunk)
     auto nd_row = [&](int q) { return ((lw + q * NW - Cfg::A_PIECES) * 64 + lane) / Cfg::CB; };
     auto nd_col = [&](int q) -> uint32_t {
-        const int chunk = (lane % Cfg::CB) ^ (ring_swizzle_nd<BN>(nd_row(q)) << 1);
+        const int chunk = (lane % Cfg::CB) ^ (swizzle_row_major<BN>(nd_row(q)) << 1);
         return (uint32_t)min(n0 * 2 + chunk * 16, p.n * 2 - 16);
     };
     uint32_t goff[NPW];
@@ -312,7 +294,7 @@ __global__ void __launch_bounds__(Cfg::THREADS) gemm_tile_ring_kernel(const Tile
     const uint32_t sa_at = Cfg::ROWS * SB + (wm * Cfg::WTM + l16) * (SC * 4) + lg, sb_at = Cfg::ROWS * SB + (BM + wn * Cfg::WTN + l16) * (SC * 4) + lg;
     // BND: this lane's 8 bytes of a k-step's first block, k rows 8 lg .. + 3
     const int nd_l = lg * 8 + (l16 >> 2);
-    const uint32_t nd_at = BM * SB + (wk * (Cfg::KW / 2) + nd_l) * Cfg::RB + ((wn * (Cfg::WTN / 16) ^ ring_swizzle_nd<BN>(nd_l)) << 5) + (l16 & 3) * 8;
+    const uint32_t nd_at = BM * SB + (wk * (Cfg::KW / 2) + nd_l) * Cfg::RB + ((wn * (Cfg::WTN / 16) ^ swizzle_row_major<BN>(nd_l)) << 5) + (l16 & 3) * 8;
     // Fragment registers.  PIPE: B's fragments and A's last row block have two sets, alternating per k-step; the other row
     // blocks of A are refilled in place right after their last matrix instruction, several of them before the next k-step
     // reads them.
@@ -332,8 +314,7 @@ __global__ void __launch_bounds__(Cfg::THREADS) gemm_tile_ring_kernel(const Tile
         const uint8_t* base = smem + b * Cfg::STAGE;
         if constexpr (Cfg::BND) {
             const uint8_t* at = base + (nd_at ^ (j << 5)) + s * 32 * Cfg::RB;
-            const uint2 lo = ring_read_transposed(at), hi = ring_read_transposed(at + 4 * Cfg::RB);
-            fb[set][j][0] = make_uint4(lo.x, lo.y, hi.x, hi.y);
+            fb[set][j][0] = read_transposed_16(at, at + 4 * Cfg::RB);
             return;
         }
 #pragma unroll

@@ -35,6 +35,26 @@ __device__ __forceinline__ uint32_t lds_address(const void* generic_ptr)
     return (uint32_t)(uintptr_t)(lds_ptr_t)(generic_ptr);
 }
 
+// A row-major B of 16-bit elements in LDS, COLS columns per k row: which of a row's 32-byte pieces (16 columns) stands where is
+// piece ^ swizzle_row_major(row).  A half wave of the transposing read takes one piece of rows 0 .. 3 and 8 .. 11 (counted from
+// a multiple of 4): they lie in different banks from 32 columns on.
+template <int COLS>
+__device__ __forceinline__ int swizzle_row_major(int row)
+{
+    const int b3 = (row >> 3) & 1;
+    return COLS == 128 ? (row & 3) | (b3 << 2) : COLS == 64 ? ((row >> 1) & 1) | (b3 << 1) : COLS == 32 ? b3 : 0;
+}
+// Eight k rows of 16 columns as the B fragment of a 16x16x32 instruction: ds_read_b64_tr_b16 reads four rows.  Every lane of a
+// group of 16 names 8 bytes -- row lane / 4, columns 4 (lane % 4) .. + 3 -- and receives its own column of the four rows.
+__device__ __forceinline__ uint4 read_transposed_16(const uint8_t* rows_0_3, const uint8_t* rows_4_7)
+{
+    typedef short s16x4 __attribute__((ext_vector_type(4)));
+    typedef __attribute__((address_space(3))) s16x4* lds_s16x4_ptr;
+    const uint2 lo = __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_ptr)(rows_0_3)));
+    const uint2 hi = __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_ptr)(rows_4_7)));
+    return make_uint4(lo.x, lo.y, hi.x, hi.y);
+}
+
 // The 4-byte form: 64 lanes x 4 bytes to LDS bytes [lds_base, lds_base + 256), lane-linear.
 __device__ __forceinline__ void lds_dma4(const uint8_t* gptr, uint32_t lds_base)
 {

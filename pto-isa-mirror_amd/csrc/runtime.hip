@@ -6,6 +6,7 @@
 #include <string.h>
 #include <unistd.h>
 
+#include <atomic>
 #include <mutex>
 #include <set>
 #include <utility>
@@ -236,9 +237,15 @@ int ptoamd_init(int device)
     }
     (void)options();
     (void)device_compute_units();
+    // the kernels' launch attributes stay with the device: a further call for it has nothing to prepare
+    static std::atomic<bool> prepared[64];
+    if (device < 64 && prepared[device].load(std::memory_order_acquire))
+        return PTOAMD_OK;
     int rc = prepare_gemm_kernels();
     if (rc == PTOAMD_OK)
         rc = prepare_gemv_kernels();
+    if (rc == PTOAMD_OK && device < 64)
+        prepared[device].store(true, std::memory_order_release);
     return rc;
 }
 

@@ -69,6 +69,23 @@ def test_row_major_b(pa, oracle, kind, shape):  # noqa: F811
         assert bool(((got.double() - ref).abs() <= bound).all()), (m, n, k)
 
 
+@pytest.mark.parametrize("k", [64, 128, 320])
+@pytest.mark.parametrize("kind", ["bf16", "f16"])
+def test_row_major_b_256x256(pa, kind, k):  # noqa: F811
+    """The 256 x 256 tile's row-major form over one, two and five slabs, with a last row of tiles that is not full and tail
+    columns that run on the deep-ring kernel: bits of the column-major product where that runs on the same tile."""
+    m, n = 4090, 4112
+    gen = torch.Generator(device="cuda").manual_seed(k)
+    tdt, t = (torch.float16, pa.F16) if kind == "f16" else (torch.bfloat16, pa.BF16)
+    a, b = (torch.rand(x, generator=gen, device="cuda").sub(0.5).to(tdt) for x in ((m, k), (k, n)))
+    got = pa.gemm(a, b, t, pa.F32, pa.B_ND)
+    assert pa.last_kernel() == f"tile256x256w8_bnd_{kind}", pa.last_kernel()
+    same = pa.gemm(a, b.t().contiguous(), t, pa.F32, pa.B_DN)
+    assert torch.equal(got[:, :4096], same[:, :4096])
+    ref, mag = a.double() @ b.double(), a.double().abs() @ b.double().abs()
+    assert bool(((got.double() - ref).abs() <= k * 2.0 ** -23 * mag).all())
+
+
 @pytest.mark.parametrize("shape", range(7))
 @pytest.mark.parametrize("ta,tb", [(ob.E4M3, ob.E4M3), (ob.E5M2, ob.E4M3), (ob.E4M3, ob.E5M2), (ob.E5M2, ob.E5M2), (ob.E2M1, ob.E2M1)])
 def test_block_scaled_types(pa, oracle, ta, tb, shape):  # noqa: F811
