@@ -367,12 +367,16 @@ constexpr int TILE_RING = 16;  // tile ids from here on: the deep-ring kernel's 
 // dtl: which of the two- and three-slab tiles take this operand as well (K and, for block-scaled types, rows of scales they can
 // stream; a row-major B)
 enum DtlTiles { DTL_NONE, DTL_256_ONLY, DTL_ALL };
-static int pick_dma_tile(int m, int n, long k_bytes, int op, DtlTiles dtl)
+// unaligned: rows that start on any byte, which the shapes with copying waves take in a form of their own; its stages take 1.9
+// times as long (bf16 600 x 8001 x 2049: 47 us on 192 x 128, 62 on the 128 x 128 that the plain estimate asks for)
+static int pick_dma_tile(int m, int n, long k_bytes, int op, DtlTiles dtl, bool unaligned = false)
 {
     const bool scaled = op >= TOP_FP8_E4E4;
     const int shapes = scaled ? RING_SHAPES_SCALED : RING_SHAPES;
-    if (options().ring >= 0 && options().ring < shapes)
-        return TILE_RING + options().ring;
+    const int first = unaligned ? RING_FIRST_UNALIGNED : 0, form = unaligned ? RING_UNALIGNED : 0;
+    const float copying = unaligned ? 1.9f : 1.0f;
+    if (options().ring >= first && options().ring < shapes)
+        return TILE_RING + form + options().ring;
     // A round or more of 256 x 256 tiles: those (with the split of a part-filled last round below) are ahead from K = 1024 on
     // -- bf16 4096 x 8192 x 2048: 105 us against 129 on 256 x 128 -- and within a tenth of the best where a sixteenth of a round
     // is left over (4096 x 4312: 192 x 128 tiles 79 against 87 us at K = 2048).
@@ -389,10 +393,10 @@ static int pick_dma_tile(int m, int n, long k_bytes, int op, DtlTiles dtl)
     for (int c = 0; c < COST_COUNT; ++c) {
         if (c < RING_SHAPES ? c >= shapes : (dtl == DTL_NONE || (dtl == DTL_256_ONLY && c != COST_TILE4) || (c == COST_TILE7 && !scaled)))
             continue;
-        if (scaled && c <= 2 && m > 64)
+        if ((scaled && c <= 2 && m > 64) || c < first)
             continue;
         static const int ids[3] = {4, 5, 7};
-        const int id = c < RING_SHAPES ? TILE_RING + c : ids[c - RING_SHAPES];
+        const int id = c < RING_SHAPES ? TILE_RING + form + c : ids[c - RING_SHAPES];
         int bm, bn;
         if (c < RING_SHAPES)
             ring_shape(c, &bm, &bn);
@@ -405,7 +409,7 @@ static int pick_dma_tile(int m, int n, long k_bytes, int op, DtlTiles dtl)
             rounds = 1.45f * (float)whole + (rest == 0 ? 0.0f : rest <= cus ? 1.0f : 1.0f + 0.45f * (float)(rest - cus) / (float)cus);
         }
         const float full = (float)tiles * (float)(bm * bn) * 1e-6f / cost[c].rate;
-        const float us = 3.0f + rounds * cost[c].round + slabs * std::max(rounds * cost[c].slab, full) * (c < RING_SHAPES ? 1.0f : ragged);
+        const float us = 3.0f + rounds * cost[c].round + slabs * std::max(rounds * copying * cost[c].slab, full) * (c < RING_SHAPES ? 1.0f : ragged);
         if (us < best_us) {
             best_us = us;
             best = id;
@@ -518,7 +522,8 @@ static const char* tile_kernel_name(int tile, int op, bool row_major_b = false)
     if (tile >= TILE_RING) {
         int bm, bn;
         ring_shape(tile - TILE_RING, &bm, &bn);
-        snprintf(buf, sizeof buf, row_major_b ? "tile%dx%d_bnd_%s" : "tile%dx%d_dtl_%s", bm, bn, ops[op]);
+        snprintf(buf, sizeof buf, row_major_b ? "tile%dx%d_bnd_%s" : tile >= TILE_RING + RING_UNALIGNED ? "tile%dx%d_any_%s" : "tile%dx%d_dtl_%s",
+                 bm, bn, ops[op]);
         return buf;
     }
     if (row_major_b)
@@ -777,9 +782,13 @@ static int gemm_common(void* c, int c_type, const void* a, const void* b, int ab
     const bool dma_ok = !b_in_kernel && aligned4(a) && aligned4(b_kmajor) && (lda_b % 4) == 0 && (ldb_kmajor % 4) == 0 &&
                         dma_offsets_fit(m, n, lda_b, ldb_kmajor, k_bytes);
     // (the deep-ring kernel reads a chunk that K ends in as the 16 bytes ending there, which must start on a dword)
+    // rows that start on other bytes, at least one chunk long: the deep-ring kernel's copies through registers (faster than the
+    // register-staged tiles, or as fast, at all of 54 sizes, m 7 .. 4000, n 1001 .. 8001, k 1023 .. 4097: 1.0 to 2.2 times)
+    const bool any_ok = ragged_k_form && !b_in_kernel && !dma_ok && k_bytes >= 16 && dma_offsets_fit(m, n, lda_b, ldb_kmajor, k_bytes);
     const int tile = nd_direct ? nd_tile
                      : options().tile < 0 && dma_ok && (k_bytes % 4) == 0 ? pick_dma_tile(m, n, k_bytes, op, dtl_k)
-                                                                          : pick_tile(m, n, k_bytes, false, false, dma_ok, ragged_k_form);
+                     : options().tile < 0 && any_ok ? pick_dma_tile(m, n, k_bytes, op, DTL_NONE, true)
+                                                    : pick_tile(m, n, k_bytes, false, false, dma_ok, ragged_k_form);
     PTOAMD_HIP_CHECK(launch_tiles(tile, op, p, stream));
     set_last_kernel(tile_kernel_name(tile_as_launched(tile, op, m, n), op, nd_direct));
     return PTOAMD_OK;
@@ -817,8 +826,10 @@ int ptoamd_gemm_w8a8(void* out_bf16, int32_t* acc_out, const int8_t* a, const in
     p.out_kind = OUT_W8A8_BF16; p.group_m = 4;
     p.b_nd = b_in_kernel; p.b_esz = 1;
     const bool dma_ok = !b_in_kernel && aligned4(a) && aligned4(b) && (lda % 4) == 0 && (ldb % 4) == 0 && dma_offsets_fit(m, n, lda, ldb, k);
+    const bool any_ok = !b_in_kernel && !dma_ok && k >= 16 && dma_offsets_fit(m, n, lda, ldb, k);
     const int tile = options().tile < 0 && dma_ok && (k % 4) == 0 ? pick_dma_tile(m, n, k, TOP_I8, (k % 128) == 0 || k > 128 ? DTL_ALL : DTL_NONE)
-                                                                  : pick_tile(m, n, k, false, false, dma_ok, true);
+                     : options().tile < 0 && any_ok ? pick_dma_tile(m, n, k, TOP_I8, DTL_NONE, true)
+                                                    : pick_tile(m, n, k, false, false, dma_ok, true);
     PTOAMD_HIP_CHECK(launch_tiles(tile, TOP_I8, p, stream));
     set_last_kernel(tile_kernel_name(tile, TOP_I8));
     return PTOAMD_OK;

@@ -27,6 +27,8 @@ struct TileGemmParams;
     X(7, 192, 128, 4, 2, 1, 128, 4, 4, 2, 1, 128, 3, 4, true)     \
     X(8, 256, 128, 4, 2, 1, 128, 3, 4, 2, 1, 128, 3, 4, true)
 constexpr int RING_SHAPES = 9, RING_SHAPES_SCALED = 7, RING_MAX_STAGE_BYTES = 1024, RING_SHAPE_128X128 = 6;
+// Added to the id of a shape with copying waves (3 and up) of the plain types: the form for rows that start on any byte.
+constexpr int RING_UNALIGNED = 16, RING_FIRST_UNALIGNED = 3;
 
 inline void ring_shape(int shape, int* bm, int* bn)
 {
@@ -35,11 +37,11 @@ inline void ring_shape(int shape, int* bm, int* bn)
         PTOAMD_RING_SHAPES_ALL(PTOAMD_RING_DIM) PTOAMD_RING_SHAPES_PLAIN(PTOAMD_RING_DIM)
 #undef PTOAMD_RING_DIM
     };
-    *bm = dims[shape][0];
-    *bn = dims[shape][1];
+    *bm = dims[shape % RING_UNALIGNED][0];
+    *bn = dims[shape % RING_UNALIGNED][1];
 }
 
-// shape: 0 .. RING_SHAPES - 1, or TILE_PREPARE_ALL
+// shape: 0 .. RING_SHAPES - 1, RING_UNALIGNED + one of the later ones, or TILE_PREPARE_ALL
 hipError_t launch_gemm_ring_bf16(int shape, const TileGemmParams& p, hipStream_t stream);
 hipError_t launch_gemm_ring_f16(int shape, const TileGemmParams& p, hipStream_t stream);
 hipError_t launch_gemm_ring_i8(int shape, const TileGemmParams& p, hipStream_t stream);

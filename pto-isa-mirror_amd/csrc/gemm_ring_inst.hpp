@@ -43,6 +43,24 @@ static hipError_t launch_ring_shape(int shape, const TileGemmParams& p, hipStrea
     return hipErrorInvalidValue;
 }
 
+// the form for rows at any alignment, shapes with copying waves only
+template <class Op>
+static hipError_t launch_ring_unaligned(int shape, const TileGemmParams& p, hipStream_t stream)
+{
+    switch (shape) {
+#define PTOAMD_RING_CASE(id, bm, bn, wm, wn, wk, sb, r, swm, swn, swk, ssb, sr, lw, pipe)                            \
+    case id:                                                                                                        \
+        if constexpr (pipe)                                                                                         \
+            return launch_ring<RingCfg<bm, bn, wm, wn, wk, sb, r, lw, pipe, Op, false, true>>(p, stream);           \
+        break;
+        PTOAMD_RING_SHAPES_ALL(PTOAMD_RING_CASE)
+        PTOAMD_RING_SHAPES_PLAIN(PTOAMD_RING_CASE)
+#undef PTOAMD_RING_CASE
+        default: break;
+    }
+    return hipErrorInvalidValue;
+}
+
 hipError_t PTOAMD_RING_FN(int shape, const TileGemmParams& p, hipStream_t stream)
 {
 #ifdef PTOAMD_RING_BND  // the 16-bit types also take a row-major B
@@ -50,6 +68,12 @@ hipError_t PTOAMD_RING_FN(int shape, const TileGemmParams& p, hipStream_t stream
 #else
     constexpr bool has_bnd = false;
 #endif
+    if (shape >= RING_UNALIGNED && shape != TILE_PREPARE_ALL) {
+        if constexpr (!PTOAMD_RING_OP::SCALED)
+            if (!p.b_nd)
+                return launch_ring_unaligned<PTOAMD_RING_OP>(shape - RING_UNALIGNED, p, stream);
+        return hipErrorInvalidValue;
+    }
     if (shape != TILE_PREPARE_ALL) {
         if (!p.b_nd)
             return launch_ring_shape<PTOAMD_RING_OP>(shape, p, stream);
@@ -63,6 +87,10 @@ hipError_t PTOAMD_RING_FN(int shape, const TileGemmParams& p, hipStream_t stream
         if constexpr (has_bnd) {
             if (e == hipSuccess)
                 e = launch_ring_shape<PTOAMD_RING_OP, true>(s, none, stream);
+        }
+        if constexpr (!PTOAMD_RING_OP::SCALED) {
+            if (e == hipSuccess && s >= RING_FIRST_UNALIGNED)
+                e = launch_ring_unaligned<PTOAMD_RING_OP>(s, none, stream);
         }
         if (e != hipSuccess)
             return e;

@@ -16,6 +16,12 @@
 //              time into fragments, so no copy of B is made and no thread moves elements.  Measured, bf16: 2048 x 4096 x 4096
 //              57 us (column-major B 56; re-ordered through a workspace first 80; scattered by the register-staged loader
 //              101), 24 x 4096 x 4096 14.2 us (column-major 9.6: here a copy takes 32 bytes of each row; loader 58)
+//   rows at any alignment (ANY, plain types): LDS-DMA wants dword-aligned addresses, so where rows start on other bytes (an odd
+//              number of 16-bit elements) the waves that copy go through registers, unaligned 16-byte loads two or three stages
+//              ahead of their ds_write_b128; everything behind the barrier is the same.
+//              A stage takes about twice as long as by LDS-DMA: the memory path serves an unaligned 16-byte load in two halves.
+//              Measured, bf16, against the register-staged tile chosen by grid size: 64 x 4097 x 4095 28 us (63), 1000 x 2049 x 2047
+//              33 (57; 2048 x 2048 by LDS-DMA: 17), 2100 x 2049 x 2047 43 (61), 4000 x 1025 x 4097 73 (110)
 //   K tail     copies never read past a row: a chunk that would is read as the 16 bytes that END at the row's end, and the
 //              last stage's fragments are masked in registers -- the same bytes of A and B, so k positions still agree
 #pragma once
@@ -41,10 +47,10 @@ struct OpFP4x16 {
 };
 
 // WM x WN x WK waves: WK groups share the tile and split every stage of SB bytes per row along K; R stages in the ring
-template <int BM_, int BN_, int WM_, int WN_, int WK_, int SB_, int R_, int LW_, bool PIPE_, class Op_, bool BND_ = false>
+template <int BM_, int BN_, int WM_, int WN_, int WK_, int SB_, int R_, int LW_, bool PIPE_, class Op_, bool BND_ = false, bool ANY_ = false>
 struct RingCfg {
     static constexpr int BM = BM_, BN = BN_, WM = WM_, WN = WN_, WK = WK_, SB = SB_, R = R_;
-    static constexpr bool PIPE = PIPE_, BND = BND_;  // BND: B is row-major [K][N]
+    static constexpr bool PIPE = PIPE_, BND = BND_, ANY = ANY_;  // BND: B is row-major [K][N]; ANY: rows start on any byte
     using Op = Op_;
     static constexpr int CW = WM * WN * WK, LW = LW_, THREADS = (CW + LW) * 64;
     static constexpr int NW = LW > 0 ? LW : CW;  // waves that copy
@@ -58,6 +64,7 @@ struct RingCfg {
     static constexpr int NV = NPW + NSW;                                  // copies a wave issues per stage
     static constexpr int STAGE = ROWS * SB + ROWS * SC * 4;
     static constexpr int KR = SB / 2, RB = BN * 2, CB = RB / 16;          // BND: k rows of a stage, bytes and chunks per row
+    static constexpr int AHEAD = NPW <= 8 ? 3 : 2;                        // ANY: stages a copying wave holds in registers
     static constexpr int RED_PITCH = BN + 4;                              // elements
     static constexpr int RED_BYTES = WK * BM * RED_PITCH * 4;
     static constexpr int LDS_BYTES = (R * STAGE > RED_BYTES ? R * STAGE : RED_BYTES);
@@ -65,6 +72,7 @@ struct RingCfg {
     static_assert(KW % KB == 0 && SB <= 1024 && 1024 % SB == 0, "a k-group's part of a stage is whole k-steps");
     static_assert(PIECES % NW == 0 && (BM * SB) % 1024 == 0, "every wave issues the same number of 1 KiB copies, each of one operand");
     static_assert(!BND || (!Op::SCALED && FR == 1 && (NB & (NB - 1)) == 0), "the row-major form is for the 16-bit types");
+    static_assert(!ANY || (PIPE && !BND && !Op::SCALED), "the register copies are the copying waves' and know no scales");
     static_assert((ROWS * SC) % 64 == 0, "scale pieces are whole");
     static_assert(LDS_BYTES <= 160 * 1024 && R >= 2 && (R - 1) * NV < 64, "LDS capacity; vmcnt is a 6-bit count");
 };
@@ -409,7 +417,54 @@ __global__ void __launch_bounds__(Cfg::THREADS) gemm_tile_ring_kernel(const Tile
         // buffer is refilled with stage st + R, and stage st + 1 has landed, whose first fragments are read under that
         // k-step's matrix instructions.
         static_assert(Cfg::LW > 0, "the pipelined form has waves that only copy");
-        if (!computes) {
+        if (Cfg::ANY && !computes) {
+            // A stage's chunks are loaded AHEAD stages before they are written.  Neither is ever skipped -- past the last
+            // stage both repeat it, into a buffer that nobody reads any more -- so that the count of loads in flight is known.
+            constexpr int G = Cfg::AHEAD;
+            uint32_t row[NPW], chunk[NPW];
+            uint4 held[G][NPW];
+#pragma unroll
+            for (int q = 0; q < NPW; ++q) {
+                row[q] = row_offset(q);
+                chunk[q] = piece_chunk(q) * 16;
+            }
+            auto load = [&](auto gc, int st) __attribute__((always_inline)) {
+                const uint32_t k0 = min(st, nst - 1) * SB;
+#pragma unroll
+                for (int q = 0; q < NPW; ++q) {
+                    const uint32_t off = row[q] + min(k0 + chunk[q], (uint32_t)(p.k_bytes - 16));
+                    held[decltype(gc)::value][q] = load_unaligned16((lw + q * NW < Cfg::A_PIECES ? p.a : p.b) + off);
+                }
+            };
+            auto store = [&](auto gc, int b) __attribute__((always_inline)) {
+#pragma unroll
+                for (int q = 0; q < NPW; ++q)
+                    *reinterpret_cast<uint4*>(smem + b * Cfg::STAGE + (lw + q * NW) * 1024 + lane * 16) = held[decltype(gc)::value][q];
+            };
+            static_for<G>([&](auto gc) { load(gc, decltype(gc)::value); });
+            static_for<R>([&](auto sc) {
+                constexpr int s = decltype(sc)::value;
+                store(integral_constant<int, s % G>{}, s);
+                load(integral_constant<int, s % G>{}, s + G);
+            });
+            ring_wait_and_barrier<63>();
+            int buf = 0, st = 0;
+            auto step = [&](auto gc) __attribute__((always_inline)) {
+                constexpr integral_constant<int, (R + decltype(gc)::value) % G> g{};
+                ring_wait_and_barrier<63>();
+                store(g, buf);
+                load(g, st + R + G);
+                buf = buf + 1 == R ? 0 : buf + 1;
+                ++st;
+            };
+#pragma unroll 1
+            while (st + G < nst)
+                static_for<G>([&](auto gc) { step(gc); });
+            static_for<G - 1>([&](auto gc) {
+                if (st < nst - 1)
+                    step(gc);
+            });
+        } else if (!computes) {
 #pragma unroll
             for (int s = 0; s < R; ++s)
                 if (s < nst)

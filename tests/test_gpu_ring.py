@@ -46,6 +46,38 @@ def test_plain_types(pa, oracle, kind, shape):  # noqa: F811
             check_f32_drain(got, ref, np.abs(fa) @ np.abs(fb).T, k, f"{kind} {m}x{n}x{k} shape {shape}")
 
 
+@pytest.mark.parametrize("shape", range(3, 9))
+@pytest.mark.parametrize("kind", ["bf16", "f16", "i8"])
+def test_rows_on_any_byte(pa, kind, shape):  # noqa: F811
+    """Rows that start on any byte (16-bit types: on any element), from one chunk of K to more stages than ring and registers
+    hold, the operands inside larger allocations whose other elements are NaN (int8: not zero): exact products of small
+    whole numbers."""
+    esz = 1 if kind == "i8" else 2
+    tdt, t, tc = {"bf16": (torch.bfloat16, pa.BF16, pa.F32), "f16": (torch.float16, pa.F16, pa.F32), "i8": (torch.int8, pa.I8, pa.I32)}[kind]
+    gen = torch.Generator(device="cuda").manual_seed(shape)
+    bm, bn, stage = SHAPES[shape][:3]
+    for m, n, kb in [(bm - 1, bn + 3, 18), (1, bn, stage + 6), (bm + 1, 2 * bn + 1, 2 * stage + 14), (bm, bn - 1, 4 * stage), (bm + 2, bn + 1, 9 * stage + 38)]:
+        k = kb // esz + (1 if kb != 4 * stage else 0)
+
+        def rows(count, pitch, start):  # whole numbers of -7 .. 7, all sums below 2^24
+            flat = torch.full((start + count * pitch + 8,), 99 if kind == "i8" else float("nan"), device="cuda").to(tdt)
+            view = flat[start:start + count * pitch].view(count, pitch)
+            view[:, :k] = torch.randint(-7, 8, (count, k), generator=gen, device="cuda").to(tdt)
+            return view
+        for pitch in (k, k + 3):
+            a, b = rows(m, pitch, 1), rows(n, pitch, 3)
+            with tile_env(PTOAMD_RING=shape):
+                got = pa.gemm(a, b, t, tc, pa.B_DN, k=k)
+                assert pa.last_kernel() == f"tile{bm}x{bn}_any_{kind}", pa.last_kernel()
+            assert torch.equal(got.double(), a[:, :k].double() @ b[:, :k].double().t()), (m, n, k, pitch)
+    if kind == "i8":  # the W8A8 entry point takes the same kernels
+        sa, sb = (torch.rand(x, generator=gen, device="cuda") for x in (m, n))
+        with tile_env(PTOAMD_RING=shape):
+            out = pa.gemm_w8a8(a[:, :k].contiguous(), b[:, :k].contiguous(), sa, sb)
+            assert pa.last_kernel() == f"tile{bm}x{bn}_any_i8", pa.last_kernel()
+        assert torch.equal(out, (got.float() * sa[:, None] * sb[None, :]).to(torch.bfloat16))
+
+
 @pytest.mark.parametrize("shape", range(9))
 @pytest.mark.parametrize("kind", ["bf16", "f16"])
 def test_row_major_b(pa, oracle, kind, shape):  # noqa: F811
