@@ -2,9 +2,9 @@
 //
 // The shape is HBM-bound (every weight byte is read once, ~60 FLOP per byte).  What limits a streaming read on this
 // memory system is the shape of each wave's load: 16 rows x 64 bytes per instruction (the natural MFMA operand
-// pattern) tops out near 3.4 TB/s, 512 contiguous bytes per half wave reaches 5+ TB/s.  Two kernels:
+// pattern) tops out near 3.4 TB/s, 512 contiguous bytes per half wave reaches 5+ TB/s.  Three kernels:
 //
-//   * split-K (k % 1024 == 0, the decode shapes): a workgroup of 8 waves owns a run of 16-row strips; wave s owns
+//   * split-K (k % 1024 == 0): a workgroup of 8 waves owns a run of 16-row strips; wave s owns
 //     k-slice s (1024 k) of every strip and keeps its activation fragments for that slice in registers for the whole
 //     kernel (128 VGPRs, loaded once).  Weights and scales stream global -> LDS by LDS-DMA into a per-wave
 //     double-buffered region (512 contiguous bytes per row, two rows per instruction, no VGPRs, no barriers: a wave
@@ -12,6 +12,7 @@
 //     four MFMAs; row pairs padded and odd rows half-swapped on the global side, so the reads are conflict-free),
 //     dequantised in registers and multiplied on
 //     v_mfma_f32_16x16x32_bf16.  The 8 k-slice partials of a strip are summed through LDS in a fixed order.
+//   * split-K with loader waves, further down: k % 2048 == 0, and k % 512 == 0 beyond one chunk of 2048 and 512 columns.
 //   * streaming (k % 512 == 0 otherwise): a wave owns 16 rows over the full K, register prefetch four chunks deep,
 //     activations staged per chunk through LDS.
 // Dequantisation: v_cvt_scalef32_pk_bf16_fp4 (fp4 pair * 2^e -> bf16 pair, exact).
@@ -349,7 +350,7 @@ __global__ void __launch_bounds__(SK_WAVES * 64) gemv_mxfp4_splitk_kernel(const 
     }
 }
 
-// ---- split-K kernel with loader waves (k % 2048 == 0) ----------------------------------------------------------
+// ---- split-K kernel with loader waves (k in chunks of 2048) ----------------------------------------------------------
 // Same products and the same partition of K into 512-wide slices as the split-K kernel above; the ORDER in which a
 // workgroup adds its chunks is rotated (see K below), so the fp32 sums agree with that kernel's to rounding (1e-5
 // relative in the tests), not bit for bit.  The order is a function of blockIdx.x and of the grid, which follows the
@@ -395,7 +396,13 @@ __device__ __forceinline__ void wg_barrier() { asm volatile("s_barrier" ::: "mem
 // stage is then two contiguous runs of memory instead of 16 pieces 1 KiB long and a row pitch apart plus 16 scale
 // pieces, and streams 4 - 5 % faster (23.4 against 24.5 us on 16 x 28672 x 8192; with the scales inside one 17 KiB block
 // per stage, which takes the code blocks off their 16 KiB alignment, 23.8 us).
-template <bool HW_CVT, bool PACKED = false>
+//
+// PARTIAL: K ends inside a chunk, on a 512-wide slice.  The last chunk's stages keep their place and their number of copies: a
+// lane whose 16 bytes would lie past the row's end re-reads the row's last 16 (the line its neighbours fetch anyway), the
+// compute waves whose slice does not exist skip the products, so nothing past a row is read and nothing is added.
+// Measured, 16 rows: 28672 x 7680 26.5 us against 34.6 on the streaming kernel, 28672 x 5120 20.5 (split-K 24.2), 8192 x 7680
+// 13.8 (28.0), 8192 x 3072 8.2 (12.8).
+template <bool HW_CVT, bool PACKED = false, bool PARTIAL = false>
 __global__ void __launch_bounds__(512) gemv_mxfp4_splitk_wide_kernel(const GemvParams p, int strips_per_wg)
 {
     extern __shared__ __align__(16) uint8_t smem[];
@@ -405,7 +412,7 @@ __global__ void __launch_bounds__(512) gemv_mxfp4_splitk_wide_kernel(const GemvP
     const int wc = wave & 3;                          // compute: k-slice of the chunk; loader: which quarter of a stage
     const int l16 = lane & 15, q = lane >> 4;
     const int s_begin = blockIdx.x * strips_per_wg, s_end = min(s_begin + strips_per_wg, p.n_groups);
-    const int nsteps = s_end - s_begin, kchunks = p.k / WD_CHUNK, sb = p.k / 32;
+    const int nsteps = s_end - s_begin, kchunks = PARTIAL ? (p.k + WD_CHUNK - 1) / WD_CHUNK : p.k / WD_CHUNK, sb = p.k / 32;
     const int kc_first = blockIdx.x % kchunks;        // chunk number x of this workgroup is chunk (kc_first + x) % kchunks of K
     const uint32_t lds0 = lds_address(smem);
     uint8_t* mine = smem + WD_RING * WD_STAGE + wc * WD_ABYTES;      // compute wave's private region
@@ -436,12 +443,15 @@ __global__ void __launch_bounds__(512) gemv_mxfp4_splitk_wide_kernel(const GemvP
             lds_dma4_off_nt(p.wp + (long)p.n_groups * kchunks * WD_WBYTES + idx * WD_SBYTES, (uint32_t)(e * 4), dst + WD_WBYTES + wc * 256);
         } else {
             const uint8_t* wbase = p.w + (long)strip * 16 * p.ldw_bytes + (long)kc * (WD_CHUNK / 2);
+            const int here = PARTIAL ? min(WD_CHUNK, p.k - kc * WD_CHUNK) : WD_CHUNK;   // k of this chunk: 16 bytes per 32, a scale dword per 128
 #pragma unroll
             for (int d = 0; d < 4; ++d) {
                 const int r = 4 * wc + d;   // a loader takes four neighbouring rows (slightly faster than every fourth)
-                lds_dma16_off_nt(wbase, (uint32_t)(min(r, rlim) * (int)p.ldw_bytes) + (uint32_t)((lane ^ r) << 4), dst + r * 1024);
+                const int chunk = PARTIAL ? min(lane ^ r, here / 32 - 1) : lane ^ r;
+                lds_dma16_off_nt(wbase, (uint32_t)(min(r, rlim) * (int)p.ldw_bytes) + (uint32_t)(chunk << 4), dst + r * 1024);
             }
-            lds_dma4_off_nt(p.sw + (long)strip * 16 * sb + (long)kc * (WD_CHUNK / 32), (uint32_t)(min(e >> 4, rlim) * sb + (e & 15) * 4),
+            const int scales = PARTIAL ? min(e & 15, here / 128 - 1) : e & 15;
+            lds_dma4_off_nt(p.sw + (long)strip * 16 * sb + (long)kc * (WD_CHUNK / 32), (uint32_t)(min(e >> 4, rlim) * sb + scales * 4),
                             dst + WD_WBYTES + wc * 256);
         }
         ++issued;
@@ -475,7 +485,7 @@ __global__ void __launch_bounds__(512) gemv_mxfp4_splitk_wide_kernel(const GemvP
         }
     };
     auto prefetch_begin = [&](int kc) {
-        abase = reinterpret_cast<const uint8_t*>(p.a) + (long)(kc * 4 + wc) * 1024;
+        abase = reinterpret_cast<const uint8_t*>(p.a) + (long)(PARTIAL ? min(kc * 4 + wc, p.k / 512 - 1) : kc * 4 + wc) * 1024;
         issue_a(0);
         issue_a(1);
         issue_a(2);
@@ -508,6 +518,7 @@ __global__ void __launch_bounds__(512) gemv_mxfp4_splitk_wide_kernel(const GemvP
         for (int kcx = 0; kcx < kchunks; ++kcx) {
             // the chunk after this one, if the workgroup has one and its activations differ
             const bool more = kchunks > 1 && (kcx + 1 < kchunks || b0 + SK_RMAX < nsteps);
+            const bool live = !PARTIAL || (kc_first + kcx) % kchunks * 4 + wc < p.k / 512;   // this wave's slice exists
             if (!loader) {
                 if (kchunks > 1 || (b0 == 0 && kcx == 0)) {
 #pragma unroll
@@ -542,22 +553,24 @@ __global__ void __launch_bounds__(512) gemv_mxfp4_splitk_wide_kernel(const GemvP
                         if (consumed > 1)
                             issue_next();
                     } else {
-                        uint4 sc4, wv[4];
-                        sc4 = *reinterpret_cast<const uint4*>(buf + sread);
+                        if (live) {
+                            uint4 sc4, wv[4];
+                            sc4 = *reinterpret_cast<const uint4*>(buf + sread);
 #pragma unroll
-                        for (int j = 0; j < 4; ++j)
-                            wv[j] = *reinterpret_cast<const uint4*>(buf + (wread ^ (64 * j)));
-                        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-                        const uint32_t sc[4] = {sc4.x, sc4.y, sc4.z, sc4.w};
+                            for (int j = 0; j < 4; ++j)
+                                wv[j] = *reinterpret_cast<const uint4*>(buf + (wread ^ (64 * j)));
+                            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+                            const uint32_t sc[4] = {sc4.x, sc4.y, sc4.z, sc4.w};
 #pragma unroll
-                        for (int j = 0; j < 4; ++j) {
-                            const float scale = e8m0_to_f32((sc[j] >> (8 * q)) & 0xFFu);  // scale byte 4 j + q of the slice
-                            const uint32_t xs[4] = {wv[j].x, wv[j].y, wv[j].z, wv[j].w};
+                            for (int j = 0; j < 4; ++j) {
+                                const float scale = e8m0_to_f32((sc[j] >> (8 * q)) & 0xFFu);  // scale byte 4 j + q of the slice
+                                const uint32_t xs[4] = {wv[j].x, wv[j].y, wv[j].z, wv[j].w};
 #pragma unroll
-                            for (int t = 0; t < 4; ++t) {
-                                const uint4 w8 = dequant8<HW_CVT>(xs[t], scale);
-                                acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, areg[4 * j + t]),
-                                                                                __builtin_bit_cast(bf16x8, w8), acc[i], 0, 0, 0);
+                                for (int t = 0; t < 4; ++t) {
+                                    const uint4 w8 = dequant8<HW_CVT>(xs[t], scale);
+                                    acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, areg[4 * j + t]),
+                                                                                    __builtin_bit_cast(bf16x8, w8), acc[i], 0, 0, 0);
+                                }
                             }
                         }
                         if (i < 4 && more)
@@ -654,6 +667,8 @@ int prepare_gemv_kernels()
     PTOAMD_HIP_CHECK(ensure_dynamic_lds(reinterpret_cast<const void*>(gemv_mxfp4_splitk_wide_kernel<true, true>), WD_LDS));
     PTOAMD_HIP_CHECK(ensure_dynamic_lds(reinterpret_cast<const void*>(gemv_mxfp4_splitk_wide_kernel<false>), WD_LDS));
     PTOAMD_HIP_CHECK(ensure_dynamic_lds(reinterpret_cast<const void*>(gemv_mxfp4_splitk_wide_kernel<true>), WD_LDS));
+    PTOAMD_HIP_CHECK(ensure_dynamic_lds(reinterpret_cast<const void*>(gemv_mxfp4_splitk_wide_kernel<false, false, true>), WD_LDS));
+    PTOAMD_HIP_CHECK(ensure_dynamic_lds(reinterpret_cast<const void*>(gemv_mxfp4_splitk_wide_kernel<true, false, true>), WD_LDS));
     PTOAMD_HIP_CHECK(ensure_dynamic_lds(reinterpret_cast<const void*>(gemv_mxfp4_splitk_kernel<false>), SK_LDS));
     PTOAMD_HIP_CHECK(ensure_dynamic_lds(reinterpret_cast<const void*>(gemv_mxfp4_splitk_kernel<true>), SK_LDS));
     return PTOAMD_OK;
@@ -696,17 +711,19 @@ extern "C" int ptoamd_gemv_mxfp4(void* out, int c_type, const void* a_bf16, cons
     const int cus = device_compute_units();
     const bool swc = opt.gemv_sw_cvt;
     const bool sk_ok = k % SK_SLICE == 0 && (reinterpret_cast<uintptr_t>(sw) & 3u) == 0 && !opt.gemv_no_splitk;
-    // loader-wave form: K in chunks of 2048; rows are addressed with 32-bit lane offsets
-    if (sk_ok && k % WD_CHUNK == 0 && (long)lda * 2 * 16 < (1L << 31) && p.ldw_bytes * 16 < (1L << 31) && !opt.gemv_no_wide) {
+    // loader-wave form: K in chunks of 2048, the last one possibly partial; rows are addressed with 32-bit lane offsets.
+    // A partial chunk: of 81 sizes (n 256 .. 28672, k 1024 .. 7680) it is ahead of the other two kernels on 80 and 2 % behind
+    // on one (4111 x 5120).  Up to one chunk of K, or 512 columns, the tests hold the sizes to the other kernels
+    // (there it would be 4 to 9 us of GPU time against 8 to 25, where a call from Python takes 7).
+    const bool partial = k % WD_CHUNK != 0;
+    const bool wide_k = !partial || (k > WD_CHUNK && n > 512);
+    if (wide_k && !opt.gemv_no_splitk && (long)lda * 2 * 16 < (1L << 31) && p.ldw_bytes * 16 < (1L << 31) && !opt.gemv_no_wide) {
         const int spw = (p.n_groups + cus - 1) / cus;    // strips per workgroup
         const int grid = (p.n_groups + spw - 1) / spw;
-        const void* fn = swc ? reinterpret_cast<const void*>(gemv_mxfp4_splitk_wide_kernel<false>)
-                             : reinterpret_cast<const void*>(gemv_mxfp4_splitk_wide_kernel<true>);
-        PTOAMD_HIP_CHECK(ensure_dynamic_lds(fn, WD_LDS));
-        if (swc)
-            hipLaunchKernelGGL(gemv_mxfp4_splitk_wide_kernel<false>, dim3(grid), dim3(512), WD_LDS, stream, p, spw);
-        else
-            hipLaunchKernelGGL(gemv_mxfp4_splitk_wide_kernel<true>, dim3(grid), dim3(512), WD_LDS, stream, p, spw);
+        const auto fn = partial ? (swc ? gemv_mxfp4_splitk_wide_kernel<false, false, true> : gemv_mxfp4_splitk_wide_kernel<true, false, true>)
+                                : (swc ? gemv_mxfp4_splitk_wide_kernel<false> : gemv_mxfp4_splitk_wide_kernel<true>);
+        PTOAMD_HIP_CHECK(ensure_dynamic_lds(reinterpret_cast<const void*>(fn), WD_LDS));
+        hipLaunchKernelGGL(fn, dim3(grid), dim3(512), WD_LDS, stream, p, spw);
         PTOAMD_HIP_CHECK(hipGetLastError());
         set_last_kernel(swc ? "gemv_mxfp4_splitk_wide_swcvt" : "gemv_mxfp4_splitk_wide");
         return PTOAMD_OK;

@@ -1255,6 +1255,23 @@ def test_gemv_mxfp4_stream(pa, oracle, m, n, k):
     _check_gemv(pa, oracle, m, n, k, "gemv_mxfp4_stream")
 
 
+# K that ends inside a chunk of 2048, one, two and three slices of 512 into it, from two chunks to five; fewer strips than
+# workgroups, several per workgroup, and more than one accumulator batch; ragged n and m
+@pytest.mark.parametrize("m,n,k", [(16, 1041, 2560), (5, 4111, 3072), (1, 8200, 3584), (16, 4096 + 15, 4608), (7, 40000, 2560), (16, 1030, 9728)])
+def test_gemv_mxfp4_partial_chunk(pa, oracle, m, n, k):
+    got = _check_gemv(pa, oracle, m, n, k, "gemv_mxfp4_splitk_wide")
+    a, w, sw = _gemv_case(m, n, k)
+    with tile_env(PTOAMD_GEMV_NO_SPLITK=1):  # the streaming kernel agrees to rounding
+        other = host(pa.gemv_mxfp4(dev(a).view(torch.bfloat16), dev(w), dev(sw), n, k, pa.F32))
+        assert pa.last_kernel() == "gemv_mxfp4_stream"
+    assert relerr(other, got) <= 1e-5
+    # what lies past a row's end is another row's: NaN scales there stay in their own output column
+    sw[n // 2] = 255
+    odd = host(pa.gemv_mxfp4(dev(a).view(torch.bfloat16), dev(w), dev(sw), n, k, pa.F32))
+    keep = np.arange(n) != n // 2
+    assert np.array_equal(odd[:, keep].view(np.uint32), got[:, keep].view(np.uint32)) and not np.isfinite(odd[:, n // 2]).any()
+
+
 def test_gemv_ragged_k_takes_the_generic_kernel(pa, oracle):
     r = np.random.default_rng(11)
     m, n, k = 3, 40, 96
