@@ -124,7 +124,8 @@ int ptoamd_event_elapsed_ms(float* ms, void* start, void* stop);
  *   relu    : flags: PTOAMD_RELU (1) = TSTORE's ReluPreMode::NormalRelu; PTOAMD_SATURATE_INF (2), quantising drains only
  * No alignment is asked of a, b or the leading dimensions beyond that of an element: rows of 16 bytes or more run on the
  * MFMA tiles whatever their alignment: the LDS-DMA kernels when rows start on 4-byte boundaries and K is a multiple of 4
- * bytes, the register-staged tiles otherwise; a row-major B is
+ * bytes, for bf16 / f16 / int8 rows on other bytes the deep-ring tiles with copies through registers, the register-staged
+ * tiles otherwise; a row-major B of 16-bit elements is read in place where its rows allow it (ptoamd_gemm_ws below) and else
  * transposed on its way into LDS by the latter.  Rows of C need no alignment either.
  * PTOAMD_F32 and PTOAMD_HIF8 operands (hif8 x hif8 only, cpu/TMatmul.hpp:38) run on the order-exact kernel: one thread
  * per output, k ascending, fmaf -- the simulator's arithmetic bit for bit.  No entry point of this group allocates.
