@@ -360,17 +360,48 @@ static const TileCost tile_costs[3][COST_COUNT] = {
     {{2.5f, 0.09f, 8.0f}, {2.1f, 0.15f, 8.0f}, {2.4f, 0.20f, 8.0f}, {3.1f, 0.235f, 5.0f}, {3.8f, 0.265f, 5.0f}, {4.5f, 0.25f, 5.3f},
      {5.0f, 0.40f, 5.5f}, {}, {}, {6.9f, 1.11f, 9.5f}, {4.2f, 0.56f, 6.7f}, {5.2f, 0.57f, 7.5f}},
 };
+// What a drain costs beside a plain one of f32, f16, bf16 or int32 values.  The deep-ring kernel drains every form in 16-byte
+// pieces, a two-slab tile some of them element by element, and an atomic addition of its 32x32 blocks touches 32 rows per
+// instruction where 16x16 blocks touch 16.  us per call, us per million elements of C, and us per call where the last columns
+// are no whole wave tile: the deep-ring kernel, the plain types' 256 x 256 tile (16x16 blocks), the tiles of 32x32 blocks.
+// Measured, on the 128 x 128 two-slab tile and on the kernel chosen now: a quantisation word per column, int8 3967 x 2560 x 320, 39
+// and 20 us; atomic additions, bf16 1981 x 7296 x 128, 355 and 180; raw accumulators, int8 17929 x 1700 x 376, 275 and 118.
+enum DrainKind { DRAIN_PLAIN, DRAIN_SCALES, DRAIN_WORD, DRAIN_COLUMN_WORDS, DRAIN_ACC_IN, DRAIN_RAW_ACC, DRAIN_ATOMIC, DRAIN_COUNT };
+enum { CLASS_RING, CLASS_256, CLASS_32X32, CLASS_COUNT };
+struct DrainCost {
+    float call[CLASS_COUNT], element[CLASS_COUNT], edge[CLASS_COUNT];
+};
+static const DrainCost drain_costs[DRAIN_COUNT] = {
+    {{0, 0, 0}, {0, 0, 0}, {0, 0, 0}},
+    {{0, 0, 0}, {0, 0, 0}, {0, 5.0f, 1.5f}},                     // W8A8: scales of rows and columns
+    {{0, 0, 2.0f}, {0, 0, 0}, {0, 5.0f, 1.5f}},                  // one quantisation word
+    {{0, 4.0f, 11.0f}, {0, 0, 2.4f}, {0, 5.0f, 1.5f}},           // one per column
+    {{0, 8.0f, 3.0f}, {0, 0, 0}, {0, 5.0f, 1.5f}},               // accumulator input
+    {{0, 6.0f, 6.0f}, {1.5f, 2.8f, 6.0f}, {0, 5.0f, 1.5f}},      // W8A8 with raw accumulators
+    {{0, 2.0f, 2.0f}, {12.5f, 12.5f, 25.0f}, {0, 5.0f, 1.5f}},   // atomic additions
+};
+// (the deep-ring kernel's scales and raw accumulators: us per round, and per round and 22000 elements of a tile)
+constexpr float RING_SCALES_ROUND = 0.5f, RING_SCALES_TILE = 22000.0f;
 constexpr int TILE_RING = 16;  // tile ids from here on: the deep-ring kernel's shapes
+
+// What the launcher may choose among.
+// dtl: which of the two- and three-slab tiles take the operands as well (K and, for block-scaled types, rows of scales they can
+// stream; a row-major B).  unaligned: rows that start on any byte, which the shapes with copying waves take in a form of their
+// own; its stages take 1.9 times as long (bf16 600 x 8001 x 2049: 47 us on 192 x 128, 62 on the 128 x 128 that the plain
+// estimate asks for).
+enum DtlTiles { DTL_NONE, DTL_256_ONLY, DTL_ALL };
+struct TileChoice {
+    DtlTiles dtl;
+    DrainKind drain;
+    bool unaligned;
+};
 
 // Block-scaled products of more than 64 rows keep away from the shapes that split K over groups of waves (0 .. 2): their sums
 // then run in k order and equal, bit for bit, those of the same product written in the tile ISA.
-// dtl: which of the two- and three-slab tiles take this operand as well (K and, for block-scaled types, rows of scales they can
-// stream; a row-major B)
-enum DtlTiles { DTL_NONE, DTL_256_ONLY, DTL_ALL };
-// unaligned: rows that start on any byte, which the shapes with copying waves take in a form of their own; its stages take 1.9
-// times as long (bf16 600 x 8001 x 2049: 47 us on 192 x 128, 62 on the 128 x 128 that the plain estimate asks for)
-static int pick_dma_tile(int m, int n, long k_bytes, int op, DtlTiles dtl, bool unaligned = false)
+static int pick_dma_tile(int m, int n, long k_bytes, int op, const TileChoice& choice)
 {
+    const DtlTiles dtl = choice.dtl;
+    const bool unaligned = choice.unaligned;
     const bool scaled = op >= TOP_FP8_E4E4;
     const int shapes = scaled ? RING_SHAPES_SCALED : RING_SHAPES;
     const int first = unaligned ? RING_FIRST_UNALIGNED : 0, form = unaligned ? RING_UNALIGNED : 0;
@@ -409,7 +440,12 @@ static int pick_dma_tile(int m, int n, long k_bytes, int op, DtlTiles dtl, bool 
             rounds = 1.45f * (float)whole + (rest == 0 ? 0.0f : rest <= cus ? 1.0f : 1.0f + 0.45f * (float)(rest - cus) / (float)cus);
         }
         const float full = (float)tiles * (float)(bm * bn) * 1e-6f / cost[c].rate;
-        const float us = 3.0f + rounds * cost[c].round + slabs * std::max(rounds * copying * cost[c].slab, full) * (c < RING_SHAPES ? 1.0f : ragged);
+        float us = 3.0f + rounds * cost[c].round + slabs * std::max(rounds * copying * cost[c].slab, full) * (c < RING_SHAPES ? 1.0f : ragged);
+        const int cl = c < RING_SHAPES ? CLASS_RING : c == COST_TILE4 && !scaled ? CLASS_256 : CLASS_32X32;
+        const DrainCost& drain = drain_costs[choice.drain];
+        us += drain.call[cl] + drain.element[cl] * (float)m * (float)n * 1e-6f + ((n % 64) != 0 ? drain.edge[cl] : 0.0f);
+        if (cl == CLASS_RING && (choice.drain == DRAIN_SCALES || choice.drain == DRAIN_RAW_ACC))
+            us += rounds * (RING_SCALES_ROUND + (float)(bm * bn) / RING_SCALES_TILE);
         if (us < best_us) {
             best_us = us;
             best = id;
@@ -755,7 +791,11 @@ static int gemm_common(void* c, int c_type, const void* a, const void* b, int ab
     const bool nd_ok = b_layout == PTOAMD_B_ND && ebytes == 2 && !options().b_nd_in_loader && options().tile < 0 && (n % 8) == 0 &&
                        aligned4(a) && aligned4(b) && (lda_b % 4) == 0 && (ldb_b % 4) == 0 && (k_bytes % 4) == 0 &&
                        dma_offsets_fit(m, RING_MAX_STAGE_BYTES / 2 + 8, lda_b, ldb_b, std::max(k_bytes, 2 * (long)n));
-    const int nd_tile = nd_ok ? pick_dma_tile(m, n, k_bytes, op, b_via_ws ? dtl_k : whole_slabs ? DTL_256_ONLY : DTL_NONE) : -1;
+    const DrainKind drain = atomic_add                 ? DRAIN_ATOMIC
+                            : qwords == nullptr        ? (c_in != nullptr ? DRAIN_ACC_IN : DRAIN_PLAIN)
+                            : q_per_column             ? DRAIN_COLUMN_WORDS
+                                                       : DRAIN_WORD;
+    const int nd_tile = nd_ok ? pick_dma_tile(m, n, k_bytes, op, {b_via_ws ? dtl_k : whole_slabs ? DTL_256_ONLY : DTL_NONE, drain, false}) : -1;
     const bool nd_direct = nd_tile >= TILE_RING || (nd_tile == 4 && whole_slabs);
     const uint8_t* b_kmajor = reinterpret_cast<const uint8_t*>(b);
     long ldb_kmajor = ldb_b;
@@ -786,8 +826,8 @@ static int gemm_common(void* c, int c_type, const void* a, const void* b, int ab
     // register-staged tiles, or as fast, at all of 54 sizes, m 7 .. 4000, n 1001 .. 8001, k 1023 .. 4097: 1.0 to 2.2 times)
     const bool any_ok = ragged_k_form && !b_in_kernel && !dma_ok && k_bytes >= 16 && dma_offsets_fit(m, n, lda_b, ldb_kmajor, k_bytes);
     const int tile = nd_direct ? nd_tile
-                     : options().tile < 0 && dma_ok && (k_bytes % 4) == 0 ? pick_dma_tile(m, n, k_bytes, op, dtl_k)
-                     : options().tile < 0 && any_ok ? pick_dma_tile(m, n, k_bytes, op, DTL_NONE, true)
+                     : options().tile < 0 && dma_ok && (k_bytes % 4) == 0 ? pick_dma_tile(m, n, k_bytes, op, {dtl_k, drain, false})
+                     : options().tile < 0 && any_ok ? pick_dma_tile(m, n, k_bytes, op, {DTL_NONE, drain, true})
                                                     : pick_tile(m, n, k_bytes, false, false, dma_ok, ragged_k_form);
     PTOAMD_HIP_CHECK(launch_tiles(tile, op, p, stream));
     set_last_kernel(tile_kernel_name(tile_as_launched(tile, op, m, n), op, nd_direct));
@@ -826,9 +866,10 @@ int ptoamd_gemm_w8a8(void* out_bf16, int32_t* acc_out, const int8_t* a, const in
     p.out_kind = OUT_W8A8_BF16; p.group_m = 4;
     p.b_nd = b_in_kernel; p.b_esz = 1;
     const bool dma_ok = !b_in_kernel && aligned4(a) && aligned4(b) && (lda % 4) == 0 && (ldb % 4) == 0 && dma_offsets_fit(m, n, lda, ldb, k);
+    const DrainKind drain = acc_out ? DRAIN_RAW_ACC : DRAIN_SCALES;
     const bool any_ok = !b_in_kernel && !dma_ok && k >= 16 && dma_offsets_fit(m, n, lda, ldb, k);
-    const int tile = options().tile < 0 && dma_ok && (k % 4) == 0 ? pick_dma_tile(m, n, k, TOP_I8, (k % 128) == 0 || k > 128 ? DTL_ALL : DTL_NONE)
-                     : options().tile < 0 && any_ok ? pick_dma_tile(m, n, k, TOP_I8, DTL_NONE, true)
+    const int tile = options().tile < 0 && dma_ok && (k % 4) == 0 ? pick_dma_tile(m, n, k, TOP_I8, {(k % 128) == 0 || k > 128 ? DTL_ALL : DTL_NONE, drain, false})
+                     : options().tile < 0 && any_ok ? pick_dma_tile(m, n, k, TOP_I8, {DTL_NONE, drain, true})
                                                     : pick_tile(m, n, k, false, false, dma_ok, true);
     PTOAMD_HIP_CHECK(launch_tiles(tile, TOP_I8, p, stream));
     set_last_kernel(tile_kernel_name(tile, TOP_I8));
@@ -974,7 +1015,7 @@ static int gemm_mx_common(const char* who, void* c, int c_type, const void* a, c
     // (the deep-ring kernel fetches them as dwords: any K that is a multiple of 128, which the row-length check above asks for)
     const bool dma_ok = !e1m2 && plain_scales && !b_in_kernel && dma_offsets_fit(m, n, lda_b, ldb_b, k_bytes);
     const int tile = e1m2 ? pick_tile(m, n, k, true, false, false)
-                     : options().tile < 0 && dma_ok && (kg % 4) == 0 ? pick_dma_tile(m, n, k_bytes, op, scale_dma_ok ? DTL_ALL : DTL_NONE)
+                     : options().tile < 0 && dma_ok && (kg % 4) == 0 ? pick_dma_tile(m, n, k_bytes, op, {scale_dma_ok ? DTL_ALL : DTL_NONE, c_in ? DRAIN_ACC_IN : DRAIN_PLAIN, false})
                                                                     : pick_tile(m, n, k_bytes, true, a4, dma_ok && scale_dma_ok);
     PTOAMD_HIP_CHECK(launch_tiles(tile, op, p, stream));
     set_last_kernel(tile_kernel_name(tile_as_launched(tile, op, m, n), op));

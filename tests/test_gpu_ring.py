@@ -169,3 +169,25 @@ def test_store_forms(pa, oracle, shape):  # noqa: F811
     assert np.array_equal(host(summed), (acc.astype(np.int64) + cin).astype(np.int32))
     assert np.array_equal(host(wide)[:, :n], oracle.store_f32(f32, ob.ST_BF16))
     assert bool((wide[:, n:] == 7.0).all())
+
+
+@pytest.mark.parametrize("drain,m,n,k", [("column words", 3967, 2560, 320), ("column words", 1324, 6144, 168), ("raw", 3788, 3968, 384), ("atomic", 1981, 7296, 128)])
+def test_drains_keep_off_the_two_slab_128x128_tile(pa, drain, m, n, k):  # noqa: F811
+    """Drains that the 128 x 128 tile stores element by element (a quantisation word per column, raw accumulators, atomic
+    additions) run on a kernel that does not, where both are candidates; the whole numbers are exact."""
+    gen = torch.Generator(device="cuda").manual_seed(n)
+    a, b = (torch.randint(-8, 9, (x, k), generator=gen, device="cuda", dtype=torch.int8) for x in (m, n))
+    acc = (a.double() @ b.double().t()).to(torch.int32)
+    if drain == "column words":  # scale 2^-4, no offset, signed bytes
+        words = torch.full((n,), (int(np.float32(2.0 ** -4).view(np.uint32)) & 0xFFFFE000) | (1 << 46), dtype=torch.int64, device="cuda")
+        got = pa.gemm_requant(a, b, pa.I8, pa.I8, words, per_column=True)
+        ref = torch.round(acc.double() / 16).clamp(-128, 127).to(torch.int8)
+    elif drain == "raw":
+        ones = torch.ones(max(m, n), device="cuda")
+        got, ref = pa.gemm_w8a8(a, b, ones[:m], ones[:n], want_acc=True)[1], acc
+    else:
+        got = torch.ones((m, n), device="cuda")
+        pa.gemm_atomic_add(got, a.bfloat16(), b.bfloat16(), pa.BF16)
+        ref = acc.float() + 1
+    assert not pa.last_kernel().startswith("tile128x128_dtl"), pa.last_kernel()
+    assert torch.equal(got, ref)
