@@ -348,8 +348,8 @@ struct TileCost {
     float round, slab;  // us per round; us per round and slab
     float rate;         // million elements of C times slabs per us
 };
-enum { COST_TILE4 = RING_SHAPES, COST_TILE5, COST_TILE7, COST_COUNT };
-static const TileCost tile_costs[3][COST_COUNT] = {
+enum { COST_TILE4 = RING_SHAPES, COST_TILE5, COST_TILE7, COST_TILE2, COST_TILE1, COST_COUNT };
+static const TileCost tile_costs[3][COST_TILE2] = {
     // plain types: 32x16, 32x32, 64x32, 64x64, 96x64, 128x64, 128x128, 192x128, 256x128; 256x256, 128x128 (two a CU), -
     {{2.2f, 0.0625f, 8.0f}, {2.0f, 0.086f, 8.0f}, {2.6f, 0.125f, 8.0f}, {2.9f, 0.165f, 7.0f}, {3.2f, 0.19f, 7.0f}, {3.6f, 0.20f, 6.3f},
      {4.7f, 0.29f, 8.0f}, {5.5f, 0.385f, 8.1f}, {6.0f, 0.49f, 7.8f}, {11.0f, 1.1f, 12.0f}, {2.9f, 0.545f, 6.6f}, {}},
@@ -360,40 +360,64 @@ static const TileCost tile_costs[3][COST_COUNT] = {
     {{2.5f, 0.09f, 8.0f}, {2.1f, 0.15f, 8.0f}, {2.4f, 0.20f, 8.0f}, {3.1f, 0.235f, 5.0f}, {3.8f, 0.265f, 5.0f}, {4.5f, 0.25f, 5.3f},
      {5.0f, 0.40f, 5.5f}, {}, {}, {6.9f, 1.11f, 9.5f}, {4.2f, 0.56f, 6.7f}, {5.2f, 0.57f, 7.5f}},
 };
+// A register-staged tile keeps several workgroups on a CU, starts with one slab where the deep ring fills its stages, and stores
+// while others multiply, so it is ahead where K is a few slabs: bf16 125 x 2624 x 64 3.8 us (deep ring 4.4), 3313 x 16112 x 56
+// 41 (53).  On rows that start on any byte it stays ahead longer, the deep ring's copies going through registers there as well:
+// 117 x 888 x 49 5.2 (8.3); with K whole 16-byte chunks, 4633 x 10496 x 512 94 (131).  us per call, per slab, per round of 64 x 64
+// or 128 x 128 tiles over the CUs (however full), and per round and slab; then what rows add that do not end on 16 bytes.  The
+// calls' constants are set against the deep ring's estimate, which is 1 to 2 us high for a few slabs, and are as much too high.
+struct StagedCost {
+    float call, slab, round, round_slab, ragged_call, ragged_slab, ragged_round_slab;
+};
+enum { STAGED_FP8 = 1, STAGED_FP4, STAGED_ROW_MAJOR, STAGED_UNALIGNED, STAGED_ROWS };  // 0: plain types
+static const StagedCost staged_costs[STAGED_ROWS][2] = {
+    {{4.6f, 0.48f, 0.74f, 0.15f, 1.4f, 0.25f, 0.12f}, {7.0f, 0.92f, 2.3f, 0.39f, 2.1f, 0.36f, 0.93f}},
+    {{4.6f, 0.55f, 0.63f, 0.2f, 1.9f, 0, 0.62f}, {}},
+    {{4.75f, 0.52f, 0.63f, 0.18f, 0, 0, 0}, {}},
+    {{4.6f, 0.58f, 0.44f, 0.6f, 3.9f, 0.1f, 0.2f}, {6.8f, 1.0f, 2.15f, 0.7f, 3.8f, 0.1f, 0.3f}},
+    {{4.25f, 0.56f, 0.79f, 0.2f, 0.75f, 0.2f, 0.11f}, {6.1f, 0.81f, 2.9f, 0.36f, 2.1f, 0.5f, 0.83f}},
+};
+// Beyond these many slabs they are never ahead of everything else.
+constexpr int STAGED_SLABS = 8, STAGED_SLABS_SCALED = 2, STAGED_SLABS_UNALIGNED = 16;
+
 // What a drain costs beside a plain one of f32, f16, bf16 or int32 values.  The deep-ring kernel drains every form in 16-byte
-// pieces, a two-slab tile some of them element by element, and an atomic addition of its 32x32 blocks touches 32 rows per
+// pieces, the other tiles some of them element by element, and an atomic addition of 32x32 blocks touches 32 rows per
 // instruction where 16x16 blocks touch 16.  us per call, us per million elements of C, and us per call where the last columns
-// are no whole wave tile: the deep-ring kernel, the plain types' 256 x 256 tile (16x16 blocks), the tiles of 32x32 blocks.
+// are no whole wave tile: the deep-ring kernel, the plain types' 256 x 256 tile (16x16 blocks), the two-slab tiles of 32x32
+// blocks, the 64 x 64 and the 128 x 128 register-staged tile.
 // Measured, on the 128 x 128 two-slab tile and on the kernel chosen now: a quantisation word per column, int8 3967 x 2560 x 320, 39
 // and 20 us; atomic additions, bf16 1981 x 7296 x 128, 355 and 180; raw accumulators, int8 17929 x 1700 x 376, 275 and 118.
 enum DrainKind { DRAIN_PLAIN, DRAIN_SCALES, DRAIN_WORD, DRAIN_COLUMN_WORDS, DRAIN_ACC_IN, DRAIN_RAW_ACC, DRAIN_ATOMIC, DRAIN_COUNT };
-enum { CLASS_RING, CLASS_256, CLASS_32X32, CLASS_COUNT };
+enum { CLASS_RING, CLASS_256, CLASS_32X32, CLASS_STAGED_64, CLASS_STAGED_128, CLASS_COUNT };
 struct DrainCost {
     float call[CLASS_COUNT], element[CLASS_COUNT], edge[CLASS_COUNT];
 };
 static const DrainCost drain_costs[DRAIN_COUNT] = {
-    {{0, 0, 0}, {0, 0, 0}, {0, 0, 0}},
-    {{0, 0, 0}, {0, 0, 0}, {0, 5.0f, 1.5f}},                     // W8A8: scales of rows and columns
-    {{0, 0, 2.0f}, {0, 0, 0}, {0, 5.0f, 1.5f}},                  // one quantisation word
-    {{0, 4.0f, 11.0f}, {0, 0, 2.4f}, {0, 5.0f, 1.5f}},           // one per column
-    {{0, 8.0f, 3.0f}, {0, 0, 0}, {0, 5.0f, 1.5f}},               // accumulator input
-    {{0, 6.0f, 6.0f}, {1.5f, 2.8f, 6.0f}, {0, 5.0f, 1.5f}},      // W8A8 with raw accumulators
-    {{0, 2.0f, 2.0f}, {12.5f, 12.5f, 25.0f}, {0, 5.0f, 1.5f}},   // atomic additions
+    {{0, 0, 0, 0, 0}, {0, 0, 0, 0, 0}, {0, 0, 0, 0.3f, 0.3f}},
+    {{0, 0, 0, 0, 0}, {0, 0, 0, 0, 0}, {0, 5.0f, 1.5f, 1.2f, 1.2f}},                                  // W8A8: scales of rows and columns
+    {{0, 0, 2.0f, 0.4f, 3.0f}, {0, 0, 0, 0, 0}, {0, 5.0f, 1.5f, 1.2f, 1.2f}},                         // one quantisation word
+    {{0, 4.0f, 11.0f, 2.1f, 12.0f}, {0, 0, 2.4f, 0.7f, 2.4f}, {0, 5.0f, 1.5f, 1.2f, 1.2f}},           // one per column
+    {{0, 8.0f, 1.0f, 0.8f, 3.2f}, {0, 0, 0, 0, 0}, {0, 5.0f, 1.5f, 1.2f, 1.2f}},                      // accumulator input
+    {{0, 6.0f, 6.0f, 2.7f, 6.0f}, {1.5f, 2.8f, 6.0f, 6.0f, 6.0f}, {0, 5.0f, 1.5f, 1.2f, 1.2f}},       // W8A8 with raw accumulators
+    {{0, 2.0f, 2.0f, 2.4f, 5.5f}, {12.5f, 12.5f, 25.0f, 25.0f, 25.0f}, {0, 5.0f, 1.5f, 1.2f, 1.2f}},  // atomic additions
 };
-// (the deep-ring kernel's scales and raw accumulators: us per round, and per round and 22000 elements of a tile)
-constexpr float RING_SCALES_ROUND = 0.5f, RING_SCALES_TILE = 22000.0f;
+// (the deep-ring kernel's scales and raw accumulators: us per round, and per round and 22000 elements of a tile; its words per
+// column, raw accumulators and atomic additions behind unaligned rows: us per call)
+constexpr float RING_SCALES_ROUND = 0.5f, RING_SCALES_TILE = 22000.0f, RING_UNALIGNED_DRAIN = 2.5f;
 constexpr int TILE_RING = 16;  // tile ids from here on: the deep-ring kernel's shapes
 
 // What the launcher may choose among.
 // dtl: which of the two- and three-slab tiles take the operands as well (K and, for block-scaled types, rows of scales they can
 // stream; a row-major B).  unaligned: rows that start on any byte, which the shapes with copying waves take in a form of their
-// own; its stages take 1.9 times as long (bf16 600 x 8001 x 2049: 47 us on 192 x 128, 62 on the 128 x 128 that the plain
-// estimate asks for).
+// own; its rounds and stages take 1.9 times as long (bf16 600 x 8001 x 2049: 47 us on 192 x 128, 62 on the 128 x 128 that the
+// plain estimate asks for).  staged: which register-staged tiles are candidates for a short K, by the state B is in for them.
 enum DtlTiles { DTL_NONE, DTL_256_ONLY, DTL_ALL };
+enum StagedTiles { STAGED_NONE, STAGED_COLUMN_MAJOR_B, STAGED_ROW_MAJOR_B };
 struct TileChoice {
     DtlTiles dtl;
     DrainKind drain;
     bool unaligned;
+    StagedTiles staged;
 };
 
 // Block-scaled products of more than 64 rows keep away from the shapes that split K over groups of waves (0 .. 2): their sums
@@ -413,39 +437,59 @@ static int pick_dma_tile(int m, int n, long k_bytes, int op, const TileChoice& c
     // is left over (4096 x 4312: 192 x 128 tiles 79 against 87 us at K = 2048).
     if (dtl != DTL_NONE && (long)((m + 255) / 256) * ((n + 255) / 256) >= device_compute_units())
         return 4;
-    const TileCost* cost = tile_costs[op == TOP_FP4 ? 2 : (scaled ? 1 : 0)];
+    const int type = op == TOP_FP4 ? STAGED_FP4 : (scaled ? STAGED_FP8 : 0);
+    const TileCost* cost = tile_costs[type];
+    const StagedCost* staged = staged_costs[choice.staged == STAGED_ROW_MAJOR_B ? STAGED_ROW_MAJOR : unaligned ? STAGED_UNALIGNED : type];
+    const DrainCost& drain = drain_costs[choice.drain];
     const int cus = device_compute_units();
-    const float slabs = (float)((k_bytes + 127) / 128);
+    const long slab_count = (k_bytes + 127) / 128;
+    const float slabs = (float)slab_count;
+    const bool staged_ok = choice.staged != STAGED_NONE && slab_count <= (scaled ? STAGED_SLABS_SCALED : unaligned ? STAGED_SLABS_UNALIGNED : STAGED_SLABS);
     // (a K that is no whole number of slabs costs the two-slab tiles half as much again: bf16 1280 x 4096, K 2048: 24.8 us,
     // K 2056: 38.4 us)
     const float ragged = (k_bytes % 128) != 0 ? 1.5f : 1.0f;
     int best = TILE_RING;
     float best_us = 1e30f;
     for (int c = 0; c < COST_COUNT; ++c) {
-        if (c < RING_SHAPES ? c >= shapes : (dtl == DTL_NONE || (dtl == DTL_256_ONLY && c != COST_TILE4) || (c == COST_TILE7 && !scaled)))
+        static const int ids[COST_COUNT - RING_SHAPES] = {4, 5, 7, 2, 1};
+        const bool ring = c < RING_SHAPES, in_registers = c >= COST_TILE2;
+        if (ring           ? c >= shapes || c < first || (scaled && c <= 2 && m > 64)
+            : in_registers ? !staged_ok || (c == COST_TILE1 && scaled)
+                           : dtl == DTL_NONE || (dtl == DTL_256_ONLY && c != COST_TILE4) || (c == COST_TILE7 && !scaled))
             continue;
-        if ((scaled && c <= 2 && m > 64) || c < first)
-            continue;
-        static const int ids[3] = {4, 5, 7};
-        const int id = c < RING_SHAPES ? TILE_RING + form + c : ids[c - RING_SHAPES];
+        const int id = ring ? TILE_RING + form + c : ids[c - RING_SHAPES];
         int bm, bn;
-        if (c < RING_SHAPES)
+        if (ring)
             ring_shape(c, &bm, &bn);
         else
             tile_shape(id, &bm, &bn);
         const long tiles = (long)((m + bm - 1) / bm) * ((n + bn - 1) / bn);
-        float rounds = (float)((tiles + cus - 1) / cus);
-        if (c == COST_TILE5) {  // two workgroups share a CU: the second adds 0.45 of the first one's time
-            const long whole = tiles / (2 * cus), rest = tiles % (2 * cus);
-            rounds = 1.45f * (float)whole + (rest == 0 ? 0.0f : rest <= cus ? 1.0f : 1.0f + 0.45f * (float)(rest - cus) / (float)cus);
+        float us;
+        if (in_registers) {
+            const StagedCost& s = staged[c - COST_TILE2];
+            const float rounds = (float)tiles / (float)cus;
+            us = s.call + slabs * s.slab + rounds * (s.round + slabs * s.round_slab);
+            if (k_bytes % 16 != 0)
+                us += s.ragged_call + slabs * (s.ragged_slab + rounds * s.ragged_round_slab);
+        } else {
+            float rounds = (float)((tiles + cus - 1) / cus);
+            if (c == COST_TILE5) {  // two workgroups share a CU: the second adds 0.45 of the first one's time
+                const long whole = tiles / (2 * cus), rest = tiles % (2 * cus);
+                rounds = 1.45f * (float)whole + (rest == 0 ? 0.0f : rest <= cus ? 1.0f : 1.0f + 0.45f * (float)(rest - cus) / (float)cus);
+            }
+            const float full = (float)tiles * (float)(bm * bn) * 1e-6f / cost[c].rate;
+            us = 3.0f + rounds * copying * cost[c].round + slabs * std::max(rounds * copying * cost[c].slab, full) * (ring ? 1.0f : ragged);
+            if (ring && (choice.drain == DRAIN_SCALES || choice.drain == DRAIN_RAW_ACC))
+                us += rounds * (RING_SCALES_ROUND + (float)(bm * bn) / RING_SCALES_TILE);
+            if (unaligned && (choice.drain == DRAIN_COLUMN_WORDS || choice.drain == DRAIN_RAW_ACC || choice.drain == DRAIN_ATOMIC))
+                us += RING_UNALIGNED_DRAIN;
         }
-        const float full = (float)tiles * (float)(bm * bn) * 1e-6f / cost[c].rate;
-        float us = 3.0f + rounds * cost[c].round + slabs * std::max(rounds * copying * cost[c].slab, full) * (c < RING_SHAPES ? 1.0f : ragged);
-        const int cl = c < RING_SHAPES ? CLASS_RING : c == COST_TILE4 && !scaled ? CLASS_256 : CLASS_32X32;
-        const DrainCost& drain = drain_costs[choice.drain];
+        const int cl = ring                           ? CLASS_RING
+                       : c == COST_TILE2              ? CLASS_STAGED_64
+                       : c == COST_TILE1              ? CLASS_STAGED_128
+                       : (c == COST_TILE4 && !scaled) ? CLASS_256
+                                                      : CLASS_32X32;
         us += drain.call[cl] + drain.element[cl] * (float)m * (float)n * 1e-6f + ((n % 64) != 0 ? drain.edge[cl] : 0.0f);
-        if (cl == CLASS_RING && (choice.drain == DRAIN_SCALES || choice.drain == DRAIN_RAW_ACC))
-            us += rounds * (RING_SCALES_ROUND + (float)(bm * bn) / RING_SCALES_TILE);
         if (us < best_us) {
             best_us = us;
             best = id;
@@ -787,7 +831,8 @@ static int gemm_common(void* c, int c_type, const void* a, const void* b, int ab
     // A row-major B of 16-bit elements is read as it is by the deep-ring kernel and, over whole slabs, by the 256 x 256 tile,
     // transposed on its way out of LDS (its rows have to be whole 16-byte chunks; a column chunk past N is fetched from the
     // row's last one).  With a workspace the tile is the one that the same product takes with a column-major B, so that both
-    // have the same bits; where that tile has no row-major form, B is re-ordered for it.
+    // have the same bits; where that tile has no row-major form, B is re-ordered for it.  (Register-staged tiles are left out with
+    // a workspace: they run a few slabs of K, for which the re-ordering launch costs more than they save.)
     const bool nd_ok = b_layout == PTOAMD_B_ND && ebytes == 2 && !options().b_nd_in_loader && options().tile < 0 && (n % 8) == 0 &&
                        aligned4(a) && aligned4(b) && (lda_b % 4) == 0 && (ldb_b % 4) == 0 && (k_bytes % 4) == 0 &&
                        dma_offsets_fit(m, RING_MAX_STAGE_BYTES / 2 + 8, lda_b, ldb_b, std::max(k_bytes, 2 * (long)n));
@@ -795,7 +840,7 @@ static int gemm_common(void* c, int c_type, const void* a, const void* b, int ab
                             : qwords == nullptr        ? (c_in != nullptr ? DRAIN_ACC_IN : DRAIN_PLAIN)
                             : q_per_column             ? DRAIN_COLUMN_WORDS
                                                        : DRAIN_WORD;
-    const int nd_tile = nd_ok ? pick_dma_tile(m, n, k_bytes, op, {b_via_ws ? dtl_k : whole_slabs ? DTL_256_ONLY : DTL_NONE, drain, false}) : -1;
+    const int nd_tile = nd_ok ? pick_dma_tile(m, n, k_bytes, op, {b_via_ws ? dtl_k : whole_slabs ? DTL_256_ONLY : DTL_NONE, drain, false, b_via_ws ? STAGED_NONE : STAGED_ROW_MAJOR_B}) : -1;
     const bool nd_direct = nd_tile >= TILE_RING || (nd_tile == 4 && whole_slabs);
     const uint8_t* b_kmajor = reinterpret_cast<const uint8_t*>(b);
     long ldb_kmajor = ldb_b;
@@ -825,9 +870,9 @@ static int gemm_common(void* c, int c_type, const void* a, const void* b, int ab
     // rows that start on other bytes, at least one chunk long: the deep-ring kernel's copies through registers (faster than the
     // register-staged tiles, or as fast, at all of 54 sizes, m 7 .. 4000, n 1001 .. 8001, k 1023 .. 4097: 1.0 to 2.2 times)
     const bool any_ok = ragged_k_form && !b_in_kernel && !dma_ok && k_bytes >= 16 && dma_offsets_fit(m, n, lda_b, ldb_kmajor, k_bytes);
-    const int tile = nd_direct ? nd_tile
-                     : options().tile < 0 && dma_ok && (k_bytes % 4) == 0 ? pick_dma_tile(m, n, k_bytes, op, {dtl_k, drain, false})
-                     : options().tile < 0 && any_ok ? pick_dma_tile(m, n, k_bytes, op, {DTL_NONE, drain, true})
+    const int tile = nd_direct || (nd_tile >= 0 && b_in_kernel) ? nd_tile
+                     : options().tile < 0 && dma_ok && (k_bytes % 4) == 0 ? pick_dma_tile(m, n, k_bytes, op, {dtl_k, drain, false, nd_ok ? STAGED_NONE : STAGED_COLUMN_MAJOR_B})
+                     : options().tile < 0 && any_ok ? pick_dma_tile(m, n, k_bytes, op, {DTL_NONE, drain, true, STAGED_COLUMN_MAJOR_B})
                                                     : pick_tile(m, n, k_bytes, false, false, dma_ok, ragged_k_form);
     PTOAMD_HIP_CHECK(launch_tiles(tile, op, p, stream));
     set_last_kernel(tile_kernel_name(tile_as_launched(tile, op, m, n), op, nd_direct));
@@ -868,8 +913,8 @@ int ptoamd_gemm_w8a8(void* out_bf16, int32_t* acc_out, const int8_t* a, const in
     const bool dma_ok = !b_in_kernel && aligned4(a) && aligned4(b) && (lda % 4) == 0 && (ldb % 4) == 0 && dma_offsets_fit(m, n, lda, ldb, k);
     const DrainKind drain = acc_out ? DRAIN_RAW_ACC : DRAIN_SCALES;
     const bool any_ok = !b_in_kernel && !dma_ok && k >= 16 && dma_offsets_fit(m, n, lda, ldb, k);
-    const int tile = options().tile < 0 && dma_ok && (k % 4) == 0 ? pick_dma_tile(m, n, k, TOP_I8, {(k % 128) == 0 || k > 128 ? DTL_ALL : DTL_NONE, drain, false})
-                     : options().tile < 0 && any_ok ? pick_dma_tile(m, n, k, TOP_I8, {DTL_NONE, drain, true})
+    const int tile = options().tile < 0 && dma_ok && (k % 4) == 0 ? pick_dma_tile(m, n, k, TOP_I8, {(k % 128) == 0 || k > 128 ? DTL_ALL : DTL_NONE, drain, false, STAGED_COLUMN_MAJOR_B})
+                     : options().tile < 0 && any_ok ? pick_dma_tile(m, n, k, TOP_I8, {DTL_NONE, drain, true, STAGED_COLUMN_MAJOR_B})
                                                     : pick_tile(m, n, k, false, false, dma_ok, true);
     PTOAMD_HIP_CHECK(launch_tiles(tile, TOP_I8, p, stream));
     set_last_kernel(tile_kernel_name(tile, TOP_I8));
@@ -1015,7 +1060,7 @@ static int gemm_mx_common(const char* who, void* c, int c_type, const void* a, c
     // (the deep-ring kernel fetches them as dwords: any K that is a multiple of 128, which the row-length check above asks for)
     const bool dma_ok = !e1m2 && plain_scales && !b_in_kernel && dma_offsets_fit(m, n, lda_b, ldb_b, k_bytes);
     const int tile = e1m2 ? pick_tile(m, n, k, true, false, false)
-                     : options().tile < 0 && dma_ok && (kg % 4) == 0 ? pick_dma_tile(m, n, k_bytes, op, {scale_dma_ok ? DTL_ALL : DTL_NONE, c_in ? DRAIN_ACC_IN : DRAIN_PLAIN, false})
+                     : options().tile < 0 && dma_ok && (kg % 4) == 0 ? pick_dma_tile(m, n, k_bytes, op, {scale_dma_ok ? DTL_ALL : DTL_NONE, c_in ? DRAIN_ACC_IN : DRAIN_PLAIN, false, STAGED_COLUMN_MAJOR_B})
                                                                     : pick_tile(m, n, k_bytes, true, a4, dma_ok && scale_dma_ok);
     PTOAMD_HIP_CHECK(launch_tiles(tile, op, p, stream));
     set_last_kernel(tile_kernel_name(tile_as_launched(tile, op, m, n), op));

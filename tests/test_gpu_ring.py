@@ -191,3 +191,27 @@ def test_drains_keep_off_the_two_slab_128x128_tile(pa, drain, m, n, k):  # noqa:
         ref = acc.float() + 1
     assert not pa.last_kernel().startswith("tile128x128_dtl"), pa.last_kernel()
     assert torch.equal(got, ref)
+
+
+@pytest.mark.parametrize("kind,m,n,k,pitch,kernel", [
+    ("bf16", 117, 888, 49, 49, "tile64x64_bf16"), ("bf16", 1609, 448, 280, 281, "tile64x64_bf16"), ("bf16", 4633, 10496, 512, 513, "tile128x128_bf16"),
+    ("bf16", 125, 2624, 64, 64, "tile64x64_bf16"), ("i8", 69, 68, 34, 34, "tile64x64_i8"), ("i8", 1609, 448, 560, 561, "tile64x64_i8"),
+    ("bf16", 64, 4097, 4095, 4095, "tile64x64_any_bf16"), ("bf16", 125, 2624, 1024, 1024, "tile64x32_dtl_bf16")])
+def test_short_k_runs_on_the_register_staged_tiles(pa, kind, m, n, k, pitch, kernel):  # noqa: F811
+    """A few slabs of K, rows on any byte (odd K; whole chunks of K at an odd pitch) and aligned, keep the register-staged tiles;
+    longer ones take the deep-ring kernel.  Exact products of small whole numbers."""
+    tdt, t, tc = (torch.int8, pa.I8, pa.I32) if kind == "i8" else (torch.bfloat16, pa.BF16, pa.F32)
+    gen = torch.Generator(device="cuda").manual_seed(k)
+    a, b = (torch.randint(-3, 4, (x, pitch), generator=gen, device="cuda").to(tdt) for x in (m, n))
+    got = pa.gemm(a, b, t, tc, pa.B_DN, k=k)
+    assert pa.last_kernel() == kernel, pa.last_kernel()
+    assert torch.equal(got.double(), a[:, :k].double() @ b[:, :k].double().t())
+
+
+def test_short_k_block_scaled_products_run_on_the_register_staged_tile(pa, oracle):  # noqa: F811
+    r = np.random.default_rng(3)
+    m, n, k = 105, 256, 256
+    a, b, sa, sb = _mx_inputs(r, ob.E2M1, m, n, k)
+    got = host(pa.gemm_mx(dev(a), dev(b), dev(sa), dev(sb), m, n, k, pa.E2M1, pa.E2M1, pa.F32))
+    assert pa.last_kernel() == "tile64x64_fp4_e2m1", pa.last_kernel()
+    assert relerr(got, oracle.matmul_mx(a, b, sa, sb, m, k, n, ob.E2M1, ob.E2M1)) <= 1e-4
