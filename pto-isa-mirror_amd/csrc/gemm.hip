@@ -503,7 +503,7 @@ static int pick_dma_tile(int m, int n, long k_bytes, int op, const TileChoice& c
 // one workgroup per CU, same wave tile as the large form) or 128x128 tiles (two workgroups per CU); a tile of the tail
 // then costs a half or a quarter of a 256x256 tile's time instead of a whole round (MXFP8 4096 x 14336 x 4096, 3.5
 // rounds of 256 CUs).  PTOAMD_TILE (an explicit tile) and PTOAMD_NO_TAIL_SPLIT=1 switch the split off;
-// PTOAMD_TAIL_TILE=5|6|7 picks the tail's tile (default: 7 for the block-scaled types, the deep-ring 128 x 128 one otherwise).
+// PTOAMD_TAIL_TILE=5|6|7 picks the tail's tile (default: 7 for the block-scaled types, the deep-ring 128 x 128 one or 5 otherwise).
 static hipError_t launch_tiles_as(int tile, int op, const TileGemmParams& p, hipStream_t stream)
 {
     if ((tile == 4 || tile == 3) && options().tile < 0 && !options().no_tail_split) {
@@ -550,9 +550,16 @@ static hipError_t launch_tiles_as(int tile, int op, const TileGemmParams& p, hip
                 tail.qwords = p.qwords + n1;
             // block-scaled types: the 256 x 128 tile with the three-slab ring unless a tail tile was asked for
             // plain types: the deep-ring kernel's 128 x 128 shape, which also reads a row-major B (bf16 4096 x 4312 x 2048: 76.8
-            // us, with tile 5 84.4); its last chunk of K starts on a dword
+            // us, with tile 5 84.4); its last chunk of K starts on a dword.  It has one workgroup on a CU where tile 5 has two: where
+            // it would take a second round tile 5 is ahead (bf16 943 x 22144 x 3168: 125 us, with a second round 134), and at a
+            // few slabs of K with W8A8's scales, which end each of its rounds late (1536 x 12416 x 384: 20 against 23 us).  Not with the
+            // drains that tile 5 stores element by element (drain_costs).
             const bool scaled_op = op >= TOP_FP8_E4E4;
-            if (p.b_nd || (!scaled_op && options().tail_tile == 0 && (p.k_bytes % 4) == 0))
+            const bool one_round = (long)((tail.m + 127) / 128) * ((tail.n + 127) / 128) <= cus;
+            const bool late_drain = p.out_kind == OUT_W8A8_BF16 && p.k_bytes <= 4 * 128;
+            const bool by_element = p.atomic_add || p.acc_out != nullptr || (p.qwords != nullptr && p.q_per_column);
+            const bool ring_ok = !scaled_op && options().tail_tile == 0 && (p.k_bytes % 4) == 0;
+            if (p.b_nd || (ring_ok && (by_element || (one_round && !late_drain))))
                 return launch_gemm_ring(RING_SHAPE_128X128, op, tail, stream);
             return launch_gemm_tile(options().tail_tile > 0 ? options().tail_tile : (scaled_op ? 7 : 5), op, tail, stream);
         }

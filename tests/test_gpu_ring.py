@@ -215,3 +215,21 @@ def test_short_k_block_scaled_products_run_on_the_register_staged_tile(pa, oracl
     got = host(pa.gemm_mx(dev(a), dev(b), dev(sa), dev(sb), m, n, k, pa.E2M1, pa.E2M1, pa.F32))
     assert pa.last_kernel() == "tile64x64_fp4_e2m1", pa.last_kernel()
     assert relerr(got, oracle.matmul_mx(a, b, sa, sb, m, k, n, ob.E2M1, ob.E2M1)) <= 1e-4
+
+
+@pytest.mark.parametrize("m,n,k,scales", [(943, 22144, 96, False), (1536, 12416, 384, True), (1536, 12416, 644, True), (4096, 4312, 64, False)])
+def test_tail_columns_on_either_kernel(pa, m, n, k, scales):  # noqa: F811
+    """Tail columns of a 256 x 256 grid that make more than a round of 128 x 128 tiles, W8A8 ones below and above the K from which
+    the deep-ring kernel takes them, and a narrow last column: the bits of the single launch."""
+    gen = torch.Generator(device="cuda").manual_seed(k)
+    if scales:
+        a, b = (torch.randint(-128, 128, (x, k), generator=gen, device="cuda", dtype=torch.int8) for x in (m, n))
+        sa, sb = (torch.rand(x, generator=gen, device="cuda") for x in (m, n))
+        run = lambda: pa.gemm_w8a8(a, b, sa, sb)  # noqa: E731
+    else:  # whole numbers: exact in any order
+        a, b = (torch.randint(-7, 8, (x, k), generator=gen, device="cuda").to(torch.bfloat16) for x in (m, n))
+        run = lambda: pa.gemm(a, b, pa.BF16, pa.F32, pa.B_DN)  # noqa: E731
+    got = run()
+    assert pa.last_kernel().startswith("tile256x256w8_dtl"), pa.last_kernel()
+    with tile_env(PTOAMD_NO_TAIL_SPLIT="1"):
+        assert torch.equal(got, run())
