@@ -374,7 +374,7 @@ static const StagedCost staged_costs[STAGED_ROWS][2] = {
     {{4.6f, 0.48f, 0.74f, 0.15f, 1.4f, 0.25f, 0.12f}, {7.0f, 0.92f, 2.3f, 0.39f, 2.1f, 0.36f, 0.93f}},
     {{4.6f, 0.55f, 0.63f, 0.2f, 1.9f, 0, 0.62f}, {}},
     {{4.75f, 0.52f, 0.63f, 0.18f, 0, 0, 0}, {}},
-    {{4.6f, 0.58f, 0.44f, 0.6f, 3.9f, 0.1f, 0.2f}, {6.8f, 1.0f, 2.15f, 0.7f, 3.8f, 0.1f, 0.3f}},
+    {{4.6f, 0.58f, 0.44f, 0.6f, 3.9f, 0.1f, 0.2f}, {6.8f, 1.0f, 2.6f, 0.7f, 3.8f, 0.1f, 0.3f}},
     {{4.25f, 0.56f, 0.79f, 0.2f, 0.75f, 0.2f, 0.11f}, {6.1f, 0.81f, 2.9f, 0.36f, 2.1f, 0.5f, 0.83f}},
 };
 // Beyond these many slabs they are never ahead of everything else.
@@ -404,6 +404,7 @@ static const DrainCost drain_costs[DRAIN_COUNT] = {
 // (the deep-ring kernel's scales and raw accumulators: us per round, and per round and 22000 elements of a tile; its words per
 // column, raw accumulators and atomic additions behind unaligned rows: us per call)
 constexpr float RING_SCALES_ROUND = 0.5f, RING_SCALES_TILE = 22000.0f, RING_UNALIGNED_DRAIN = 2.5f;
+constexpr int TILE256_ROW_MAJOR_K_BYTES = 1024;  // (see pick_dma_tile)
 constexpr int TILE_RING = 16;  // tile ids from here on: the deep-ring kernel's shapes
 
 // What the launcher may choose among.
@@ -434,8 +435,12 @@ static int pick_dma_tile(int m, int n, long k_bytes, int op, const TileChoice& c
         return TILE_RING + form + options().ring;
     // A round or more of 256 x 256 tiles: those (with the split of a part-filled last round below) are ahead from K = 1024 on
     // -- bf16 4096 x 8192 x 2048: 105 us against 129 on 256 x 128 -- and within a tenth of the best where a sixteenth of a round
-    // is left over (4096 x 4312: 192 x 128 tiles 79 against 87 us at K = 2048).
-    if (dtl != DTL_NONE && (long)((m + 255) / 256) * ((n + 255) / 256) >= device_compute_units())
+    // is left over (4096 x 4312: 192 x 128 tiles 79 against 87 us at K = 2048).  From a row-major B without a workspace they
+    // compete at a short K where more than a tenth of them lies past the matrix (640 x 22848 x 192: 39 us, 192 x 128
+    // deep-ring tiles 25; 4000 x 4288 x 64: 16 us, the others from 22).
+    const long tiles256 = (long)((m + 255) / 256) * ((n + 255) / 256);
+    const bool compete = dtl == DTL_256_ONLY && k_bytes < TILE256_ROW_MAJOR_K_BYTES && 10.0 * m * n < 9.0 * 65536 * tiles256;
+    if (dtl != DTL_NONE && tiles256 >= device_compute_units() && !compete)
         return 4;
     const int type = op == TOP_FP4 ? STAGED_FP4 : (scaled ? STAGED_FP8 : 0);
     const TileCost* cost = tile_costs[type];

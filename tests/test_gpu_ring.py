@@ -233,3 +233,15 @@ def test_tail_columns_on_either_kernel(pa, m, n, k, scales):  # noqa: F811
     assert pa.last_kernel().startswith("tile256x256w8_dtl"), pa.last_kernel()
     with tile_env(PTOAMD_NO_TAIL_SPLIT="1"):
         assert torch.equal(got, run())
+
+
+@pytest.mark.parametrize("m,n,k,kernel", [(640, 22848, 192, "tile192x128_bnd_bf16"), (640, 22848, 384, "tile192x128_bnd_bf16"), (640, 22848, 1024, "tile256x256w8_bnd_bf16"),
+                                          (4000, 4288, 64, "tile256x256w8_bnd_bf16")])
+def test_row_major_b_short_k_off_the_256x256_tile(pa, m, n, k, kernel):  # noqa: F811
+    """A round of 256 x 256 tiles from a row-major B: below 512 elements of K the other kernels compete for it where more than a
+    tenth of those tiles lies past the matrix."""
+    gen = torch.Generator(device="cuda").manual_seed(k)
+    a, b = (torch.randint(-3, 4, x, generator=gen, device="cuda").to(torch.bfloat16) for x in ((m, k), (k, n)))
+    got = pa.gemm(a, b, pa.BF16, pa.F32, pa.B_ND)
+    assert pa.last_kernel() == kernel, pa.last_kernel()
+    assert torch.equal(got.double(), a.double() @ b.double())
