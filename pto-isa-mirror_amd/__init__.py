@@ -79,8 +79,33 @@ for _name, _sig in _SIGNATURES.items():
     getattr(_lib, _name).argtypes = [{"p": C.c_void_p, "i": C.c_int, "z": C.c_size_t}[c] for c in _sig]
 
 
+class _EntryPoint(C.CFUNCTYPE(C.c_int)):
+    """An entry point as lib() hands it out: besides what the declared types take, any of ctypes' integer types for any of
+    them (c_long, c_uint, c_bool, an address as c_ulong ...)."""
+    _flags_, _restype_ = C.CFUNCTYPE(C.c_int)._flags_, C.c_int
+
+    def __call__(self, *args):
+        try:
+            return super().__call__(*args)
+        except C.ArgumentError:
+            if len(args) < len(self.argtypes):
+                raise
+            return super().__call__(*[t(a.value) if isinstance(a, C._SimpleCData) and not isinstance(a, t) else a
+                                      for t, a in zip(self.argtypes, args)], *args[len(self.argtypes):])
+
+
+# The library for callers of lib(), a handle of its own: types that a caller declares on it are not those of the calls below.
+_callers_lib = C.CDLL(LIB_PATH)
+for _name in EXPORTS:
+    if _name in _SIGNATURES:
+        setattr(_callers_lib, _name, _EntryPoint((_name, _callers_lib)))
+        getattr(_callers_lib, _name).argtypes = getattr(_lib, _name).argtypes
+    else:
+        getattr(_callers_lib, _name).restype = getattr(_lib, _name).restype
+
+
 def lib():
-    return _lib
+    return _callers_lib
 
 
 def _check(rc, what):

@@ -57,3 +57,25 @@ def test_argument_errors_are_reported_without_a_gpu():
     lib.ptoamd_gemm_mx_workspace_bytes.restype = ctypes.c_size_t
     assert lib.ptoamd_gemm_mx_workspace_bytes(64, 48, 256, 0, 3) == 64 * 8 + 48 * 8  # ZZ / NN: both scale arrays re-laid
     assert lib.ptoamd_gemm_mx_workspace_bytes(64, 48, 256, 1, 5) == 0                # the natural layouts need none
+
+
+def test_lib_takes_any_ctypes_integer():
+    """pa.lib() takes plain numbers and ctypes objects of any integer type, also where they are not the declared ones."""
+    import __graft_entry__ as ge
+
+    pa = ge.load_package()
+    f = pa.lib().ptoamd_gemm
+    c_int, c_long, c_uint, c_bool, c_ulong, c_void_p = (ctypes.c_int, ctypes.c_long, ctypes.c_uint, ctypes.c_bool, ctypes.c_ulong, ctypes.c_void_p)
+    buf = ctypes.create_string_buffer(64)
+    at = ctypes.addressof(buf)
+    for integer in (int, c_int, c_long, c_uint, ctypes.c_ubyte, ctypes.c_longlong):
+        for address in (int, c_void_p, c_ulong):
+            args = [address(at), 0, address(at), address(at), 1, None, integer(4), integer(4), integer(4), integer(4), integer(4), integer(3), 1,
+                    c_bool(True), None]
+            assert f(*args) == -1 and "leading dimension" in pa.lib().ptoamd_last_error().decode()
+            args[8] = integer(0)
+            assert f(*args) == -1 and "must be positive (4, 4, 0)" in pa.lib().ptoamd_last_error().decode()
+    with pytest.raises(ctypes.ArgumentError):
+        f(buf, "f32", buf, buf, 1, None, 4, 4, 4, 4, 4, 3, 1, 0, None)
+    with pytest.raises((ctypes.ArgumentError, TypeError)):
+        f(buf, c_long(0))
