@@ -147,12 +147,18 @@ def _cin(c_in, out):
     return _ptr(c_in, True)
 
 
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def _stream(stream):
     """The HIP stream to launch on.  The current one is asked for by its handle: a torch.cuda.Stream object for it costs 2.7 us
-    of a call's 10.4 (m = 16, out allocated), its handle 0.1."""
+    of a call's 10.4 (m = 16, out allocated), its handle 0.1.  torch has no public function for it; without the private one the
+    object is made."""
     if stream is not None:
         return stream.cuda_stream
-    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
+    if _raw_stream is None:
+        return torch.cuda.current_stream().cuda_stream
+    return _raw_stream(torch.cuda.current_device())
 
 
 _TORCH_OUT = {F32: torch.float32, F16: torch.float16, BF16: torch.bfloat16, I32: torch.int32}

@@ -79,3 +79,19 @@ def test_lib_takes_any_ctypes_integer():
         f(buf, "f32", buf, buf, 1, None, 4, 4, 4, 4, 4, 3, 1, 0, None)
     with pytest.raises((ctypes.ArgumentError, TypeError)):
         f(buf, c_long(0))
+
+
+def test_current_stream_without_the_private_torch_function(monkeypatch):
+    import types
+
+    import __graft_entry__ as ge
+    import torch
+
+    pa = ge.load_package()
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: 0)
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda device=None: types.SimpleNamespace(cuda_stream=0x1234))
+    monkeypatch.setattr(pa, "_raw_stream", None)
+    assert pa._stream(None) == 0x1234
+    monkeypatch.setattr(pa, "_raw_stream", lambda device: 0x5678 + device)
+    assert pa._stream(None) == 0x5678
+    assert pa._stream(types.SimpleNamespace(cuda_stream=0x9abc)) == 0x9abc
