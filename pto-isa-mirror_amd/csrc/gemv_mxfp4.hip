@@ -12,7 +12,8 @@
 //     four MFMAs; row pairs padded and odd rows half-swapped on the global side, so the reads are conflict-free),
 //     dequantised in registers and multiplied on
 //     v_mfma_f32_16x16x32_bf16.  The 8 k-slice partials of a strip are summed through LDS in a fixed order.
-//   * split-K with loader waves, further down: k % 2048 == 0, and k % 512 == 0 beyond one chunk of 2048 and 512 columns.
+//   * split-K with loader waves, further down: k % 2048 == 0, and most of k % 512 == 0 beyond one
+//     chunk of 2048 and 512 columns (the launcher's rule).
 //   * streaming (k % 512 == 0 otherwise): a wave owns 16 rows over the full K, register prefetch four chunks deep,
 //     activations staged per chunk through LDS.
 // Dequantisation: v_cvt_scalef32_pk_bf16_fp4 (fp4 pair * 2^e -> bf16 pair, exact).
@@ -712,11 +713,20 @@ extern "C" int ptoamd_gemv_mxfp4(void* out, int c_type, const void* a_bf16, cons
     const bool swc = opt.gemv_sw_cvt;
     const bool sk_ok = k % SK_SLICE == 0 && (reinterpret_cast<uintptr_t>(sw) & 3u) == 0 && !opt.gemv_no_splitk;
     // loader-wave form: K in chunks of 2048, the last one possibly partial; rows are addressed with 32-bit lane offsets.
-    // A partial chunk: of 81 sizes (n 256 .. 28672, k 1024 .. 7680) it is ahead of the other two kernels on 80 and 2 % behind
-    // on one (4111 x 5120).  Up to one chunk of K, or 512 columns, the tests hold the sizes to the other kernels
-    // (there it would be 4 to 9 us of GPU time against 8 to 25, where a call from Python takes 7).
+    // Partial chunks (n 520 .. 60000, k 2560 .. 15360, m 1 .. 16, us with weights from HBM, which is a decode step's case): it is ahead
+    // of both other kernels except
+    //   * beyond 8192 in whole slices of 1024 on the split-K kernel, up to about 16384 columns: few strips per workgroup, and its
+    //     rounds of chunks are not spread over them (16 x 1152 x 11264: 12.2 against 10.4; 1 x 4111 x 15360: 18.4 against 15.5;
+    //     16 x 8192 x 9216: 15.5 against 14.6; 16 x 20000 x 11264: 27.6 against 29.8);
+    //   * one slice of 512 behind the first chunk, many columns and few rows, on the streaming kernel (1 x 28672 x 2560: 12.3 against
+    //     11.6; 16 x 28672 x 2560: 13.0 against 14.2).
+    // With the same weights over and over, from the caches, the line would lie elsewhere (16 x 6144 x 7168: 12.1 against 11.4 on the
+    // split-K kernel, from HBM 12.4 against 13.5).  Up to one chunk of K, or 512 columns, the older kernels run, as they did before
+    // this form came in (it would be 4 to 9 us of GPU time there against 8 to 25, where a call from Python takes 7).
     const bool partial = k % WD_CHUNK != 0;
-    const bool wide_k = !partial || (k > WD_CHUNK && n > 512);
+    const bool split_ahead = k % SK_SLICE == 0 && k > 8192 && n <= 16384;
+    const bool stream_ahead = k < WD_CHUNK + SK_SLICE && k % SK_SLICE != 0 && n > 20480 && m <= 4;
+    const bool wide_k = !partial || (k > WD_CHUNK && n > 512 && !split_ahead && !stream_ahead);
     if (wide_k && !opt.gemv_no_splitk && (long)lda * 2 * 16 < (1L << 31) && p.ldw_bytes * 16 < (1L << 31) && !opt.gemv_no_wide) {
         const int spw = (p.n_groups + cus - 1) / cus;    // strips per workgroup
         const int grid = (p.n_groups + spw - 1) / spw;

@@ -1272,6 +1272,14 @@ def test_gemv_mxfp4_partial_chunk(pa, oracle, m, n, k):
     assert np.array_equal(odd[:, keep].view(np.uint32), got[:, keep].view(np.uint32)) and not np.isfinite(odd[:, n // 2]).any()
 
 
+# a partial last chunk where another kernel is ahead of the loader-wave one, and the other side of each line
+@pytest.mark.parametrize("m,n,k,kernel", [(16, 1152, 11264, "gemv_mxfp4_splitk"), (3, 4111, 9216, "gemv_mxfp4_splitk"), (2, 16400, 9216, "gemv_mxfp4_splitk_wide"),
+                                          (16, 2048, 7168, "gemv_mxfp4_splitk_wide"), (4, 20481, 2560, "gemv_mxfp4_stream"),
+                                          (5, 20481, 2560, "gemv_mxfp4_splitk_wide"), (4, 20480, 2560, "gemv_mxfp4_splitk_wide")])
+def test_gemv_mxfp4_partial_chunk_on_the_kernel_ahead(pa, oracle, m, n, k, kernel):
+    _check_gemv(pa, oracle, m, n, k, kernel)
+
+
 def test_gemv_ragged_k_takes_the_generic_kernel(pa, oracle):
     r = np.random.default_rng(11)
     m, n, k = 3, 40, 96
