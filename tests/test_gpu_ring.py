@@ -138,6 +138,47 @@ def test_block_scaled_types(pa, oracle, ta, tb, shape):  # noqa: F811
                         max_rel=1e-4 if fp4 else 1e-3, eps=None if fp4 else 2.0 ** -11)
 
 
+def _fp8_operands(r, ta, tb, m, n, k):
+    """Codes without NaN and infinities, on the device with rows at a wider pitch whose other bytes are NaN codes."""
+    a, _, _, _ = _mx_inputs(r, ta, m, n, k)
+    _, b, _, _ = _mx_inputs(r, tb, m, n, k)
+    wide = []
+    for x, pad in ((a, 4), (b, 20)):
+        w = torch.full((x.shape[0], k + pad), 0x7F, dtype=torch.uint8, device="cuda")
+        w[:, :k] = dev(x)
+        wide.append(w[:, :k])
+    return a, b, wide[0], wide[1]
+
+
+@pytest.mark.parametrize("shape", range(7))
+@pytest.mark.parametrize("ta,tb", [(ob.E4M3, ob.E4M3), (ob.E5M2, ob.E4M3), (ob.E4M3, ob.E5M2), (ob.E5M2, ob.E5M2)])
+def test_fp8_without_scales(pa, oracle, ta, tb, shape):  # noqa: F811
+    """No scale arrays, and a K that ends inside a stage, inside a fragment of 32 bytes and inside a chunk of 16."""
+    r = np.random.default_rng(300 + shape + 16 * ta + tb)
+    bm, bn, stage = SHAPES[shape][0], SHAPES[shape][1], SHAPES[shape][3]
+    for m, n, k in ((bm - 1, bn + 3, 16), (1, bn, stage + 4), (bm + 1, 2 * bn + 1, 2 * stage), (bm, bn - 1, 6 * stage + 36)):
+        a, b, da, db = _fp8_operands(r, ta, tb, m, n, k)
+        ref = oracle.matmul_fp8(a, b, b_dn=True, a_type=ta, b_type=tb)
+        with tile_env(PTOAMD_RING=shape):
+            got = host(pa.gemm_fp8(da, db, PA_T[ta], PA_T[tb]))
+            assert pa.last_kernel().startswith(f"tile{bm}x{bn}_dtl_fp8"), pa.last_kernel()
+        mag = np.abs(_mx_unpack(oracle, a, ta)) @ np.abs(_mx_unpack(oracle, b, tb)).T
+        # (the fp8 form of the scaled instruction keeps about 13 bits below the largest of a block's products: 2^-11 of sum|a||b|)
+        check_f32_drain(got, ref, mag, k, f"fp8 {ta}x{tb} {m}x{n}x{k} shape {shape}", max_rel=1e-3, eps=2.0 ** -11)
+
+
+@pytest.mark.parametrize("m,n,k,kernel", [(24, 1000, 1024, "tile32x16_dtl"), (384, 2048, 1060, "tile64x64_dtl"), (1000, 2048, 1024, "tile128x64_dtl"),
+                                          (2048, 2560, 512, "tile128x128_dtl"), (1024, 6144, 1024, "tile256x128r3_dtl"), (4096, 4096, 256, "tile256x256w8_dtl")])
+def test_fp8_without_scales_on_the_kernel_of_its_size(pa, m, n, k, kernel):  # noqa: F811
+    """No switch set: products of small whole numbers, whose sums are exact, on the kernel that the sizes ask for."""
+    gen = torch.Generator(device="cuda").manual_seed(k)
+    a, b = (torch.randint(-2, 3, (x, k), generator=gen, device="cuda").float().to(torch.float8_e4m3fn).view(torch.uint8) for x in (m, n))
+    got = pa.gemm(a, b, pa.E4M3, pa.F32, pa.B_DN)
+    assert pa.last_kernel() == f"{kernel}_fp8_e4m3_e4m3", pa.last_kernel()
+    value = lambda x: x.view(torch.float8_e4m3fn).double()  # noqa: E731
+    assert torch.equal(got.double(), value(a) @ value(b).t())
+
+
 @pytest.mark.parametrize("shape", [0, 3, 7])
 def test_store_forms(pa, oracle, shape):  # noqa: F811
     """Accumulator input, bias, relu, 16-bit rows at an odd pitch, W8A8 with raw accumulators, per-column requantisation and
