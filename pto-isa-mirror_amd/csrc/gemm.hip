@@ -283,14 +283,11 @@ static bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 
 static long ws_row_bytes(long k_bytes) { return (k_bytes + 15) / 16 * 16; }  // row pitch of a transposed B in a workspace
 static bool aligned4(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 3u) == 0; }
 
-// Which tile shape to run where the operands are not the DMA kernels' (pick_dma_tile, below, chooses among those): the largest
-// whose grid still fills most of the 256 CUs.  PTOAMD_TILE=0..7 overrides (both choices),
-// PTOAMD_FORCE_GENERIC=1 sends everything to the order-exact kernel (used by the parity tests).
-// Tiles 0-2 stage slabs through registers (any K); tiles 3-7 DMA slabs straight into LDS and need K to be a whole
-// number of 128-byte slabs (7: the 256 x 128 tile with a ring of three slabs, block-scaled types only -- for the other
-// types the id selects tile 6).  Measured on MI355X: the 8-wave 256x256 DMA tile (4) is the
-// fastest for every operand type once the grid fills the chip (the block-scaled types included: their scales come
-// through LDS, which leaves the 32-byte fp8 fragments just enough registers); smaller grids take the 128x128 DMA tile.
+// Which tile shape to run where pick_dma_tile, below, does not choose (rows of a row-major B that no kernel reads in place,
+// scales in other layouts, 64-bit offsets, a K that is not whole dwords): the largest whose grid still fills most of the 256 CUs.
+// PTOAMD_TILE=0..7 overrides (both choices), PTOAMD_FORCE_GENERIC=1 sends everything to the order-exact kernel (used by the
+// parity tests).  Tiles 0-2 stage slabs through registers (any K); tiles 3-7 DMA slabs straight into LDS (7: the 256 x 128 tile
+// with a ring of three slabs, block-scaled types only -- for the other types the id selects tile 6).
 // The DMA tiles address an operand as a wave-uniform 64-bit base plus a 32-bit per-lane byte offset: the last row's offset
 // plus the K extent must fit 32 bits, or the tile has to take the register-staged form (64-bit addresses per lane).
 static bool dma_offsets_fit(int m, int n, long lda_bytes, long ldb_bytes, long k_bytes)
@@ -299,11 +296,11 @@ static bool dma_offsets_fit(int m, int n, long lda_bytes, long ldb_bytes, long k
     return last <= (long)UINT32_MAX;
 }
 
-// dma_ok: what the DMA tiles need besides whole slabs -- 16-byte aligned operand rows, 32-bit lane offsets, and for the
+// dma_ok: what the DMA tiles need besides whole slabs -- operand rows that start on dwords, 32-bit lane offsets, and for the
 // block-scaled types scale rows they can stream.
 // The plain types' tiles 4 and 5 also take a K that is not a whole number of slabs (at least one slab long).
 // (ragged_k_ok: the operand type has them -- bf16, f16, int8)
-static int pick_tile(int m, int n, long k_bytes, bool scaled, bool fp4 = false, bool dma_ok = true, bool ragged_k_ok = false)
+static int pick_tile(int m, int n, long k_bytes, bool scaled, bool dma_ok, bool ragged_k_ok = false)
 {
     const bool ragged_k = (k_bytes % 128) != 0;
     const bool dtl_ok = dma_ok && (!ragged_k || (ragged_k_ok && k_bytes > 128));
@@ -319,17 +316,8 @@ static int pick_tile(int m, int n, long k_bytes, bool scaled, bool fp4 = false, 
     }
     const long t256 = (long)((m + 255) / 256) * ((n + 255) / 256);
     const long t128 = (long)((m + 127) / 128) * ((n + 127) / 128);
-    const long t256x128 = (long)((m + 255) / 256) * ((n + 127) / 128);
     const int cus = device_compute_units();
-    // Block-scaled types between half and three quarters of a round of 256 x 256 tiles: the 256 x 128 tile with the
-    // three-slab ring puts a workgroup on (nearly) every CU (MXFP4 2048 x 4096 x 4096: 22.5 against 24.9 us)
-    if (scaled && dtl_ok && t256 >= cus / 2 && t256 < 3 * cus / 4 && t256x128 <= cus)
-        return 7;
-    if (scaled && dtl_ok && t256 >= cus / 2)
-        return 4;  // half the copy-in bytes per MFMA of the 128x128 tile
-    if (scaled)
-        return t128 >= 3 * cus / 8 ? (dtl_ok ? 5 : 1) : 2;
-    if (t256 >= cus / 2)
+    if (!scaled && t256 >= cus / 2)
         return dtl_ok ? 4 : 1;
     if (t128 >= 3 * cus / 8)
         return dtl_ok ? 5 : 1;
@@ -878,14 +866,15 @@ static int gemm_common(void* c, int c_type, const void* a, const void* b, int ab
     // (LDS-DMA needs dword-aligned global addresses, no more: rows at 4-byte alignment run 114 against 100 us on bf16 4096^3)
     const bool dma_ok = !b_in_kernel && aligned4(a) && aligned4(b_kmajor) && (lda_b % 4) == 0 && (ldb_kmajor % 4) == 0 &&
                         dma_offsets_fit(m, n, lda_b, ldb_kmajor, k_bytes);
-    // (the deep-ring kernel reads a chunk that K ends in as the 16 bytes ending there, which must start on a dword)
     // rows that start on other bytes, at least one chunk long: the deep-ring kernel's copies through registers (faster than the
     // register-staged tiles, or as fast, at all of 54 sizes, m 7 .. 4000, n 1001 .. 8001, k 1023 .. 4097: 1.0 to 2.2 times)
     const bool any_ok = ragged_k_form && !b_in_kernel && !dma_ok && k_bytes >= 16 && dma_offsets_fit(m, n, lda_b, ldb_kmajor, k_bytes);
+    // (a K of whole dwords: the deep-ring kernel reads a chunk that K ends in as the 16 bytes ending there.  A K that is not, in
+    // rows that start on dwords, keeps to the tiles of pick_tile)
     const int tile = nd_direct || (nd_tile >= 0 && b_in_kernel) ? nd_tile
                      : options().tile < 0 && dma_ok && (k_bytes % 4) == 0 ? pick_dma_tile(m, n, k_bytes, op, {dtl_k, drain, false, nd_ok ? STAGED_NONE : STAGED_COLUMN_MAJOR_B})
                      : options().tile < 0 && any_ok ? pick_dma_tile(m, n, k_bytes, op, {DTL_NONE, drain, true, STAGED_COLUMN_MAJOR_B})
-                                                    : pick_tile(m, n, k_bytes, false, false, dma_ok, ragged_k_form);
+                                                    : pick_tile(m, n, k_bytes, false, dma_ok, ragged_k_form);
     PTOAMD_HIP_CHECK(launch_tiles(tile, op, p, stream));
     set_last_kernel(tile_kernel_name(tile_as_launched(tile, op, m, n), op, nd_direct));
     return PTOAMD_OK;
@@ -927,7 +916,7 @@ int ptoamd_gemm_w8a8(void* out_bf16, int32_t* acc_out, const int8_t* a, const in
     const bool any_ok = !b_in_kernel && !dma_ok && k >= 16 && dma_offsets_fit(m, n, lda, ldb, k);
     const int tile = options().tile < 0 && dma_ok && (k % 4) == 0 ? pick_dma_tile(m, n, k, TOP_I8, {(k % 128) == 0 || k > 128 ? DTL_ALL : DTL_NONE, drain, false, STAGED_COLUMN_MAJOR_B})
                      : options().tile < 0 && any_ok ? pick_dma_tile(m, n, k, TOP_I8, {DTL_NONE, drain, true, STAGED_COLUMN_MAJOR_B})
-                                                    : pick_tile(m, n, k, false, false, dma_ok, true);
+                                                    : pick_tile(m, n, k, false, dma_ok, true);
     PTOAMD_HIP_CHECK(launch_tiles(tile, TOP_I8, p, stream));
     set_last_kernel(tile_kernel_name(tile, TOP_I8));
     return PTOAMD_OK;
@@ -1071,9 +1060,9 @@ static int gemm_mx_common(const char* who, void* c, int c_type, const void* a, c
                               (k_slabs % (a4 ? 2 : 4)) == 0;
     // (the deep-ring kernel fetches them as dwords: any K that is a multiple of 128, which the row-length check above asks for)
     const bool dma_ok = !e1m2 && plain_scales && !b_in_kernel && dma_offsets_fit(m, n, lda_b, ldb_b, k_bytes);
-    const int tile = e1m2 ? pick_tile(m, n, k, true, false, false)
+    const int tile = e1m2 ? pick_tile(m, n, k, true, false)
                      : options().tile < 0 && dma_ok && (kg % 4) == 0 ? pick_dma_tile(m, n, k_bytes, op, {scale_dma_ok ? DTL_ALL : DTL_NONE, c_in ? DRAIN_ACC_IN : DRAIN_PLAIN, false, STAGED_COLUMN_MAJOR_B})
-                                                                    : pick_tile(m, n, k_bytes, true, a4, dma_ok && scale_dma_ok);
+                                                                    : pick_tile(m, n, k_bytes, true, dma_ok && scale_dma_ok);
     PTOAMD_HIP_CHECK(launch_tiles(tile, op, p, stream));
     set_last_kernel(tile_kernel_name(tile_as_launched(tile, op, m, n), op));
     return PTOAMD_OK;
