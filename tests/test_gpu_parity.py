@@ -1608,12 +1608,18 @@ def test_row_major_b_through_a_workspace(pa, oracle):
     assert ws.numel() == n * k * 2 and pa.gemm_workspace_bytes(n, k, pa.BF16, pa.B_DN) == 0
     assert pa.gemm_workspace_bytes(10, 33, pa.I8, pa.B_ND) == 10 * 48   # rows of the re-ordered copy are padded to 16 bytes
     got = pa.gemm(a, b, pa.BF16, pa.F32, pa.B_ND, workspace=ws)
-    assert "dtl" in pa.last_kernel(), pa.last_kernel()
+    assert pa.last_kernel() == "tile128x128_dtl_bf16", pa.last_kernel()
     same = pa.gemm(a, b.t().contiguous(), pa.BF16, pa.F32, pa.B_DN)
+    assert pa.last_kernel() == "tile128x128_dtl_bf16", pa.last_kernel()
     assert torch.equal(got, same)
-    in_loader = pa.gemm(a, b, pa.BF16, pa.F32, pa.B_ND)   # no workspace: the register-staged loader transposes, nothing is allocated
-    assert pa.last_kernel().startswith("tile") and "dtl" not in pa.last_kernel()
-    assert relerr(host(in_loader), host(same)) <= 1e-5
+    in_place = pa.gemm(a, b, pa.BF16, pa.F32, pa.B_ND)   # no workspace: the deep-ring kernel reads B as it lies
+    assert pa.last_kernel() == "tile128x128_bnd_bf16", pa.last_kernel()
+    assert relerr(host(in_place), host(same)) <= 1e-5
+    with tile_env(PTOAMD_B_ND_IN_LOADER=1):              # the register-staged loader transposes; the workspace is not written
+        ws.fill_(7)
+        in_loader = pa.gemm(a, b, pa.BF16, pa.F32, pa.B_ND, workspace=ws)
+        assert pa.last_kernel() == "tile128x128_bf16", pa.last_kernel()
+    assert bool((ws == 7).all()) and relerr(host(in_loader), host(same)) <= 1e-5
     with pytest.raises(pa.PtoAmdError, match="workspace"):
         pa.gemm(a, b, pa.BF16, pa.F32, pa.B_ND, workspace=ws[: ws.numel() // 2])
 
