@@ -124,9 +124,13 @@ int ptoamd_event_elapsed_ms(float* ms, void* start, void* stop);
  *   relu    : flags: PTOAMD_RELU (1) = TSTORE's ReluPreMode::NormalRelu; PTOAMD_SATURATE_INF (2), quantising drains only
  * No alignment is asked of a, b or the leading dimensions beyond that of an element: rows of 16 bytes or more run on the
  * MFMA tiles whatever their alignment: the LDS-DMA kernels when rows start on 4-byte boundaries and K is a multiple of 4
- * bytes, for bf16 / f16 / int8 rows on other bytes the deep-ring tiles with copies through registers, the register-staged
- * tiles otherwise; a row-major B of 16-bit elements is read in place where its rows allow it (ptoamd_gemm_ws below) and else
+ * bytes; for bf16 / f16 / int8 rows that start on other bytes the deep-ring tiles with copies through registers; for
+ * bf16 / f16 / int8 rows that start on 4-byte boundaries with a K that is not a multiple of 4 bytes the two-slab DMA tiles
+ * where K is longer than 128 bytes and the grid large enough (a few dozen 128 x 128 tiles of C), else, as for everything left
+ * over and for a short K, the register-staged tiles; a row-major B of 16-bit elements is read in place where its rows allow it (ptoamd_gemm_ws below) and else
  * transposed on its way into LDS by the latter.  Rows of C need no alignment either.
+ * The kernel follows from the whole shape, m included, and kernels add the k products of an output in different orders: a
+ * row's f32 sums agree from one batch size to another to rounding, not bit for bit (int8 sums are exact).
  * PTOAMD_F32 and PTOAMD_HIF8 operands (hif8 x hif8 only, cpu/TMatmul.hpp:38) run on the order-exact kernel: one thread
  * per output, k ascending, fmaf -- the simulator's arithmetic bit for bit.  No entry point of this group allocates.
  */
@@ -150,6 +154,9 @@ int ptoamd_gemm_bias(void* c, int c_type, const void* a, const void* b, int ab_t
  * b_layout) bytes, 256-byte aligned) first.  The deep-ring tiles read a row-major B of 16-bit elements in place, with or
  * without a workspace, where n is a multiple of 8, k and both pitches are even and the operands lie on 4-byte addresses;
  * otherwise ptoamd_gemm transposes B inside the loader of the register-staged tiles, for every tile row of C.
+ * With a workspace the tile is the one that the column-major product takes (but for a K of a few slabs, where that may be a
+ * register-staged one), and its sums have the same order; reading in place can be faster than the re-ordering that this asks
+ * for, so pass a workspace where B is not readable in place, or for that order.
  * workspace == NULL is ptoamd_gemm_bias.  No counterpart in
  * the reference (its TLOAD re-orders an ND panel into L1 per tile, cpu/TLoad.hpp:287-321).
  */

@@ -24,7 +24,7 @@ inline hipStream_t as_stream(void* s) { return reinterpret_cast<hipStream_t>(s);
 // The environment switches of the dispatchers, read once per process (and again by ptoamd_reload_options): a launch
 // tests plain fields instead of calling getenv.
 struct Options {
-    int tile = -1;               // PTOAMD_TILE=0..6: run this tile shape; -1 = choose by problem size
+    int tile = -1;               // PTOAMD_TILE=0..7: run this tile shape; -1 = choose by problem size
     int ring = -1;               // PTOAMD_RING=0..8: run this shape of the deep-ring kernel where it applies; -1 = choose
     bool mx_16x16 = false;       // PTOAMD_MX_16X16=1: the block-scaled fp8 256 x 256 tile runs on the 16x16x128 instruction
     bool no_tail_split = false;  // PTOAMD_NO_TAIL_SPLIT=1: never split a half-full last round off as smaller tiles

@@ -329,9 +329,10 @@ static int pick_tile(int m, int n, long k_bytes, bool scaled, bool dma_ok, bool 
 // (first copies, store) and a time per 128-byte slab of K -- what a round costs hardly depends on how full it is, each CU
 // waits for its own copies -- and no less than its slabs at the rate a full chip sustains (power, and the copies from the
 // L2s).  The numbers are fits to the times of every kernel on 110 sizes per operand type (m 1 .. 4096, n 256 .. 14336, k
-// 256 .. 8192).  Summed over those sizes, the fitted estimate's choices take 3.22, 2.74, 2.54 and 1.81 ms (bf16, int8, MXFP8,
-// MXFP4) where the best kernel for each takes 3.12, 2.64, 2.42 and 1.73 and the two- and three-slab tiles chosen by grid size
-// alone 4.74, 3.51, 3.23 and 2.10.
+// 256 .. 8192).  On 14686 other sizes of every operand form the choices take 249.5 ms where the best kernel for each takes 234.7
+// and the tiles chosen by grid size alone 405.7; 154 sizes run more than a tenth slower than on the latter.  On full grids with
+// aligned rows the estimate itself is up to a third high (2048 x 4096 x 4096 on 256 x 128 tiles: 58 us, 78 estimated), for all
+// deep-ring shapes alike.
 struct TileCost {
     float round, slab;  // us per round; us per round and slab
     float rate;         // million elements of C times slabs per us
@@ -438,8 +439,9 @@ static int pick_dma_tile(int m, int n, long k_bytes, int op, const TileChoice& c
     const long slab_count = (k_bytes + 127) / 128;
     const float slabs = (float)slab_count;
     const bool staged_ok = choice.staged != STAGED_NONE && slab_count <= (scaled ? STAGED_SLABS_SCALED : unaligned ? STAGED_SLABS_UNALIGNED : STAGED_SLABS);
-    // (a K that is no whole number of slabs costs the two-slab tiles half as much again: bf16 1280 x 4096, K 2048: 24.8 us,
-    // K 2056: 38.4 us)
+    // (bf16 1280 x 4096 on two-slab tiles, K 2048: 24.8 us, K 2056: 38.4 us.  Most of it is that the rows no longer start on
+    // 128-byte lines, which costs the deep-ring shapes a fifth to a third per slab on a full chip as well; that is not in their
+    // estimate)
     const float ragged = (k_bytes % 128) != 0 ? 1.5f : 1.0f;
     int best = TILE_RING;
     float best_us = 1e30f;
