@@ -441,8 +441,9 @@ static int pick_dma_tile(int m, int n, long k_bytes, int op, const TileChoice& c
     const bool staged_ok = choice.staged != STAGED_NONE && slab_count <= (scaled ? STAGED_SLABS_SCALED : unaligned ? STAGED_SLABS_UNALIGNED : STAGED_SLABS);
     // (bf16 1280 x 4096 on two-slab tiles, K 2048: 24.8 us, K 2056: 38.4 us.  Most of it is that the rows no longer start on
     // 128-byte lines, which costs the deep-ring shapes a fifth to a third per slab on a full chip as well; that is not in their
-    // estimate)
-    const float ragged = (k_bytes % 128) != 0 ? 1.5f : 1.0f;
+    // estimate.  The 256 x 256 tile loses less over a long K: bf16 1391 x 9546, K 6800, takes it 177 us, 255 on deep-ring tiles)
+    const bool whole_slabs = (k_bytes % 128) == 0;
+    const float ragged = whole_slabs ? 1.0f : 1.5f, ragged_256 = whole_slabs ? 1.0f : k_bytes > 4096 ? 1.25f : 1.5f;
     int best = TILE_RING;
     float best_us = 1e30f;
     for (int c = 0; c < COST_COUNT; ++c) {
@@ -473,7 +474,7 @@ static int pick_dma_tile(int m, int n, long k_bytes, int op, const TileChoice& c
                 rounds = 1.45f * (float)whole + (rest == 0 ? 0.0f : rest <= cus ? 1.0f : 1.0f + 0.45f * (float)(rest - cus) / (float)cus);
             }
             const float full = (float)tiles * (float)(bm * bn) * 1e-6f / cost[c].rate;
-            us = 3.0f + rounds * copying * cost[c].round + slabs * std::max(rounds * copying * cost[c].slab, full) * (ring ? 1.0f : ragged);
+            us = 3.0f + rounds * copying * cost[c].round + slabs * std::max(rounds * copying * cost[c].slab, full) * (ring ? 1.0f : c == COST_TILE4 ? ragged_256 : ragged);
             if (ring && (choice.drain == DRAIN_SCALES || choice.drain == DRAIN_RAW_ACC))
                 us += rounds * (RING_SCALES_ROUND + (float)(bm * bn) / RING_SCALES_TILE);
             if (unaligned && (choice.drain == DRAIN_COLUMN_WORDS || choice.drain == DRAIN_RAW_ACC || choice.drain == DRAIN_ATOMIC))

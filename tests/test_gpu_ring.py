@@ -286,3 +286,16 @@ def test_row_major_b_short_k_off_the_256x256_tile(pa, m, n, k, kernel):  # noqa:
     got = pa.gemm(a, b, pa.BF16, pa.F32, pa.B_ND)
     assert pa.last_kernel() == kernel, pa.last_kernel()
     assert torch.equal(got.double(), a.double() @ b.double())
+
+
+@pytest.mark.parametrize("kind,m,n,k,kernel", [("bf16", 1391, 9546, 6800, "tile256x256w8_dtl_bf16"), ("i8", 2117, 5492, 9300, "tile256x256w8_dtl_i8"),
+                                               ("bf16", 1237, 4100, 2056, "tile192x128_dtl_bf16")])
+def test_long_k_off_the_lines(pa, kind, m, n, k, kernel):  # noqa: F811
+    """A long K that is no whole number of slabs, on a grid that nearly fills the chip, runs on the 256 x 256 tile, a smaller grid
+    on the deep-ring kernel.  Exact products of small whole numbers."""
+    tdt, t, tc = (torch.int8, pa.I8, pa.I32) if kind == "i8" else (torch.bfloat16, pa.BF16, pa.F32)
+    gen = torch.Generator(device="cuda").manual_seed(k)
+    a, b = (torch.randint(-3, 4, (x, k), generator=gen, device="cuda").to(tdt) for x in (m, n))
+    got = pa.gemm(a, b, t, tc, pa.B_DN)
+    assert pa.last_kernel() == kernel, pa.last_kernel()
+    assert torch.equal(got.double(), a.double() @ b.double().t())
