@@ -329,8 +329,8 @@ static int pick_tile(int m, int n, long k_bytes, bool scaled, bool dma_ok, bool 
 // (first copies, store) and a time per 128-byte slab of K -- what a round costs hardly depends on how full it is, each CU
 // waits for its own copies -- and no less than its slabs at the rate a full chip sustains (power, and the copies from the
 // L2s).  The numbers are fits to the times of every kernel on 110 sizes per operand type (m 1 .. 4096, n 256 .. 14336, k
-// 256 .. 8192).  On 14686 other sizes of every operand form the choices take 249.5 ms where the best kernel for each takes 234.7
-// and the tiles chosen by grid size alone 405.7; 154 sizes run more than a tenth slower than on the latter.  On full grids with
+// 256 .. 8192).  On 14686 other sizes of every operand form the choices take 249.1 ms where the best kernel for each takes 234.7
+// and the tiles chosen by grid size alone 405.7; 144 sizes run more than a tenth slower than on the latter.  On full grids with
 // aligned rows the estimate itself is up to a third high (2048 x 4096 x 4096 on 256 x 128 tiles: 58 us, 78 estimated), for all
 // deep-ring shapes alike.
 struct TileCost {
@@ -441,9 +441,10 @@ static int pick_dma_tile(int m, int n, long k_bytes, int op, const TileChoice& c
     const bool staged_ok = choice.staged != STAGED_NONE && slab_count <= (scaled ? STAGED_SLABS_SCALED : unaligned ? STAGED_SLABS_UNALIGNED : STAGED_SLABS);
     // (bf16 1280 x 4096 on two-slab tiles, K 2048: 24.8 us, K 2056: 38.4 us.  Most of it is that the rows no longer start on
     // 128-byte lines, which costs the deep-ring shapes a fifth to a third per slab on a full chip as well; that is not in their
-    // estimate.  The 256 x 256 tile loses less over a long K: bf16 1391 x 9546, K 6800, takes it 177 us, 255 on deep-ring tiles)
+    // estimate.  The 256 x 256 tile loses less over a long K: bf16 1391 x 9546, K 6800, takes it 177 us, 255 on deep-ring tiles; charged 1.25
+    // it is taken where it is not ahead, 3044 x 3712, K 2392, 91 us against 76)
     const bool whole_slabs = (k_bytes % 128) == 0;
-    const float ragged = whole_slabs ? 1.0f : 1.5f, ragged_256 = whole_slabs ? 1.0f : k_bytes > 4096 ? 1.25f : 1.5f;
+    const float ragged = whole_slabs ? 1.0f : 1.5f, ragged_256 = whole_slabs ? 1.0f : k_bytes > 4096 ? 1.35f : 1.5f;
     int best = TILE_RING;
     float best_us = 1e30f;
     for (int c = 0; c < COST_COUNT; ++c) {

@@ -289,7 +289,7 @@ def test_row_major_b_short_k_off_the_256x256_tile(pa, m, n, k, kernel):  # noqa:
 
 
 @pytest.mark.parametrize("kind,m,n,k,kernel", [("bf16", 1391, 9546, 6800, "tile256x256w8_dtl_bf16"), ("i8", 2117, 5492, 9300, "tile256x256w8_dtl_i8"),
-                                               ("bf16", 1237, 4100, 2056, "tile192x128_dtl_bf16")])
+                                               ("bf16", 1237, 4100, 2056, "tile192x128_dtl_bf16"), ("bf16", 3044, 3712, 2392, "tile192x128_dtl_bf16")])
 def test_long_k_off_the_lines(pa, kind, m, n, k, kernel):  # noqa: F811
     """A long K that is no whole number of slabs, on a grid that nearly fills the chip, runs on the 256 x 256 tile, a smaller grid
     on the deep-ring kernel.  Exact products of small whole numbers."""
