@@ -12,8 +12,8 @@ static hipError_t launch_ring(const TileGemmParams& p, hipStream_t stream)
     const hipError_t e = ensure_dynamic_lds(reinterpret_cast<const void*>(&gemm_tile_ring_kernel<Cfg>), Cfg::LDS_BYTES);
     if (e != hipSuccess || p.m <= 0)  // m = 0: only make the kernel ready to launch on the current device
         return e;
-    const int tiles = ((p.m + Cfg::BM - 1) / Cfg::BM) * ((p.n + Cfg::BN - 1) / Cfg::BN);
-    hipLaunchKernelGGL((gemm_tile_ring_kernel<Cfg>), dim3(tiles), dim3(Cfg::THREADS), Cfg::LDS_BYTES, stream, p);
+    const RingTiles tiles = ring_tiles(p, Cfg::BM, Cfg::BN);
+    hipLaunchKernelGGL((gemm_tile_ring_kernel<Cfg>), dim3(tiles.grid), dim3(Cfg::THREADS), Cfg::LDS_BYTES, stream, p, tiles);
     return hipGetLastError();
 }
 

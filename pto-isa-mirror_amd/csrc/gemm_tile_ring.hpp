@@ -196,8 +196,53 @@ __device__ __forceinline__ void ring_store(const TileGemmParams& p, Elem (&v)[NE
     }
 }
 
+// n / d for 0 <= n < 2^31 as a product: with l = ceil(log2 d) and magic = ceil(2^(31 + l) / d), which is below 2^32, the error of
+// n * magic / 2^(31 + l) is below 1 / d.
+struct RingDivisor {
+    uint32_t magic, shift;
+    __host__ static RingDivisor of(uint32_t d)
+    {
+        uint32_t l = 0;
+        while ((1ull << l) < d)
+            ++l;
+        return {(uint32_t)(((1ull << (31 + l)) + d - 1) / d), 31 + l};
+    }
+    __device__ __forceinline__ int divide(int n) const { return (int)(((uint64_t)(uint32_t)n * magic) >> shift); }
+};
+// Workgroup -> tile, worked out by the host: `grid` tiles in tiles_m rows, walked in groups of group_m rows (the last group of
+// group_last); per_group tiles make a group.  Two divisions of run-time values in the kernel took 90 scalar instructions.
+struct RingTiles {
+    int grid, tiles_m, group_m, per_group;
+    RingDivisor by_group, by_group_m, by_group_last;
+};
+inline RingTiles ring_tiles(const TileGemmParams& p, int bm, int bn)
+{
+    RingTiles t;
+    const int tiles_n = (p.n + bn - 1) / bn;
+    t.tiles_m = (p.m + bm - 1) / bm;
+    t.grid = t.tiles_m * tiles_n;
+    t.group_m = p.group_m;
+    t.per_group = p.group_m * tiles_n;
+    t.by_group = RingDivisor::of(t.per_group);
+    t.by_group_m = RingDivisor::of(p.group_m);
+    t.by_group_last = RingDivisor::of(t.tiles_m % p.group_m ? t.tiles_m % p.group_m : p.group_m);
+    return t;
+}
+// Has the arguments in scalar registers from here on: they arrive in one wait, where the compiler's own loads, each in front of
+// its first use, stand one after the other on the way to the first copy and again in front of the store.
+template <class T>
+__device__ __forceinline__ void ring_argument(const T v)
+{
+    asm volatile("" : : "s"(v));
+}
+template <class... T>
+__device__ __forceinline__ void ring_arguments(const T... v)
+{
+    (ring_argument(v), ...);
+}
+
 template <class Cfg>
-__global__ void __launch_bounds__(Cfg::THREADS) gemm_tile_ring_kernel(const TileGemmParams p)
+__global__ void __launch_bounds__(Cfg::THREADS) gemm_tile_ring_kernel(const TileGemmParams p, const RingTiles tiles)
 {
     using Op = typename Cfg::Op;
     using Acc = typename Op::Acc;
@@ -215,13 +260,14 @@ __global__ void __launch_bounds__(Cfg::THREADS) gemm_tile_ring_kernel(const Tile
 
     // ---- workgroup -> tile.  Workgroup ids go round-robin to the 8 XCDs; XCD x takes a contiguous run of tiles, walked in
     // groups of group_m tile rows, so that what an L2 holds is a few panels of A and of B.
-    const int tiles_m = (p.m + BM - 1) / BM, tiles_n = (p.n + BN - 1) / BN, grid = tiles_m * tiles_n;
+    ring_arguments(p.a, p.b, p.c, p.c_in, p.bias, p.acc_out, p.sa, p.sb, p.row_scale, p.col_scale, p.m, p.n, p.k_bytes, p.lda_bytes, p.ldb_bytes,
+                   p.ldc, p.scale_ld, p.relu, p.out_kind, p.qwords, p.q_per_column, p.atomic_add, tiles.grid);
     const int xcd = blockIdx.x & 7;
-    const int lid = xcd * (grid >> 3) + min(xcd, grid & 7) + (blockIdx.x >> 3);
-    const int per_group = p.group_m * tiles_n;
-    const int first_m = (lid / per_group) * p.group_m;
-    const int gsize = min(tiles_m - first_m, p.group_m);
-    const int m0 = (first_m + (lid % per_group) % gsize) * BM, n0 = ((lid % per_group) / gsize) * BN;
+    const int lid = xcd * (tiles.grid >> 3) + min(xcd, tiles.grid & 7) + (blockIdx.x >> 3);
+    const int group = tiles.by_group.divide(lid), in_group = lid - group * tiles.per_group, first_m = group * tiles.group_m;
+    const int gsize = min(tiles.tiles_m - first_m, tiles.group_m);
+    const int column = (gsize == tiles.group_m ? tiles.by_group_m : tiles.by_group_last).divide(in_group);
+    const int m0 = (first_m + in_group - column * gsize) * BM, n0 = column * BN;
 
     // ---- TLOAD addressing: piece w + q * NW of a stage, lane -> (row, position) linear, fetching chunk position ^ swizzle
     const int nst = (p.k_bytes + SB - 1) / SB;
@@ -540,27 +586,28 @@ __global__ void __launch_bounds__(Cfg::THREADS) gemm_tile_ring_kernel(const Tile
 
     // ---- TSTORE: the k-groups' partial sums meet in LDS (the ring is free), are added in group order and leave as 16
     // bytes per thread.  A block is transposed in its lanes: lane (l16, lg) holds row l16, columns 4 lg .. + 3.
-    __syncthreads();
-    Elem* red = reinterpret_cast<Elem*>(smem) + wk * (BM * Cfg::RED_PITCH);
-    if (computes) {
-#pragma unroll
-        for (int i = 0; i < MB; ++i)
-#pragma unroll
-            for (int j = 0; j < NB; ++j)
-                *reinterpret_cast<Acc*>(red + (wm * Cfg::WTM + i * 16 + l16) * Cfg::RED_PITCH + wn * Cfg::WTN + j * 16 + 4 * lg) = acc[i][j];
-    }
-    __syncthreads();
     auto drain = [&](auto kc) __attribute__((always_inline)) {
         constexpr int KIND = decltype(kc)::value, NE = ring_cols<KIND>, CT = BN / NE, RSTEP = Cfg::THREADS / CT;
         static_assert(Cfg::THREADS % CT == 0, "a thread keeps its columns from row to row");
         const int c = (tid % CT) * NE, gj = n0 + c;
+        // (what the columns and the first row bring is fetched while the sums are exchanged)
+        RingColumns<KIND, NE, Elem> cols;
+        cols.load(p, min(gj, p.n - 1));
+        float rs = KIND == OUT_W8A8_BF16 ? p.row_scale[min(m0 + tid / CT, p.m - 1)] : 1.0f;
+        __syncthreads();
+        Elem* red = reinterpret_cast<Elem*>(smem) + wk * (BM * Cfg::RED_PITCH);
+        if (computes) {
+#pragma unroll
+            for (int i = 0; i < MB; ++i)
+#pragma unroll
+                for (int j = 0; j < NB; ++j)
+                    *reinterpret_cast<Acc*>(red + (wm * Cfg::WTM + i * 16 + l16) * Cfg::RED_PITCH + wn * Cfg::WTN + j * 16 + 4 * lg) = acc[i][j];
+        }
+        __syncthreads();
         if (gj >= p.n)
             return;
-        RingColumns<KIND, NE, Elem> cols;
-        cols.load(p, gj);
 #pragma unroll 1
         for (int r = tid / CT; r < BM && m0 + r < p.m; r += RSTEP) {
-            const float rs = KIND == OUT_W8A8_BF16 ? p.row_scale[m0 + r] : 1.0f;
             Elem v[NE];
 #pragma unroll
             for (int e = 0; e < NE; ++e)
@@ -574,7 +621,10 @@ __global__ void __launch_bounds__(Cfg::THREADS) gemm_tile_ring_kernel(const Tile
                     for (int e = 0; e < 4; ++e)
                         v[4 * q + e] += x[e];
                 }
-            ring_store<KIND>(p, v, cols, rs, m0 + r, gj);
+            const float row_scale = rs;
+            if (KIND == OUT_W8A8_BF16)
+                rs = p.row_scale[min(m0 + r + RSTEP, p.m - 1)];
+            ring_store<KIND>(p, v, cols, row_scale, m0 + r, gj);
         }
     };
     if (p.out_kind == OUT_Q8)
