@@ -59,22 +59,38 @@ struct RingCfg {
     static constexpr int KW = SB / WK, KSTEPS = KW / KB;
     static constexpr int ROWS = BM + BN, CPR = SB / 16, RPP = 1024 / SB;  // chunks per row, rows per 1 KiB piece
     static constexpr int PIECES = ROWS * SB / 1024, A_PIECES = BM * SB / 1024, NPW = PIECES / NW;
-    static constexpr int SC = Op::SCALED ? SB / KB : 0;                   // scale dwords (four groups each) per row and stage
-    static constexpr int SPC = ROWS * SC / 64, NSW = (SPC + NW - 1) / NW; // 64-dword scale pieces; per wave
+    // Block scales, SPS dwords (of four groups each) per row and stage.  A copy's cost is the 128-byte lines it touches, whatever it
+    // takes of them: a dword or two per row, as each stage needs them, made them half as expensive as the operands (96 x 64 tile,
+    // fp8: 160 lines beside 320 per stage).  Such tiles of 160 rows and more (CHUNKED) copy a row's scales 64 or 32 bytes at a
+    // time, for SPC stages, into SBUFS buffers behind the ring (20 lines per stage; MXFP8 384 x 4096 x 4096 16.0 -> 13.5 us, on
+    // 128 x 128 tiles up to a fifth less).  So does the narrow fp4 tile, whose stage takes 64 bytes (5 % less).  With fewer rows the
+    // start counts more, which takes longer so (32 x 32 tile, fp8 5 x 4352 x 640 3.4 -> 3.6 us), and where a stage takes 16 bytes of
+    // a row there is nothing to gain (fp4 on 96 x 64: 1 % more): these copy dwords into the stage itself.
+    static constexpr int SPS = Op::SCALED ? SB / KB : 0;
+    static constexpr bool CHUNKED = Op::SCALED && ((ROWS >= 160 && SPS <= 2) || SPS >= 16);
+    static constexpr int STAGE_SPS = CHUNKED ? 0 : SPS;                        // (scale dwords inside a stage)
+    static constexpr int SPIECES = ROWS * STAGE_SPS / 64, NSW = (SPIECES + NW - 1) / NW; // 64-dword scale pieces; per wave
     static constexpr int NV = NPW + NSW;                                  // copies a wave issues per stage
-    static constexpr int STAGE = ROWS * SB + ROWS * SC * 4;
+    static constexpr int STAGE = ROWS * SB + ROWS * STAGE_SPS * 4;
+    // (the chunk of the stage that is being copied finds a buffer whose last reader is past)
+    static constexpr int scale_buffers(int scb) { return !CHUNKED ? 0 : 1 + (R - 1 + scb / 4 / SPS - 1) / (scb / 4 / SPS); }
+    static constexpr int SCB = !CHUNKED ? 64 : R * STAGE + scale_buffers(64) * ROWS * 64 <= 160 * 1024 ? 64 : 32;
+    static constexpr int SPC = CHUNKED ? SCB / 4 / SPS : 1, SBUFS = scale_buffers(SCB);
+    static constexpr int SCALE_BYTES = SBUFS * ROWS * SCB;
     static constexpr int KR = SB / 2, RB = BN * 2, CB = RB / 16;          // BND: k rows of a stage, bytes and chunks per row
     static constexpr int AHEAD = NPW <= 8 ? 3 : 2;                        // ANY: stages a copying wave holds in registers
     static constexpr int RED_PITCH = BN + 4;                              // elements
     static constexpr int RED_BYTES = WK * BM * RED_PITCH * 4;
-    static constexpr int LDS_BYTES = (R * STAGE > RED_BYTES ? R * STAGE : RED_BYTES);
+    static constexpr int LDS_BYTES = (R * STAGE + SCALE_BYTES > RED_BYTES ? R * STAGE + SCALE_BYTES : RED_BYTES);
     static_assert(BM % (16 * WM) == 0 && BN % (16 * WN) == 0, "wave tiles are made of 16x16 blocks");
     static_assert(KW % KB == 0 && SB <= 1024 && 1024 % SB == 0, "a k-group's part of a stage is whole k-steps");
     static_assert(PIECES % NW == 0 && (BM * SB) % 1024 == 0, "every wave issues the same number of 1 KiB copies, each of one operand");
     static_assert(!BND || (!Op::SCALED && FR == 1 && (NB & (NB - 1)) == 0), "the row-major form is for the 16-bit types");
     static_assert(!ANY || (PIPE && !BND && !Op::SCALED), "the register copies are the copying waves' and know no scales");
-    static_assert((ROWS * SC) % 64 == 0, "scale pieces are whole");
-    static_assert(LDS_BYTES <= 160 * 1024 && R >= 2 && (R - 1) * NV < 64, "LDS capacity; vmcnt is a 6-bit count");
+    static_assert((ROWS * STAGE_SPS) % 64 == 0, "scale pieces are whole");
+    static_assert(!CHUNKED || (SCB / 4 % SPS == 0 && (SBUFS - 1) * SPC >= R - 1 && BM * SCB % 1024 == 0 && BN * SCB % 1024 == 0 && ROWS <= NW * 64),
+                  "a chunk of scales is whole stages; a 1 KiB copy of them is of one operand; a thread can hold a row's");
+    static_assert(LDS_BYTES <= 160 * 1024 && R >= 2 && R * NV + (CHUNKED ? ROWS * SCB / 1024 / NW + 1 : 0) < 64, "LDS capacity; vmcnt is a 6-bit count");
 };
 
 // position of a row's 16-byte chunk is chunk ^ ring_swizzle(row)
@@ -82,6 +98,13 @@ template <int SB>
 __device__ __forceinline__ int ring_swizzle(int row)
 {
     return SB == 128 ? swizzle_chunk(row, 0) : (row & 15);
+}
+
+// position of a row's 16-byte piece of scales is piece ^ ring_scale_swizzle(row): the byte reads of 16 rows hit different banks
+template <int SCB>
+__device__ __forceinline__ int ring_scale_swizzle(int row)
+{
+    return (row / (256 / SCB)) % (SCB / 16);
 }
 
 template <int N>
@@ -248,7 +271,8 @@ __global__ void __launch_bounds__(Cfg::THREADS) gemm_tile_ring_kernel(const Tile
     using Acc = typename Op::Acc;
     using Elem = typename Op::Elem;
     constexpr int BM = Cfg::BM, BN = Cfg::BN, MB = Cfg::MB, NB = Cfg::NB, FR = Cfg::FR, SB = Cfg::SB, R = Cfg::R, NW = Cfg::NW;
-    constexpr int NPW = Cfg::NPW, NSW = Cfg::NSW, NV = Cfg::NV, SC = Cfg::SC, CPR = Cfg::CPR;
+    constexpr int NPW = Cfg::NPW, NSW = Cfg::NSW, NV = Cfg::NV, CPR = Cfg::CPR;
+    constexpr bool CHUNKED = Cfg::CHUNKED;
     extern __shared__ __align__(16) uint8_t smem[];
 
     const int tid = threadIdx.x, lane = tid & 63;
@@ -289,7 +313,7 @@ __global__ void __launch_bounds__(Cfg::THREADS) gemm_tile_ring_kernel(const Tile
 #pragma unroll
     for (int q = 0; q < NPW; ++q)
         goff[q] = Cfg::BND && lw + q * NW >= Cfg::A_PIECES ? (uint32_t)(nd_row(q) * p.ldb_bytes) + nd_col(q) : row_offset(q) + piece_chunk(q) * 16;
-    // scales: dword e = row * SC + d of a stage's scale area; without scale arrays the copies fetch bytes of A that are not used
+    // Scales in the stage: dword e = row * STAGE_SPS + d; without scale arrays the copies fetch bytes of A that are not used.
     const bool has_scales = Op::SCALED && p.sa != nullptr;
     const uint8_t* sc_row[NSW > 0 ? NSW : 1];
     int sc_d[NSW > 0 ? NSW : 1];
@@ -297,11 +321,55 @@ __global__ void __launch_bounds__(Cfg::THREADS) gemm_tile_ring_kernel(const Tile
     if constexpr (NSW > 0) {
 #pragma unroll
         for (int q = 0; q < NSW; ++q) {
-            const int e = ((lw + q * NW) % Cfg::SPC) * 64 + lane, r = e / SC;
-            sc_d[q] = e % SC;
+            const int e = ((lw + q * NW) % Cfg::SPIECES) * 64 + lane, r = e / Cfg::STAGE_SPS;
+            sc_d[q] = e % Cfg::STAGE_SPS;
             sc_row[q] = !has_scales ? p.a : r < BM ? p.sa + (long)min(m0 + r, p.m - 1) * p.scale_ld : p.sb + (long)min(n0 + r - BM, p.n - 1) * p.scale_ld;
         }
     }
+    // Scales in chunks: without scale arrays nothing is copied and the fragments' bytes, whatever they hold, are not used.  A row's
+    // last 16 bytes are the 16 that END there, so where scale_ld is no multiple of 16 its last dwords lie scale_shift further on; a
+    // row shorter than that (K < 512) goes through registers.
+    const bool short_scales = CHUNKED && has_scales && p.scale_ld < 16;
+    const int scale_last = CHUNKED ? p.scale_ld / 16 * 4 : 0, scale_shift = CHUNKED ? (4 - p.scale_ld / 4 % 4) % 4 : 0;
+    auto issue_scales = [&](int chunk) __attribute__((always_inline)) {
+        if constexpr (CHUNKED) {
+            constexpr int SCB = Cfg::SCB, LANES = SCB / 16, RPI = 64 / LANES, COPIES = Cfg::ROWS / RPI;  // lanes per row, rows per copy
+            const uint32_t dst = lds0 + R * Cfg::STAGE + (chunk % Cfg::SBUFS) * (Cfg::ROWS * SCB);
+#pragma unroll
+            for (int q = 0; q < (COPIES + NW - 1) / NW; ++q) {
+                const int c = lw + q * NW, r = c * RPI + lane / LANES;
+                if (COPIES % NW != 0 && c >= COPIES)
+                    break;
+                const int byte = min(chunk * SCB + ((lane % LANES) ^ ring_scale_swizzle<SCB>(r)) * 16, p.scale_ld - 16);
+                const bool is_a = c * RPI < BM;
+                const int row = is_a ? min(m0 + r, p.m - 1) : min(n0 + r - BM, p.n - 1);
+                lds_dma16_off(is_a ? p.sa : p.sb, (uint32_t)(row * p.scale_ld + byte), dst + c * 1024);
+            }
+        }
+    };
+    uint32_t held_scales[3];
+    const int held_row = lw * 64 + lane;
+    auto hold_short_scales = [&]() __attribute__((always_inline)) {
+        if constexpr (CHUNKED) {
+            if (short_scales && held_row < Cfg::ROWS) {
+                const uint8_t* row = held_row < BM ? p.sa + (long)min(m0 + held_row, p.m - 1) * p.scale_ld : p.sb + (long)min(n0 + held_row - BM, p.n - 1) * p.scale_ld;
+#pragma unroll
+                for (int d = 0; d < 3; ++d)
+                    held_scales[d] = *reinterpret_cast<const uint32_t*>(row + min(4 * d, p.scale_ld - 4));
+            }
+        }
+    };
+    auto write_short_scales = [&]() __attribute__((always_inline)) {
+        if constexpr (CHUNKED) {
+            if (short_scales && held_row < Cfg::ROWS) {
+                uint8_t* at = smem + R * Cfg::STAGE + held_row * Cfg::SCB + ring_scale_swizzle<Cfg::SCB>(held_row) * 16 + scale_shift * 4;
+#pragma unroll
+                for (int d = 0; d < 3; ++d)
+                    if (4 * d < p.scale_ld)
+                        *reinterpret_cast<uint32_t*>(at + 4 * d) = held_scales[d];
+            }
+        }
+    };
     auto issue = [&](int st, int buf) __attribute__((always_inline)) {
         const uint32_t dst = __builtin_amdgcn_readfirstlane(lds0 + buf * Cfg::STAGE);
         const long kb = (long)st * SB, kb_b = Cfg::BND ? (long)st * Cfg::KR * p.ldb_bytes : kb;
@@ -329,7 +397,11 @@ __global__ void __launch_bounds__(Cfg::THREADS) gemm_tile_ring_kernel(const Tile
         if constexpr (NSW > 0) {
 #pragma unroll
             for (int q = 0; q < NSW; ++q)
-                lds_dma4(sc_row[q] + 4 * min(st * SC + sc_d[q], sc_last), dst + Cfg::ROWS * SB + ((lw + q * NW) % Cfg::SPC) * 256);
+                lds_dma4(sc_row[q] + 4 * min(st * Cfg::STAGE_SPS + sc_d[q], sc_last), dst + Cfg::ROWS * SB + ((lw + q * NW) % Cfg::SPIECES) * 256);
+        }
+        if constexpr (CHUNKED) {
+            if (has_scales && !short_scales && st % Cfg::SPC == 0)  // ahead of the next stage's copies, which stages are counted by
+                issue_scales(st / Cfg::SPC);
         }
     };
 
@@ -345,7 +417,25 @@ __global__ void __launch_bounds__(Cfg::THREADS) gemm_tile_ring_kernel(const Tile
     // ---- fragments: chunk c0 + lg of row l16 of a block, c0 a multiple of 4, sits at position c0 ^ (lg ^ swizzle(l16))
     const uint32_t lane_x = (uint32_t)((lg ^ ring_swizzle<SB>(l16)) ^ (wk * (Cfg::KW / 16))) << 4;
     const uint32_t fa_row = (wm * Cfg::WTM + l16) * SB, fb_row = (BM + wn * Cfg::WTN + l16) * SB;
-    const uint32_t sa_at = Cfg::ROWS * SB + (wm * Cfg::WTM + l16) * (SC * 4) + lg, sb_at = Cfg::ROWS * SB + (BM + wn * Cfg::WTN + l16) * (SC * 4) + lg;
+    // Scale bytes.  In the stage: k-step s, row block i at {sa_at, sb_at} + 4 s + i * 16 * 4 STAGE_SPS of the stage.  In chunks: at
+    // {a, b} of scale_rows(st) + 4 s + i * 16 * SCB; a chunk's dwords are 4 bytes apart but for the swizzle, which touches the bits of
+    // a row's 16-byte pieces only, and a wave's k-steps lie in one piece.
+    struct ScaleRows {
+        uint32_t a, b;
+    };
+    constexpr int SCALE_ROW = CHUNKED ? Cfg::SCB : Cfg::STAGE_SPS * 4;
+    const uint32_t scale_lane = (CHUNKED ? R * Cfg::STAGE + ((ring_scale_swizzle<Cfg::SCB>(l16) * 16) ^ (wk * Cfg::KSTEPS * 4)) : Cfg::ROWS * SB + wk * Cfg::KSTEPS * 4) + lg;
+    const uint32_t sa_at = scale_lane + (wm * Cfg::WTM + l16) * SCALE_ROW, sb_at = scale_lane + (BM + wn * Cfg::WTN + l16) * SCALE_ROW;
+    auto scale_rows = [&](uint32_t st) __attribute__((always_inline)) -> ScaleRows {
+        if constexpr (!CHUNKED)
+            return {0, 0};
+        else {
+            static_assert(Cfg::KSTEPS <= 4 && R * Cfg::STAGE % 64 == 0 && (Cfg::ROWS * Cfg::SCB) % 64 == 0, "a wave's k-steps of a stage lie in one 16-byte piece");
+            const uint32_t in_chunk = (st * Cfg::SPS * 4) % Cfg::SCB;
+            const uint32_t buf = (st / Cfg::SPC % Cfg::SBUFS) * (Cfg::ROWS * Cfg::SCB) + (st * Cfg::SPS + wk * Cfg::KSTEPS >= (uint32_t)scale_last ? scale_shift * 4 : 0);
+            return {(sa_at ^ in_chunk) + buf, (sb_at ^ in_chunk) + buf};
+        }
+    };
     // BND: this lane's 8 bytes of a k-step's first block, k rows 8 lg .. + 3
     const int nd_l = lg * 8 + (l16 >> 2);
     const uint32_t nd_at = BM * SB + (wk * (Cfg::KW / 2) + nd_l) * Cfg::RB + ((wn * (Cfg::WTN / 16) ^ swizzle_row_major<BN>(nd_l)) << 5) + (l16 & 3) * 8;
@@ -356,15 +446,15 @@ __global__ void __launch_bounds__(Cfg::THREADS) gemm_tile_ring_kernel(const Tile
     uint4 fa[SETS][MB][FR], fb[SETS][NB][FR];
     uint32_t xa[SETS][MB], xb[SETS][NB];
     auto aset = [](int set, int i) constexpr { return i == MB - 1 ? set : 0; };
-    auto read_a = [&](int set, int i, int s, int b) __attribute__((always_inline)) {
+    auto read_a = [&](int set, int i, int s, int b, const ScaleRows& sc) __attribute__((always_inline)) {
         const uint8_t* base = smem + b * Cfg::STAGE;
 #pragma unroll
         for (int f = 0; f < FR; ++f)
             fa[set][i][f] = *reinterpret_cast<const uint4*>(base + fa_row + i * (16 * SB) + (lane_x ^ ((s * 4 * FR + 4 * f) << 4)));
         if constexpr (Op::SCALED)
-            xa[set][i] = base[sa_at + (wk * Cfg::KSTEPS + s) * 4 + i * (16 * SC * 4)];
+            xa[set][i] = (CHUNKED ? smem + sc.a : base + sa_at)[s * 4 + i * (16 * SCALE_ROW)];
     };
-    auto read_b = [&](int set, int j, int s, int b) __attribute__((always_inline)) {
+    auto read_b = [&](int set, int j, int s, int b, const ScaleRows& sc) __attribute__((always_inline)) {
         const uint8_t* base = smem + b * Cfg::STAGE;
         if constexpr (Cfg::BND) {
             const uint8_t* at = base + (nd_at ^ (j << 5)) + s * 32 * Cfg::RB;
@@ -375,15 +465,15 @@ __global__ void __launch_bounds__(Cfg::THREADS) gemm_tile_ring_kernel(const Tile
         for (int f = 0; f < FR; ++f)
             fb[set][j][f] = *reinterpret_cast<const uint4*>(base + fb_row + j * (16 * SB) + (lane_x ^ ((s * 4 * FR + 4 * f) << 4)));
         if constexpr (Op::SCALED)
-            xb[set][j] = base[sb_at + (wk * Cfg::KSTEPS + s) * 4 + j * (16 * SC * 4)];
+            xb[set][j] = (CHUNKED ? smem + sc.b : base + sb_at)[s * 4 + j * (16 * SCALE_ROW)];
     };
-    auto read_all = [&](int set, int s, int b) __attribute__((always_inline)) {
+    auto read_all = [&](int set, int s, int b, const ScaleRows& sc) __attribute__((always_inline)) {
 #pragma unroll
         for (int j = 0; j < NB; ++j)
-            read_b(set, j, s, b);
+            read_b(set, j, s, b, sc);
 #pragma unroll
         for (int i = 0; i < MB; ++i)
-            read_a(Cfg::PIPE ? aset(set, i) : 0, i, s, b);
+            read_a(Cfg::PIPE ? aset(set, i) : 0, i, s, b, sc);
     };
     auto mma = [&](int set, int i, int j) __attribute__((always_inline)) {
         const int as = Cfg::PIPE ? aset(set, i) : 0;
@@ -424,10 +514,12 @@ __global__ void __launch_bounds__(Cfg::THREADS) gemm_tile_ring_kernel(const Tile
     if constexpr (!Cfg::PIPE) {
         // Barrier st: stage st has landed and no wave reads stage st - 1 any more, whose buffer is refilled.
         if (loads) {
+            hold_short_scales();
 #pragma unroll
             for (int s = 0; s < R - 1; ++s)
                 if (s < nst)
                     issue(s, s);
+            write_short_scales();
         }
         int buf = 0;
         auto step = [&](int st) __attribute__((always_inline)) {
@@ -440,10 +532,11 @@ __global__ void __launch_bounds__(Cfg::THREADS) gemm_tile_ring_kernel(const Tile
             }
         };
         for (int st = 0; st < nst - 1; ++st) {
+            const ScaleRows rows = scale_rows(st);
             step(st);
             if (computes)
                 static_for<Cfg::KSTEPS>([&](auto sc) {
-                    read_all(0, decltype(sc)::value, buf);
+                    read_all(0, decltype(sc)::value, buf, rows);
 #pragma unroll
                     for (int i = 0; i < MB; ++i)
 #pragma unroll
@@ -452,10 +545,11 @@ __global__ void __launch_bounds__(Cfg::THREADS) gemm_tile_ring_kernel(const Tile
                 });
             buf = buf + 1 == R ? 0 : buf + 1;
         }
+        const ScaleRows rows = scale_rows(nst - 1);
         step(nst - 1);
         if (computes)
             static_for<Cfg::KSTEPS>([&](auto sc) {
-                read_all(0, decltype(sc)::value, buf);
+                read_all(0, decltype(sc)::value, buf, rows);
                 tail_step(0, decltype(sc)::value);
             });
     } else {
@@ -511,10 +605,12 @@ __global__ void __launch_bounds__(Cfg::THREADS) gemm_tile_ring_kernel(const Tile
                     step(gc);
             });
         } else if (!computes) {
+            hold_short_scales();
 #pragma unroll
             for (int s = 0; s < R; ++s)
                 if (s < nst)
                     issue(s, s);
+            write_short_scales();
             loader_barrier(min(R - 1, nst - 1));
             int buf = 0;
             for (int st = 0; st < nst - 1; ++st) {
@@ -524,9 +620,11 @@ __global__ void __launch_bounds__(Cfg::THREADS) gemm_tile_ring_kernel(const Tile
                 buf = buf + 1 == R ? 0 : buf + 1;
             }
         } else {
+            // the scale addresses of a stage and the next one's: computed a stage ahead, off the way from barrier to matrix instruction
+            ScaleRows rows = scale_rows(0), next_rows = scale_rows(1);
             ring_wait_and_barrier<63>();
-            read_all(0, 0, 0);
-            int buf = 0;
+            read_all(0, 0, 0, rows);
+            int buf = 0, st = 0;
             auto body = [&](auto parc) __attribute__((always_inline)) {
                 constexpr int PAR = decltype(parc)::value;
                 const int nbuf = buf + 1 == R ? 0 : buf + 1;
@@ -535,6 +633,7 @@ __global__ void __launch_bounds__(Cfg::THREADS) gemm_tile_ring_kernel(const Tile
                     constexpr bool LASTSTEP = s + 1 == Cfg::KSTEPS;
                     constexpr int rs = LASTSTEP ? 0 : s + 1;
                     const int rb = LASTSTEP ? nbuf : buf;
+                    const ScaleRows& rsc = LASTSTEP ? next_rows : rows;
                     if constexpr (LASTSTEP)
                         ring_wait_and_barrier<63>();
                     // (reads pinned behind the instruction that frees their registers; B first, each next k-step needs all of it)
@@ -545,32 +644,34 @@ __global__ void __launch_bounds__(Cfg::THREADS) gemm_tile_ring_kernel(const Tile
                         if constexpr (x < NB || x == AL || (j == NB - 1 && i < MB - 1)) {
                             __builtin_amdgcn_sched_barrier(0);
                             if constexpr (x < NB)
-                                read_b(SET ^ 1, x, rs, rb);
+                                read_b(SET ^ 1, x, rs, rb, rsc);
                             if constexpr (x == AL)
-                                read_a(SET ^ 1, MB - 1, rs, rb);
+                                read_a(SET ^ 1, MB - 1, rs, rb, rsc);
                             if constexpr (j == NB - 1 && i < MB - 1)
-                                read_a(0, i, rs, rb);
+                                read_a(0, i, rs, rb, rsc);
                             __builtin_amdgcn_sched_barrier(0);
                         }
                     });
                 });
                 buf = nbuf;
+                ++st;
+                rows = next_rows;
+                next_rows = scale_rows(st + 1);
             };
             auto last = [&](auto parc) __attribute__((always_inline)) {
                 static_for<Cfg::KSTEPS>([&](auto sc) {
                     constexpr int s = decltype(sc)::value, SET = (decltype(parc)::value + s) & 1;
                     if constexpr (s > 0)
-                        read_all(SET, s, buf);
+                        read_all(SET, s, buf, rows);
                     tail_step(SET, s);
                 });
             };
             if constexpr (Cfg::KSTEPS % 2 == 0) {
-                for (int st = 0; st < nst - 1; ++st)
+                while (st < nst - 1)
                     body(integral_constant<int, 0>{});
                 last(integral_constant<int, 0>{});
             } else {  // the register sets change places from stage to stage
-                int st = 0;
-                for (; st + 2 < nst; st += 2) {
+                while (st + 2 < nst) {
                     body(integral_constant<int, 0>{});
                     body(integral_constant<int, 1>{});
                 }

@@ -138,6 +138,29 @@ def test_block_scaled_types(pa, oracle, ta, tb, shape):  # noqa: F811
                         max_rel=1e-4 if fp4 else 1e-3, eps=None if fp4 else 2.0 ** -11)
 
 
+@pytest.mark.parametrize("shape", range(7))
+@pytest.mark.parametrize("fp4", [False, True])
+def test_block_scales_over_several_chunks(pa, oracle, fp4, shape):  # noqa: F811
+    """Scales are copied 1024 or 2048 elements of K at a time: K of several such chunks, the last one short, its rows' scales
+    ending on 16 bytes and off them; and rows of scales shorter than 16 bytes."""
+    r = np.random.default_rng(400 + shape)
+    bm, bn = SHAPES[shape][:2]
+    t = ob.E2M1 if fp4 else ob.E4M3
+    for m, n, k in ((bm + 1, bn - 1, 2560), (bm - 1, bn + 3, 6400 if fp4 else 6272), (bm, bn + 1, 256), (1, bn + 1, 256 if fp4 else 384)):
+        one = 2 if fp4 else 0x38  # 1.0; the sign bit of a random half of the codes
+        a, b = ((one | (r.integers(0, 2, (x, k)) << (3 if fp4 else 7))).astype(np.uint8) for x in (m, n))
+        if fp4:
+            a, b = ((x[:, 0::2] | (x[:, 1::2] << 4)).astype(np.uint8) for x in (a, b))
+        sa, sb = (r.integers(120, 135, (x, k // 32)).astype(np.uint8) for x in (m, n))
+        with tile_env(PTOAMD_RING=shape):
+            got = host(pa.gemm_mx(dev(a), dev(b), dev(sa), dev(sb), m, n, k, PA_T[t], PA_T[t], pa.F32))
+            assert pa.last_kernel().startswith(f"tile{bm}x{bn}_dtl"), pa.last_kernel()
+        ua, ub = (_mx_unpack(oracle, x, t) * np.repeat(2.0 ** (s.astype(np.float64) - 127), 32, 1) for x, s in ((a, sa), (b, sb)))
+        # (bounds as in test_block_scaled_types)
+        check_f32_drain(got, ua @ ub.T, np.abs(ua) @ np.abs(ub).T, k, f"{m}x{n}x{k} shape {shape} fp4 {fp4}",
+                        max_rel=1e-4 if fp4 else 1e-3, eps=None if fp4 else 2.0 ** -11)
+
+
 def _fp8_operands(r, ta, tb, m, n, k):
     """Codes without NaN and infinities, on the device with rows at a wider pitch whose other bytes are NaN codes."""
     a, _, _, _ = _mx_inputs(r, ta, m, n, k)
