@@ -315,9 +315,11 @@ struct TileCfg {
     static constexpr int SLAB = 128;                              // bytes of K per slab row
     static constexpr int KSTEPS = SLAB / (LG * Op::FRAG_BYTES);
     static constexpr int A_BYTES = BM * SLAB, B_BYTES = BN * SLAB, STAGE_BYTES = A_BYTES + B_BYTES;
-    // the direct-to-LDS kernel of a block-scaled operand type keeps two buffers of 16 scale bytes per tile row behind
-    // the operand ring
-    static constexpr int SCALE_BYTES = Op::SCALED ? 2 * (BM + BN) * 16 : 0;
+    // the direct-to-LDS kernel of a block-scaled operand type keeps two buffers of SCALE_CHUNK scale bytes per tile row behind
+    // the operand ring.  fp8 takes 32 bytes where they fit: a copy costs the lines it touches, and 16 bytes of a row touch as many
+    // (MXFP8 4096 x 14336 x 4096 193.4 -> 191.8 us); fp4, whose slab takes 8 of them, is no faster with 32 (75.6 against 74.5 us).
+    static constexpr int SCALE_CHUNK = Op::SCALED && Op::GROUPS_PER_SLAB == 4 && RING * STAGE_BYTES + 2 * (BM + BN) * 32 <= 160 * 1024 ? 32 : 16;
+    static constexpr int SCALE_BYTES = Op::SCALED ? 2 * (BM + BN) * SCALE_CHUNK : 0;
     static constexpr int LDS_BYTES = RING * STAGE_BYTES + SCALE_BYTES;
     static_assert(LDS_BYTES <= 160 * 1024, "the ring and the scale buffers fit the CU's LDS");
     static constexpr int LA = BM * 8 / THREADS, LB = BN * 8 / THREADS;  // 16-byte chunks per thread per slab

@@ -181,14 +181,15 @@ __global__ void __launch_bounds__(Cfg::THREADS) gemm_tile_dtl_kernel(const TileG
 
     // ---- MX block scales.  A lane needs the E8M0 bytes of its own rows, 4 (fp8) or 8 (fp4) per row per slab; fetched
     // per lane from global memory they are 64 separate small requests per load instruction and keep the CU's address
-    // unit busier than the operand DMAs do.  Instead the 16 scale bytes of every row of the tile -- SPG slabs' worth --
-    // are DMAed into one of two LDS scale buffers, one instruction per 64 rows, and each wave reads the dwords of its
+    // unit busier than the operand DMAs do.  Instead the next 16 or 32 scale bytes of every row of the tile -- SPG slabs' worth --
+    // are DMAed into one of two LDS scale buffers, one instruction per KiB, and each wave reads the dwords of its
     // rows from there.  Chunk g + 1 is requested when slab g * SPG starts and read from the last k-step of
     // slab (g + 1) * SPG - 1 on, i.e. at least one slab barrier (with its vmcnt(0)) later.
     constexpr int GPS = Op::SCALED ? Op::GROUPS_PER_SLAB : 4;  // scale bytes per row per slab
-    constexpr int SW = GPS / 4, SPG = 16 / GPS;
-    constexpr int SROWS = BM + BN, NSI = SROWS / 64, NW = NT / 64, NSW = (NSI + NW - 1) / NW;
-    static_assert(SROWS % 64 == 0 && BM % 64 == 0, "one scale DMA covers 64 rows of one operand");
+    constexpr int CB = Cfg::SCALE_CHUNK, SW = GPS / 4, SPG = CB / GPS, CL = CB / 16;  // bytes per row and chunk; lanes that copy them
+    constexpr int SROWS = BM + BN, NSI = SROWS * CL / 64, NW = NT / 64, NSW = (NSI + NW - 1) / NW;
+    static_assert(SROWS * CL % 64 == 0 && BM * CL % 64 == 0, "one scale DMA covers rows of one operand");
+    auto scale_swizzle = [](int row) { return CL == 1 ? 0 : ((row >> 3) & 1) * 16; };
     // The scale dwords of slab kt + 1 are read one k-step ahead (after slab kt's barrier), so that the slab's first
     // MFMA does not wait for an LDS round trip.  PTOAMD_SCALES_AT_SLAB_START reads them when the slab starts instead
     // (one register set fewer) for the 32-byte fragments of a large wave tile.
@@ -213,7 +214,7 @@ __global__ void __launch_bounds__(Cfg::THREADS) gemm_tile_dtl_kernel(const TileG
     if (has_scales) {
 #pragma unroll
         for (int w = 0; w < NSW; ++w) {
-            const int r = (wave + w * NW) * 64 + lane;  // row of [A rows | B rows]; past the end for idle waves (unused)
+            const int r = ((wave + w * NW) * 64 + lane) / CL;  // row of [A rows | B rows]; past the end for idle waves (unused)
             sc_src[w] = r < BM ? p.sa + (long)min(m0 + r, p.m - 1) * p.scale_ld
                                : p.sb + (long)min(n0 + max(r - BM, 0), p.n - 1) * p.scale_ld;
         }
@@ -223,8 +224,9 @@ __global__ void __launch_bounds__(Cfg::THREADS) gemm_tile_dtl_kernel(const TileG
 #pragma unroll
             for (int w = 0; w < NSW; ++w) {
                 const int i = wave + w * NW;
+                const int at = CL == 1 ? g * 16 : min(g * CB + ((lane % CL * 16) ^ scale_swizzle(lane / CL)), p.scale_ld - 16);
                 if (i < NSI)
-                    lds_dma16(sc_src[w] + (long)g * 16, lds_scales + (g & 1) * (SROWS * 16) + i * 1024);
+                    lds_dma16(sc_src[w] + at, lds_scales + (g & 1) * (SROWS * CB) + i * 1024);
             }
         }
     };
@@ -234,15 +236,16 @@ __global__ void __launch_bounds__(Cfg::THREADS) gemm_tile_dtl_kernel(const TileG
     // with E8M0 127 once, in the prologue.)
     auto read_scales = [&](int kt) __attribute__((always_inline)) {
         if (Op::SCALED) {
-            const uint8_t* base = smem + RING * Cfg::STAGE_BYTES + ((kt / SPG) & 1) * (SROWS * 16) + (kt % SPG) * GPS;
+            const uint8_t* base = smem + RING * Cfg::STAGE_BYTES + ((kt / SPG) & 1) * (SROWS * CB);
+            const uint32_t at = (l32 * CB + scale_swizzle(l32)) ^ ((kt % SPG) * GPS);
 #pragma unroll
             for (int w = 0; w < SW; ++w) {
 #pragma unroll
                 for (int i = 0; i < MB; ++i)
-                    sca_n[i][w] = *reinterpret_cast<const uint32_t*>(base + (wm * Cfg::WTM + i * BLK + l32) * 16 + w * 4);
+                    sca_n[i][w] = *reinterpret_cast<const uint32_t*>(base + at + (wm * Cfg::WTM + i * BLK) * CB + w * 4);
 #pragma unroll
                 for (int j = 0; j < NB; ++j)
-                    scb_n[j][w] = *reinterpret_cast<const uint32_t*>(base + (BM + wn * Cfg::WTN + j * BLK + l32) * 16 + w * 4);
+                    scb_n[j][w] = *reinterpret_cast<const uint32_t*>(base + at + (BM + wn * Cfg::WTN + j * BLK) * CB + w * 4);
             }
         }
     };
@@ -361,7 +364,7 @@ __global__ void __launch_bounds__(Cfg::THREADS) gemm_tile_dtl_kernel(const TileG
     tload(0, 0);
     tload_scales(0);
     if (Op::SCALED && !has_scales) {
-        for (int o = tid * 16; o < 2 * SROWS * 16; o += NT * 16)
+        for (int o = tid * 16; o < 2 * SROWS * CB; o += NT * 16)
             *reinterpret_cast<uint4*>(smem + RING * Cfg::STAGE_BYTES + o) = make_uint4(0x7F7F7F7Fu, 0x7F7F7F7Fu, 0x7F7F7F7Fu, 0x7F7F7F7Fu);
     }
     // slab 1's first DMAs go out now but only slab 0 (and the scales) are waited for: the counter retires loads in

@@ -161,6 +161,20 @@ def test_block_scales_over_several_chunks(pa, oracle, fp4, shape):  # noqa: F811
                         max_rel=1e-4 if fp4 else 1e-3, eps=None if fp4 else 2.0 ** -11)
 
 
+@pytest.mark.parametrize("tile", [4, 5, 7])
+@pytest.mark.parametrize("k", [512, 1536, 2560])
+def test_block_scales_of_the_two_and_three_slab_tiles(pa, oracle, tile, k):  # noqa: F811
+    """fp8 scales are copied 1024 elements of K at a time where they fit: half a chunk, one and a half, two and a half."""
+    r = np.random.default_rng(tile + k)
+    m, n = 259, 261
+    a, b, sa, sb = _mx_inputs(r, ob.E4M3, m, n, k)
+    with tile_env(PTOAMD_TILE=tile):
+        got = host(pa.gemm_mx(dev(a), dev(b), dev(sa), dev(sb), m, n, k, pa.E4M3, pa.E4M3, pa.F32))
+        assert "_dtl_fp8" in pa.last_kernel(), pa.last_kernel()
+    ua, ub = (_mx_unpack(oracle, x, ob.E4M3) * np.repeat(2.0 ** (s.astype(np.float64) - 127), 32, 1) for x, s in ((a, sa), (b, sb)))
+    check_f32_drain(got, ua @ ub.T, np.abs(ua) @ np.abs(ub).T, k, f"{m}x{n}x{k} tile {tile}", max_rel=1e-3, eps=2.0 ** -11)
+
+
 def _fp8_operands(r, ta, tb, m, n, k):
     """Codes without NaN and infinities, on the device with rows at a wider pitch whose other bytes are NaN codes."""
     a, _, _, _ = _mx_inputs(r, ta, m, n, k)
