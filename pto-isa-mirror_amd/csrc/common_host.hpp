@@ -2,7 +2,10 @@
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdarg.h>
+#include <stdint.h>
 #include <stdio.h>
+
+#include <atomic>
 
 #include "../../include/ptoamd.h"
 
@@ -10,8 +13,24 @@ namespace ptoamd {
 
 void set_error(const char* fmt, ...);
 void set_last_kernel(const char* name);
-// sets hipFuncAttributeMaxDynamicSharedMemorySize once per (kernel, current device); thread-safe
-hipError_t ensure_dynamic_lds(const void* kernel, int bytes);
+// The kernel of a matmul by what its name is made of: spelling it on every launch took 0.2 us.
+struct KernelName {
+    const char* (*spell)(int tile, int op, bool row_major_b);
+    int tile, op;
+    bool row_major_b;
+};
+void set_last_kernel(const KernelName& name);
+// Sets hipFuncAttributeMaxDynamicSharedMemorySize of one kernel once per current device; thread-safe, one object per kernel.
+struct DynamicLds {
+    std::atomic<uint64_t> devices{0};  // those it is set on
+    hipError_t allow(const void* kernel, int bytes);
+};
+template <auto* KERNEL>
+hipError_t ensure_dynamic_lds(int bytes)
+{
+    static DynamicLds lds;
+    return lds.allow(reinterpret_cast<const void*>(KERNEL), bytes);
+}
 
 // Everything a first launch would otherwise set up lazily, done for the current device: the dynamic-LDS attribute of
 // every tile and GEMV kernel and the device address of the library's static scratch array.  After it, no entry point

@@ -596,7 +596,7 @@ static int tile_as_launched(int tile, int op, int m, int n)
     return tile == 3 ? 4 : tile;
 }
 
-static const char* tile_kernel_name(int tile, int op, bool row_major_b = false)
+static const char* tile_kernel_name(int tile, int op, bool row_major_b)
 {
     static const char* ops[TOP_COUNT] = {"bf16", "f16", "i8", "fp8_e4m3_e4m3", "fp8_e5m2_e5m2", "fp8_e4m3_e5m2",
                                          "fp8_e5m2_e4m3", "fp4_e2m1"};
@@ -880,7 +880,7 @@ static int gemm_common(void* c, int c_type, const void* a, const void* b, int ab
                      : options().tile < 0 && any_ok ? pick_dma_tile(m, n, k_bytes, op, {DTL_NONE, drain, true, STAGED_COLUMN_MAJOR_B})
                                                     : pick_tile(m, n, k_bytes, false, dma_ok, ragged_k_form);
     PTOAMD_HIP_CHECK(launch_tiles(tile, op, p, stream));
-    set_last_kernel(tile_kernel_name(tile_as_launched(tile, op, m, n), op, nd_direct));
+    set_last_kernel(KernelName{tile_kernel_name, tile_as_launched(tile, op, m, n), op, nd_direct});
     return PTOAMD_OK;
 }
 
@@ -922,7 +922,7 @@ int ptoamd_gemm_w8a8(void* out_bf16, int32_t* acc_out, const int8_t* a, const in
                      : options().tile < 0 && any_ok ? pick_dma_tile(m, n, k, TOP_I8, {DTL_NONE, drain, true, STAGED_COLUMN_MAJOR_B})
                                                     : pick_tile(m, n, k, false, dma_ok, true);
     PTOAMD_HIP_CHECK(launch_tiles(tile, TOP_I8, p, stream));
-    set_last_kernel(tile_kernel_name(tile, TOP_I8));
+    set_last_kernel(KernelName{tile_kernel_name, tile, TOP_I8, false});
     return PTOAMD_OK;
 }
 
@@ -1068,7 +1068,7 @@ static int gemm_mx_common(const char* who, void* c, int c_type, const void* a, c
                      : options().tile < 0 && dma_ok && (kg % 4) == 0 ? pick_dma_tile(m, n, k_bytes, op, {scale_dma_ok ? DTL_ALL : DTL_NONE, c_in ? DRAIN_ACC_IN : DRAIN_PLAIN, false, STAGED_COLUMN_MAJOR_B})
                                                                     : pick_tile(m, n, k_bytes, true, dma_ok && scale_dma_ok);
     PTOAMD_HIP_CHECK(launch_tiles(tile, op, p, stream));
-    set_last_kernel(tile_kernel_name(tile_as_launched(tile, op, m, n), op));
+    set_last_kernel(KernelName{tile_kernel_name, tile_as_launched(tile, op, m, n), op, false});
     return PTOAMD_OK;
 }
 

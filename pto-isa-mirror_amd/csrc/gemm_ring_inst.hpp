@@ -9,7 +9,7 @@ namespace ptoamd {
 template <class Cfg>
 static hipError_t launch_ring(const TileGemmParams& p, hipStream_t stream)
 {
-    const hipError_t e = ensure_dynamic_lds(reinterpret_cast<const void*>(&gemm_tile_ring_kernel<Cfg>), Cfg::LDS_BYTES);
+    const hipError_t e = ensure_dynamic_lds<&gemm_tile_ring_kernel<Cfg>>(Cfg::LDS_BYTES);
     if (e != hipSuccess || p.m <= 0)  // m = 0: only make the kernel ready to launch on the current device
         return e;
     const RingTiles tiles = ring_tiles(p, Cfg::BM, Cfg::BN);

@@ -10,9 +10,9 @@ namespace ptoamd {
 template <class Cfg>
 static hipError_t launch_cfg(const TileGemmParams& p, hipStream_t stream)
 {
-    hipError_t e = ensure_dynamic_lds(reinterpret_cast<const void*>(&gemm_tile_kernel<Cfg, false>), Cfg::LDS_BYTES);
+    hipError_t e = ensure_dynamic_lds<&gemm_tile_kernel<Cfg, false>>(Cfg::LDS_BYTES);
     if (e == hipSuccess)
-        e = ensure_dynamic_lds(reinterpret_cast<const void*>(&gemm_tile_kernel<Cfg, true>), Cfg::LDS_BYTES);
+        e = ensure_dynamic_lds<&gemm_tile_kernel<Cfg, true>>(Cfg::LDS_BYTES);
     if (e != hipSuccess || p.m <= 0)  // m = 0: only make the kernels ready to launch on the current device
         return e;
     const int tiles = ((p.m + Cfg::BM - 1) / Cfg::BM) * ((p.n + Cfg::BN - 1) / Cfg::BN);
@@ -31,14 +31,14 @@ static hipError_t launch_cfg(const TileGemmParams& p, hipStream_t stream)
 template <class Cfg, bool RAGGED_K = false, bool ROW_MAJOR_B = false>
 static hipError_t launch_dtl(const TileGemmParams& p, hipStream_t stream)
 {
-    hipError_t e = ensure_dynamic_lds(reinterpret_cast<const void*>(&gemm_tile_dtl_kernel<Cfg, false>), Cfg::LDS_BYTES);
+    hipError_t e = ensure_dynamic_lds<&gemm_tile_dtl_kernel<Cfg, false>>(Cfg::LDS_BYTES);
     if constexpr (RAGGED_K) {
         if (e == hipSuccess)
-            e = ensure_dynamic_lds(reinterpret_cast<const void*>(&gemm_tile_dtl_kernel<Cfg, true>), Cfg::LDS_BYTES);
+            e = ensure_dynamic_lds<&gemm_tile_dtl_kernel<Cfg, true>>(Cfg::LDS_BYTES);
     }
     if constexpr (ROW_MAJOR_B) {
         if (e == hipSuccess)
-            e = ensure_dynamic_lds(reinterpret_cast<const void*>(&gemm_tile_dtl_kernel<Cfg, false, true>), Cfg::LDS_BYTES);
+            e = ensure_dynamic_lds<&gemm_tile_dtl_kernel<Cfg, false, true>>(Cfg::LDS_BYTES);
     }
     if (e != hipSuccess || p.m <= 0)
         return e;
@@ -67,7 +67,7 @@ static hipError_t launch_dtl(const TileGemmParams& p, hipStream_t stream)
 template <class Cfg>
 static hipError_t launch_mx16(const TileGemmParams& p, hipStream_t stream)
 {
-    const hipError_t e = ensure_dynamic_lds(reinterpret_cast<const void*>(&gemm_tile_mx16_kernel<Cfg>), Cfg::LDS_BYTES);
+    const hipError_t e = ensure_dynamic_lds<&gemm_tile_mx16_kernel<Cfg>>(Cfg::LDS_BYTES);
     if (e != hipSuccess || p.m <= 0)
         return e;
     if (p.k_bytes % 128 != 0)

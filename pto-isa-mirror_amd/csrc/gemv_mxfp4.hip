@@ -665,13 +665,13 @@ __global__ void __launch_bounds__(256) gemv_mxfp4_pack_kernel(uint8_t* __restric
 
 int prepare_gemv_kernels()
 {
-    PTOAMD_HIP_CHECK(ensure_dynamic_lds(reinterpret_cast<const void*>(gemv_mxfp4_splitk_wide_kernel<true, true>), WD_LDS));
-    PTOAMD_HIP_CHECK(ensure_dynamic_lds(reinterpret_cast<const void*>(gemv_mxfp4_splitk_wide_kernel<false>), WD_LDS));
-    PTOAMD_HIP_CHECK(ensure_dynamic_lds(reinterpret_cast<const void*>(gemv_mxfp4_splitk_wide_kernel<true>), WD_LDS));
-    PTOAMD_HIP_CHECK(ensure_dynamic_lds(reinterpret_cast<const void*>(gemv_mxfp4_splitk_wide_kernel<false, false, true>), WD_LDS));
-    PTOAMD_HIP_CHECK(ensure_dynamic_lds(reinterpret_cast<const void*>(gemv_mxfp4_splitk_wide_kernel<true, false, true>), WD_LDS));
-    PTOAMD_HIP_CHECK(ensure_dynamic_lds(reinterpret_cast<const void*>(gemv_mxfp4_splitk_kernel<false>), SK_LDS));
-    PTOAMD_HIP_CHECK(ensure_dynamic_lds(reinterpret_cast<const void*>(gemv_mxfp4_splitk_kernel<true>), SK_LDS));
+    PTOAMD_HIP_CHECK((ensure_dynamic_lds<&gemv_mxfp4_splitk_wide_kernel<true, true>>(WD_LDS)));
+    PTOAMD_HIP_CHECK((ensure_dynamic_lds<&gemv_mxfp4_splitk_wide_kernel<false>>(WD_LDS)));
+    PTOAMD_HIP_CHECK((ensure_dynamic_lds<&gemv_mxfp4_splitk_wide_kernel<true>>(WD_LDS)));
+    PTOAMD_HIP_CHECK((ensure_dynamic_lds<&gemv_mxfp4_splitk_wide_kernel<false, false, true>>(WD_LDS)));
+    PTOAMD_HIP_CHECK((ensure_dynamic_lds<&gemv_mxfp4_splitk_wide_kernel<true, false, true>>(WD_LDS)));
+    PTOAMD_HIP_CHECK((ensure_dynamic_lds<&gemv_mxfp4_splitk_kernel<false>>(SK_LDS)));
+    PTOAMD_HIP_CHECK((ensure_dynamic_lds<&gemv_mxfp4_splitk_kernel<true>>(SK_LDS)));
     return PTOAMD_OK;
 }
 
@@ -732,7 +732,10 @@ extern "C" int ptoamd_gemv_mxfp4(void* out, int c_type, const void* a_bf16, cons
         const int grid = (p.n_groups + spw - 1) / spw;
         const auto fn = partial ? (swc ? gemv_mxfp4_splitk_wide_kernel<false, false, true> : gemv_mxfp4_splitk_wide_kernel<true, false, true>)
                                 : (swc ? gemv_mxfp4_splitk_wide_kernel<false> : gemv_mxfp4_splitk_wide_kernel<true>);
-        PTOAMD_HIP_CHECK(ensure_dynamic_lds(reinterpret_cast<const void*>(fn), WD_LDS));
+        PTOAMD_HIP_CHECK((partial ? (swc ? ensure_dynamic_lds<&gemv_mxfp4_splitk_wide_kernel<false, false, true>>(WD_LDS)
+                                        : ensure_dynamic_lds<&gemv_mxfp4_splitk_wide_kernel<true, false, true>>(WD_LDS))
+                                 : (swc ? ensure_dynamic_lds<&gemv_mxfp4_splitk_wide_kernel<false>>(WD_LDS)
+                                        : ensure_dynamic_lds<&gemv_mxfp4_splitk_wide_kernel<true>>(WD_LDS))));
         hipLaunchKernelGGL(fn, dim3(grid), dim3(512), WD_LDS, stream, p, spw);
         PTOAMD_HIP_CHECK(hipGetLastError());
         set_last_kernel(swc ? "gemv_mxfp4_splitk_wide_swcvt" : "gemv_mxfp4_splitk_wide");
@@ -748,9 +751,7 @@ extern "C" int ptoamd_gemv_mxfp4(void* out, int c_type, const void* a_bf16, cons
         int spw = (p.n_groups + cus - 1) / cus;          // strips per workgroup, a multiple of the row-group count
         spw = (spw + rgs - 1) / rgs * rgs;
         const int grid = (p.n_groups + spw - 1) / spw;
-        const void* fn = swc ? reinterpret_cast<const void*>(gemv_mxfp4_splitk_kernel<false>)
-                             : reinterpret_cast<const void*>(gemv_mxfp4_splitk_kernel<true>);
-        PTOAMD_HIP_CHECK(ensure_dynamic_lds(fn, SK_LDS));
+        PTOAMD_HIP_CHECK((swc ? ensure_dynamic_lds<&gemv_mxfp4_splitk_kernel<false>>(SK_LDS) : ensure_dynamic_lds<&gemv_mxfp4_splitk_kernel<true>>(SK_LDS)));
         if (swc)
             hipLaunchKernelGGL(gemv_mxfp4_splitk_kernel<false>, dim3(grid), dim3(SK_WAVES * 64), SK_LDS, stream, p, ksw_log2, spw);
         else
@@ -832,7 +833,7 @@ extern "C" int ptoamd_gemv_mxfp4_packed(void* out, int c_type, const void* a_bf1
     const int cus = device_compute_units();
     const int spw = (p.n_groups + cus - 1) / cus;
     const int grid = (p.n_groups + spw - 1) / spw;
-    PTOAMD_HIP_CHECK(ensure_dynamic_lds(reinterpret_cast<const void*>(gemv_mxfp4_splitk_wide_kernel<true, true>), WD_LDS));
+    PTOAMD_HIP_CHECK((ensure_dynamic_lds<&gemv_mxfp4_splitk_wide_kernel<true, true>>(WD_LDS)));
     hipLaunchKernelGGL((gemv_mxfp4_splitk_wide_kernel<true, true>), dim3(grid), dim3(512), WD_LDS, stream, p, spw);
     PTOAMD_HIP_CHECK(hipGetLastError());
     set_last_kernel("gemv_mxfp4_splitk_wide_packed");

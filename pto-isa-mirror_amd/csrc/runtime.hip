@@ -8,8 +8,6 @@
 
 #include <atomic>
 #include <mutex>
-#include <set>
-#include <utility>
 
 #include "common_host.hpp"
 
@@ -25,11 +23,24 @@ void set_error(const char* fmt, ...)
     va_end(ap);
 }
 static thread_local unsigned long g_launches = 0;
+static thread_local KernelName g_kernel_name{};  // spelled out into g_kernel when somebody asks
 void set_last_kernel(const char* name)
 {
     strncpy(g_kernel, name, sizeof g_kernel - 1);
     g_kernel[sizeof g_kernel - 1] = 0;
+    g_kernel_name.spell = nullptr;
     ++g_launches;
+}
+void set_last_kernel(const KernelName& name)
+{
+    g_kernel_name = name;
+    ++g_launches;
+}
+static const char* last_kernel()
+{
+    if (g_kernel_name.spell != nullptr)
+        set_last_kernel(g_kernel_name.spell(g_kernel_name.tile, g_kernel_name.op, g_kernel_name.row_major_b)), --g_launches;
+    return g_kernel;
 }
 
 // ---- environment switches ---------------------------------------------------------------------------------------------
@@ -178,7 +189,7 @@ TraceScope::~TraceScope()
     TraceSink& sink = trace_sink();
     std::lock_guard<std::mutex> lock(sink.mu);
     fprintf(sink.file, "{\"sequence_id\": %lu, \"opcode\": \"%s\", \"pipeline\": \"%s\", \"kernel\": \"%s\", \"m\": %ld, \"n\": %ld, \"k\": %ld",
-            sink.sequence++, opcode_, pipeline_, g_kernel, m_, n_, k_);
+            sink.sequence++, opcode_, pipeline_, last_kernel(), m_, n_, k_);
     for (int side = 0; side < 2; ++side) {
         const Tile* t = side == 0 ? in_ : out_;
         const int cnt = side == 0 ? nin_ : nout_;
@@ -194,21 +205,20 @@ TraceScope::~TraceScope()
 
 // hipFuncAttributeMaxDynamicSharedMemorySize is a property of (kernel, device): it is set once per pair, under a lock,
 // so that launches from several host threads or on several devices of one process all see it.
-hipError_t ensure_dynamic_lds(const void* kernel, int bytes)
+hipError_t DynamicLds::allow(const void* kernel, int bytes)
 {
-    static std::mutex mu;
-    static std::set<std::pair<int, const void*>> done;
     int dev = 0;
     hipError_t e = hipGetDevice(&dev);
     if (e != hipSuccess)
         return e;
-    std::lock_guard<std::mutex> lock(mu);
-    const auto key = std::make_pair(dev, kernel);
-    if (done.count(key))
+    const uint64_t bit = dev < 64 ? 1ull << dev : 0;  // (devices past 64 set it on every call)
+    if (devices.load(std::memory_order_acquire) & bit)
         return hipSuccess;
+    static std::mutex mu;
+    std::lock_guard<std::mutex> lock(mu);
     e = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
     if (e == hipSuccess)
-        done.insert(key);
+        devices.fetch_or(bit, std::memory_order_release);
     return e;
 }
 }  // namespace ptoamd
@@ -218,7 +228,7 @@ using namespace ptoamd;
 extern "C" {
 
 const char* ptoamd_last_error(void) { return g_error; }
-const char* ptoamd_last_kernel(void) { return g_kernel; }
+const char* ptoamd_last_kernel(void) { return last_kernel(); }
 
 int ptoamd_init(int device)
 {
