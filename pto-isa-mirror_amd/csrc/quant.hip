@@ -14,6 +14,19 @@ static_assert(PTOAMD_OCP_MXFP8 == MX_OCP_FP8 && PTOAMD_NV_MXFP8 == MX_NV_FP8 && 
                   PTOAMD_NV_MXFP4 == MX_NV_FP4,
               "the C ABI's algorithm ids are the kernels' template arguments");
 
+// The largest of 4 or 8 neighbouring lanes' values, in all of them: lane ^ 1 and lane ^ 2 by quad permutations; then a quad agrees,
+// and the mirror of eight lanes brings the other quad's.
+template <int ALG, int LANES>
+__device__ __forceinline__ uint32_t group_max(uint32_t run)
+{
+    static_assert(LANES == 4 || LANES == 8, "a group of 32 is four or eight pieces of 16 bytes");
+    run = max_merge<ALG>(run, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)run, 0xB1, 0xF, 0xF, true));
+    run = max_merge<ALG>(run, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)run, 0x4E, 0xF, 0xF, true));
+    if (LANES == 8)
+        run = max_merge<ALG>(run, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)run, 0x141, 0xF, 0xF, true));
+    return run;
+}
+
 // ---- axis 1: 32-element groups along a row.  A lane owns one 16-byte piece of the source (4 f32 or 8 half / bf16
 // elements), so a group is 8 or 4 neighbouring lanes and a wave reads 1 KiB per load instruction; every thread handles
 // UNITS such pieces, one block-wide span apart, with all its loads in flight before the first is used.
@@ -24,11 +37,11 @@ static_assert(PTOAMD_OCP_MXFP8 == MX_OCP_FP8 && PTOAMD_NV_MXFP8 == MX_NV_FP8 && 
 // NaN scaling) are resolved per group last.  The bf16 source's re-rounding of
 // the scaled value (TQuant.hpp:68-76) is the identity here: the scaling is a power of two, so the product of a bf16
 // value is a bf16 value again unless it is subnormal, and then it is far below the smallest code either way.
-template <int ALG, typename T, bool SRC_BF16>
+template <int ALG, typename T, bool SRC_BF16, int UNITS>
 __global__ void __launch_bounds__(256) tquant_mx_rows_kernel(uint8_t* dst, uint8_t* exp, float* mx, float* scaling, const T* src, long units)
 {
     constexpr bool FP4 = ALG == PTOAMD_OCP_MXFP4 || ALG == PTOAMD_NV_MXFP4;
-    constexpr int EPL = 16 / (int)sizeof(T), LPG = 32 / EPL, UNITS = 4;
+    constexpr int EPL = 16 / (int)sizeof(T), LPG = 32 / EPL;
     const long first = (long)blockIdx.x * (UNITS * 256) + threadIdx.x;
     uint4 raw[UNITS];
 #pragma unroll
@@ -56,9 +69,7 @@ __global__ void __launch_bounds__(256) tquant_mx_rows_kernel(uint8_t* dst, uint8
 #pragma unroll
         for (int i = 0; i < EPL; ++i)
             run = max_step<ALG>(run, v[i], (int)(threadIdx.x & (LPG - 1)) * EPL + i);
-#pragma unroll
-        for (int off = 1; off < LPG; off <<= 1)
-            run = max_merge<ALG>(run, (uint32_t)__shfl_xor((int)run, off, LPG));
+        run = group_max<ALG, LPG>(run);
         const float maxabs = max_value<ALG>(run);
         const uint32_t e = shared_exponent<ALG>(maxabs);
         const float sc = group_scaling<ALG>(maxabs, e);
@@ -283,6 +294,10 @@ __global__ void tdequant_kernel(float* dst, const T* src, const float* scale, co
     dst[idx] = __fmul_rn(__fsub_rn((float)src[idx], offset[pi]), scale[pi]);
 }
 
+// Up to 16 MiB of source one piece per thread, beyond it two: what a small matrix waits for is the chain of one piece (bf16 to MXFP8,
+// 384 x 4096: 2.5 us with one, 2.9 with two, 3.7 with four); a large one is bound by its streams and better off with two loads in
+// flight (4096 x 4096 f32: 16.4, 15.4, 15.3 us; 28672 x 8192 bf16 to MXFP4: 118, 115, 120).
+constexpr long TQUANT_ONE_PIECE = 1 << 20;
 template <int ALG, typename T, bool SRC_BF16>
 static int launch_tquant_mx(uint8_t* dst, uint8_t* exp, float* mx, float* scaling, const void* src, int rows, int cols,
                             int axis, hipStream_t stream)
@@ -290,8 +305,12 @@ static int launch_tquant_mx(uint8_t* dst, uint8_t* exp, float* mx, float* scalin
     const T* s = reinterpret_cast<const T*>(src);
     if (axis == 1) {
         const long units = (long)rows * cols * (long)sizeof(T) / 16;  // 16-byte pieces; a row is a whole number of them
-        hipLaunchKernelGGL((tquant_mx_rows_kernel<ALG, T, SRC_BF16>), dim3((unsigned)((units + 1023) / 1024)), dim3(256),
-                           0, stream, dst, exp, mx, scaling, s, units);
+        if (units <= TQUANT_ONE_PIECE)
+            hipLaunchKernelGGL((tquant_mx_rows_kernel<ALG, T, SRC_BF16, 1>), dim3((unsigned)((units + 255) / 256)), dim3(256), 0, stream, dst, exp, mx,
+                               scaling, s, units);
+        else
+            hipLaunchKernelGGL((tquant_mx_rows_kernel<ALG, T, SRC_BF16, 2>), dim3((unsigned)((units + 511) / 512)), dim3(256), 0, stream, dst, exp,
+                               mx, scaling, s, units);
     } else {
         dim3 block(128), grid((cols / 2 + 127) / 128, rows / 32);
         hipLaunchKernelGGL((tquant_mx_cols_kernel<ALG, T, SRC_BF16>), grid, block, 0, stream, dst, exp, mx, scaling, s,
