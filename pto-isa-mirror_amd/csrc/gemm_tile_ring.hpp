@@ -22,6 +22,10 @@
 //              A stage takes about twice as long as by LDS-DMA.
 //              Measured, bf16, against the register-staged tile chosen by grid size: 64 x 4097 x 4095 28 us (63), 1000 x 2049 x 2047
 //              33 (57; 2048 x 2048 by LDS-DMA: 17), 2100 x 2049 x 2047 43 (61), 4000 x 1025 x 4097 73 (110)
+//   rows on 16 bytes off the 128-byte lines (SKEW, plain types, shapes with four stages): a copy's cost is the lines it touches, and
+//              a stage of such a row lies across two per 128 bytes.  Each row's copies are cut at its lines instead, up to 112 bytes
+//              ahead of the row's k, so a stage is multiplied when the next one has landed as well.  bf16 1237 x 4100 x 2056 with
+//              bias and relu 32.2 -> 25.6 us, 24.3 where the pitch is a multiple of 128 bytes
 //   K tail     copies never read past a row: a chunk that would is read as the 16 bytes that END at the row's end, and the
 //              last stage's fragments are masked in registers -- the same bytes of A and B, so k positions still agree
 #pragma once
@@ -47,10 +51,10 @@ struct OpFP4x16 {
 };
 
 // WM x WN x WK waves: WK groups share the tile and split every stage of SB bytes per row along K; R stages in the ring
-template <int BM_, int BN_, int WM_, int WN_, int WK_, int SB_, int R_, int LW_, bool PIPE_, class Op_, bool BND_ = false, bool ANY_ = false>
+template <int BM_, int BN_, int WM_, int WN_, int WK_, int SB_, int R_, int LW_, bool PIPE_, class Op_, bool BND_ = false, bool ANY_ = false, bool SKEW_ = false>
 struct RingCfg {
     static constexpr int BM = BM_, BN = BN_, WM = WM_, WN = WN_, WK = WK_, SB = SB_, R = R_;
-    static constexpr bool PIPE = PIPE_, BND = BND_, ANY = ANY_;  // BND: B is row-major [K][N]; ANY: rows start on any byte
+    static constexpr bool PIPE = PIPE_, BND = BND_, ANY = ANY_, SKEW = SKEW_;  // B is row-major [K][N]; rows start on any byte; on any 16
     using Op = Op_;
     static constexpr int CW = WM * WN * WK, LW = LW_, THREADS = (CW + LW) * 64;
     static constexpr int NW = LW > 0 ? LW : CW;  // waves that copy
@@ -86,6 +90,7 @@ struct RingCfg {
     static_assert(KW % KB == 0 && SB <= 1024 && 1024 % SB == 0, "a k-group's part of a stage is whole k-steps");
     static_assert(PIECES % NW == 0 && (BM * SB) % 1024 == 0, "every wave issues the same number of 1 KiB copies, each of one operand");
     static_assert(!BND || (!Op::SCALED && FR == 1 && (NB & (NB - 1)) == 0), "the row-major form is for the 16-bit types");
+    static_assert(!SKEW || (PIPE && !BND && !ANY && !Op::SCALED && R >= 4), "two stages have to have landed where one is multiplied");
     static_assert(!ANY || (PIPE && !BND && !Op::SCALED), "the register copies are the copying waves' and know no scales");
     static_assert((ROWS * STAGE_SPS) % 64 == 0, "scale pieces are whole");
     static_assert(!CHUNKED || (SCB / 4 % SPS == 0 && (SBUFS - 1) * SPC >= R - 1 && BM * SCB % 1024 == 0 && BN * SCB % 1024 == 0 && ROWS <= NW * 64),
@@ -295,6 +300,7 @@ __global__ void __launch_bounds__(Cfg::THREADS) gemm_tile_ring_kernel(const Tile
 
     // ---- TLOAD addressing: piece w + q * NW of a stage, lane -> (row, position) linear, fetching chunk position ^ swizzle
     const int nst = (p.k_bytes + SB - 1) / SB;
+    const int ncopy = Cfg::SKEW ? (p.k_bytes + 7 * 16 + SB - 1) / SB : nst;  // stages copied
     const bool k_tail = p.k_bytes % SB != 0;
     const uint32_t lds0 = lds_address(smem);
     auto piece_row = [&](int q) { return (lw + q * NW) * Cfg::RPP + lane / CPR; };
@@ -309,10 +315,20 @@ __global__ void __launch_bounds__(Cfg::THREADS) gemm_tile_ring_kernel(const Tile
         const int chunk = (lane % Cfg::CB) ^ (swizzle_row_major<BN>(nd_row(q)) << 1);
         return (uint32_t)min(n0 * 2 + chunk * 16, p.n * 2 - 16);
     };
+    // SKEW: a stage of a row is whole 128-byte lines, so it starts `skew` chunks ahead of its own k.  Of the chunks of a stage's lines
+    // that belong to this k stage and to the one before, each stands where its k has it: fragment reads find it at the same place
+    // in either buffer, and their banks are those of rows that start on a line.
+    auto skewed_chunk = [&](int q) -> int {
+        if constexpr (!Cfg::SKEW)
+            return piece_chunk(q);
+        const int skew = ((uint32_t)(uintptr_t)(lw + q * NW < Cfg::A_PIECES ? p.a : p.b) + row_offset(q)) >> 4 & 7;
+        return (piece_chunk(q) + skew) % CPR - skew;
+    };
+    constexpr int LINE = Cfg::SKEW ? 128 : 0;  // (added to the lanes' offsets, taken off the base: they stay positive)
     uint32_t goff[NPW];
 #pragma unroll
     for (int q = 0; q < NPW; ++q)
-        goff[q] = Cfg::BND && lw + q * NW >= Cfg::A_PIECES ? (uint32_t)(nd_row(q) * p.ldb_bytes) + nd_col(q) : row_offset(q) + piece_chunk(q) * 16;
+        goff[q] = Cfg::BND && lw + q * NW >= Cfg::A_PIECES ? (uint32_t)(nd_row(q) * p.ldb_bytes) + nd_col(q) : row_offset(q) + skewed_chunk(q) * 16 + LINE;
     // Scales in the stage: dword e = row * STAGE_SPS + d; without scale arrays the copies fetch bytes of A that are not used.
     const bool has_scales = Op::SCALED && p.sa != nullptr;
     const uint8_t* sc_row[NSW > 0 ? NSW : 1];
@@ -373,7 +389,7 @@ __global__ void __launch_bounds__(Cfg::THREADS) gemm_tile_ring_kernel(const Tile
     auto issue = [&](int st, int buf) __attribute__((always_inline)) {
         const uint32_t dst = __builtin_amdgcn_readfirstlane(lds0 + buf * Cfg::STAGE);
         const long kb = (long)st * SB, kb_b = Cfg::BND ? (long)st * Cfg::KR * p.ldb_bytes : kb;
-        if (k_tail && st == nst - 1) {
+        if (Cfg::SKEW ? st == 0 || (st + 1) * SB > p.k_bytes : k_tail && st == nst - 1) {
 #pragma unroll
             for (int q = 0; q < NPW; ++q) {
                 const int piece = lw + q * NW;
@@ -384,14 +400,15 @@ __global__ void __launch_bounds__(Cfg::THREADS) gemm_tile_ring_kernel(const Tile
                     lds_dma16_off(p.b + (long)base_row * p.ldb_bytes, (uint32_t)((src - base_row) * p.ldb_bytes) + nd_col(q), dst + piece * 1024);
                     continue;
                 }
-                const uint32_t off = row_offset(q) + (uint32_t)min(st * SB + piece_chunk(q) * 16, p.k_bytes - 16);
+                const int at = min(st * SB + skewed_chunk(q) * 16, p.k_bytes - 16);
+                const uint32_t off = row_offset(q) + (uint32_t)(Cfg::SKEW ? max(at, 0) : at);
                 lds_dma16_off(piece < Cfg::A_PIECES ? p.a : p.b, off, dst + piece * 1024);
             }
         } else {
 #pragma unroll
             for (int q = 0; q < NPW; ++q) {
                 const int piece = lw + q * NW;
-                lds_dma16_off(piece < Cfg::A_PIECES ? p.a + kb : p.b + kb_b, goff[q], dst + piece * 1024);
+                lds_dma16_off((piece < Cfg::A_PIECES ? p.a + kb : p.b + kb_b) - LINE, goff[q], dst + piece * 1024);
             }
         }
         if constexpr (NSW > 0) {
@@ -446,7 +463,39 @@ __global__ void __launch_bounds__(Cfg::THREADS) gemm_tile_ring_kernel(const Tile
     uint4 fa[SETS][MB][FR], fb[SETS][NB][FR];
     uint32_t xa[SETS][MB], xb[SETS][NB];
     auto aset = [](int set, int i) constexpr { return i == MB - 1 ? set : 0; };
-    auto read_a = [&](int set, int i, int s, int b, const ScaleRows& sc) __attribute__((always_inline)) {
+    // SKEW: a chunk that is `skew` chunks or less from its stage's end came with the next one's lines.  Rows of a lane are 16 apart and
+    // so have one skew.  {a, b}[s]: where the lane's chunk of k-step s is; next_a, next_b: behind the stage.
+    struct Skewed {
+        uint32_t a[Cfg::SKEW ? Cfg::KSTEPS : 1], b[Cfg::SKEW ? Cfg::KSTEPS : 1];
+    };
+    bool next_a[Cfg::SKEW ? Cfg::KSTEPS : 1], next_b[Cfg::SKEW ? Cfg::KSTEPS : 1];
+    if constexpr (Cfg::SKEW) {
+        static_assert(FR == 1, "a fragment is one chunk");
+        const int skew_a = ((uint32_t)(uintptr_t)p.a + (uint32_t)((m0 + wm * Cfg::WTM + l16) * p.lda_bytes)) >> 4 & 7;
+        const int skew_b = ((uint32_t)(uintptr_t)p.b + (uint32_t)((n0 + wn * Cfg::WTN + l16) * p.ldb_bytes)) >> 4 & 7;
+#pragma unroll
+        for (int s = 0; s < Cfg::KSTEPS; ++s) {
+            next_a[s] = wk * (Cfg::KW / 16) + s * 4 + lg + skew_a >= CPR;
+            next_b[s] = wk * (Cfg::KW / 16) + s * 4 + lg + skew_b >= CPR;
+        }
+    }
+    auto skewed = [&](int b) __attribute__((always_inline)) -> Skewed {
+        Skewed r{};
+        if constexpr (Cfg::SKEW) {
+            const uint32_t here = b * Cfg::STAGE, behind = (b + 1 == R ? 0 : b + 1) * Cfg::STAGE;
+#pragma unroll
+            for (int s = 0; s < Cfg::KSTEPS; ++s) {
+                r.a[s] = fa_row + (lane_x ^ (s << 6)) + (next_a[s] ? behind : here);
+                r.b[s] = fb_row + (lane_x ^ (s << 6)) + (next_b[s] ? behind : here);
+            }
+        }
+        return r;
+    };
+    auto read_a = [&](int set, int i, int s, int b, const ScaleRows& sc, const Skewed& sk) __attribute__((always_inline)) {
+        if constexpr (Cfg::SKEW) {
+            fa[set][i][0] = *reinterpret_cast<const uint4*>(smem + sk.a[s] + i * (16 * SB));
+            return;
+        }
         const uint8_t* base = smem + b * Cfg::STAGE;
 #pragma unroll
         for (int f = 0; f < FR; ++f)
@@ -454,7 +503,11 @@ __global__ void __launch_bounds__(Cfg::THREADS) gemm_tile_ring_kernel(const Tile
         if constexpr (Op::SCALED)
             xa[set][i] = (CHUNKED ? smem + sc.a : base + sa_at)[s * 4 + i * (16 * SCALE_ROW)];
     };
-    auto read_b = [&](int set, int j, int s, int b, const ScaleRows& sc) __attribute__((always_inline)) {
+    auto read_b = [&](int set, int j, int s, int b, const ScaleRows& sc, const Skewed& sk) __attribute__((always_inline)) {
+        if constexpr (Cfg::SKEW) {
+            fb[set][j][0] = *reinterpret_cast<const uint4*>(smem + sk.b[s] + j * (16 * SB));
+            return;
+        }
         const uint8_t* base = smem + b * Cfg::STAGE;
         if constexpr (Cfg::BND) {
             const uint8_t* at = base + (nd_at ^ (j << 5)) + s * 32 * Cfg::RB;
@@ -467,13 +520,13 @@ __global__ void __launch_bounds__(Cfg::THREADS) gemm_tile_ring_kernel(const Tile
         if constexpr (Op::SCALED)
             xb[set][j] = (CHUNKED ? smem + sc.b : base + sb_at)[s * 4 + j * (16 * SCALE_ROW)];
     };
-    auto read_all = [&](int set, int s, int b, const ScaleRows& sc) __attribute__((always_inline)) {
+    auto read_all = [&](int set, int s, int b, const ScaleRows& sc, const Skewed& sk) __attribute__((always_inline)) {
 #pragma unroll
         for (int j = 0; j < NB; ++j)
-            read_b(set, j, s, b, sc);
+            read_b(set, j, s, b, sc, sk);
 #pragma unroll
         for (int i = 0; i < MB; ++i)
-            read_a(Cfg::PIPE ? aset(set, i) : 0, i, s, b, sc);
+            read_a(Cfg::PIPE ? aset(set, i) : 0, i, s, b, sc, sk);
     };
     auto mma = [&](int set, int i, int j) __attribute__((always_inline)) {
         const int as = Cfg::PIPE ? aset(set, i) : 0;
@@ -536,7 +589,7 @@ __global__ void __launch_bounds__(Cfg::THREADS) gemm_tile_ring_kernel(const Tile
             step(st);
             if (computes)
                 static_for<Cfg::KSTEPS>([&](auto sc) {
-                    read_all(0, decltype(sc)::value, buf, rows);
+                    read_all(0, decltype(sc)::value, buf, rows, Skewed{});
 #pragma unroll
                     for (int i = 0; i < MB; ++i)
 #pragma unroll
@@ -549,7 +602,7 @@ __global__ void __launch_bounds__(Cfg::THREADS) gemm_tile_ring_kernel(const Tile
         step(nst - 1);
         if (computes)
             static_for<Cfg::KSTEPS>([&](auto sc) {
-                read_all(0, decltype(sc)::value, buf, rows);
+                read_all(0, decltype(sc)::value, buf, rows, Skewed{});
                 tail_step(0, decltype(sc)::value);
             });
     } else {
@@ -608,22 +661,25 @@ __global__ void __launch_bounds__(Cfg::THREADS) gemm_tile_ring_kernel(const Tile
             hold_short_scales();
 #pragma unroll
             for (int s = 0; s < R; ++s)
-                if (s < nst)
+                if (s < ncopy)
                     issue(s, s);
             write_short_scales();
-            loader_barrier(min(R - 1, nst - 1));
+            // (SKEW: two stages, copies, up to a stage more of them)
+            constexpr int AHEAD = Cfg::SKEW ? 2 : 1;
+            loader_barrier(max(0, min(R - AHEAD, ncopy - AHEAD)));
             int buf = 0;
             for (int st = 0; st < nst - 1; ++st) {
-                loader_barrier(min(R - 2, nst - 2 - st));
-                if (st + R < nst)
+                loader_barrier(max(0, min(R - 1 - AHEAD, ncopy - 1 - AHEAD - st)));
+                if (st + R < ncopy)
                     issue(st + R, buf);
                 buf = buf + 1 == R ? 0 : buf + 1;
             }
         } else {
             // the scale addresses of a stage and the next one's: computed a stage ahead, off the way from barrier to matrix instruction
             ScaleRows rows = scale_rows(0), next_rows = scale_rows(1);
+            Skewed skew = skewed(0), next_skew = skewed(1);
             ring_wait_and_barrier<63>();
-            read_all(0, 0, 0, rows);
+            read_all(0, 0, 0, rows, skew);
             int buf = 0, st = 0;
             auto body = [&](auto parc) __attribute__((always_inline)) {
                 constexpr int PAR = decltype(parc)::value;
@@ -634,6 +690,7 @@ __global__ void __launch_bounds__(Cfg::THREADS) gemm_tile_ring_kernel(const Tile
                     constexpr int rs = LASTSTEP ? 0 : s + 1;
                     const int rb = LASTSTEP ? nbuf : buf;
                     const ScaleRows& rsc = LASTSTEP ? next_rows : rows;
+                    const Skewed& rsk = LASTSTEP ? next_skew : skew;
                     if constexpr (LASTSTEP)
                         ring_wait_and_barrier<63>();
                     // (reads pinned behind the instruction that frees their registers; B first, each next k-step needs all of it)
@@ -644,11 +701,11 @@ __global__ void __launch_bounds__(Cfg::THREADS) gemm_tile_ring_kernel(const Tile
                         if constexpr (x < NB || x == AL || (j == NB - 1 && i < MB - 1)) {
                             __builtin_amdgcn_sched_barrier(0);
                             if constexpr (x < NB)
-                                read_b(SET ^ 1, x, rs, rb, rsc);
+                                read_b(SET ^ 1, x, rs, rb, rsc, rsk);
                             if constexpr (x == AL)
-                                read_a(SET ^ 1, MB - 1, rs, rb, rsc);
+                                read_a(SET ^ 1, MB - 1, rs, rb, rsc, rsk);
                             if constexpr (j == NB - 1 && i < MB - 1)
-                                read_a(0, i, rs, rb, rsc);
+                                read_a(0, i, rs, rb, rsc, rsk);
                             __builtin_amdgcn_sched_barrier(0);
                         }
                     });
@@ -657,12 +714,14 @@ __global__ void __launch_bounds__(Cfg::THREADS) gemm_tile_ring_kernel(const Tile
                 ++st;
                 rows = next_rows;
                 next_rows = scale_rows(st + 1);
+                skew = next_skew;
+                next_skew = skewed(nbuf + 1 == R ? 0 : nbuf + 1);
             };
             auto last = [&](auto parc) __attribute__((always_inline)) {
                 static_for<Cfg::KSTEPS>([&](auto sc) {
                     constexpr int s = decltype(sc)::value, SET = (decltype(parc)::value + s) & 1;
                     if constexpr (s > 0)
-                        read_all(SET, s, buf, rows);
+                        read_all(SET, s, buf, rows, skew);
                     tail_step(SET, s);
                 });
             };

@@ -78,6 +78,33 @@ def test_rows_on_any_byte(pa, kind, shape):  # noqa: F811
         assert torch.equal(out, (got.float() * sa[:, None] * sb[None, :]).to(torch.bfloat16))
 
 
+@pytest.mark.parametrize("shape", [3, 4, 6, 7])
+@pytest.mark.parametrize("kind", ["bf16", "f16", "i8"])
+def test_rows_on_16_bytes_off_the_lines(pa, kind, shape):  # noqa: F811
+    """Rows that start on 16 bytes but not on 128: pitches that leave one, four and eight different offsets, A and B apart, K from the
+    six stages on that whole lines are copied for (and a chunk less), ending on a stage, a chunk and inside one; what is around the operands is NaN (int8: not zero).
+    The bits of the product of the same operands on whole lines."""
+    esz = 1 if kind == "i8" else 2
+    tdt, t, tc = {"bf16": (torch.bfloat16, pa.BF16, pa.F32), "f16": (torch.float16, pa.F16, pa.F32), "i8": (torch.int8, pa.I8, pa.I32)}[kind]
+    gen = torch.Generator(device="cuda").manual_seed(shape)
+    bm, bn, stage = SHAPES[shape][:3]
+
+    def rows(values, pitch, start):  # (in bytes)
+        flat = torch.full((start // esz + values.shape[0] * pitch // esz,), 99 if kind == "i8" else float("nan"), device="cuda").to(tdt)
+        view = flat[start // esz:].view(values.shape[0], pitch // esz)[:, :values.shape[1]]
+        view.copy_(values)
+        return view
+    for m, n, kb in [(bm - 1, bn + 3, 6 * stage - 16), (1, bn, 6 * stage), (bm + 1, 2 * bn + 1, 6 * stage + 20), (bm, bn - 1, 8 * stage - 112), (bm + 2, bn + 1, 9 * stage + 100)]:
+        a, b = ((torch.rand((x, kb // esz), generator=gen, device="cuda") * 200 - 100).to(tdt) for x in (m, n))
+        line = (kb + 127) // 128 * 128
+        with tile_env(PTOAMD_RING=shape):
+            ref = pa.gemm(rows(a, line, 0), rows(b, line, 0), t, tc, pa.B_DN)
+            for pa_, sa, pb, sb in [(line + 16, 0, line + 16, 0), (line + 64, 32, line + 32, 112), (line, 48, line + 240, 0), (line + 128, 0, line, 96)]:
+                got = pa.gemm(rows(a, pa_, sa), rows(b, pb, sb), t, tc, pa.B_DN)
+                assert torch.equal(got, ref), (m, n, kb, pa_, sa, pb, sb)
+        assert torch.isfinite(got.double()).all()
+
+
 @pytest.mark.parametrize("shape", range(9))
 @pytest.mark.parametrize("kind", ["bf16", "f16"])
 def test_row_major_b(pa, oracle, kind, shape):  # noqa: F811
