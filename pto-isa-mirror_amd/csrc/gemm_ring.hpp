@@ -18,15 +18,14 @@ struct TileGemmParams;
     X(0, 32, 16, 1, 1, 8, 1024, 3, 1, 1, 8, 1024, 3, 0, false)    \
     X(1, 32, 32, 1, 1, 8, 512, 4, 1, 2, 4, 512, 4, 0, false)      \
     X(2, 64, 32, 1, 1, 8, 512, 3, 2, 1, 4, 512, 3, 0, false)      \
-    X(3, 64, 64, 2, 2, 2, 256, 4, 2, 4, 1, 256, 4, 4, true)       \
-    X(4, 96, 64, 2, 2, 2, 256, 4, 2, 4, 1, 256, 3, 4, true)       \
-    X(5, 128, 64, 2, 2, 2, 256, 3, 4, 2, 1, 256, 3, 4, true)      \
-    X(6, 128, 128, 2, 4, 1, 128, 4, 2, 4, 1, 128, 4, 4, true)
-// the plain types only (the block-scaled columns are empty): a block-scaled wave tile of this size does not fit the 168 registers
-// of twelve waves
+    X(3, 64, 64, 2, 1, 2, 256, 4, 2, 2, 1, 256, 4, 4, true)       \
+    X(4, 96, 64, 2, 1, 2, 256, 4, 2, 2, 1, 256, 3, 4, true)       \
+    X(5, 128, 64, 2, 1, 2, 256, 3, 2, 2, 1, 256, 3, 4, true)      \
+    X(6, 128, 128, 2, 2, 1, 128, 4, 2, 2, 1, 128, 4, 4, true)
+// the plain types only (the block-scaled columns are empty)
 #define PTOAMD_RING_SHAPES_PLAIN(X)                               \
-    X(7, 192, 128, 4, 2, 1, 128, 4, 0, 0, 0, 0, 0, 4, true)       \
-    X(8, 256, 128, 4, 2, 1, 128, 3, 0, 0, 0, 0, 0, 4, true)
+    X(7, 192, 128, 2, 2, 1, 128, 4, 0, 0, 0, 0, 0, 4, true)       \
+    X(8, 256, 128, 2, 2, 1, 128, 3, 0, 0, 0, 0, 0, 4, true)
 constexpr int RING_SHAPES = 9, RING_SHAPES_SCALED = 7, RING_MAX_STAGE_BYTES = 1024, RING_SHAPE_128X128 = 6;
 // Added to the id of a shape with copying waves (3 and up) of the plain types: the form for rows that start on any byte.
 constexpr int RING_UNALIGNED = 16, RING_FIRST_UNALIGNED = 3;
