@@ -452,7 +452,8 @@ template <int KIND>
 constexpr bool out_quant = KIND == OUT_Q8 || KIND == OUT_QF16;  // (OUT_QF16 instances also serve OUT_QBF16 and OUT_QS16)
 
 // Element-wise form: any alignment, any edge.  A lane's elements are 4-column runs of one row, so this form is slow
-// (short scattered stores); whole, aligned wave tiles take the staged form below.
+// (short scattered stores); it serves what the staged form below does not: atomic additions, raw accumulators beside the scaled
+// result, and the quantising kinds where a wave tile's columns reach past N.
 template <int KIND, bool FULL, class Cfg, class Acc>
 __device__ __forceinline__ void tstore_block(const TileGemmParams& p, const Acc& acc, int row_b, int col_b, int l32, int lhi)
 {
@@ -484,7 +485,7 @@ __device__ __forceinline__ void tstore_block(const TileGemmParams& p, const Acc&
     }
 }
 
-// float accumulators drain to f32 / f16 / bf16, int32 accumulators to int32 or (W8A8) scaled bf16: only those forms are
+// int32 accumulators drain to int32 or (W8A8) scaled bf16, float ones element by element to f32 only: only those forms are
 // compiled for an operand type (the host rejects the other combinations)
 template <bool FULL, class Cfg, class Acc>
 __device__ __forceinline__ void tstore_block_kind(const TileGemmParams& p, const Acc& acc, int row_b, int col_b, int l32, int lhi)
@@ -499,11 +500,7 @@ __device__ __forceinline__ void tstore_block_kind(const TileGemmParams& p, const
         else
             tstore_block<OUT_W8A8_BF16, FULL, Cfg>(p, acc, row_b, col_b, l32, lhi);
     } else {
-        switch (p.out_kind) {
-            case OUT_F32: tstore_block<OUT_F32, FULL, Cfg>(p, acc, row_b, col_b, l32, lhi); break;
-            case OUT_F16: tstore_block<OUT_F16, FULL, Cfg>(p, acc, row_b, col_b, l32, lhi); break;
-            default: tstore_block<OUT_BF16, FULL, Cfg>(p, acc, row_b, col_b, l32, lhi); break;
-        }
+        tstore_block<OUT_F32, FULL, Cfg>(p, acc, row_b, col_b, l32, lhi);
     }
 }
 
@@ -520,11 +517,16 @@ struct StagedStore {
     static_assert((32 * Cfg::WTN / 16) % 64 == 0, "a band is a whole number of 64-lane reads, down to one-byte outputs");
 };
 
-// `stage` is the calling wave's private LDS region of StagedStore<Cfg>::WAVE_BYTES bytes.  The wave tile's columns lie
-// inside the matrix (checked by the caller); its last rows may lie past row m - 1: they are computed on clamped row
-// indices and not stored.  Rows of C need no alignment: a row piece leaves as 16-byte stores at whatever address it
-// starts (the part takes unaligned vector stores; on 16-byte aligned rows they are whole 128-byte lines).
-template <int KIND, class Cfg, class Acc>
+// `stage` is the calling wave's private LDS region of StagedStore<Cfg>::WAVE_BYTES bytes.  The wave tile starts inside the matrix
+// (checked by the caller); its last rows may lie past row m - 1: they are computed on clamped row indices and not stored.  Its
+// last columns may lie past column n - 1 (not for the quantising kinds): a row piece is then its whole 16-byte chunks and, from one
+// lane per row, the elements of the chunk that N ends in, as 8-, 4- and 2-byte stores.  Rows of C need no alignment: a row piece
+// leaves as 16-byte stores at whatever address it starts (the part takes unaligned vector stores; on 16-byte aligned rows they are
+// whole 128-byte lines).
+// One wave tile that crosses N used to be stored element by element, and the launch waited for it.  n = 2020 and k = 2048 (fp4 4096),
+// us, element by element and now (2048 columns): bf16 1024 rows on 256 x 256 tiles 61.8 / 38.5 (38.3), W8A8 44.0 / 22.1 (21.8), on 128 x
+// 128 tiles 17.5 / 9.7 (9.2); MXFP4 on 256 x 256 27.4 / 22.2 (22.0), on 128 x 128 14.2 / 11.6 (11.2).
+template <int KIND, bool EDGE, class Cfg, class Acc>
 __device__ __forceinline__ void tstore_staged(const TileGemmParams& p, Acc (&acc)[Cfg::MB][Cfg::NB], int row0, int col0,
                                               int l32, int lhi, uint8_t* stage)
 {
@@ -545,14 +547,19 @@ __device__ __forceinline__ void tstore_staged(const TileGemmParams& p, Acc (&acc
     constexpr bool PRE_BIAS = PRE && !out_quant<KIND>, PRE_QW = PRE && out_quant<KIND>;
     Elem bias_pre[Cfg::NB][Cfg::Op::ACC_REGS];
     const bool has_bias = PRE_BIAS && p.bias != nullptr;
-    if (has_bias) {
+    static_assert(!EDGE || !out_quant<KIND>, "the quantising kinds' edges are stored element by element");
+    auto fetch_columns = [&](auto& dst, const auto* src) __attribute__((always_inline)) {
         static_for<Cfg::NB>([&](auto jc) {
             constexpr int j = decltype(jc)::value;
 #pragma unroll
-            for (int r = 0; r < Cfg::Op::ACC_REGS; ++r)
-                bias_pre[j][r] = reinterpret_cast<const Elem*>(p.bias)[col0 + j * BLK + acc_col<BLK>(r, lhi)];
+            for (int r = 0; r < Cfg::Op::ACC_REGS; ++r) {
+                const int c = col0 + j * BLK + acc_col<BLK>(r, lhi);
+                dst[j][r] = src[EDGE ? min(c, p.n - 1) : c];
+            }
         });
-    }
+    };
+    if (has_bias)
+        fetch_columns(bias_pre, reinterpret_cast<const Elem*>(p.bias));
     // (byte targets keep the words decoded -- three floats per column instead of a 64-bit word taken apart per element)
     constexpr bool Q8 = KIND == OUT_Q8;
     uint64_t qw_pre[Cfg::NB][Cfg::Op::ACC_REGS];
@@ -582,13 +589,12 @@ __device__ __forceinline__ void tstore_staged(const TileGemmParams& p, Acc (&acc
 #pragma unroll
         for (int i = 0; i < Cfg::MB; ++i)  // the row scales likewise: one load latency instead of one per block row
             rs_pre[i] = p.row_scale[min(row0 + i * BLK + l32, p.m - 1)];
-        static_for<Cfg::NB>([&](auto jc) {
-            constexpr int j = decltype(jc)::value;
-#pragma unroll
-            for (int r = 0; r < Cfg::Op::ACC_REGS; ++r)
-                cs_pre[j][r] = p.col_scale[col0 + j * BLK + acc_col<BLK>(r, lhi)];
-        });
+        fetch_columns(cs_pre, p.col_scale);
     }
+    constexpr int EPC = 16 / ESZ;  // elements of a chunk
+    const int live = EDGE ? p.n - col0 : Cfg::WTN, whole = live / EPC, rest = live % EPC;
+    static_assert(64 % CHUNKS == 0, "a lane stores the same chunk of several rows");
+    const int row_end = !EDGE || (lane % CHUNKS) < whole ? p.m : 0;
     static_for<Cfg::MB / BPB>([&](auto bc) {
         constexpr int band = decltype(bc)::value;
         static_for<BPB>([&](auto hc) {
@@ -600,8 +606,8 @@ __device__ __forceinline__ void tstore_staged(const TileGemmParams& p, Acc (&acc
                 constexpr int j = decltype(jc)::value;
                 __builtin_amdgcn_sched_barrier(0);
                 const int col_b = col0 + j * BLK;
-                const Acc v = tstore_terms<true, !out_quant<KIND>, Cfg>(p, acc[i][j], gi, col_b, lhi,
-                                                                      PRE_BIAS ? bias_pre[j] : nullptr);  // (read only where p.bias is set)
+                const Acc v = tstore_terms<!EDGE, !out_quant<KIND>, Cfg>(p, acc[i][j], gi, col_b, lhi,
+                                                                       PRE_BIAS ? bias_pre[j] : nullptr);  // (read only where p.bias is set)
 #pragma unroll
                 for (int g = 0; g < Cfg::Op::ACC_REGS / 4; ++g) {
                     const int qc = acc_col<BLK>(4 * g, lhi);  // first of the quad's four columns
@@ -645,36 +651,65 @@ __device__ __forceinline__ void tstore_staged(const TileGemmParams& p, Acc (&acc
             nt_u32x4* dst = reinterpret_cast<nt_u32x4*>(reinterpret_cast<uint8_t*>(p.c) +
                                                         ((long)(row0 + band * 32 + row) * p.ldc + col0) * ESZ + ch * 16);
             const nt_u32x4 vv = {v.x, v.y, v.z, v.w};
-            if (row0 + band * 32 + row < p.m)
+            if (row0 + band * 32 + row < row_end)
                 __builtin_nontemporal_store(vv, dst);  // C is not read again by this kernel: keep it out of the L2's way (plain stores end TSTORE
                                                    // 0.3 us sooner, but their write-backs cost the next launch 1 us)
+        }
+        if constexpr (EDGE) {
+            if (rest != 0 && lane < 32 && row0 + band * 32 + lane < p.m) {
+                const uint4 v = *reinterpret_cast<const uint4*>(stage + lane * ROW_BYTES + whole * 16);
+                uint8_t* dst = reinterpret_cast<uint8_t*>(p.c) + ((long)(row0 + band * 32 + lane) * p.ldc + col0) * ESZ + whole * 16;
+                const int bytes = rest * ESZ;
+                typedef unsigned int u32x2 __attribute__((ext_vector_type(2), aligned(1)));
+                typedef unsigned int u32 __attribute__((aligned(1)));
+                if (bytes & 8)
+                    *reinterpret_cast<u32x2*>(dst) = u32x2{v.x, v.y};
+                if (bytes & 4)
+                    *reinterpret_cast<u32*>(dst + (bytes & 8)) = bytes & 8 ? v.z : v.x;
+                if (bytes & 2)
+                    *reinterpret_cast<uint16_t*>(dst + (bytes & 12)) = (uint16_t)(bytes & 8 ? (bytes & 4 ? v.w : v.z) : (bytes & 4 ? v.y : v.x));
+            }
         }
     });
 }
 
-// `stage`: the wave's private LDS region for the staged form, free of other uses from here on; nullptr = element-wise
+// `stage`: the wave's private LDS region for the staged form, free of other uses from here on
 template <class Cfg, class Acc>
 __device__ __forceinline__ void tstore(const TileGemmParams& p, Acc (&acc)[Cfg::MB][Cfg::NB], int row0, int col0, int l32,
-                                       int lhi, uint8_t* stage = nullptr)
+                                       int lhi, uint8_t* stage)
 {
-    // the staged form takes wave tiles whose columns are all inside the matrix (rows past m - 1 are skipped row by row)
-    const bool cols_inside = row0 < p.m && col0 + Cfg::WTN <= p.n;
+    if (row0 >= p.m || col0 >= p.n)
+        return;
     const bool raw_acc = p.out_kind == OUT_W8A8_BF16 && p.acc_out != nullptr;
-    if (stage != nullptr && cols_inside && !p.atomic_add && !raw_acc) {
+    // (the two forms apart: with the edge's code in its way the plain one took longer, W8A8 1024 x 2048 x 2048 on 128 x 128 tiles 9.1 -> 9.6
+    // us, apart 9.2)
+    const bool edge = col0 + Cfg::WTN > p.n;
+    auto staged = [&](auto kind) __attribute__((always_inline)) {
+        constexpr int KIND = decltype(kind)::value;
+        if constexpr (!out_quant<KIND>) {
+            if (edge) {
+                tstore_staged<KIND, true, Cfg>(p, acc, row0, col0, l32, lhi, stage);
+                return;
+            }
+        }
+        tstore_staged<KIND, false, Cfg>(p, acc, row0, col0, l32, lhi, stage);
+    };
+    using std::integral_constant;
+    if (!(edge && p.out_kind >= OUT_Q8) && !p.atomic_add && !raw_acc) {
         if (p.out_kind >= OUT_QF16) {
-            tstore_staged<OUT_QF16, Cfg>(p, acc, row0, col0, l32, lhi, stage);
+            staged(integral_constant<int, OUT_QF16>{});
         } else if (p.out_kind == OUT_Q8) {
-            tstore_staged<OUT_Q8, Cfg>(p, acc, row0, col0, l32, lhi, stage);
+            staged(integral_constant<int, OUT_Q8>{});
         } else if constexpr (std::is_same<typename Cfg::Op::Elem, int32_t>::value) {
             if (p.out_kind == OUT_I32)
-                tstore_staged<OUT_I32, Cfg>(p, acc, row0, col0, l32, lhi, stage);
+                staged(integral_constant<int, OUT_I32>{});
             else
-                tstore_staged<OUT_W8A8_BF16, Cfg>(p, acc, row0, col0, l32, lhi, stage);
+                staged(integral_constant<int, OUT_W8A8_BF16>{});
         } else {
             switch (p.out_kind) {
-                case OUT_F32: tstore_staged<OUT_F32, Cfg>(p, acc, row0, col0, l32, lhi, stage); break;
-                case OUT_F16: tstore_staged<OUT_F16, Cfg>(p, acc, row0, col0, l32, lhi, stage); break;
-                default: tstore_staged<OUT_BF16, Cfg>(p, acc, row0, col0, l32, lhi, stage); break;
+                case OUT_F32: staged(integral_constant<int, OUT_F32>{}); break;
+                case OUT_F16: staged(integral_constant<int, OUT_F16>{}); break;
+                default: staged(integral_constant<int, OUT_BF16>{}); break;
             }
         }
         return;

@@ -1,0 +1,64 @@
+"""The staged store where a wave tile's columns reach past N: every element of C inside a wider buffer, nothing around it."""
+import pytest
+import torch
+
+from test_gpu_parity import pa, tile_env  # noqa: F401
+
+pytestmark = pytest.mark.gpu
+
+# columns past the last whole 256, 128 or 64: each remainder of a 16-byte chunk, first and last columns of a wave tile
+COLUMNS = [1, 2, 3, 63, 65, 100, 127, 132, 161, 254, 261]
+
+
+def _product(pa, kind, a, b, out, bias, c_in):  # noqa: F811
+    """The call, and what it has to give before the rounding to out's type: exact, all sums being small multiples of 1/4."""
+    if kind == "w8a8":
+        sa, sb = (2.0 ** -(torch.arange(x.shape[0], device="cuda") % 3).float() for x in (a, b))
+        pa.gemm_w8a8(a.to(torch.int8), b.to(torch.int8), sa, sb, out=out)
+        return (a.double() @ b.double().T) * sa.double()[:, None] * sb.double()
+    if kind in ("fp8", "fp4"):
+        m, k = a.shape
+        table = {1: 2, 2: 4, 3: 5, 0: 0} if kind == "fp4" else {0: 0, 1: 0x38, 2: 0x40, 3: 0x44}
+        sign = 8 if kind == "fp4" else 0x80
+
+        def codes(x):
+            lut = torch.tensor([table[i] for i in range(4)], device="cuda", dtype=torch.uint8)
+            c = lut[x.abs().long()] | (sign * (x < 0)).to(torch.uint8)
+            return (c[:, 0::2] | (c[:, 1::2] << 4)).contiguous() if kind == "fp4" else c
+        ones = [torch.full((x.shape[0], k // 32), 127, dtype=torch.uint8, device="cuda") for x in (a, b)]
+        t = pa.E2M1 if kind == "fp4" else pa.E4M3
+        c_type = {torch.float32: pa.F32, torch.bfloat16: pa.BF16}[out.dtype]
+        pa.gemm_mx(codes(a), codes(b), ones[0], ones[1], m, b.shape[0], k, t, t, c_type, out=out, c_in=c_in, bias=bias if c_in is None else None)
+    else:
+        tdt, t = {"bf16": (torch.bfloat16, pa.BF16), "f16": (torch.float16, pa.F16), "i8": (torch.int8, pa.I8)}[kind]
+        c_type = {torch.float32: pa.F32, torch.bfloat16: pa.BF16, torch.float16: pa.F16, torch.int32: pa.I32}[out.dtype]
+        pa.gemm(a.to(tdt), b.to(tdt), t, c_type, pa.B_DN, c_in=c_in, relu=c_in is not None, bias=bias, out=out)
+    ref = a.double() @ b.double().T
+    if c_in is not None:
+        ref = ref + c_in.double()
+    if bias is not None and not (kind in ("fp8", "fp4") and c_in is not None):
+        ref = ref + bias.double()
+    return ref.clamp_min(0) if c_in is not None and kind not in ("fp8", "fp4") else ref
+
+
+@pytest.mark.parametrize("tile", [1, 2, 4, 5, 6, 7])
+@pytest.mark.parametrize("kind,types", [("bf16", [torch.float32, torch.bfloat16]), ("f16", [torch.float16]), ("i8", [torch.int32]), ("w8a8", [torch.bfloat16]),
+                                        ("fp8", [torch.bfloat16]), ("fp4", [torch.float32, torch.bfloat16])])
+def test_wave_tiles_that_cross_n(pa, kind, types, tile):  # noqa: F811
+    gen = torch.Generator(device="cuda").manual_seed(tile)
+    for i, n in enumerate(COLUMNS):
+        m, k, dtype = (1, 33, 129, 258)[i % 4], 512, types[i % len(types)]
+        a, b = (torch.randint(-3, 4, (x, k), generator=gen, device="cuda") for x in (m, n))
+        acc = torch.int32 if kind == "i8" else torch.float32
+        bias = torch.randint(-9, 10, (n,), generator=gen, device="cuda").to(acc) if i % 3 == 1 and kind != "w8a8" else None
+        lead = i % 3  # columns in front of C: its rows start on any element
+        wide = torch.full((m, n + lead + 9), 77, device="cuda", dtype=dtype)
+        # (the accumulator input has C's row pitch)
+        c_in = torch.randint(-9, 10, wide.shape, generator=gen, device="cuda").to(acc)[:, lead:lead + n] if i % 3 == 2 and kind != "w8a8" else None
+        with tile_env(PTOAMD_TILE=tile):
+            ref = _product(pa, kind, a, b, wide[:, lead:lead + n], bias, c_in)
+            name = pa.last_kernel()
+        assert name.startswith("tile") and "ring" not in name, name
+        # (one rounding: f32 and int32 hold the sums, the 16-bit types round what f32 holds)
+        assert torch.equal(wide[:, lead:lead + n], ref.float().to(dtype)), (kind, tile, m, n, name)
+        assert (wide[:, :lead] == 77).all() and (wide[:, lead + n:] == 77).all(), (kind, tile, m, n, name)
