@@ -224,7 +224,7 @@ __global__ void __launch_bounds__(Cfg::THREADS) gemm_tile_dtl_kernel(const TileG
 #pragma unroll
             for (int w = 0; w < NSW; ++w) {
                 const int i = wave + w * NW;
-                const int at = CL == 1 ? g * 16 : min(g * CB + ((lane % CL * 16) ^ scale_swizzle(lane / CL)), p.scale_ld - 16);
+                const long at = CL == 1 ? (long)g * 16 : min(g * CB + ((lane % CL * 16) ^ scale_swizzle(lane / CL)), p.scale_ld - 16);
                 if (i < NSI)
                     lds_dma16(sc_src[w] + at, lds_scales + (g & 1) * (SROWS * CB) + i * 1024);
             }
@@ -236,16 +236,22 @@ __global__ void __launch_bounds__(Cfg::THREADS) gemm_tile_dtl_kernel(const TileG
     // with E8M0 127 once, in the prologue.)
     auto read_scales = [&](int kt) __attribute__((always_inline)) {
         if (Op::SCALED) {
-            const uint8_t* base = smem + RING * Cfg::STAGE_BYTES + ((kt / SPG) & 1) * (SROWS * CB);
-            const uint32_t at = (l32 * CB + scale_swizzle(l32)) ^ ((kt % SPG) * GPS);
+            // (without a swizzle the slab's place goes into the wave-uniform part: the lanes' offsets are the same for every slab.
+            // MXFP4 1024 x 2048 x 4096 on 256 x 256 tiles 21.4 us, 14.05 on 256 x 128 ones; worked out per lane 22.0 and 14.5)
+            const uint32_t in_chunk = (kt % SPG) * GPS;
+            const uint8_t* base = smem + RING * Cfg::STAGE_BYTES + ((kt / SPG) & 1) * (SROWS * CB) + (CL == 1 ? in_chunk : 0);
+            const uint32_t swizzled = (l32 * CB + scale_swizzle(l32)) ^ in_chunk;
+            auto dword = [&](int row, int w) __attribute__((always_inline)) {
+                return *reinterpret_cast<const uint32_t*>(CL == 1 ? base + (row + l32) * CB + w * 4 : base + swizzled + row * CB + w * 4);
+            };
 #pragma unroll
             for (int w = 0; w < SW; ++w) {
 #pragma unroll
                 for (int i = 0; i < MB; ++i)
-                    sca_n[i][w] = *reinterpret_cast<const uint32_t*>(base + at + (wm * Cfg::WTM + i * BLK) * CB + w * 4);
+                    sca_n[i][w] = dword(wm * Cfg::WTM + i * BLK, w);
 #pragma unroll
                 for (int j = 0; j < NB; ++j)
-                    scb_n[j][w] = *reinterpret_cast<const uint32_t*>(base + at + (BM + wn * Cfg::WTN + j * BLK) * CB + w * 4);
+                    scb_n[j][w] = dword(BM + wn * Cfg::WTN + j * BLK, w);
             }
         }
     };
