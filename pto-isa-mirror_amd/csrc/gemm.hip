@@ -372,7 +372,9 @@ constexpr int STAGED_SLABS = 8, STAGED_SLABS_SCALED = 2, STAGED_SLABS_UNALIGNED 
 // What a drain costs beside a plain one of f32, f16, bf16 or int32 values.  The deep-ring kernel drains every form in 16-byte
 // pieces, the other tiles some of them element by element, and an atomic addition of 32x32 blocks touches 32 rows per
 // instruction where 16x16 blocks touch 16.  us per call, us per million elements of C, and us per call where the last columns
-// are no whole wave tile: the deep-ring kernel, the plain types' 256 x 256 tile (16x16 blocks), the two-slab tiles of 32x32
+// are no whole wave tile (plain and scaled results are stored there as everywhere, W8A8 1024 x 2020 x 2048 0.3 us over 2048 columns
+// on 256 x 256 tiles, 0.5 on 128 x 128; charged 5 and 1.5 while that was element by element, 1857 x 6445 x 640 took 128 x 128
+// tiles, 29.6 us, 256 x 256 now 19.8): the deep-ring kernel, the plain types' 256 x 256 tile (16x16 blocks), the two-slab tiles of 32x32
 // blocks, the 64 x 64 and the 128 x 128 register-staged tile.
 // Measured, on the 128 x 128 two-slab tile and on the kernel chosen now: a quantisation word per column, int8 3967 x 2560 x 320, 39
 // and 20 us; atomic additions, bf16 1981 x 7296 x 128, 355 and 180; raw accumulators, int8 17929 x 1700 x 376, 275 and 118.
@@ -383,7 +385,7 @@ struct DrainCost {
 };
 static const DrainCost drain_costs[DRAIN_COUNT] = {
     {{0, 0, 0, 0, 0}, {0, 0, 0, 0, 0}, {0, 0, 0, 0.3f, 0.3f}},
-    {{0, 0, 0, 0, 0}, {0, 0, 0, 0, 0}, {0, 5.0f, 1.5f, 1.2f, 1.2f}},                                  // W8A8: scales of rows and columns
+    {{0, 0, 0, 0, 0}, {0, 0, 0, 0, 0}, {0, 0.3f, 0.6f, 0.6f, 0.6f}},                                  // W8A8: scales of rows and columns
     {{0, 0, 2.0f, 0.4f, 3.0f}, {0, 0, 0, 0, 0}, {0, 5.0f, 1.5f, 1.2f, 1.2f}},                         // one quantisation word
     {{0, 4.0f, 11.0f, 2.1f, 12.0f}, {0, 0, 2.4f, 0.7f, 2.4f}, {0, 5.0f, 1.5f, 1.2f, 1.2f}},           // one per column
     {{0, 8.0f, 1.0f, 0.8f, 3.2f}, {0, 0, 0, 0, 0}, {0, 5.0f, 1.5f, 1.2f, 1.2f}},                      // accumulator input
