@@ -452,8 +452,8 @@ template <int KIND>
 constexpr bool out_quant = KIND == OUT_Q8 || KIND == OUT_QF16;  // (OUT_QF16 instances also serve OUT_QBF16 and OUT_QS16)
 
 // Element-wise form: any alignment, any edge.  A lane's elements are 4-column runs of one row, so this form is slow
-// (short scattered stores); it serves what the staged form below does not: atomic additions, raw accumulators beside the scaled
-// result, and the quantising kinds where a wave tile's columns reach past N.
+// (short scattered stores); it serves what the staged form below does not: atomic additions, and raw accumulators beside the scaled
+// result.
 template <int KIND, bool FULL, class Cfg, class Acc>
 __device__ __forceinline__ void tstore_block(const TileGemmParams& p, const Acc& acc, int row_b, int col_b, int l32, int lhi)
 {
@@ -485,16 +485,11 @@ __device__ __forceinline__ void tstore_block(const TileGemmParams& p, const Acc&
     }
 }
 
-// int32 accumulators drain to int32 or (W8A8) scaled bf16, float ones element by element to f32 only: only those forms are
-// compiled for an operand type (the host rejects the other combinations)
+// (what is stored this way is int32 or, from int32, scaled bf16, and f32 from float accumulators)
 template <bool FULL, class Cfg, class Acc>
 __device__ __forceinline__ void tstore_block_kind(const TileGemmParams& p, const Acc& acc, int row_b, int col_b, int l32, int lhi)
 {
-    if (p.out_kind == OUT_Q8) {
-        tstore_block<OUT_Q8, FULL, Cfg>(p, acc, row_b, col_b, l32, lhi);
-    } else if (p.out_kind >= OUT_QF16) {
-        tstore_block<OUT_QF16, FULL, Cfg>(p, acc, row_b, col_b, l32, lhi);
-    } else if constexpr (std::is_same<typename Cfg::Op::Elem, int32_t>::value) {
+    if constexpr (std::is_same<typename Cfg::Op::Elem, int32_t>::value) {
         if (p.out_kind == OUT_I32)
             tstore_block<OUT_I32, FULL, Cfg>(p, acc, row_b, col_b, l32, lhi);
         else
@@ -519,13 +514,14 @@ struct StagedStore {
 
 // `stage` is the calling wave's private LDS region of StagedStore<Cfg>::WAVE_BYTES bytes.  The wave tile starts inside the matrix
 // (checked by the caller); its last rows may lie past row m - 1: they are computed on clamped row indices and not stored.  Its
-// last columns may lie past column n - 1 (not for the quantising kinds): a row piece is then its whole 16-byte chunks and, from one
-// lane per row, the elements of the chunk that N ends in, as 8-, 4- and 2-byte stores.  Rows of C need no alignment: a row piece
+// last columns may lie past column n - 1: a row piece is then its whole 16-byte chunks and, from one lane per row, the elements of the
+// chunk that N ends in, as stores of 8 bytes down to one.  Rows of C need no alignment: a row piece
 // leaves as 16-byte stores at whatever address it starts (the part takes unaligned vector stores; on 16-byte aligned rows they are
 // whole 128-byte lines).
 // One wave tile that crosses N used to be stored element by element, and the launch waited for it.  n = 2020 and k = 2048 (fp4 4096),
 // us, element by element and now (2048 columns): bf16 1024 rows on 256 x 256 tiles 61.8 / 38.5 (38.3), W8A8 44.0 / 22.1 (21.8), on 128 x
-// 128 tiles 17.5 / 9.7 (9.2); MXFP4 on 256 x 256 27.4 / 22.2 (22.0), on 128 x 128 14.2 / 11.6 (11.2).
+// 128 tiles 17.5 / 9.7 (9.2); MXFP4 on 256 x 256 27.4 / 22.2 (22.0), on 128 x 128 14.2 / 11.6 (11.2); int8 to int8 by
+// a word, 256 x 256 46.1 / 25.3 (24.7), by a word per column 52.6 / 27.5 (27.0).
 template <int KIND, bool EDGE, class Cfg, class Acc>
 __device__ __forceinline__ void tstore_staged(const TileGemmParams& p, Acc (&acc)[Cfg::MB][Cfg::NB], int row0, int col0,
                                               int l32, int lhi, uint8_t* stage)
@@ -547,7 +543,6 @@ __device__ __forceinline__ void tstore_staged(const TileGemmParams& p, Acc (&acc
     constexpr bool PRE_BIAS = PRE && !out_quant<KIND>, PRE_QW = PRE && out_quant<KIND>;
     Elem bias_pre[Cfg::NB][Cfg::Op::ACC_REGS];
     const bool has_bias = PRE_BIAS && p.bias != nullptr;
-    static_assert(!EDGE || !out_quant<KIND>, "the quantising kinds' edges are stored element by element");
     auto fetch_columns = [&](auto& dst, const auto* src) __attribute__((always_inline)) {
         static_for<Cfg::NB>([&](auto jc) {
             constexpr int j = decltype(jc)::value;
@@ -575,7 +570,8 @@ __device__ __forceinline__ void tstore_staged(const TileGemmParams& p, Acc (&acc
                 constexpr int j = decltype(jc)::value;
 #pragma unroll
                 for (int r = 0; r < Cfg::Op::ACC_REGS; ++r) {
-                    const uint64_t w = p.qwords[col0 + j * BLK + acc_col<BLK>(r, lhi)];
+                    const int c = col0 + j * BLK + acc_col<BLK>(r, lhi);
+                    const uint64_t w = p.qwords[EDGE ? min(c, p.n - 1) : c];
                     if (Q8)
                         bq_pre[j][r] = decode_byte_quant<true>(w);
                     else
@@ -629,7 +625,7 @@ __device__ __forceinline__ void tstore_staged(const TileGemmParams& p, Acc (&acc
                                 bits[e] = byte_quant_bits((float)v[4 * g + e], p.q_per_column ? bq_pre[j][4 * g + e] : bq0, (p.relu & 1) != 0);
                                 continue;
                             }
-                            const uint64_t qw = !out_quant<KIND> ? 0 : !p.q_per_column ? qw0 : (PRE_QW && !Q8) ? qw_pre[j][4 * g + e] : p.qwords[col_b + qc + e];
+                            const uint64_t qw = !out_quant<KIND> ? 0 : !p.q_per_column ? qw0 : (PRE_QW && !Q8) ? qw_pre[j][4 * g + e] : p.qwords[EDGE ? min(col_b + qc + e, p.n - 1) : col_b + qc + e];
                             bits[e] = tstore_bits<KIND>(v[4 * g + e], rs, 1.0f, qw, p.q_per_column != 0, p.relu, p.out_kind);
                         }
                         if (ESZ == 4)
@@ -666,8 +662,12 @@ __device__ __forceinline__ void tstore_staged(const TileGemmParams& p, Acc (&acc
                     *reinterpret_cast<u32x2*>(dst) = u32x2{v.x, v.y};
                 if (bytes & 4)
                     *reinterpret_cast<u32*>(dst + (bytes & 8)) = bytes & 8 ? v.z : v.x;
+                const uint32_t last = bytes & 8 ? (bytes & 4 ? v.w : v.z) : (bytes & 4 ? v.y : v.x);
+                typedef uint16_t u16 __attribute__((aligned(1)));
                 if (bytes & 2)
-                    *reinterpret_cast<uint16_t*>(dst + (bytes & 12)) = (uint16_t)(bytes & 8 ? (bytes & 4 ? v.w : v.z) : (bytes & 4 ? v.y : v.x));
+                    *reinterpret_cast<u16*>(dst + (bytes & 12)) = (uint16_t)last;
+                if (ESZ == 1 && (bytes & 1))
+                    dst[bytes & 14] = (uint8_t)(bytes & 2 ? last >> 16 : last);
             }
         }
     });
@@ -686,16 +686,13 @@ __device__ __forceinline__ void tstore(const TileGemmParams& p, Acc (&acc)[Cfg::
     const bool edge = col0 + Cfg::WTN > p.n;
     auto staged = [&](auto kind) __attribute__((always_inline)) {
         constexpr int KIND = decltype(kind)::value;
-        if constexpr (!out_quant<KIND>) {
-            if (edge) {
-                tstore_staged<KIND, true, Cfg>(p, acc, row0, col0, l32, lhi, stage);
-                return;
-            }
-        }
-        tstore_staged<KIND, false, Cfg>(p, acc, row0, col0, l32, lhi, stage);
+        if (edge)
+            tstore_staged<KIND, true, Cfg>(p, acc, row0, col0, l32, lhi, stage);
+        else
+            tstore_staged<KIND, false, Cfg>(p, acc, row0, col0, l32, lhi, stage);
     };
     using std::integral_constant;
-    if (!(edge && p.out_kind >= OUT_Q8) && !p.atomic_add && !raw_acc) {
+    if (!p.atomic_add && !raw_acc) {
         if (p.out_kind >= OUT_QF16) {
             staged(integral_constant<int, OUT_QF16>{});
         } else if (p.out_kind == OUT_Q8) {

@@ -62,3 +62,30 @@ def test_wave_tiles_that_cross_n(pa, kind, types, tile):  # noqa: F811
         # (one rounding: f32 and int32 hold the sums, the 16-bit types round what f32 holds)
         assert torch.equal(wide[:, lead:lead + n], ref.float().to(dtype)), (kind, tile, m, n, name)
         assert (wide[:, :lead] == 77).all() and (wide[:, lead + n:] == 77).all(), (kind, tile, m, n, name)
+
+
+@pytest.mark.parametrize("tile", [1, 2, 4, 5, 6])
+@pytest.mark.parametrize("kind", ["bf16", "i8"])
+@pytest.mark.parametrize("per_column", [False, True])
+def test_quantised_wave_tiles_that_cross_n(pa, per_column, kind, tile):  # noqa: F811
+    """The same bits as the first columns of a product of whole tiles."""
+    gen = torch.Generator(device="cuda").manual_seed(tile)
+    tdt, t = (torch.bfloat16, pa.BF16) if kind == "bf16" else (torch.int8, pa.I8)
+    names = {pa.I8: torch.int8, pa.U8: torch.uint8, pa.F16: torch.float16, pa.BF16: torch.bfloat16, pa.I16: torch.int16}
+    m, k, most = 130, 256, 512
+    a, b = (torch.randint(-3, 4, (x, k), generator=gen, device="cuda").to(tdt) for x in (m, most))
+    scale = (torch.rand(most, generator=gen, device="cuda") * 0.5 + 0.25).view(torch.int32).to(torch.int64) & 0xFFFFE000
+    words = scale | (torch.randint(0, 8, (most,), generator=gen, device="cuda") << 37) | (3 << 32)
+    for i, n in enumerate(COLUMNS + [12, 77, 190]):
+        c_type = [pa.I8, pa.U8, pa.F16, pa.I16 if kind == "i8" else pa.BF16][i % 4]
+        signed = (1 << 46) if c_type == pa.I8 else 0
+        q = (words if per_column else words[:1]) | signed
+        wide = torch.full((m, n + 20), 77, device="cuda", dtype=names[c_type])
+        lead = i % 3
+        with tile_env(PTOAMD_TILE=tile):
+            ref = pa.gemm_requant(a, b, t, c_type, q, per_column=per_column)
+            pa.gemm_requant(a, b[:n], t, c_type, q[:n].contiguous(), per_column=per_column, out=wide[:, lead:lead + n])
+        raw = torch.int8 if c_type in (pa.I8, pa.U8) else torch.int16
+        assert torch.equal(wide[:, lead:lead + n].contiguous().view(raw), ref[:, :n].contiguous().view(raw)), (kind, tile, n, c_type)
+        assert ref[:, :n].unique().numel() > 4
+        assert (wide[:, :lead] == 77).all() and (wide[:, lead + n:] == 77).all(), (kind, tile, n, c_type)
