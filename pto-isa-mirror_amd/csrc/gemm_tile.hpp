@@ -316,8 +316,10 @@ struct TileCfg {
     static constexpr int KSTEPS = SLAB / (LG * Op::FRAG_BYTES);
     static constexpr int A_BYTES = BM * SLAB, B_BYTES = BN * SLAB, STAGE_BYTES = A_BYTES + B_BYTES;
     // the direct-to-LDS kernel of a block-scaled operand type keeps two buffers of SCALE_CHUNK scale bytes per tile row behind
-    // the operand ring.  fp8 takes 32 bytes where they fit: a copy costs the lines it touches, and 16 bytes of a row touch as many
-    // (MXFP8 4096 x 14336 x 4096 193.4 -> 191.8 us); fp4, whose slab takes 8 of them, is no faster with 32 (75.6 against 74.5 us).
+    // the operand ring.  fp8 takes 32 bytes where they fit: a copy costs the lines it touches, and 16 bytes of a row touch as many.
+    // MXFP8, us, by 16 and by 32 bytes: 256 x 256 tiles, 1024 x 2048 x 4096 42.0 and 41.0, 2048 x 4096 x 8192 79.6 and 77.0; 256 x
+    // 128 tiles 31.9 and 29.3, 69.0 and 65.4; a short K waits longer for the first ones, 1024 x 2048 x 512 9.7 and 9.9, 6.33 and
+    // 6.40.  fp4, whose slab takes 8 of them, is no faster with 32 (74.5 and 75.6 us).
     static constexpr int SCALE_CHUNK = Op::SCALED && Op::GROUPS_PER_SLAB == 4 && RING * STAGE_BYTES + 2 * (BM + BN) * 32 <= 160 * 1024 ? 32 : 16;
     static constexpr int SCALE_BYTES = Op::SCALED ? 2 * (BM + BN) * SCALE_CHUNK : 0;
     static constexpr int LDS_BYTES = RING * STAGE_BYTES + SCALE_BYTES;
@@ -673,26 +675,33 @@ __device__ __forceinline__ void tstore_staged(const TileGemmParams& p, Acc (&acc
     });
 }
 
-// `stage`: the wave's private LDS region for the staged form, free of other uses from here on
-template <class Cfg, class Acc>
+// `stage`: the wave's private LDS region for the staged form, free of other uses from here on.
+// EDGE: the last columns of the matrix are no whole wave tile.  A kernel of its own: next to the edge's code the form for whole wave
+// tiles took 12 to 44 registers more, and a return in front of both forms took the K loop's addresses apart.  Launches without an edge
+// lost 1 to 4 % by them, and bf16 2381 x 6298 x 256 from a row-major B, where a SIMD then held a wave less, ran 55.4 instead of 38.5
+// us (now 37.1).  Whole tiles, us, both forms in one kernel and now (before there was an edge form): MXFP4 1024 x 2048 x 4096 on 256 x
+// 256 tiles 21.3 / 20.9 (20.9), int8 1024 x 2048 x 2048 to int8 by a word on 256 x 128 16.8 / 16.5 (16.4), bf16 from a row-major B on
+// 128 x 128 register-staged ones 44.9 / 42.6 (42.7).
+template <class Cfg, bool EDGE, class Acc>
 __device__ __forceinline__ void tstore(const TileGemmParams& p, Acc (&acc)[Cfg::MB][Cfg::NB], int row0, int col0, int l32,
                                        int lhi, uint8_t* stage)
 {
-    if (row0 >= p.m || col0 >= p.n)
-        return;
     const bool raw_acc = p.out_kind == OUT_W8A8_BF16 && p.acc_out != nullptr;
-    // (the two forms apart: with the edge's code in its way the plain one took longer, W8A8 1024 x 2048 x 2048 on 128 x 128 tiles 9.1 -> 9.6
-    // us, apart 9.2)
-    const bool edge = col0 + Cfg::WTN > p.n;
+    // (both are the same for the whole wave)
+    const bool crosses = EDGE && __builtin_amdgcn_readfirstlane(col0) + Cfg::WTN > p.n;
+    const bool inside = __builtin_amdgcn_readfirstlane(row0) < p.m && __builtin_amdgcn_readfirstlane(col0) < p.n;
     auto staged = [&](auto kind) __attribute__((always_inline)) {
         constexpr int KIND = decltype(kind)::value;
-        if (edge)
-            tstore_staged<KIND, true, Cfg>(p, acc, row0, col0, l32, lhi, stage);
-        else
-            tstore_staged<KIND, false, Cfg>(p, acc, row0, col0, l32, lhi, stage);
+        if constexpr (EDGE) {
+            if (crosses) {
+                tstore_staged<KIND, true, Cfg>(p, acc, row0, col0, l32, lhi, stage);
+                return;
+            }
+        }
+        tstore_staged<KIND, false, Cfg>(p, acc, row0, col0, l32, lhi, stage);
     };
     using std::integral_constant;
-    if (!p.atomic_add && !raw_acc) {
+    if (inside && !p.atomic_add && !raw_acc) {
         if (p.out_kind >= OUT_QF16) {
             staged(integral_constant<int, OUT_QF16>{});
         } else if (p.out_kind == OUT_Q8) {
@@ -711,6 +720,8 @@ __device__ __forceinline__ void tstore(const TileGemmParams& p, Acc (&acc)[Cfg::
         }
         return;
     }
+    if (!p.atomic_add && !raw_acc)
+        return;
     static_for<Cfg::MB * Cfg::NB>([&](auto bc) {
         constexpr int i = decltype(bc)::value / Cfg::NB, j = decltype(bc)::value % Cfg::NB;
         // keep the address arithmetic of one 32x32 block from being hoisted over the others (register pressure)
@@ -753,8 +764,14 @@ __device__ __forceinline__ uint4 load_chunk_tail(const uint8_t* g, int rem)
 
 // RAGGED: some row of A or B does not end on a 16-byte chunk boundary (see the loader below).  A compile-time form, so
 // that the kernel for whole chunks carries neither the tail-masking code nor a branch in its K loop.
+// EDGE: see tstore.  The rows that RAGGED is for have a last wave tile that is not whole more often than not: it comes with EDGE only.
+// The waves of a SIMD that the plain types are compiled for are those that the tile's LDS admits: by itself the compiler takes 260
+// registers for the 128 x 128 tile's RAGGED form, 136 for int8's 64 x 64 one, and a wave less fits.
 template <class Cfg, bool RAGGED>
-__global__ void __launch_bounds__(Cfg::THREADS) gemm_tile_kernel(const TileGemmParams p)
+constexpr int staged_waves = Cfg::Op::SCALED ? 1 : Cfg::BM == 64 ? 4 : RAGGED ? 2 : 1;
+template <class Cfg, bool RAGGED, bool EDGE>
+__global__ void __launch_bounds__(Cfg::THREADS) __attribute__((amdgpu_waves_per_eu(staged_waves<Cfg, RAGGED>, staged_waves<Cfg, RAGGED> > 1 ? staged_waves<Cfg, RAGGED> : 8)))
+    gemm_tile_kernel(const TileGemmParams p)
 {
     using Op = typename Cfg::Op;
     using Acc = typename Op::Acc;
@@ -1026,7 +1043,7 @@ __global__ void __launch_bounds__(Cfg::THREADS) gemm_tile_kernel(const TileGemmP
     }
 
     // ---- TSTORE: drain the accumulators through the epilogue (the ring is free after the loop's last barrier)
-    tstore<Cfg>(p, acc, m0 + wm * Cfg::WTM, n0 + wn * Cfg::WTN, l32, lhi, smem + wave * StagedStore<Cfg>::WAVE_BYTES);
+    tstore<Cfg, EDGE>(p, acc, m0 + wm * Cfg::WTM, n0 + wn * Cfg::WTN, l32, lhi, smem + wave * StagedStore<Cfg>::WAVE_BYTES);
 }
 
 // One launcher per (tile shape, operand type); defined in gemm_tile_<op>.hip, called from gemm.hip.

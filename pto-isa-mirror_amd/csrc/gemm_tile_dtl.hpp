@@ -89,7 +89,8 @@ __host__ __device__ constexpr int dma_phase_begin(int phase)
 // BND: B is row-major [K][N] of 16-bit elements (a whole number of slabs of K).  A slab of B is then 64 k rows as they lie in
 // memory, and the fragment reads transpose them (read_transposed_16, lds_dma.hpp); products, order and results are those
 // of a column-major B.  bf16 4096^3: 95 us (column-major 94, re-ordered through a workspace first 131).
-template <class Cfg, bool RAGGED = false, bool BND = false>
+// EDGE: see tstore.
+template <class Cfg, bool RAGGED, bool BND, bool EDGE>
 __global__ void __launch_bounds__(Cfg::THREADS) gemm_tile_dtl_kernel(const TileGemmParams p)
 {
     static_assert(!RAGGED || (Cfg::RING == 2 && !Cfg::Op::SCALED), "the ragged-K form exists for the two-slab ring of the plain types");
@@ -236,8 +237,8 @@ __global__ void __launch_bounds__(Cfg::THREADS) gemm_tile_dtl_kernel(const TileG
     // with E8M0 127 once, in the prologue.)
     auto read_scales = [&](int kt) __attribute__((always_inline)) {
         if (Op::SCALED) {
-            // (without a swizzle the slab's place goes into the wave-uniform part: the lanes' offsets are the same for every slab.
-            // MXFP4 1024 x 2048 x 4096 on 256 x 256 tiles 21.4 us, 14.05 on 256 x 128 ones; worked out per lane 22.0 and 14.5)
+            // (without a swizzle the slab's place goes into the wave-uniform part: the lanes' offsets are the same for every slab.  Worked
+            // out per lane, MXFP4 1024 x 2048 x 4096 takes 3 % more on 256 x 256 tiles and 4 % on 256 x 128 ones)
             const uint32_t in_chunk = (kt % SPG) * GPS;
             const uint8_t* base = smem + RING * Cfg::STAGE_BYTES + ((kt / SPG) & 1) * (SROWS * CB) + (CL == 1 ? in_chunk : 0);
             const uint32_t swizzled = (l32 * CB + scale_swizzle(l32)) ^ in_chunk;
@@ -481,7 +482,7 @@ __global__ void __launch_bounds__(Cfg::THREADS) gemm_tile_dtl_kernel(const TileG
 
     // ---- TSTORE.  No wave reads the ring after the last slab's barrier (its fragment reads were issued before it) and
     // no DMA is in flight, so each wave may reuse a piece of it for the staged store without another barrier.
-    tstore<Cfg>(p, acc, m0 + wm * Cfg::WTM, n0 + wn * Cfg::WTN, l32, lhi, smem + wave * StagedStore<Cfg>::WAVE_BYTES);
+    tstore<Cfg, EDGE>(p, acc, m0 + wm * Cfg::WTM, n0 + wn * Cfg::WTN, l32, lhi, smem + wave * StagedStore<Cfg>::WAVE_BYTES);
 }
 
 }  // namespace ptoamd

@@ -7,22 +7,49 @@
 
 namespace ptoamd {
 
+// One kernel on a tile grid; m = 0: only make it ready to launch on the current device.
+template <auto* KERNEL, class Cfg>
+static hipError_t launch_kernel(const TileGemmParams& p, hipStream_t stream)
+{
+    const hipError_t e = ensure_dynamic_lds<KERNEL>(Cfg::LDS_BYTES);
+    if (e != hipSuccess || p.m <= 0)
+        return e;
+    const int tiles = ((p.m + Cfg::BM - 1) / Cfg::BM) * ((p.n + Cfg::BN - 1) / Cfg::BN);
+    hipLaunchKernelGGL((*KERNEL), dim3(tiles), dim3(Cfg::THREADS), Cfg::LDS_BYTES, stream, p);
+    return hipGetLastError();
+}
+
+// (the block-scaled types have the EDGE kernel only: theirs is no slower over whole wave tiles, MXFP8 1024 x 2048 x 2048 on 128 x 128
+// tiles 26.0 us, without the edge's code 27.0)
 template <class Cfg>
 static hipError_t launch_cfg(const TileGemmParams& p, hipStream_t stream)
 {
-    hipError_t e = ensure_dynamic_lds<&gemm_tile_kernel<Cfg, false>>(Cfg::LDS_BYTES);
-    if (e == hipSuccess)
-        e = ensure_dynamic_lds<&gemm_tile_kernel<Cfg, true>>(Cfg::LDS_BYTES);
-    if (e != hipSuccess || p.m <= 0)  // m = 0: only make the kernels ready to launch on the current device
+    constexpr bool BOTH = !Cfg::Op::SCALED;
+    if (p.m <= 0) {
+        hipError_t e = launch_kernel<&gemm_tile_kernel<Cfg, false, true>, Cfg>(p, stream);
+        if (e == hipSuccess)
+            e = launch_kernel<&gemm_tile_kernel<Cfg, true, true>, Cfg>(p, stream);
+        if (e == hipSuccess && BOTH)
+            e = launch_kernel<&gemm_tile_kernel<Cfg, false, !BOTH>, Cfg>(p, stream);
         return e;
-    const int tiles = ((p.m + Cfg::BM - 1) / Cfg::BM) * ((p.n + Cfg::BN - 1) / Cfg::BN);
+    }
     // rows that do not end on a 16-byte chunk boundary take the kernel with the tail-masking loader
     const bool ragged = (p.k_bytes & 15) != 0 || (p.b_nd && (((long)p.n * p.b_esz) & 15) != 0);
     if (ragged)
-        hipLaunchKernelGGL((gemm_tile_kernel<Cfg, true>), dim3(tiles), dim3(Cfg::THREADS), Cfg::LDS_BYTES, stream, p);
-    else
-        hipLaunchKernelGGL((gemm_tile_kernel<Cfg, false>), dim3(tiles), dim3(Cfg::THREADS), Cfg::LDS_BYTES, stream, p);
-    return hipGetLastError();
+        return launch_kernel<&gemm_tile_kernel<Cfg, true, true>, Cfg>(p, stream);
+    if (p.n % Cfg::WTN != 0)
+        return launch_kernel<&gemm_tile_kernel<Cfg, false, true>, Cfg>(p, stream);
+    return launch_kernel<&gemm_tile_kernel<Cfg, false, !BOTH>, Cfg>(p, stream);
+}
+
+// whole wave tiles of columns, or not
+template <class Cfg, bool RAGGED_K, bool ROW_MAJOR_B>
+static hipError_t launch_dtl_form(const TileGemmParams& p, hipStream_t stream)
+{
+    if (p.m > 0 && p.n % Cfg::WTN == 0)
+        return launch_kernel<&gemm_tile_dtl_kernel<Cfg, RAGGED_K, ROW_MAJOR_B, false>, Cfg>(p, stream);
+    const hipError_t e = launch_kernel<&gemm_tile_dtl_kernel<Cfg, RAGGED_K, ROW_MAJOR_B, true>, Cfg>(p, stream);
+    return e == hipSuccess && p.m <= 0 ? launch_kernel<&gemm_tile_dtl_kernel<Cfg, RAGGED_K, ROW_MAJOR_B, false>, Cfg>(p, stream) : e;
 }
 
 // RAGGED_K: this tile also exists in the form that takes a K extent of any length (the plain types' 256 x 256 and
@@ -31,50 +58,40 @@ static hipError_t launch_cfg(const TileGemmParams& p, hipStream_t stream)
 template <class Cfg, bool RAGGED_K = false, bool ROW_MAJOR_B = false>
 static hipError_t launch_dtl(const TileGemmParams& p, hipStream_t stream)
 {
-    hipError_t e = ensure_dynamic_lds<&gemm_tile_dtl_kernel<Cfg, false>>(Cfg::LDS_BYTES);
-    if constexpr (RAGGED_K) {
-        if (e == hipSuccess)
-            e = ensure_dynamic_lds<&gemm_tile_dtl_kernel<Cfg, true>>(Cfg::LDS_BYTES);
-    }
-    if constexpr (ROW_MAJOR_B) {
-        if (e == hipSuccess)
-            e = ensure_dynamic_lds<&gemm_tile_dtl_kernel<Cfg, false, true>>(Cfg::LDS_BYTES);
-    }
-    if (e != hipSuccess || p.m <= 0)
+    if (p.m <= 0) {
+        hipError_t e = launch_dtl_form<Cfg, false, false>(p, stream);
+        if constexpr (RAGGED_K) {
+            if (e == hipSuccess)
+                e = launch_dtl_form<Cfg, true, false>(p, stream);
+        }
+        if constexpr (ROW_MAJOR_B) {
+            if (e == hipSuccess)
+                e = launch_dtl_form<Cfg, false, true>(p, stream);
+        }
         return e;
-    const int tiles = ((p.m + Cfg::BM - 1) / Cfg::BM) * ((p.n + Cfg::BN - 1) / Cfg::BN);
+    }
+    const bool whole_slabs = p.k_bytes % 128 == 0;
     if (p.b_nd) {
         if constexpr (ROW_MAJOR_B) {
-            if (p.k_bytes % 128 == 0) {
-                hipLaunchKernelGGL((gemm_tile_dtl_kernel<Cfg, false, true>), dim3(tiles), dim3(Cfg::THREADS), Cfg::LDS_BYTES, stream, p);
-                return hipGetLastError();
-            }
+            if (whole_slabs)
+                return launch_dtl_form<Cfg, false, true>(p, stream);
         }
         return hipErrorInvalidValue;  // (as below)
     }
-    if (p.k_bytes % 128 != 0) {
-        if constexpr (RAGGED_K) {
-            hipLaunchKernelGGL((gemm_tile_dtl_kernel<Cfg, true>), dim3(tiles), dim3(Cfg::THREADS), Cfg::LDS_BYTES, stream, p);
-            return hipGetLastError();
-        }
-        return hipErrorInvalidValue;  // the dispatcher sends such a K to this form only where it exists
-    }
-    hipLaunchKernelGGL((gemm_tile_dtl_kernel<Cfg, false>), dim3(tiles), dim3(Cfg::THREADS), Cfg::LDS_BYTES, stream, p);
-    return hipGetLastError();
+    if (whole_slabs)
+        return launch_dtl_form<Cfg, false, false>(p, stream);
+    if constexpr (RAGGED_K)
+        return launch_dtl_form<Cfg, true, false>(p, stream);
+    return hipErrorInvalidValue;  // the dispatcher sends such a K to this form only where it exists
 }
 
 // the 256 x 256 tile of the block-scaled fp8 types on the 16x16x128 instruction (whole 128-byte slabs of K only)
 template <class Cfg>
 static hipError_t launch_mx16(const TileGemmParams& p, hipStream_t stream)
 {
-    const hipError_t e = ensure_dynamic_lds<&gemm_tile_mx16_kernel<Cfg>>(Cfg::LDS_BYTES);
-    if (e != hipSuccess || p.m <= 0)
-        return e;
-    if (p.k_bytes % 128 != 0)
+    if (p.m > 0 && p.k_bytes % 128 != 0)
         return hipErrorInvalidValue;
-    const int tiles = ((p.m + Cfg::BM - 1) / Cfg::BM) * ((p.n + Cfg::BN - 1) / Cfg::BN);
-    hipLaunchKernelGGL((gemm_tile_mx16_kernel<Cfg>), dim3(tiles), dim3(Cfg::THREADS), Cfg::LDS_BYTES, stream, p);
-    return hipGetLastError();
+    return launch_kernel<&gemm_tile_mx16_kernel<Cfg>, Cfg>(p, stream);
 }
 
 #ifdef PTOAMD_TILE_RAGGED_K

@@ -200,7 +200,7 @@ __global__ void __launch_bounds__(Cfg::THREADS) gemm_tile_mx16_kernel(const Tile
     }
     slab(kt, kt & 1, false, false);
 
-    tstore<Cfg>(p, acc, m0 + wm * Cfg::WTM, n0 + wn * Cfg::WTN, l16, lg, smem + wave * StagedStore<Cfg>::WAVE_BYTES);
+    tstore<Cfg, false>(p, acc, m0 + wm * Cfg::WTM, n0 + wn * Cfg::WTN, l16, lg, smem + wave * StagedStore<Cfg>::WAVE_BYTES);
 }
 
 }  // namespace ptoamd

@@ -78,3 +78,24 @@ def test_large_tiles_keep_two_waves_per_simd(kernels):
     for k in big:
         assert k[".vgpr_count"] + k.get(".agpr_count", 0) <= 256, (k[".name"], k[".vgpr_count"], k.get(".agpr_count"))
         assert k[".max_flat_workgroup_size"] == 512
+
+
+def test_register_staged_tiles_of_the_plain_types_share_a_simd(kernels):
+    """Several workgroups of a register-staged tile run on a CU as long as its waves' registers let them: 128 x 128 tiles two waves
+    a SIMD (their LDS admits two workgroups), 64 x 64 tiles four.  A SIMD has 512 registers per lane, given out by eights."""
+    for edge, waves in (("Li128ELi128E", 2), ("Li64ELi64E", 4)):
+        ks = [k for k in kernels if "16gemm_tile_kernel" in k[".name"] and edge in k[".name"] and any(op in k[".name"] for op in ("OpBF16", "OpF16", "OpI8"))]
+        assert len(ks) >= 6, [k[".name"] for k in kernels if "gemm_tile_kernel" in k[".name"]]
+        over = {k[".name"]: k[".vgpr_count"] for k in ks if (k[".vgpr_count"] + 7) // 8 * 8 * waves > 512}
+        assert not over, over
+
+
+def test_tiles_without_an_edge_carry_no_code_for_one(kernels):
+    """Launches of whole wave tiles have kernels of their own (last template argument false) with no more registers than those that
+    also store a wave tile that crosses N."""
+    by_name = {k[".name"]: k[".vgpr_count"] for k in kernels if "gemm_tile_dtl_kernel" in k[".name"]}
+    assert by_name
+    for name, count in by_name.items():
+        assert ("ELb0EEEv" in name) != ("ELb1EEEv" in name), name
+        if "ELb1EEEv" in name:
+            assert by_name[name.replace("ELb1EEEv", "ELb0EEEv")] <= count, name
