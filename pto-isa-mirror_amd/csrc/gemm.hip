@@ -329,10 +329,12 @@ static int pick_tile(int m, int n, long k_bytes, bool scaled, bool dma_ok, bool 
 // (first copies, store) and a time per 128-byte slab of K -- what a round costs hardly depends on how full it is, each CU
 // waits for its own copies -- and no less than its slabs at the rate a full chip sustains (power, and the copies from the
 // L2s).  The numbers are fits to the times of every kernel on 110 sizes per operand type (m 1 .. 4096, n 256 .. 14336, k
-// 256 .. 8192).  On 14686 other sizes of every operand form the choices take 249.1 ms where the best kernel for each takes 234.7
-// and the tiles chosen by grid size alone 405.7; 144 sizes run more than a tenth slower than on the latter.  On full grids with
-// aligned rows the estimate itself is up to a third high (2048 x 4096 x 4096 on 256 x 128 tiles: 58 us, 78 estimated), for all
-// deep-ring shapes alike.
+// 256 .. 8192).  They were fitted, and the totals that follow taken, before the deep-ring kernel copied rows off the lines by whole lines and
+// block scales by chunks, and before its four multiplying waves and the staged store of wave tiles that cross N; the kernels
+// have become 0 to 25 % faster since, unevenly (profile of the kernel choice), and only the drains' costs were set again.  On 14686
+// other sizes of every operand form the choices took 249.1 ms where the best kernel for each took 234.7 and the tiles chosen by grid size
+// alone 405.7; 144 sizes ran more than a tenth slower than on the latter.  On full grids with aligned rows the estimate itself is
+// up to a third high (2048 x 4096 x 4096 on 256 x 128 tiles: 58 us, 78 estimated), for all deep-ring shapes alike.
 struct TileCost {
     float round, slab;  // us per round; us per round and slab
     float rate;         // million elements of C times slabs per us
@@ -370,12 +372,17 @@ static const StagedCost staged_costs[STAGED_ROWS][2] = {
 constexpr int STAGED_SLABS = 8, STAGED_SLABS_SCALED = 2, STAGED_SLABS_UNALIGNED = 16;
 
 // What a drain costs beside a plain one of f32, f16, bf16 or int32 values.  The deep-ring kernel drains every form in 16-byte
-// pieces, the other tiles some of them element by element, and an atomic addition of 32x32 blocks touches 32 rows per
-// instruction where 16x16 blocks touch 16.  us per call, us per million elements of C, and us per call where the last columns
-// are no whole wave tile (plain and scaled results are stored there as everywhere, W8A8 1024 x 2020 x 2048 0.3 us over 2048 columns
-// on 256 x 256 tiles, 0.5 on 128 x 128; charged 5 and 1.5 while that was element by element, 1857 x 6445 x 640 took 128 x 128
-// tiles, 29.6 us, 256 x 256 now 19.8): the deep-ring kernel, the plain types' 256 x 256 tile (16x16 blocks), the two-slab tiles of 32x32
-// blocks, the 64 x 64 and the 128 x 128 register-staged tile.
+// pieces; so do the other tiles, but for atomic additions and raw accumulators, which go element by element, and the accumulator
+// input, which is read so where a wave tile crosses N.  An atomic addition of 32x32 blocks touches 32 rows per instruction where 16x16
+// blocks touch 16.  us per call, us per million elements of C, and us per call where the last columns are no whole wave tile: the
+// deep-ring kernel, the plain types' 256 x 256 tile (16x16 blocks), the two-slab tiles of 32x32 blocks, the 64 x 64 and the 128 x 128
+// register-staged tile.
+// The edge, measured (m 512 and 1024, n 1101 .. 4050 against whole tiles, k 2048): W8A8 0.4, 0.8, 0.5, 0.6, one quantisation word 0.5,
+// 0.8, 0.6, 0.9, one per column 0.6, 0.5, 0.5, 0.6.  Charged 5 and 1.5 while it was stored element by element, the 256 x 256 tile lost to 128 x
+// 128 ones: W8A8 1857 x 6445 x 640 29.6 us for 19.8; by a word 2914 x 4275 x 256 20.1 for 13.4, 2504 x 5006 x 384 20.2 for 14.1, by
+// a word per column 2256 x 6604 x 768 28.2 for 24.3.  The accumulator input's measures 5 to 6 us, 2.5 to 5 (two- and three-slab), 1.2 and
+// 5; charged so, of 210 sizes three change kernel and lose (bf16 1209 x 7624 x 384 23.6 -> 37.1 us): the rest of the estimate
+// makes up for it, and its charge stays.
 // Measured, on the 128 x 128 two-slab tile and on the kernel chosen now: a quantisation word per column, int8 3967 x 2560 x 320, 39
 // and 20 us; atomic additions, bf16 1981 x 7296 x 128, 355 and 180; raw accumulators, int8 17929 x 1700 x 376, 275 and 118.
 enum DrainKind { DRAIN_PLAIN, DRAIN_SCALES, DRAIN_WORD, DRAIN_COLUMN_WORDS, DRAIN_ACC_IN, DRAIN_RAW_ACC, DRAIN_ATOMIC, DRAIN_COUNT };
@@ -386,8 +393,8 @@ struct DrainCost {
 static const DrainCost drain_costs[DRAIN_COUNT] = {
     {{0, 0, 0, 0, 0}, {0, 0, 0, 0, 0}, {0, 0, 0, 0.3f, 0.3f}},
     {{0, 0, 0, 0, 0}, {0, 0, 0, 0, 0}, {0, 0.3f, 0.6f, 0.6f, 0.6f}},                                  // W8A8: scales of rows and columns
-    {{0, 0, 2.0f, 0.4f, 3.0f}, {0, 0, 0, 0, 0}, {0, 5.0f, 1.5f, 1.2f, 1.2f}},                         // one quantisation word
-    {{0, 4.0f, 11.0f, 2.1f, 12.0f}, {0, 0, 2.4f, 0.7f, 2.4f}, {0, 5.0f, 1.5f, 1.2f, 1.2f}},           // one per column
+    {{0, 0, 2.0f, 0.4f, 3.0f}, {0, 0, 0, 0, 0}, {0, 0.5f, 0.8f, 0.6f, 0.9f}},                         // one quantisation word
+    {{0, 4.0f, 11.0f, 2.1f, 12.0f}, {0, 0, 2.4f, 0.7f, 2.4f}, {0, 0.6f, 0.5f, 0.5f, 0.6f}},           // one per column
     {{0, 8.0f, 1.0f, 0.8f, 3.2f}, {0, 0, 0, 0, 0}, {0, 5.0f, 1.5f, 1.2f, 1.2f}},                      // accumulator input
     {{0, 6.0f, 6.0f, 2.7f, 6.0f}, {1.5f, 2.8f, 6.0f, 6.0f, 6.0f}, {0, 5.0f, 1.5f, 1.2f, 1.2f}},       // W8A8 with raw accumulators
     {{0, 2.0f, 2.0f, 2.4f, 5.5f}, {12.5f, 12.5f, 25.0f, 25.0f, 25.0f}, {0, 5.0f, 1.5f, 1.2f, 1.2f}},  // atomic additions
@@ -442,9 +449,10 @@ static int pick_dma_tile(int m, int n, long k_bytes, int op, const TileChoice& c
     const float slabs = (float)slab_count;
     const bool staged_ok = choice.staged != STAGED_NONE && slab_count <= (scaled ? STAGED_SLABS_SCALED : unaligned ? STAGED_SLABS_UNALIGNED : STAGED_SLABS);
     // (bf16 1280 x 4096 on two-slab tiles, K 2048: 24.8 us, K 2056: 38.4 us.  Most of it is that the rows no longer start on
-    // 128-byte lines, which costs the deep-ring shapes a fifth to a third per slab on a full chip as well; that is not in their
-    // estimate.  The 256 x 256 tile loses less over a long K: bf16 1391 x 9546, K 6800, takes it 177 us, 255 on deep-ring tiles; charged 1.25
-    // it is taken where it is not ahead, 3044 x 3712, K 2392, 91 us against 76)
+    // 128-byte lines, which costs the deep-ring shapes without a form for such rows (three stages in the ring, or fewer than six of K) a
+    // fifth to a third per slab on a full chip as well; that is not in their estimate.  The 256 x 256 tile loses less over a long K: bf16
+    // 1391 x 9546, K 6800, takes it 177 us, 255 on deep-ring tiles; charged 1.25 it is taken where it is not ahead, 3044 x 3712, K 2392,
+    // 91 us against 76)
     const bool whole_slabs = (k_bytes % 128) == 0;
     const float ragged = whole_slabs ? 1.0f : 1.5f, ragged_256 = whole_slabs ? 1.0f : k_bytes > 4096 ? 1.35f : 1.5f;
     int best = TILE_RING;
@@ -551,14 +559,14 @@ static hipError_t launch_tiles_as(int tile, int op, const TileGemmParams& p, hip
             // plain types: the deep-ring kernel's 128 x 128 shape, which also reads a row-major B (bf16 4096 x 4312 x 2048: 76.8
             // us, with tile 5 84.4); its last chunk of K starts on a dword.  It has one workgroup on a CU where tile 5 has two: where
             // it would take a second round tile 5 is ahead (bf16 943 x 22144 x 3168: 125 us, with a second round 134), and at a
-            // few slabs of K with W8A8's scales, which end each of its rounds late (1536 x 12416 x 384: 20 against 23 us).  Not with the
-            // drains that tile 5 stores element by element (drain_costs).
+            // few slabs of K with W8A8's scales, which end each of its rounds late (1536 x 12416 x 384: 20 against 23 us).  Never with the
+            // drains that tile 5 is slow at (drain_costs).
             const bool scaled_op = op >= TOP_FP8_E4E4;
             const bool one_round = (long)((tail.m + 127) / 128) * ((tail.n + 127) / 128) <= cus;
             const bool late_drain = p.out_kind == OUT_W8A8_BF16 && p.k_bytes <= 4 * 128;
-            const bool by_element = p.atomic_add || p.acc_out != nullptr || (p.qwords != nullptr && p.q_per_column);
+            const bool slow_drain = p.atomic_add || p.acc_out != nullptr || (p.qwords != nullptr && p.q_per_column);
             const bool ring_ok = !scaled_op && options().tail_tile == 0 && (p.k_bytes % 4) == 0;
-            if (p.b_nd || (ring_ok && (by_element || (one_round && !late_drain))))
+            if (p.b_nd || (ring_ok && (slow_drain || (one_round && !late_drain))))
                 return launch_gemm_ring(RING_SHAPE_128X128, op, tail, stream);
             return launch_gemm_tile(options().tail_tile > 0 ? options().tail_tile : (scaled_op ? 7 : 5), op, tail, stream);
         }
@@ -1070,7 +1078,7 @@ static int gemm_mx_common(const char* who, void* c, int c_type, const void* a, c
                      : options().tile < 0 && dma_ok && (kg % 4) == 0 ? pick_dma_tile(m, n, k_bytes, op, {scale_dma_ok ? DTL_ALL : DTL_NONE, c_in ? DRAIN_ACC_IN : DRAIN_PLAIN, false, STAGED_COLUMN_MAJOR_B})
                                                                     : pick_tile(m, n, k_bytes, true, dma_ok && scale_dma_ok);
     PTOAMD_HIP_CHECK(launch_tiles(tile, op, p, stream));
-    set_last_kernel(KernelName{tile_kernel_name, tile_as_launched(tile, op, m, n), op, false});
+    set_last_kernel(KernelName{tile_kernel_name, tile_as_launched(tile, op, m, n), op, false, false});
     return PTOAMD_OK;
 }
 

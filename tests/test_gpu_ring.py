@@ -363,3 +363,16 @@ def test_long_k_off_the_lines(pa, kind, m, n, k, kernel):  # noqa: F811
     got = pa.gemm(a, b, t, tc, pa.B_DN)
     assert pa.last_kernel() == kernel, pa.last_kernel()
     assert torch.equal(got.double(), a.double() @ b.double().t())
+
+
+@pytest.mark.parametrize("m,n,k,per_column", [(2914, 4275, 256, False), (2504, 5006, 384, False), (2256, 6604, 768, True)])
+def test_requantised_columns_that_end_inside_a_wave_tile(pa, m, n, k, per_column):  # noqa: F811
+    """The 256 x 256 tile, which stores such columns as it does whole wave tiles, where it is ahead; the bits of a smaller tile."""
+    gen = torch.Generator(device="cuda").manual_seed(k)
+    a, b = (torch.randint(-99, 100, (x, k), generator=gen, device="cuda", dtype=torch.int8) for x in (m, n))
+    words = ((torch.rand(n if per_column else 1, generator=gen, device="cuda") * 1e-4 + 1e-4).view(torch.int32).to(torch.int64) & 0xFFFFE000) | (1 << 46)
+    got = pa.gemm_requant(a, b, pa.I8, pa.I8, words, per_column=per_column)
+    assert pa.last_kernel() == "tile256x256w8_dtl_i8", pa.last_kernel()
+    with tile_env(PTOAMD_TILE=2):
+        assert torch.equal(got, pa.gemm_requant(a, b, pa.I8, pa.I8, words, per_column=per_column))
+    assert got.unique().numel() > 100
