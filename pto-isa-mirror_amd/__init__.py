@@ -382,20 +382,24 @@ def mx_scale_relayout(src, src_layout, dst_layout, rows, cols, stream=None):
     return out
 
 
-# ---- the entry points above as native callables (binding/entry_points.cpp): they take the plain calls, 4.2 us where ctypes takes
-# 7.2 (m = n = k = 512), and hand every other one to the function of that name above
-_BINDING_PATH = os.path.join(_HERE, "lib", "ptoamd_binding.so")
-
-
+# ---- the entry points above as native callables (binding/entry_points.cpp): they take the plain calls and hand every other one to the
+# function of that name above
 def _native_entry_points():
+    """The binding reads torch's and Python's own structures: it is taken for the Python and, to the commit, the torch that it was
+    built against.  Otherwise, or not built, the functions above stay: they do the same, more slowly."""
     import importlib.machinery
     import importlib.util
-    loader = importlib.machinery.ExtensionFileLoader("ptoamd_binding", _BINDING_PATH)
+    import sysconfig
+    path = os.path.join(_HERE, "lib", "ptoamd_binding" + sysconfig.get_config_var("EXT_SUFFIX"))  # (the Python version is in the name)
+    here = f"{torch.__version__} {torch.version.git_version}"
+    loader = importlib.machinery.ExtensionFileLoader("ptoamd_binding", path)
     try:
-        binding = importlib.util.module_from_spec(importlib.util.spec_from_file_location("ptoamd_binding", _BINDING_PATH, loader=loader))
+        binding = importlib.util.module_from_spec(importlib.util.spec_from_file_location("ptoamd_binding", path, loader=loader))
         loader.exec_module(binding)
-    except ImportError as e:  # (built against another torch, or not built: the functions above do the same, more slowly)
-        warnings.warn(f"{_BINDING_PATH} does not load, calls take the slower way through ctypes: {e}", RuntimeWarning, stacklevel=2)
+        if binding.torch_id != here:
+            raise ImportError(f"built against torch {binding.torch_id}, this is {here}")
+    except ImportError as e:
+        warnings.warn(f"{path} is not used, calls take the slower way through ctypes: {e}", RuntimeWarning, stacklevel=2)
         return
     binding.set_error(PtoAmdError)
     for f in (gemm, gemm_w8a8, gemm_mx, gemv_mxfp4, gemv_mxfp4_packed, tquant_int8, tquant_mx, tdequant):

@@ -1,8 +1,13 @@
 """The native entry points against the package's Python functions that they take the plain calls off (`__wrapped__`)."""
 import copy
+import importlib.util
 import inspect
+import os
 import pickle
+import subprocess
+import sys
 import threading
+import warnings
 
 import pytest
 import torch
@@ -45,6 +50,48 @@ def test_refused_calls_raise_what_the_function_raises(name):
              ((a, a, "f32"), {}), ((a, a, 2 ** 70), {})]
     for args, kw in calls:
         assert outcome(f, *args, **kw) == outcome(f.__wrapped__, *args, **kw), (name, args, kw)
+
+
+def _package_anew():
+    spec = importlib.util.spec_from_file_location("package_loaded_anew", os.path.join(ge.PKG_DIR, "__init__.py"), submodule_search_locations=[ge.PKG_DIR])
+    module = importlib.util.module_from_spec(spec)
+    with warnings.catch_warnings(record=True) as raised:
+        warnings.simplefilter("always")
+        spec.loader.exec_module(module)
+    return module, [w for w in raised if issubclass(w.category, RuntimeWarning)]
+
+
+@pytest.mark.parametrize("what", ["version", "commit", "python", "none"])
+def test_another_torch_or_python_keeps_the_functions(monkeypatch, what):
+    import sysconfig
+    if what == "version":
+        monkeypatch.setattr(torch, "__version__", torch.__version__ + ".post1")
+    elif what == "commit":
+        monkeypatch.setattr(torch.version, "git_version", "0" * 40)
+    elif what == "python":
+        suffix = sysconfig.get_config_var("EXT_SUFFIX")
+        monkeypatch.setattr(sysconfig, "get_config_var", lambda name: ".other" + suffix)
+    module, raised = _package_anew()
+    assert [inspect.isfunction(getattr(module, n)) for n in NAMES] == [what != "none"] * len(NAMES)
+    assert len(raised) == (what != "none")
+
+
+def _make(python, *targets):
+    return subprocess.run(["make", "-C", ge.PKG_DIR, "-n", "-B", f"PYTHON={python}", *targets], capture_output=True, text=True)
+
+
+def test_the_build_needs_no_torch():
+    """Without a torch (an interpreter without its packages, no interpreter at all) everything but the binding is built; with one the
+    binding is named and compiled for the interpreter that was asked for."""
+    for python in (sys.executable + " -S", "/no/such/python"):
+        steps = _make(python)
+        assert steps.returncode == 0 and "entry_points.cpp" not in steps.stdout, steps.stdout[-2000:] + steps.stderr
+        for lib in ("libptoamd.so", "libpto_gemm_performance.so", "libpto_gemm_tiled.so", "libpto_mxmatmul_performance.so"):
+            assert f"-o lib/{lib}" in steps.stdout, lib
+    import sysconfig
+    steps = _make(sys.executable)
+    assert steps.returncode == 0 and "ptoamd_binding" + sysconfig.get_config_var("EXT_SUFFIX") in steps.stdout
+    assert f"{torch.__version__} {torch.version.git_version}" in steps.stdout and sysconfig.get_paths()["include"] in steps.stdout
 
 
 def _cases(p):
@@ -158,3 +205,17 @@ def test_capture_and_replay(pa):  # noqa: F811
         a.mul_(1.5)
         graph.replay()
         assert torch.equal(got, pa.gemm.__wrapped__(a, b, t)), i
+
+
+@pytest.mark.gpu
+def test_compiled_and_traced_callers(pa):  # noqa: F811
+    """torch.compile breaks its graph at an entry point and calls it: the eager result.  torch.jit.trace records what it records of
+    the Python function (the allocation of the result, which nothing fills when the trace is run)."""
+    (a, b, t), _ = _cases(pa)["gemm"][0]
+    ref = pa.gemm.__wrapped__(a + 1, b, t) * 2
+    torch._dynamo.reset()
+    compiled = torch.compile(lambda x: pa.gemm(x + 1, b, t) * 2, backend="eager")
+    for _ in range(2):
+        assert torch.equal(compiled(a), ref)
+    code = [torch.jit.trace(lambda x: f(x + 1, b, t) * 2, (a,), check_trace=False).code for f in (pa.gemm, pa.gemm.__wrapped__)]  # noqa: B023
+    assert code[0] == code[1], code
