@@ -15,9 +15,9 @@ void set_error(const char* fmt, ...);
 void set_last_kernel(const char* name);
 // The kernel of a matmul by what its name is made of: spelling it on every launch took 0.2 us.
 struct KernelName {
-    const char* (*spell)(int tile, int op, bool row_major_b);
+    const char* (*spell)(int tile, int op, bool row_major_b, bool by_lines);
     int tile, op;
-    bool row_major_b;
+    bool row_major_b, by_lines;
 };
 void set_last_kernel(const KernelName& name);
 // Sets hipFuncAttributeMaxDynamicSharedMemorySize of one kernel once per current device; thread-safe, one object per kernel.

@@ -606,7 +606,7 @@ static int tile_as_launched(int tile, int op, int m, int n)
     return tile == 3 ? 4 : tile;
 }
 
-static const char* tile_kernel_name(int tile, int op, bool row_major_b)
+static const char* tile_kernel_name(int tile, int op, bool row_major_b, bool by_lines)
 {
     static const char* ops[TOP_COUNT] = {"bf16", "f16", "i8", "fp8_e4m3_e4m3", "fp8_e5m2_e5m2", "fp8_e4m3_e5m2",
                                          "fp8_e5m2_e4m3", "fp4_e2m1"};
@@ -616,7 +616,7 @@ static const char* tile_kernel_name(int tile, int op, bool row_major_b)
     if (tile >= TILE_RING) {
         int bm, bn;
         ring_shape(tile - TILE_RING, &bm, &bn);
-        snprintf(buf, sizeof buf, row_major_b ? "tile%dx%d_bnd_%s" : tile >= TILE_RING + RING_UNALIGNED ? "tile%dx%d_any_%s" : "tile%dx%d_dtl_%s",
+        snprintf(buf, sizeof buf, row_major_b ? "tile%dx%d_bnd_%s" : tile >= TILE_RING + RING_UNALIGNED ? "tile%dx%d_any_%s" : by_lines ? "tile%dx%d_dtl_lines_%s" : "tile%dx%d_dtl_%s",
                  bm, bn, ops[op]);
         return buf;
     }
@@ -625,6 +625,12 @@ static const char* tile_kernel_name(int tile, int op, bool row_major_b)
     else
         snprintf(buf, sizeof buf, "%s_%s", tiles[tile], ops[op]);
     return buf;
+}
+
+// (spelled out where a shape is asked for, so that which form ran can be told; the names of the kernels that are chosen stay)
+static bool launched_by_lines(int tile, int op, const TileGemmParams& p)
+{
+    return options().ring >= 0 && op < TOP_FP8_E4E4 && !p.b_nd && ring_by_lines(tile - TILE_RING, p.a, p.b, p.m, p.n, p.k_bytes, p.lda_bytes, p.ldb_bytes);
 }
 
 template <typename T>
@@ -890,7 +896,7 @@ static int gemm_common(void* c, int c_type, const void* a, const void* b, int ab
                      : options().tile < 0 && any_ok ? pick_dma_tile(m, n, k_bytes, op, {DTL_NONE, drain, true, STAGED_COLUMN_MAJOR_B})
                                                     : pick_tile(m, n, k_bytes, false, dma_ok, ragged_k_form);
     PTOAMD_HIP_CHECK(launch_tiles(tile, op, p, stream));
-    set_last_kernel(KernelName{tile_kernel_name, tile_as_launched(tile, op, m, n), op, nd_direct});
+    set_last_kernel(KernelName{tile_kernel_name, tile_as_launched(tile, op, m, n), op, nd_direct, launched_by_lines(tile, op, p)});
     return PTOAMD_OK;
 }
 
@@ -932,7 +938,7 @@ int ptoamd_gemm_w8a8(void* out_bf16, int32_t* acc_out, const int8_t* a, const in
                      : options().tile < 0 && any_ok ? pick_dma_tile(m, n, k, TOP_I8, {DTL_NONE, drain, true, STAGED_COLUMN_MAJOR_B})
                                                     : pick_tile(m, n, k, false, dma_ok, true);
     PTOAMD_HIP_CHECK(launch_tiles(tile, TOP_I8, p, stream));
-    set_last_kernel(KernelName{tile_kernel_name, tile, TOP_I8, false});
+    set_last_kernel(KernelName{tile_kernel_name, tile, TOP_I8, false, launched_by_lines(tile, TOP_I8, p)});
     return PTOAMD_OK;
 }
 

@@ -1,6 +1,9 @@
 // The tile shapes of the deep-ring kernel (gemm_tile_ring.hpp) and its launchers, one per operand type.
 #pragma once
 #include <hip/hip_runtime.h>
+#include <stdint.h>
+
+#include <algorithm>
 
 namespace ptoamd {
 
@@ -43,6 +46,37 @@ inline void ring_shape(int shape, int* bm, int* bn)
     };
     *bm = dims[shape % RING_UNALIGNED][0];
     *bn = dims[shape % RING_UNALIGNED][1];
+}
+
+// Rows that start on 16 bytes but not all on 128: a stage's 128 bytes of a row lie across two lines, and a copy costs the lines it
+// touches.  The shapes with four stages in the ring then copy whole lines (SKEW), from six stages of K on: with fewer the stage more
+// that has to land before the first product costs as much (bf16 423 x 1600 x 328 on 64 x 64 tiles 4.8 us, by lines 5.3; 187 x 4502 x
+// 248 5.2 and 5.6).  500 sizes (m 33 .. 4096, n 256 .. 8192), by lines against not: 192 x 128 tiles 0.83, 128 x 128 0.80, 96 x 64 0.88, 64 x
+// 64 0.92 from 2 KiB of K on, and 0.92 to 0.97 where half of the rows start on a line (pitches of 64 bytes).
+inline bool rows_off_lines(const void* a, const void* b, int m, int n, int k_bytes, long lda_bytes, long ldb_bytes, int stage_bytes)
+{
+    if (k_bytes < 6 * stage_bytes)
+        return false;
+    const uint64_t last = std::max((uint64_t)(m - 1) * (uint64_t)lda_bytes, (uint64_t)(n - 1) * (uint64_t)ldb_bytes) + (uint64_t)k_bytes;
+    if (last + 1024 > UINT32_MAX)  // (lane offsets of whole lines reach a little past a row's)
+        return false;
+    const uint64_t bits = reinterpret_cast<uintptr_t>(a) | reinterpret_cast<uintptr_t>(b) | (uint64_t)lda_bytes | (uint64_t)ldb_bytes;
+    return bits % 16 == 0 && bits % 128 != 0;
+}
+constexpr int RING_LINES_DEPTH = 4;
+// whether a launch of a shape takes that form (plain types, B column-major)
+inline bool ring_by_lines(int shape, const void* a, const void* b, int m, int n, int k_bytes, long lda_bytes, long ldb_bytes)
+{
+    static const struct {
+        int stage_bytes, depth;
+        bool pipelined;
+    } forms[RING_SHAPES] = {
+#define PTOAMD_RING_FORM(id, bm, bn, wm, wn, wk, sb, r, swm, swn, swk, ssb, sr, lw, pipe) {sb, r, pipe},
+        PTOAMD_RING_SHAPES_ALL(PTOAMD_RING_FORM) PTOAMD_RING_SHAPES_PLAIN(PTOAMD_RING_FORM)
+#undef PTOAMD_RING_FORM
+    };
+    return shape >= 0 && shape < RING_SHAPES && forms[shape].pipelined && forms[shape].depth >= RING_LINES_DEPTH &&
+           rows_off_lines(a, b, m, n, k_bytes, lda_bytes, ldb_bytes, forms[shape].stage_bytes);
 }
 
 // shape: 0 .. RING_SHAPES - 1, RING_UNALIGNED + one of the later ones, or TILE_PREPARE_ALL

@@ -39,7 +39,7 @@ void set_last_kernel(const KernelName& name)
 static const char* last_kernel()
 {
     if (g_kernel_name.spell != nullptr)
-        set_last_kernel(g_kernel_name.spell(g_kernel_name.tile, g_kernel_name.op, g_kernel_name.row_major_b)), --g_launches;
+        set_last_kernel(g_kernel_name.spell(g_kernel_name.tile, g_kernel_name.op, g_kernel_name.row_major_b, g_kernel_name.by_lines)), --g_launches;
     return g_kernel;
 }
 

@@ -106,6 +106,44 @@ def test_rows_on_16_bytes_off_the_lines(pa, kind, shape):  # noqa: F811
 
 
 @pytest.mark.parametrize("shape", range(9))
+@pytest.mark.parametrize("kind", ["bf16", "f16", "i8"])
+def test_which_rows_are_copied_by_lines(pa, kind, shape):  # noqa: F811
+    """The form for rows off the lines runs on the shapes with four stages in the ring from six stages of K on, and on no other: by the
+    kernel's name, and exact products of small whole numbers either way."""
+    esz = 1 if kind == "i8" else 2
+    tdt, t, tc = {"bf16": (torch.bfloat16, pa.BF16, pa.F32), "f16": (torch.float16, pa.F16, pa.F32), "i8": (torch.int8, pa.I8, pa.I32)}[kind]
+    gen = torch.Generator(device="cuda").manual_seed(shape)
+    bm, bn, stage = SHAPES[shape][:3]
+    for kb, pitch, start, off in [(6 * stage, 6 * stage + 16, 0, True), (6 * stage - 16, 6 * stage + 16, 0, False), (6 * stage, 6 * stage + 128, 0, False),
+                                  (6 * stage, 6 * stage + 128, 64, True), (6 * stage + 36, 6 * stage + 68, 0, False), (7 * stage + 36, 7 * stage + 48, 80, True)]:
+        def rows(count):  # whole numbers of -7 .. 7, all sums below 2^24
+            flat = torch.full(((start + count * pitch) // esz,), 99 if kind == "i8" else float("nan"), device="cuda").to(tdt)
+            view = flat[start // esz:].view(count, pitch // esz)[:, :kb // esz]
+            view.copy_(torch.randint(-7, 8, view.shape, generator=gen, device="cuda"))
+            return view
+        a, b = rows(bm + 1), rows(2 * bn - 1)
+        with tile_env(PTOAMD_RING=shape):
+            got = pa.gemm(a, b, t, tc, pa.B_DN)
+            name = pa.last_kernel()
+        form = "dtl_lines" if off and shape in (3, 4, 6, 7) else "dtl"
+        assert name == f"tile{bm}x{bn}_{form}_{kind}", (kb, pitch, start, name)
+        assert torch.equal(got.double(), a.double() @ b.double().t()), (kb, pitch, start)
+
+
+def test_rows_copied_by_lines_beyond_2_gib(pa):  # noqa: F811
+    """Lane offsets past 2^31 bytes: rows 17 MB apart."""
+    m, n, k, pitch = 130, 65, 1024, (17 << 20) // 2 + 8
+    gen = torch.Generator(device="cuda").manual_seed(0)
+    a = torch.empty(m * pitch, dtype=torch.bfloat16, device="cuda").view(m, pitch)[:, :k]
+    a.copy_(torch.randint(-7, 8, (m, k), generator=gen, device="cuda"))
+    b = torch.randint(-7, 8, (n, k), generator=gen, device="cuda").to(torch.bfloat16)
+    with tile_env(PTOAMD_RING=3):
+        got = pa.gemm(a, b, pa.BF16, pa.F32, pa.B_DN)
+        assert pa.last_kernel() == "tile64x64_dtl_lines_bf16", pa.last_kernel()
+    assert torch.equal(got.double(), a.double() @ b.double().t())
+
+
+@pytest.mark.parametrize("shape", range(9))
 @pytest.mark.parametrize("kind", ["bf16", "f16"])
 def test_row_major_b(pa, oracle, kind, shape):  # noqa: F811
     """B as [K][N] with columns that end in part of a tile and rows at a wider pitch (the columns past N hold NaN), K ending
