@@ -93,7 +93,7 @@ struct RingCfg {
     static_assert(!SKEW || (PIPE && !BND && !ANY && !Op::SCALED && R >= 4), "two stages have to have landed where one is multiplied");
     static_assert(!ANY || (PIPE && !BND && !Op::SCALED), "the register copies are the copying waves' and know no scales");
     static_assert((ROWS * STAGE_SPS) % 64 == 0, "scale pieces are whole");
-    static_assert(!CHUNKED || (SCB / 4 % SPS == 0 && (SBUFS - 1) * SPC >= R - 1 && BM * SCB % 1024 == 0 && BN * SCB % 1024 == 0 && ROWS <= NW * 64),
+    static_assert(!CHUNKED || (SCB / 4 % SPS == 0 && (SBUFS - 1) * SPC >= R - 1 && BM * SCB % 1024 == 0 && BN * SCB % 1024 == 0 && ROWS <= CW * 64),
                   "a chunk of scales is whole stages; a 1 KiB copy of them is of one operand; a thread can hold a row's");
     static_assert(LDS_BYTES <= 160 * 1024 && R >= 2 && R * NV + (CHUNKED ? ROWS * SCB / 1024 / NW + 1 : 0) < 64, "LDS capacity; vmcnt is a 6-bit count");
 };
@@ -344,7 +344,9 @@ __global__ void __launch_bounds__(Cfg::THREADS) gemm_tile_ring_kernel(const Tile
     }
     // Scales in chunks: without scale arrays nothing is copied and the fragments' bytes, whatever they hold, are not used.  A row's
     // last 16 bytes are the 16 that END there, so where scale_ld is no multiple of 16 its last dwords lie scale_shift further on; a
-    // row shorter than that (K < 512) goes through registers.
+    // row shorter than that (K < 512) goes through registers, of the waves that multiply where others copy: these have nothing else under
+    // way, while in a copying wave the wait for the scales was one for all stages copied behind them (MXFP8 2048 x 4096 x 384 on 128 x
+    // 128 tiles 14.8 -> 14.2 us, 384 x 4096 x 384 7.75 -> 7.5).  Out of line: in the way, K of 512 and more took 2 % longer.
     const bool short_scales = CHUNKED && has_scales && p.scale_ld < 16;
     const int scale_last = CHUNKED ? p.scale_ld / 16 * 4 : 0, scale_shift = CHUNKED ? (4 - p.scale_ld / 4 % 4) % 4 : 0;
     auto issue_scales = [&](int chunk) __attribute__((always_inline)) {
@@ -364,10 +366,10 @@ __global__ void __launch_bounds__(Cfg::THREADS) gemm_tile_ring_kernel(const Tile
         }
     };
     uint32_t held_scales[3];
-    const int held_row = lw * 64 + lane;
+    const int held_row = tid;  // (a wave that multiplies)
     auto hold_short_scales = [&]() __attribute__((always_inline)) {
         if constexpr (CHUNKED) {
-            if (short_scales && held_row < Cfg::ROWS) {
+            if (__builtin_expect(short_scales, 0) && held_row < Cfg::ROWS) {
                 const uint8_t* row = held_row < BM ? p.sa + (long)min(m0 + held_row, p.m - 1) * p.scale_ld : p.sb + (long)min(n0 + held_row - BM, p.n - 1) * p.scale_ld;
 #pragma unroll
                 for (int d = 0; d < 3; ++d)
@@ -377,7 +379,7 @@ __global__ void __launch_bounds__(Cfg::THREADS) gemm_tile_ring_kernel(const Tile
     };
     auto write_short_scales = [&]() __attribute__((always_inline)) {
         if constexpr (CHUNKED) {
-            if (short_scales && held_row < Cfg::ROWS) {
+            if (__builtin_expect(short_scales, 0) && held_row < Cfg::ROWS) {
                 uint8_t* at = smem + R * Cfg::STAGE + held_row * Cfg::SCB + ring_scale_swizzle<Cfg::SCB>(held_row) * 16 + scale_shift * 4;
 #pragma unroll
                 for (int d = 0; d < 3; ++d)
@@ -658,12 +660,10 @@ __global__ void __launch_bounds__(Cfg::THREADS) gemm_tile_ring_kernel(const Tile
                     step(gc);
             });
         } else if (!computes) {
-            hold_short_scales();
 #pragma unroll
             for (int s = 0; s < R; ++s)
                 if (s < ncopy)
                     issue(s, s);
-            write_short_scales();
             // (SKEW: two stages, copies, up to a stage more of them)
             constexpr int AHEAD = Cfg::SKEW ? 2 : 1;
             loader_barrier(max(0, min(R - AHEAD, ncopy - AHEAD)));
@@ -675,6 +675,8 @@ __global__ void __launch_bounds__(Cfg::THREADS) gemm_tile_ring_kernel(const Tile
                 buf = buf + 1 == R ? 0 : buf + 1;
             }
         } else {
+            hold_short_scales();
+            write_short_scales();
             // the scale addresses of a stage and the next one's: computed a stage ahead, off the way from barrier to matrix instruction
             ScaleRows rows = scale_rows(0), next_rows = scale_rows(1);
             Skewed skew = skewed(0), next_skew = skewed(1);
