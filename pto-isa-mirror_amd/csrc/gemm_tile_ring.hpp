@@ -132,9 +132,11 @@ __device__ __forceinline__ uint4 ring_mask_chunk(uint4 v, int valid)
     return make_uint4(w[0], w[1], w[2], w[3]);
 }
 
-// Consecutive columns of an output row that one thread drains: 16 bytes of 16- and 32-bit outputs.
-template <int KIND>
-constexpr int ring_cols = out_bytes<KIND> == 2 ? 8 : 4;
+// Consecutive columns of an output row that one thread drains: 16 bytes of 16- and 32-bit outputs, 4 of one-byte outputs and, where a thread
+// would have more than four such pieces, 8 (int8 by a word: 256 x 128 tiles 0.91 to 0.97 of the time with 4, 128 x 128 0.93 to 0.97; on 128 x
+// 64, four pieces, 1.02).
+template <int KIND, class Cfg>
+constexpr int ring_cols = out_bytes<KIND> == 2 || (out_bytes<KIND> == 1 && Cfg::BM * Cfg::BN > 16 * Cfg::THREADS) ? 8 : 4;
 // What depends on the column only.  A thread drains the same columns of several rows and fetches these once (fetched with
 // every row they cost bf16 1237 x 4100 x 2056 with a bias row 8 us).
 template <int KIND, int NE, class Elem>
@@ -200,8 +202,11 @@ __device__ __forceinline__ void ring_store(const TileGemmParams& p, Elem (&v)[NE
         // Vector stores go to any address.  Non-temporal: C is not read again here, and written back from the L2s it slows the
         // next launch (2048 x 4096 x 4096 to f32: 82 us with plain stores, 67 with these).
         if constexpr (out_bytes<KIND> == 1) {
-            const uint32_t w = bits[0] | (bits[1] << 8) | (bits[2] << 16) | (bits[3] << 24);
-            __builtin_memcpy(dst, &w, 4);
+            uint32_t w[NE / 4];
+#pragma unroll
+            for (int i = 0; i < NE / 4; ++i)
+                w[i] = bits[4 * i] | (bits[4 * i + 1] << 8) | (bits[4 * i + 2] << 16) | (bits[4 * i + 3] << 24);
+            __builtin_memcpy(dst, w, NE);
         } else {
             typedef uint32_t nt4 __attribute__((ext_vector_type(4), aligned(1)));
             nt4 w;
@@ -749,7 +754,7 @@ __global__ void __launch_bounds__(Cfg::THREADS) gemm_tile_ring_kernel(const Tile
     // ---- TSTORE: the k-groups' partial sums meet in LDS (the ring is free), are added in group order and leave as 16
     // bytes per thread.  A block is transposed in its lanes: lane (l16, lg) holds row l16, columns 4 lg .. + 3.
     auto drain = [&](auto kc) __attribute__((always_inline)) {
-        constexpr int KIND = decltype(kc)::value, NE = ring_cols<KIND>, CT = BN / NE, RSTEP = Cfg::THREADS / CT;
+        constexpr int KIND = decltype(kc)::value, NE = ring_cols<KIND, Cfg>, CT = BN / NE, RSTEP = Cfg::THREADS / CT;
         static_assert(Cfg::THREADS % CT == 0, "a thread keeps its columns from row to row");
         const int c = (tid % CT) * NE, gj = n0 + c;
         // (what the columns and the first row bring is fetched while the sums are exchanged)

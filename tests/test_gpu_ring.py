@@ -314,6 +314,29 @@ def test_store_forms(pa, oracle, shape):  # noqa: F811
     assert bool((wide[:, n:] == 7.0).all())
 
 
+@pytest.mark.parametrize("shape", [3, 5, 6, 7, 8])
+@pytest.mark.parametrize("per_column", [False, True])
+def test_one_byte_results_in_pieces(pa, oracle, per_column, shape):  # noqa: F811
+    """A thread stores 4 or (shapes 6 to 8) 8 one-byte columns at a time: N ending on each of 8 columns of a piece, on rows at an odd
+    pitch whose other columns are kept."""
+    r = np.random.default_rng(60 + shape)
+    m, k = SHAPES[shape][0] + 5, 196
+    n_most = SHAPES[shape][1] + 16
+    a, b = (r.integers(-128, 128, (x, k)).astype(np.int8) for x in (m, n_most))
+    words = np.array([(int(np.float32(r.uniform(1e-4, 1e-3)).view(np.uint32)) & 0xFFFFE000) | (int(r.integers(0, 16)) << 37) | (1 << 46)
+                      for _ in range(n_most if per_column else 1)], np.uint64)
+    acc = oracle.matmul_i8(a, b, b_dn=True)
+    for n in range(n_most - 8, n_most):
+        w = words[:n] if per_column else words
+        wide = torch.full((m, n + 6 + n % 2), 7, dtype=torch.int8, device="cuda")
+        with tile_env(PTOAMD_RING=shape):
+            pa.gemm_requant(dev(a), dev(b[:n].copy()), pa.I8, pa.I8, dev(w.view(np.int64)), per_column=per_column, out=wide[:, 3:3 + n])
+            assert "_dtl_" in pa.last_kernel()
+        ref = np.asarray(oracle.store_quant(acc[:, :n].copy(), ob.ST_I8, w, per_column)).view(np.int8).reshape(m, n)
+        assert np.array_equal(host(wide)[:, 3:3 + n].view(np.int8), ref), n
+        assert bool((wide[:, :3] == 7).all()) and bool((wide[:, 3 + n:] == 7).all()), n
+
+
 @pytest.mark.parametrize("drain,m,n,k", [("column words", 3967, 2560, 320), ("column words", 1324, 6144, 168), ("raw", 3788, 3968, 384), ("atomic", 1981, 7296, 128)])
 def test_drains_keep_off_the_two_slab_128x128_tile(pa, drain, m, n, k):  # noqa: F811
     """Drains that the 128 x 128 tile stores element by element (a quantisation word per column, raw accumulators, atomic
