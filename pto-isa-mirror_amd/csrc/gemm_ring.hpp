@@ -18,9 +18,9 @@ struct TileGemmParams;
 // that issues copies stands still while the CU's memory queue is full (128 x 128, bf16 2048 x 2048 x 4096: 50 us with every
 // wave copying and multiplying, 33 us with the roles split).  From 64 x 64 on four waves multiply: eight on half of their wave
 // tiles read half as much again from LDS per product.  Four against eight, over full grids and part-filled ones: 64 x 64 0.92 to 0.99,
-// 96 x 64 and 128 x 64 fp8 0.93 and 0.98, plain types there level, 128 x 128 level, W8A8 on it 0.93; 256 x 128 on a full grid 0.96 to
-// 0.98, but on a part-filled one 1 to 3 % more (bf16 512 x 1024 x 1024 15.8 and 16.0 us): their last stage and drain have nothing
-// beside them.
+// 96 x 64 and 128 x 64 fp8 0.93 and 0.98, plain types there level, 128 x 128 level, W8A8 on it 0.93, MXFP8 1.02 up
+// to K 640 and 0.9 to 1 beyond; 256 x 128 0.94 to 0.98 on a full grid and with one-byte results, and level on a part-filled one and over few
+// slabs with 16- or 32-bit results, whose last stage and drain have nothing beside them (bf16 512 x 1024 x 1024 16.0 and 16.2 us).
 #define PTOAMD_RING_SHAPES_ALL(X)                                 \
     X(0, 32, 16, 1, 1, 8, 1024, 3, 1, 1, 8, 1024, 3, 0, false)    \
     X(1, 32, 32, 1, 1, 8, 512, 4, 1, 2, 4, 512, 4, 0, false)      \

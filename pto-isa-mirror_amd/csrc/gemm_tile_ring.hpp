@@ -792,11 +792,12 @@ __global__ void __launch_bounds__(Cfg::THREADS) gemm_tile_ring_kernel(const Tile
                 rs = p.row_scale[min(m0 + r + RSTEP, p.m - 1)];
             ring_store<KIND>(p, v, cols, row_scale, m0 + r, gj);
         };
-        // (Where a thread has more than one row piece, four of them in flight: one after the other each waits for its LDS reads, which
-        // showed where four waves multiply and fewer threads drain.  256 x 128 tiles, bf16 1536 x 2560 x 640 14.5 -> 13.9 us, W8A8 512 x
-        // 1024 x 1024 0.95 of before; eight in flight int8 to int32 2 % less, W8A8 on 192 x 128 3 % more.)
+        // (Where a thread has more than one row piece, four of them in flight, eight of sixteen: one after the other each waits for its LDS
+        // reads, which showed where four waves multiply and fewer threads drain.  256 x 128 tiles, bf16 1536 x 2560 x 640 14.5 -> 13.9 us, W8A8
+        // 512 x 1024 x 1024 0.95 of before; with eight in flight int8 to int32 512 x 1024 x 1024 11.95 -> 11.7 us, but W8A8 on 192 x 128 3 % more.)
         if constexpr (RSTEP < BM) {
-#pragma unroll 4
+            constexpr int FLIGHT = BM / RSTEP >= 16 ? 8 : 4;
+#pragma unroll FLIGHT
             for (int r = tid / CT; r < BM && m0 + r < p.m; r += RSTEP)
                 drain_row(r);
         } else {
