@@ -589,6 +589,14 @@ __device__ __forceinline__ void tstore_staged(const TileGemmParams& p, Acc (&acc
             rs_pre[i] = p.row_scale[min(row0 + i * BLK + l32, p.m - 1)];
         fetch_columns(cs_pre, p.col_scale);
     }
+    // C is not read again by this kernel: pieces of whole 64-byte sectors are stored non-temporally (plain stores end TSTORE 0.3 us
+    // sooner, but their write-backs cost the next launch 1 us).  Where rows start off the sectors, two wave tiles share one at every
+    // seam: streamed, its parts go to memory one by one, written plainly they meet in the L2.  4096 x n x 1024 on 256 x 256 tiles, us,
+    // streamed and plain: bf16 n 4096 27.6 / 28.4, 4128 46.6 / 45.9, 4104 51.9 / 46.3, 4100 52.6 / 46.3; f32 4128 51.6 / 50.2, 4104 58.6 /
+    // 50.7; one byte 4104 56.3 / 53.2; 128 x 128 tiles bf16 4100 45.7 / 42.8, f32 4100 55.3 / 50.0, but one byte 57.2 / 58.8 (a wave's
+    // pieces are a sector long there, and its drain is bound by the conversions); MXFP4 2040 x 8100 x 8192 72.1 / 66.0.
+    constexpr bool NARROW = ESZ == 1 && Cfg::BM * Cfg::BN < 65536;
+    const bool streamed = NARROW || ((reinterpret_cast<uintptr_t>(p.c) | (uintptr_t)p.ldc * ESZ) & 63) == 0;
     constexpr int EPC = 16 / ESZ;  // elements of a chunk
     const int live = EDGE ? p.n - col0 : Cfg::WTN, whole = live / EPC, rest = live % EPC;
     static_assert(64 % CHUNKS == 0, "a lane stores the same chunk of several rows");
@@ -649,9 +657,15 @@ __device__ __forceinline__ void tstore_staged(const TileGemmParams& p, Acc (&acc
             nt_u32x4* dst = reinterpret_cast<nt_u32x4*>(reinterpret_cast<uint8_t*>(p.c) +
                                                         ((long)(row0 + band * 32 + row) * p.ldc + col0) * ESZ + ch * 16);
             const nt_u32x4 vv = {v.x, v.y, v.z, v.w};
-            if (row0 + band * 32 + row < row_end)
-                __builtin_nontemporal_store(vv, dst);  // C is not read again by this kernel: keep it out of the L2's way (plain stores end TSTORE
-                                                   // 0.3 us sooner, but their write-backs cost the next launch 1 us)
+            if (row0 + band * 32 + row < row_end) {
+                if (streamed) {
+                    __builtin_nontemporal_store(vv, dst);
+                } else {
+                    asm volatile("");  // (both stores would be made one, a plain one)
+                    *dst = vv;
+                    asm volatile("");
+                }
+            }
         }
         if constexpr (EDGE) {
             if (rest != 0 && lane < 32 && row0 + band * 32 + lane < p.m) {

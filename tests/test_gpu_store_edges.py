@@ -89,3 +89,24 @@ def test_quantised_wave_tiles_that_cross_n(pa, per_column, kind, tile):  # noqa:
         assert torch.equal(wide[:, lead:lead + n].contiguous().view(raw), ref[:, :n].contiguous().view(raw)), (kind, tile, n, c_type)
         assert ref[:, :n].unique().numel() > 4
         assert (wide[:, :lead] == 77).all() and (wide[:, lead + n:] == 77).all(), (kind, tile, n, c_type)
+
+
+@pytest.mark.parametrize("tile", [1, 2, 4, 5, 6])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_rows_on_and_off_the_64_byte_sectors(pa, dtype, tile):  # noqa: F811
+    """Rows of C on whole sectors are stored non-temporally, others plainly: the same bits, nothing around them."""
+    gen = torch.Generator(device="cuda").manual_seed(tile)
+    m, n, k = 130, 261, 256
+    a, b = (torch.randint(-3, 4, (x, k), generator=gen, device="cuda") for x in (m, n))
+    ref = (a.double() @ b.double().T).float().to(dtype)
+    sector = 64 // ref.element_size()
+    wide = torch.empty(m * 400 + 2 * sector, device="cuda", dtype=dtype)
+    assert wide.data_ptr() % 64 == 0
+    # (row pitch in elements, columns in front of C): on the sectors; the pitch off them; the first row off them
+    for pitch, lead in [(288, 0), (288, sector), (288 + sector // 2, 0), (289, 0), (288, 1), (288, sector // 2)]:
+        wide.fill_(77)
+        view = wide[:m * pitch].view(m, pitch) if lead == 0 else wide[lead:lead + m * pitch].view(m, pitch)
+        with tile_env(PTOAMD_TILE=tile):
+            pa.gemm(a.bfloat16(), b.bfloat16(), pa.BF16, pa.F32 if dtype == torch.float32 else pa.BF16, pa.B_DN, out=view[:, :n])
+        assert torch.equal(view[:, :n], ref), (tile, pitch, lead)
+        assert (view[:, n:] == 77).all() and (wide[:lead] == 77).all() and (wide[lead + m * pitch:] == 77).all(), (tile, pitch, lead)
