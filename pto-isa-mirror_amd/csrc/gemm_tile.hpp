@@ -649,23 +649,29 @@ __device__ __forceinline__ void tstore_staged(const TileGemmParams& p, Acc (&acc
             });
         });
         __builtin_amdgcn_sched_barrier(0);
+        auto store_band = [&](auto nt) __attribute__((always_inline)) {
 #pragma unroll
-        for (int it = 0; it < ITERS; ++it) {
-            const int q = it * 64 + lane, row = q / CHUNKS, ch = q % CHUNKS;
-            const uint4 v = *reinterpret_cast<const uint4*>(stage + row * ROW_BYTES + ch * 16);
-            typedef unsigned int nt_u32x4 __attribute__((ext_vector_type(4), aligned(1)));
-            nt_u32x4* dst = reinterpret_cast<nt_u32x4*>(reinterpret_cast<uint8_t*>(p.c) +
-                                                        ((long)(row0 + band * 32 + row) * p.ldc + col0) * ESZ + ch * 16);
-            const nt_u32x4 vv = {v.x, v.y, v.z, v.w};
-            if (row0 + band * 32 + row < row_end) {
-                if (streamed) {
-                    __builtin_nontemporal_store(vv, dst);
-                } else {
-                    asm volatile("");  // (both stores would be made one, a plain one)
-                    *dst = vv;
-                    asm volatile("");
+            for (int it = 0; it < ITERS; ++it) {
+                const int q = it * 64 + lane, row = q / CHUNKS, ch = q % CHUNKS;
+                const uint4 v = *reinterpret_cast<const uint4*>(stage + row * ROW_BYTES + ch * 16);
+                typedef unsigned int nt_u32x4 __attribute__((ext_vector_type(4), aligned(1)));
+                nt_u32x4* dst = reinterpret_cast<nt_u32x4*>(reinterpret_cast<uint8_t*>(p.c) +
+                                                            ((long)(row0 + band * 32 + row) * p.ldc + col0) * ESZ + ch * 16);
+                const nt_u32x4 vv = {v.x, v.y, v.z, v.w};
+                if (row0 + band * 32 + row < row_end) {
+                    if constexpr (decltype(nt)::value)
+                        __builtin_nontemporal_store(vv, dst);
+                    else
+                        *dst = vv;
                 }
             }
+        };
+        if (streamed) {
+            store_band(std::true_type{});
+        } else {
+            asm volatile("");  // (the two would be made one, of plain stores)
+            store_band(std::false_type{});
+            asm volatile("");
         }
         if constexpr (EDGE) {
             if (rest != 0 && lane < 32 && row0 + band * 32 + lane < p.m) {
