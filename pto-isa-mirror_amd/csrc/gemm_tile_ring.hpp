@@ -120,17 +120,17 @@ __device__ __forceinline__ void ring_wait_and_barrier()
 }
 
 // the K tail: of the 16 bytes of a fragment chunk only `valid` belong to the row, the last ones (valid >= 16: all)
-__device__ __forceinline__ uint4 ring_mask_chunk(uint4 v, int valid)
+__device__ __forceinline__ uint4 ring_chunk_mask(int valid)
 {
-    const int drop = 16 - valid;  // low bytes to clear
-    uint32_t w[4] = {v.x, v.y, v.z, v.w};
+    uint32_t m[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-        const int n = drop - 4 * i;
-        w[i] = n <= 0 ? w[i] : (n >= 4 ? 0u : w[i] & (0xFFFFFFFFu << (8 * n)));
+        const int n = 16 - valid - 4 * i;  // low bytes of the dword to clear
+        m[i] = n <= 0 ? 0xFFFFFFFFu : (n >= 4 ? 0u : 0xFFFFFFFFu << (8 * n));
     }
-    return make_uint4(w[0], w[1], w[2], w[3]);
+    return make_uint4(m[0], m[1], m[2], m[3]);
 }
+__device__ __forceinline__ uint4 ring_masked(uint4 v, uint4 m) { return make_uint4(v.x & m.x, v.y & m.y, v.z & m.z, v.w & m.w); }
 
 // Consecutive columns of an output row that one thread drains: 16 bytes of 16- and 32-bit outputs, 4 of one-byte outputs and, where a thread
 // would have more than four such pieces, 8 (int8 by a word: 256 x 128 tiles 0.91 to 0.97 of the time with 4, 128 x 128 0.93 to 0.97; on 128 x
@@ -347,7 +347,8 @@ __global__ void __launch_bounds__(Cfg::THREADS) gemm_tile_ring_kernel(const Tile
             sc_row[q] = !has_scales ? p.a : r < BM ? p.sa + (long)min(m0 + r, p.m - 1) * p.scale_ld : p.sb + (long)min(n0 + r - BM, p.n - 1) * p.scale_ld;
         }
     }
-    // Scales in chunks: without scale arrays nothing is copied and the fragments' bytes, whatever they hold, are not used.  A row's
+    // Scales in chunks: without scale arrays nothing is copied and the buffers hold E8M0 127 (selected per fragment, the scales cost
+    // a VALU instruction and a wait for each in front of the matrix instructions).  A row's
     // last 16 bytes are the 16 that END there, so where scale_ld is no multiple of 16 its last dwords lie scale_shift further on; a
     // row shorter than that (K < 512) goes through registers, of the waves that multiply where others copy: these have nothing else under
     // way, while in a copying wave the wait for the scales was one for all stages copied behind them (MXFP8 2048 x 4096 x 384 on 128 x
@@ -391,6 +392,13 @@ __global__ void __launch_bounds__(Cfg::THREADS) gemm_tile_ring_kernel(const Tile
                     if (4 * d < p.scale_ld)
                         *reinterpret_cast<uint32_t*>(at + 4 * d) = held_scales[d];
             }
+        }
+    };
+    auto fill_scales = [&]() __attribute__((always_inline)) {
+        if constexpr (CHUNKED) {
+            if (__builtin_expect(!has_scales, 0))
+                for (int o = tid * 16; o < Cfg::SCALE_BYTES; o += Cfg::CW * 64 * 16)
+                    *reinterpret_cast<uint4*>(smem + R * Cfg::STAGE + o) = make_uint4(0x7F7F7F7Fu, 0x7F7F7F7Fu, 0x7F7F7F7Fu, 0x7F7F7F7Fu);
         }
     };
     auto issue = [&](int st, int buf) __attribute__((always_inline)) {
@@ -533,26 +541,28 @@ __global__ void __launch_bounds__(Cfg::THREADS) gemm_tile_ring_kernel(const Tile
             read_b(set, j, s, b, sc, sk);
 #pragma unroll
         for (int i = 0; i < MB; ++i)
-            read_a(Cfg::PIPE ? aset(set, i) : 0, i, s, b, sc, sk);
+            read_a(aset(set, i), i, s, b, sc, sk);
     };
     auto mma = [&](int set, int i, int j) __attribute__((always_inline)) {
-        const int as = Cfg::PIPE ? aset(set, i) : 0;
-        Op::mma(acc[i][j], fa[as][i], fb[set][j], Op::SCALED ? (has_scales ? xa[as][i] : 127u) : 0u, Op::SCALED ? (has_scales ? xb[set][j] : 127u) : 0u);
+        const int as = aset(set, i);
+        Op::mma(acc[i][j], fa[as][i], fb[set][j], Op::SCALED ? (CHUNKED || has_scales ? xa[as][i] : 127u) : 0u, Op::SCALED ? (CHUNKED || has_scales ? xb[set][j] : 127u) : 0u);
     };
     // k-step s of the last stage, which may reach past K
     auto tail_step = [&](int set, int s) __attribute__((always_inline)) {
         const int k0 = (nst - 1) * SB + wk * Cfg::KW + s * Cfg::KB;  // first K byte of the step
         if (k0 >= p.k_bytes)
             return;
+        if (k_tail) {
 #pragma unroll
-        for (int f = 0; f < FR; ++f) {
-            const int valid = p.k_bytes - (k0 + (4 * f + lg) * 16);
+            for (int f = 0; f < FR; ++f) {
+                const uint4 mask = ring_chunk_mask(p.k_bytes - (k0 + (4 * f + lg) * 16));
 #pragma unroll
-            for (int i = 0; i < MB; ++i)
-                fa[Cfg::PIPE ? aset(set, i) : 0][i][f] = ring_mask_chunk(fa[Cfg::PIPE ? aset(set, i) : 0][i][f], valid);
+                for (int i = 0; i < MB; ++i)
+                    fa[aset(set, i)][i][f] = ring_masked(fa[aset(set, i)][i][f], mask);
 #pragma unroll
-            for (int j = 0; j < NB; ++j)
-                fb[set][j][f] = ring_mask_chunk(fb[set][j][f], valid);
+                for (int j = 0; j < NB; ++j)
+                    fb[set][j][f] = ring_masked(fb[set][j][f], mask);
+            }
         }
 #pragma unroll
         for (int i = 0; i < MB; ++i)
@@ -575,6 +585,7 @@ __global__ void __launch_bounds__(Cfg::THREADS) gemm_tile_ring_kernel(const Tile
         // Barrier st: stage st has landed and no wave reads stage st - 1 any more, whose buffer is refilled.
         if (loads) {
             hold_short_scales();
+            fill_scales();
 #pragma unroll
             for (int s = 0; s < R - 1; ++s)
                 if (s < nst)
@@ -613,7 +624,7 @@ __global__ void __launch_bounds__(Cfg::THREADS) gemm_tile_ring_kernel(const Tile
                 tail_step(0, decltype(sc)::value);
             });
     } else {
-        // Barrier st stands before the last k-step of stage st: every wave holds that k-step's fragments, so the stage's
+        // Barrier st stands in front of or in the last k-step of stage st: every wave holds that k-step's fragments, so the stage's
         // buffer is refilled with stage st + R, and stage st + 1 has landed, whose first fragments are read under that
         // k-step's matrix instructions.
         static_assert(Cfg::LW > 0, "the pipelined form has waves that only copy");
@@ -665,13 +676,20 @@ __global__ void __launch_bounds__(Cfg::THREADS) gemm_tile_ring_kernel(const Tile
                     step(gc);
             });
         } else if (!computes) {
-#pragma unroll
-            for (int s = 0; s < R; ++s)
+            // (SKEW: two stages, copies, up to a stage more of them)
+            // The first barrier stands behind one stage more than the multiplying waves need, not behind the whole ring: to issue that takes 1.3
+            // to 2 us on a cold start, long after the first stage has landed.  First product at 1.55 instead of 1.95 us (MXFP8 384 x 4096 x 4096
+            // on 96 x 64 tiles, launch 12.2 -> 11.8 us), 0.9 instead of 1.45 (bf16 2048 x 2048 x 4096 on 128 x 128, 32.0 -> 31.3); behind just what
+            // they need it is 0.1 us earlier and the launch no shorter.
+            constexpr int AHEAD = Cfg::SKEW ? 2 : 1, EARLY = AHEAD + 1;
+            static_assert(EARLY < R, "the ring holds more than the first barrier waits for");
+            static_for<R>([&](auto sc) {
+                constexpr int s = decltype(sc)::value;
+                if constexpr (s == EARLY)
+                    loader_barrier(max(0, min(EARLY - AHEAD, ncopy - AHEAD)));
                 if (s < ncopy)
                     issue(s, s);
-            // (SKEW: two stages, copies, up to a stage more of them)
-            constexpr int AHEAD = Cfg::SKEW ? 2 : 1;
-            loader_barrier(max(0, min(R - AHEAD, ncopy - AHEAD)));
+            });
             int buf = 0;
             for (int st = 0; st < nst - 1; ++st) {
                 loader_barrier(max(0, min(R - 1 - AHEAD, ncopy - 1 - AHEAD - st)));
@@ -681,6 +699,7 @@ __global__ void __launch_bounds__(Cfg::THREADS) gemm_tile_ring_kernel(const Tile
             }
         } else {
             hold_short_scales();
+            fill_scales();
             write_short_scales();
             // the scale addresses of a stage and the next one's: computed a stage ahead, off the way from barrier to matrix instruction
             ScaleRows rows = scale_rows(0), next_rows = scale_rows(1);
@@ -688,8 +707,9 @@ __global__ void __launch_bounds__(Cfg::THREADS) gemm_tile_ring_kernel(const Tile
             ring_wait_and_barrier<63>();
             read_all(0, 0, 0, rows, skew);
             int buf = 0, st = 0;
-            auto body = [&](auto parc) __attribute__((always_inline)) {
+            auto body = [&](auto parc, auto lastc) __attribute__((always_inline)) {
                 constexpr int PAR = decltype(parc)::value;
+                constexpr bool LASTSTAGE = decltype(lastc)::value;
                 const int nbuf = buf + 1 == R ? 0 : buf + 1;
                 static_for<Cfg::KSTEPS>([&](auto sc) {
                     constexpr int s = decltype(sc)::value, SET = (PAR + s) & 1;
@@ -698,18 +718,26 @@ __global__ void __launch_bounds__(Cfg::THREADS) gemm_tile_ring_kernel(const Tile
                     const int rb = LASTSTEP ? nbuf : buf;
                     const ScaleRows& rsc = LASTSTEP ? next_rows : rows;
                     const Skewed& rsk = LASTSTEP ? next_skew : skew;
-                    if constexpr (LASTSTEP)
-                        ring_wait_and_barrier<63>();
-                    // (reads pinned behind the instruction that frees their registers; B first, each next k-step needs all of it)
+                    // The barrier waits for the wave's own reads, the last of which go out a row of matrix instructions before the k-step's end:
+                    // it stands a row into the last k-step, so that two rows cover them (and nothing is moved across it: the compiler put
+                    // all but one of that row's instructions behind it).  128 x 128 tiles 700 -> 680 clocks a stage, 256 x 128 1211 -> 1160, 192 x
+                    // 128 970 -> 953, MXFP8 on 96 x 64 936 -> 880.
+                    constexpr int BAR = LASTSTEP && MB > 1 && NMMA >= 6 ? NB : 0;
                     static_for<NMMA>([&](auto xc) {
                         constexpr int x = decltype(xc)::value, i = x / NB, j = x % NB;
-                        mma(SET, i, j);
-                        constexpr int AL = NB < NMMA ? NB : NMMA - 1;
-                        if constexpr (x < NB || x == AL || (j == NB - 1 && i < MB - 1)) {
+                        if constexpr (LASTSTEP && !LASTSTAGE && x == BAR) {
                             __builtin_amdgcn_sched_barrier(0);
-                            if constexpr (x < NB)
-                                read_b(SET ^ 1, x, rs, rb, rsc, rsk);
-                            if constexpr (x == AL)
+                            ring_wait_and_barrier<63>();
+                        }
+                        mma(SET, i, j);
+                        constexpr int y = x - BAR, AL = NB < NMMA - BAR ? NB : NMMA - BAR - 1;
+                        if constexpr (!(LASTSTEP && LASTSTAGE) && y >= 0 && (y < NB || y == AL || (j == NB - 1 && i < MB - 1))) {
+                            __builtin_amdgcn_sched_barrier(0);
+                            if constexpr (y < NB)
+                                read_b(SET ^ 1, y, rs, rb, rsc, rsk);
+                            if constexpr (y == 0)
+                                static_for<BAR / NB>([&](auto rc) { read_a(0, decltype(rc)::value, rs, rb, rsc, rsk); });
+                            if constexpr (y == AL)
                                 read_a(SET ^ 1, MB - 1, rs, rb, rsc, rsk);
                             if constexpr (j == NB - 1 && i < MB - 1)
                                 read_a(0, i, rs, rb, rsc, rsk);
@@ -717,6 +745,8 @@ __global__ void __launch_bounds__(Cfg::THREADS) gemm_tile_ring_kernel(const Tile
                         }
                     });
                 });
+                if constexpr (LASTSTAGE)
+                    return;
                 buf = nbuf;
                 ++st;
                 rows = next_rows;
@@ -725,6 +755,14 @@ __global__ void __launch_bounds__(Cfg::THREADS) gemm_tile_ring_kernel(const Tile
                 next_skew = skewed(nbuf + 1 == R ? 0 : nbuf + 1);
             };
             auto last = [&](auto parc) __attribute__((always_inline)) {
+                // (K of whole stages: as any other stage.  Larger wave tiles have no registers for a second copy of the loop's body: 256 x 128
+                // tiles kept 164 bytes of it in scratch memory and took 65 us instead of 55)
+                if constexpr (NMMA * FR <= 16) {
+                    if (!k_tail) {
+                        body(parc, std::true_type{});
+                        return;
+                    }
+                }
                 static_for<Cfg::KSTEPS>([&](auto sc) {
                     constexpr int s = decltype(sc)::value, SET = (decltype(parc)::value + s) & 1;
                     if constexpr (s > 0)
@@ -734,15 +772,15 @@ __global__ void __launch_bounds__(Cfg::THREADS) gemm_tile_ring_kernel(const Tile
             };
             if constexpr (Cfg::KSTEPS % 2 == 0) {
                 while (st < nst - 1)
-                    body(integral_constant<int, 0>{});
+                    body(integral_constant<int, 0>{}, std::false_type{});
                 last(integral_constant<int, 0>{});
             } else {  // the register sets change places from stage to stage
                 while (st + 2 < nst) {
-                    body(integral_constant<int, 0>{});
-                    body(integral_constant<int, 1>{});
+                    body(integral_constant<int, 0>{}, std::false_type{});
+                    body(integral_constant<int, 1>{}, std::false_type{});
                 }
                 if (st + 1 < nst) {
-                    body(integral_constant<int, 0>{});
+                    body(integral_constant<int, 0>{}, std::false_type{});
                     last(integral_constant<int, 1>{});
                 } else {
                     last(integral_constant<int, 0>{});

@@ -437,3 +437,34 @@ def test_requantised_columns_that_end_inside_a_wave_tile(pa, m, n, k, per_column
     with tile_env(PTOAMD_TILE=2):
         assert torch.equal(got, pa.gemm_requant(a, b, pa.I8, pa.I8, words, per_column=per_column))
     assert got.unique().numel() > 100
+
+
+@pytest.mark.parametrize("shape", range(9))
+@pytest.mark.parametrize("kind", ["bf16", "i8", "fp8"])
+def test_every_count_of_stages(pa, kind, shape):  # noqa: F811
+    """One stage of K to three more than a ring holds, whole and with a chunk and four bytes more (fp8: MX blocks), every remainder of a
+    thread's columns, 32- and 16-bit results: exact, the sums being whole numbers below 2^24."""
+    scaled = kind == "fp8"
+    if scaled and SHAPES[shape][3] is None:
+        pytest.skip("the plain types' shape")
+    bm, bn, stage = SHAPES[shape][0], SHAPES[shape][1], SHAPES[shape][3 if scaled else 2]
+    gen = torch.Generator(device="cuda").manual_seed(shape)
+    for count in range(1, 8):
+        for tail in (0, 128 if scaled else 20):
+            kb, m, n = count * stage + tail, bm + 1, bn + count
+            k = kb // 2 if kind == "bf16" else kb
+            a, b = (torch.randint(-3, 4, (x, k), generator=gen, device="cuda") for x in (m, n))
+            ref = a.double() @ b.double().T
+            with tile_env(PTOAMD_RING=shape):
+                if kind == "fp8":
+                    lut = torch.tensor([0, 0x38, 0x40, 0x44], device="cuda", dtype=torch.uint8)  # 0, 1, 2, 3 in E4M3
+                    ca, cb = (lut[x.abs()] | (0x80 * (x < 0)).to(torch.uint8) for x in (a, b))
+                    got = pa.gemm_fp8(ca, cb, pa.E4M3, pa.E4M3, pa.F32 if count % 2 else pa.BF16)
+                elif kind == "bf16":
+                    bias = torch.randint(-9, 10, (n,), generator=gen, device="cuda").float()
+                    got = pa.gemm(a.bfloat16(), b.bfloat16(), pa.BF16, pa.F32 if count % 2 else pa.BF16, pa.B_DN, bias=bias)
+                    ref = ref + bias.double()
+                else:
+                    got = pa.gemm(a.to(torch.int8), b.to(torch.int8), pa.I8, pa.I32, pa.B_DN)
+                assert pa.last_kernel().startswith(f"tile{bm}x{bn}_"), pa.last_kernel()
+            assert torch.equal(got, ref.float().to(got.dtype)), (kind, m, n, kb)
