@@ -135,8 +135,19 @@ __device__ __forceinline__ uint4 ring_masked(uint4 v, uint4 m) { return make_uin
 // Consecutive columns of an output row that one thread drains: 16 bytes of 16- and 32-bit outputs, 4 of one-byte outputs and, where a thread
 // would have more than four such pieces, 8 (int8 by a word: 256 x 128 tiles 0.91 to 0.97 of the time with 4, 128 x 128 0.93 to 0.97; on 128 x
 // 64, four pieces, 1.02).
+// Half or a quarter of that on the narrow tiles, which have fewer elements than that many times their threads: the pieces of a thread are
+// added and stored one after the other while most threads have none.  bf16 24 x 4096 x 4096 on 32 x 16 tiles 7.48 -> 7.09 us, 64 x 8192 x
+// 1024 on 64 x 32 6.0 -> 5.5.
 template <int KIND, class Cfg>
-constexpr int ring_cols = out_bytes<KIND> == 2 || (out_bytes<KIND> == 1 && Cfg::BM * Cfg::BN > 16 * Cfg::THREADS) ? 8 : 4;
+constexpr int ring_columns()
+{
+    int ne = out_bytes<KIND> == 2 || (out_bytes<KIND> == 1 && Cfg::BM * Cfg::BN > 16 * Cfg::THREADS) ? 8 : 4;
+    while (out_bytes<KIND> > 1 && ne > 2 && Cfg::BM * Cfg::BN < ne * Cfg::THREADS)
+        ne /= 2;
+    return ne;
+}
+template <int KIND, class Cfg>
+constexpr int ring_cols = ring_columns<KIND, Cfg>();
 // What depends on the column only.  A thread drains the same columns of several rows and fetches these once (fetched with
 // every row they cost bf16 1237 x 4100 x 2056 with a bias row 8 us).
 template <int KIND, int NE, class Elem>
@@ -146,12 +157,15 @@ struct RingColumns {
     uint64_t qw[NE];
     __device__ __forceinline__ void load(const TileGemmParams& p, int gj)
     {
+        if (p.bias != nullptr) {
+#pragma unroll
+            for (int e = 0; e < NE; ++e)
+                bias[e] = reinterpret_cast<const Elem*>(p.bias)[min(gj + e, p.n - 1)];
+        }
 #pragma unroll
         for (int e = 0; e < NE; ++e) {
-            const int c = min(gj + e, p.n - 1);
-            bias[e] = p.bias != nullptr ? reinterpret_cast<const Elem*>(p.bias)[c] : 0;
-            scale[e] = KIND == OUT_W8A8_BF16 ? p.col_scale[c] : 1.0f;
-            qw[e] = out_quant<KIND> ? p.qwords[p.q_per_column ? c : 0] : 0;
+            scale[e] = KIND == OUT_W8A8_BF16 ? p.col_scale[min(gj + e, p.n - 1)] : 1.0f;
+            qw[e] = out_quant<KIND> ? p.qwords[p.q_per_column ? min(gj + e, p.n - 1) : 0] : 0;
         }
     }
 };
@@ -208,12 +222,20 @@ __device__ __forceinline__ void ring_store(const TileGemmParams& p, Elem (&v)[NE
                 w[i] = bits[4 * i] | (bits[4 * i + 1] << 8) | (bits[4 * i + 2] << 16) | (bits[4 * i + 3] << 24);
             __builtin_memcpy(dst, w, NE);
         } else {
-            typedef uint32_t nt4 __attribute__((ext_vector_type(4), aligned(1)));
-            nt4 w;
+            constexpr int WORDS = NE * out_bytes<KIND> / 4;
+            uint32_t w[WORDS];
 #pragma unroll
-            for (int i = 0; i < 4; ++i)
-                w[i] = out_bytes<KIND> == 2 ? bits[(2 * i) % NE] | (bits[(2 * i + 1) % NE] << 16) : bits[i];
-            __builtin_nontemporal_store(w, reinterpret_cast<nt4*>(dst));
+            for (int i = 0; i < WORDS; ++i)
+                w[i] = out_bytes<KIND> == 2 ? bits[(2 * i) % NE] | (bits[(2 * i + 1) % NE] << 16) : bits[i % NE];
+            typedef uint32_t nt1 __attribute__((aligned(1)));
+            typedef uint32_t nt2 __attribute__((ext_vector_type(2), aligned(1)));
+            typedef uint32_t nt4 __attribute__((ext_vector_type(4), aligned(1)));
+            if constexpr (WORDS == 1)
+                __builtin_nontemporal_store(w[0], reinterpret_cast<nt1*>(dst));
+            else if constexpr (WORDS == 2)
+                __builtin_nontemporal_store(nt2{w[0], w[1]}, reinterpret_cast<nt2*>(dst));
+            else
+                __builtin_nontemporal_store(nt4{w[0], w[1], w[2], w[3]}, reinterpret_cast<nt4*>(dst));
         }
     } else {
 #pragma unroll
@@ -789,11 +811,13 @@ __global__ void __launch_bounds__(Cfg::THREADS) gemm_tile_ring_kernel(const Tile
         }
     }
 
-    // ---- TSTORE: the k-groups' partial sums meet in LDS (the ring is free), are added in group order and leave as 16
-    // bytes per thread.  A block is transposed in its lanes: lane (l16, lg) holds row l16, columns 4 lg .. + 3.
+    // ---- TSTORE: the k-groups' partial sums meet in LDS (the ring is free), are added in group order and leave as up to 16
+    // bytes per thread and row.  A block is transposed in its lanes: lane (l16, lg) holds row l16, columns 4 lg .. + 3.
     auto drain = [&](auto kc) __attribute__((always_inline)) {
         constexpr int KIND = decltype(kc)::value, NE = ring_cols<KIND, Cfg>, CT = BN / NE, RSTEP = Cfg::THREADS / CT;
         static_assert(Cfg::THREADS % CT == 0, "a thread keeps its columns from row to row");
+        constexpr int VW = NE < 4 ? NE : 4;
+        typedef Elem Piece __attribute__((ext_vector_type(VW)));
         const int c = (tid % CT) * NE, gj = n0 + c;
         // (what the columns and the first row bring is fetched while the sums are exchanged)
         RingColumns<KIND, NE, Elem> cols;
@@ -819,11 +843,11 @@ __global__ void __launch_bounds__(Cfg::THREADS) gemm_tile_ring_kernel(const Tile
 #pragma unroll
             for (int g = 0; g < Cfg::WK; ++g)
 #pragma unroll
-                for (int q = 0; q < NE / 4; ++q) {
-                    const Acc x = *reinterpret_cast<const Acc*>(reinterpret_cast<const Elem*>(smem) + (g * BM + r) * Cfg::RED_PITCH + c + 4 * q);
+                for (int q = 0; q < NE / VW; ++q) {
+                    const Piece x = *reinterpret_cast<const Piece*>(reinterpret_cast<const Elem*>(smem) + (g * BM + r) * Cfg::RED_PITCH + c + VW * q);
 #pragma unroll
-                    for (int e = 0; e < 4; ++e)
-                        v[4 * q + e] += x[e];
+                    for (int e = 0; e < VW; ++e)
+                        v[VW * q + e] += x[e];
                 }
             const float row_scale = rs;
             if (KIND == OUT_W8A8_BF16)
