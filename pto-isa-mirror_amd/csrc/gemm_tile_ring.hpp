@@ -264,11 +264,13 @@ struct RingDivisor {
     }
     __device__ __forceinline__ int divide(int n) const { return (int)(((uint64_t)(uint32_t)n * magic) >> shift); }
 };
-// Workgroup -> tile, worked out by the host: `grid` tiles in tiles_m rows, walked in groups of group_m rows (the last group of
-// group_last); per_group tiles make a group.  Two divisions of run-time values in the kernel took 90 scalar instructions.
+// Workgroup -> tile, prepared by the host: `grid` tiles in tiles_m rows, walked in groups of rows; per_group tiles make a group of
+// RING_GROUP rows (the last one has fewer), or all tiles are one group of tiles_m rows (per_group = grid).  divisor: of per_group,
+// or of tiles_m.  Two divisions of run-time values in the kernel took 90 scalar instructions.
+constexpr int RING_GROUP = 4;
 struct RingTiles {
-    int grid, tiles_m, group_m, per_group;
-    RingDivisor by_group, by_group_m, by_group_last;
+    int grid, tiles_m, per_group;
+    RingDivisor divisor;
 };
 inline RingTiles ring_tiles(const TileGemmParams& p, int bm, int bn)
 {
@@ -276,15 +278,13 @@ inline RingTiles ring_tiles(const TileGemmParams& p, int bm, int bn)
     const int tiles_n = (p.n + bn - 1) / bn;
     t.tiles_m = (p.m + bm - 1) / bm;
     t.grid = t.tiles_m * tiles_n;
-    t.group_m = p.group_m;
-    t.per_group = p.group_m * tiles_n;
-    t.by_group = RingDivisor::of(t.per_group);
-    t.by_group_m = RingDivisor::of(p.group_m);
-    t.by_group_last = RingDivisor::of(t.tiles_m % p.group_m ? t.tiles_m % p.group_m : p.group_m);
+    const bool one_group = p.group_m >= t.tiles_m;
+    t.per_group = one_group ? t.grid : RING_GROUP * tiles_n;
+    t.divisor = RingDivisor::of(one_group ? t.tiles_m : t.per_group);
     return t;
 }
-// Has the arguments in scalar registers from here on: they arrive in one wait, where the compiler's own loads, each in front of
-// its first use, stand one after the other on the way to the first copy and again in front of the store.
+// Has arguments in scalar registers from here on: they arrive in one wait, where the compiler's own loads, each in front of its first
+// use, stand one after the other.
 template <class T>
 __device__ __forceinline__ void ring_argument(const T v)
 {
@@ -296,8 +296,21 @@ __device__ __forceinline__ void ring_arguments(const T... v)
     (ring_argument(v), ...);
 }
 
+// The kernel's arguments as they lie in memory.  What is in front of `rest` are the fourteen scalar registers that the hardware fills
+// before a wave starts (the units are compiled with kernel argument preloading): tile, addresses and first copies do not wait 0.3 to
+// 0.4 us for the argument load.  `rest` is read through this, where it is needed: taken from the kernel's parameter it is loaded on
+// entry, all of it, and the registers that it takes away are missed (MXFP8 384 x 4096 x 4096 11.3 us for 10.9).
+struct RingArguments {
+    const uint8_t *a, *b;
+    uint32_t lda_bytes, ldb_bytes;
+    int m, n, k_bytes, grid, tiles_m, per_group;
+    uint32_t magic, shift;
+    TileGemmParams rest;
+};
+static_assert(sizeof(RingArguments) == 56 + sizeof(TileGemmParams), "the parameters' offsets, each aligned by itself");
 template <class Cfg>
-__global__ void __launch_bounds__(Cfg::THREADS) gemm_tile_ring_kernel(const TileGemmParams p, const RingTiles tiles)
+__global__ void __launch_bounds__(Cfg::THREADS) gemm_tile_ring_kernel(const uint8_t* a, const uint8_t* b, const uint32_t lda_bytes, const uint32_t ldb_bytes, const int m, const int n, const int k_bytes,
+                                                                     const int grid, const int tiles_m, const int per_group, const uint32_t magic, const uint32_t shift, const TileGemmParams)
 {
     using Op = typename Cfg::Op;
     using Acc = typename Op::Acc;
@@ -316,14 +329,43 @@ __global__ void __launch_bounds__(Cfg::THREADS) gemm_tile_ring_kernel(const Tile
 
     // ---- workgroup -> tile.  Workgroup ids go round-robin to the 8 XCDs; XCD x takes a contiguous run of tiles, walked in
     // groups of group_m tile rows, so that what an L2 holds is a few panels of A and of B.
-    ring_arguments(p.a, p.b, p.c, p.c_in, p.bias, p.acc_out, p.sa, p.sb, p.row_scale, p.col_scale, p.m, p.n, p.k_bytes, p.lda_bytes, p.ldb_bytes,
-                   p.ldc, p.scale_ld, p.relu, p.out_kind, p.qwords, p.q_per_column, p.atomic_add, tiles.grid);
+    const TileGemmParams& rest = reinterpret_cast<const RingArguments*>((const void*)__builtin_amdgcn_kernarg_segment_ptr())->rest;
+    TileGemmParams p;
+    p.a = a;
+    p.b = b;
+    p.m = m;
+    p.n = n;
+    p.k_bytes = k_bytes;
+    p.lda_bytes = lda_bytes;
+    p.ldb_bytes = ldb_bytes;
+    // Has the cache lines of `rest` fetched, so that the drain's loads find them; behind the first copies, where the wait costs nothing.
+    auto touch_arguments = [&]() __attribute__((always_inline)) { ring_arguments(rest.c, rest.ldc, rest.q_per_column); };
+    // for the drain, in one wait
+    auto drain_arguments = [&]() __attribute__((always_inline)) {
+        p.c = rest.c;
+        p.c_in = rest.c_in;
+        p.bias = rest.bias;
+        p.acc_out = rest.acc_out;
+        p.row_scale = rest.row_scale;
+        p.col_scale = rest.col_scale;
+        p.ldc = rest.ldc;
+        p.relu = rest.relu;
+        p.out_kind = rest.out_kind;
+        p.qwords = rest.qwords;
+        p.q_per_column = rest.q_per_column;
+        p.atomic_add = rest.atomic_add;
+        ring_arguments(p.c, p.c_in, p.bias, p.acc_out, p.row_scale, p.col_scale, p.ldc, p.relu, p.out_kind, p.qwords, p.q_per_column, p.atomic_add);
+    };
     const int xcd = blockIdx.x & 7;
-    const int lid = xcd * (tiles.grid >> 3) + min(xcd, tiles.grid & 7) + (blockIdx.x >> 3);
-    const int group = tiles.by_group.divide(lid), in_group = lid - group * tiles.per_group, first_m = group * tiles.group_m;
-    const int gsize = min(tiles.tiles_m - first_m, tiles.group_m);
-    const int column = (gsize == tiles.group_m ? tiles.by_group_m : tiles.by_group_last).divide(in_group);
-    const int m0 = (first_m + in_group - column * gsize) * BM, n0 = column * BN;
+    const int lid = xcd * (grid >> 3) + min(xcd, grid & 7) + (blockIdx.x >> 3);
+    const int quotient = RingDivisor{magic, shift}.divide(lid);
+    int row = lid - quotient * tiles_m, column = quotient;
+    if (per_group != grid) {
+        const int in_group = lid - quotient * per_group, first = quotient * RING_GROUP, gsize = min(tiles_m - first, RING_GROUP);
+        column = gsize == 4 ? in_group >> 2 : gsize == 3 ? (int)(uint32_t)(((uint64_t)(uint32_t)in_group * 0xAAAAAAABu) >> 33) : in_group >> (gsize - 1);
+        row = first + in_group - column * gsize;
+    }
+    const int m0 = row * BM, n0 = column * BN;
 
     // ---- TLOAD addressing: piece w + q * NW of a stage, lane -> (row, position) linear, fetching chunk position ^ swizzle
     const int nst = (p.k_bytes + SB - 1) / SB;
@@ -357,26 +399,38 @@ __global__ void __launch_bounds__(Cfg::THREADS) gemm_tile_ring_kernel(const Tile
     for (int q = 0; q < NPW; ++q)
         goff[q] = Cfg::BND && lw + q * NW >= Cfg::A_PIECES ? (uint32_t)(nd_row(q) * p.ldb_bytes) + nd_col(q) : row_offset(q) + skewed_chunk(q) * 16 + LINE;
     // Scales in the stage: dword e = row * STAGE_SPS + d; without scale arrays the copies fetch bytes of A that are not used.
-    const bool has_scales = Op::SCALED && p.sa != nullptr;
+    // (All that depends on the scales' arguments is worked out by scale_arguments(), which a copying wave calls behind its first copies.)
+    bool has_scales = false, short_scales = false;
+    int scale_last = 0, scale_shift = 0;
     const uint8_t* sc_row[NSW > 0 ? NSW : 1];
-    int sc_d[NSW > 0 ? NSW : 1];
-    const int sc_last = has_scales ? p.scale_ld / 4 - 1 : 0;  // last scale dword of a row
-    if constexpr (NSW > 0) {
+    int sc_d[NSW > 0 ? NSW : 1], sc_last = 0;  // last scale dword of a row
+    auto scale_arguments = [&]() __attribute__((always_inline)) {
+        if constexpr (Op::SCALED) {
+            p.sa = rest.sa;
+            p.sb = rest.sb;
+            p.scale_ld = rest.scale_ld;
+            ring_arguments(p.sa, p.sb, p.scale_ld);
+            has_scales = p.sa != nullptr;
+            sc_last = has_scales ? p.scale_ld / 4 - 1 : 0;
+            short_scales = CHUNKED && has_scales && p.scale_ld < 16;
+            scale_last = CHUNKED ? p.scale_ld / 16 * 4 : 0;
+            scale_shift = CHUNKED ? (4 - p.scale_ld / 4 % 4) % 4 : 0;
+            if constexpr (NSW > 0) {
 #pragma unroll
-        for (int q = 0; q < NSW; ++q) {
-            const int e = ((lw + q * NW) % Cfg::SPIECES) * 64 + lane, r = e / Cfg::STAGE_SPS;
-            sc_d[q] = e % Cfg::STAGE_SPS;
-            sc_row[q] = !has_scales ? p.a : r < BM ? p.sa + (long)min(m0 + r, p.m - 1) * p.scale_ld : p.sb + (long)min(n0 + r - BM, p.n - 1) * p.scale_ld;
+                for (int q = 0; q < NSW; ++q) {
+                    const int e = ((lw + q * NW) % Cfg::SPIECES) * 64 + lane, r = e / Cfg::STAGE_SPS;
+                    sc_d[q] = e % Cfg::STAGE_SPS;
+                    sc_row[q] = !has_scales ? p.a : r < BM ? p.sa + (long)min(m0 + r, p.m - 1) * p.scale_ld : p.sb + (long)min(n0 + r - BM, p.n - 1) * p.scale_ld;
+                }
+            }
         }
-    }
+    };
     // Scales in chunks: without scale arrays nothing is copied and the buffers hold E8M0 127 (selected per fragment, the scales cost
     // a VALU instruction and a wait for each in front of the matrix instructions).  A row's
     // last 16 bytes are the 16 that END there, so where scale_ld is no multiple of 16 its last dwords lie scale_shift further on; a
     // row shorter than that (K < 512) goes through registers, of the waves that multiply where others copy: these have nothing else under
     // way, while in a copying wave the wait for the scales was one for all stages copied behind them (MXFP8 2048 x 4096 x 384 on 128 x
     // 128 tiles 14.8 -> 14.2 us, 384 x 4096 x 384 7.75 -> 7.5).  Out of line: in the way, K of 512 and more took 2 % longer.
-    const bool short_scales = CHUNKED && has_scales && p.scale_ld < 16;
-    const int scale_last = CHUNKED ? p.scale_ld / 16 * 4 : 0, scale_shift = CHUNKED ? (4 - p.scale_ld / 4 % 4) % 4 : 0;
     auto issue_scales = [&](int chunk) __attribute__((always_inline)) {
         if constexpr (CHUNKED) {
             constexpr int SCB = Cfg::SCB, LANES = SCB / 16, RPI = 64 / LANES, COPIES = Cfg::ROWS / RPI;  // lanes per row, rows per copy
@@ -423,7 +477,7 @@ __global__ void __launch_bounds__(Cfg::THREADS) gemm_tile_ring_kernel(const Tile
                     *reinterpret_cast<uint4*>(smem + R * Cfg::STAGE + o) = make_uint4(0x7F7F7F7Fu, 0x7F7F7F7Fu, 0x7F7F7F7Fu, 0x7F7F7F7Fu);
         }
     };
-    auto issue = [&](int st, int buf) __attribute__((always_inline)) {
+    auto issue_operands = [&](int st, int buf) __attribute__((always_inline)) {
         const uint32_t dst = __builtin_amdgcn_readfirstlane(lds0 + buf * Cfg::STAGE);
         const long kb = (long)st * SB, kb_b = Cfg::BND ? (long)st * Cfg::KR * p.ldb_bytes : kb;
         if (Cfg::SKEW ? st == 0 || (st + 1) * SB > p.k_bytes : k_tail && st == nst - 1) {
@@ -448,7 +502,10 @@ __global__ void __launch_bounds__(Cfg::THREADS) gemm_tile_ring_kernel(const Tile
                 lds_dma16_off((piece < Cfg::A_PIECES ? p.a + kb : p.b + kb_b) - LINE, goff[q], dst + piece * 1024);
             }
         }
+    };
+    auto issue_stage_scales = [&](int st, int buf) __attribute__((always_inline)) {
         if constexpr (NSW > 0) {
+            const uint32_t dst = __builtin_amdgcn_readfirstlane(lds0 + buf * Cfg::STAGE);
 #pragma unroll
             for (int q = 0; q < NSW; ++q)
                 lds_dma4(sc_row[q] + 4 * min(st * Cfg::STAGE_SPS + sc_d[q], sc_last), dst + Cfg::ROWS * SB + ((lw + q * NW) % Cfg::SPIECES) * 256);
@@ -457,6 +514,10 @@ __global__ void __launch_bounds__(Cfg::THREADS) gemm_tile_ring_kernel(const Tile
             if (has_scales && !short_scales && st % Cfg::SPC == 0)  // ahead of the next stage's copies, which stages are counted by
                 issue_scales(st / Cfg::SPC);
         }
+    };
+    auto issue = [&](int st, int buf) __attribute__((always_inline)) {
+        issue_operands(st, buf);
+        issue_stage_scales(st, buf);
     };
 
     Acc acc[MB][NB];
@@ -606,12 +667,19 @@ __global__ void __launch_bounds__(Cfg::THREADS) gemm_tile_ring_kernel(const Tile
     if constexpr (!Cfg::PIPE) {
         // Barrier st: stage st has landed and no wave reads stage st - 1 any more, whose buffer is refilled.
         if (loads) {
+            if constexpr (CHUNKED)
+                scale_arguments();
             hold_short_scales();
             fill_scales();
+            issue_operands(0, 0);
+            if constexpr (!CHUNKED)
+                scale_arguments();
+            issue_stage_scales(0, 0);
 #pragma unroll
-            for (int s = 0; s < R - 1; ++s)
+            for (int s = 1; s < R - 1; ++s)
                 if (s < nst)
                     issue(s, s);
+            touch_arguments();
             write_short_scales();
         }
         int buf = 0;
@@ -681,6 +749,7 @@ __global__ void __launch_bounds__(Cfg::THREADS) gemm_tile_ring_kernel(const Tile
                 load(integral_constant<int, s % G>{}, s + G);
             });
             ring_wait_and_barrier<63>();
+            touch_arguments();
             int buf = 0, st = 0;
             auto step = [&](auto gc) __attribute__((always_inline)) {
                 constexpr integral_constant<int, (R + decltype(gc)::value) % G> g{};
@@ -709,9 +778,15 @@ __global__ void __launch_bounds__(Cfg::THREADS) gemm_tile_ring_kernel(const Tile
                 constexpr int s = decltype(sc)::value;
                 if constexpr (s == EARLY)
                     loader_barrier(max(0, min(EARLY - AHEAD, ncopy - AHEAD)));
-                if (s < ncopy)
+                if constexpr (s == 0) {
+                    issue_operands(0, 0);
+                    scale_arguments();
+                    issue_stage_scales(0, 0);
+                } else if (s < ncopy) {
                     issue(s, s);
+                }
             });
+            touch_arguments();
             int buf = 0;
             for (int st = 0; st < nst - 1; ++st) {
                 loader_barrier(max(0, min(R - 1 - AHEAD, ncopy - 1 - AHEAD - st)));
@@ -720,6 +795,8 @@ __global__ void __launch_bounds__(Cfg::THREADS) gemm_tile_ring_kernel(const Tile
                 buf = buf + 1 == R ? 0 : buf + 1;
             }
         } else {
+            scale_arguments();
+            touch_arguments();
             hold_short_scales();
             fill_scales();
             write_short_scales();
@@ -811,6 +888,7 @@ __global__ void __launch_bounds__(Cfg::THREADS) gemm_tile_ring_kernel(const Tile
         }
     }
 
+    drain_arguments();
     // ---- TSTORE: the k-groups' partial sums meet in LDS (the ring is free), are added in group order and leave as up to 16
     // bytes per thread and row.  A block is transposed in its lanes: lane (l16, lg) holds row l16, columns 4 lg .. + 3.
     auto drain = [&](auto kc) __attribute__((always_inline)) {
