@@ -402,6 +402,9 @@ static const DrainCost drain_costs[DRAIN_COUNT] = {
 // (the deep-ring kernel's scales and raw accumulators: us per round, and per round and 22000 elements of a tile; its words per
 // column, raw accumulators and atomic additions behind unaligned rows: us per call)
 constexpr float RING_SCALES_ROUND = 0.5f, RING_SCALES_TILE = 22000.0f, RING_UNALIGNED_DRAIN = 2.5f;
+// Up to so many slabs the 32 x 32 shape on rows of any byte is behind the register-staged tiles: bf16 1 x 301 x 257, five slabs, 6.25 us, 7.15
+// on it; int8 18 x 5001 x 385, four, 6.9 and 7.9; bf16 1 x 301 x 385, seven, 7.5 and 6.2.
+constexpr int RING_NARROW_SLABS = 5;
 constexpr int TILE256_ROW_MAJOR_K_BYTES = 1024;  // (see pick_dma_tile)
 constexpr int TILE_RING = 16;  // tile ids from here on: the deep-ring kernel's shapes
 
@@ -427,9 +430,9 @@ static int pick_dma_tile(int m, int n, long k_bytes, int op, const TileChoice& c
     const bool unaligned = choice.unaligned;
     const bool scaled = op >= TOP_FP8_E4E4;
     const int shapes = scaled ? RING_SHAPES_SCALED : RING_SHAPES;
-    const int first = unaligned ? RING_FIRST_UNALIGNED : 0, form = unaligned ? RING_UNALIGNED : 0;
+    const int form = unaligned ? RING_UNALIGNED : 0;
     const float copying = unaligned ? 1.9f : 1.0f;
-    if (options().ring >= first && options().ring < shapes)
+    if (options().ring >= 0 && options().ring < shapes && (!unaligned || ring_unaligned_shape(options().ring)))
         return TILE_RING + form + options().ring;
     // A round or more of 256 x 256 tiles: those (with the split of a part-filled last round below) are ahead from K = 1024 on
     // -- bf16 4096 x 8192 x 2048: 105 us against 129 on 256 x 128 -- and within a tenth of the best where a sixteenth of a round
@@ -460,7 +463,7 @@ static int pick_dma_tile(int m, int n, long k_bytes, int op, const TileChoice& c
     for (int c = 0; c < COST_COUNT; ++c) {
         static const int ids[COST_COUNT - RING_SHAPES] = {4, 5, 7, 2, 1};
         const bool ring = c < RING_SHAPES, in_registers = c >= COST_TILE2;
-        if (ring           ? c >= shapes || c < first || (scaled && c <= 2 && m > 64)
+        if (ring           ? c >= shapes || (unaligned && !ring_unaligned_shape(c)) || (c == RING_NARROW_UNALIGNED && unaligned && staged_ok && slab_count <= RING_NARROW_SLABS) || (scaled && c <= 2 && m > 64)
             : in_registers ? !staged_ok || (c == COST_TILE1 && scaled)
                            : dtl == DTL_NONE || (dtl == DTL_256_ONLY && c != COST_TILE4) || (c == COST_TILE7 && !scaled))
             continue;
@@ -616,7 +619,7 @@ static const char* tile_kernel_name(int tile, int op, bool row_major_b, bool by_
     if (tile >= TILE_RING) {
         int bm, bn;
         ring_shape(tile - TILE_RING, &bm, &bn);
-        snprintf(buf, sizeof buf, row_major_b ? "tile%dx%d_bnd_%s" : tile >= TILE_RING + RING_UNALIGNED ? "tile%dx%d_any_%s" : by_lines ? "tile%dx%d_dtl_lines_%s" : "tile%dx%d_dtl_%s",
+        snprintf(buf, sizeof buf, row_major_b ? (tile >= TILE_RING + RING_UNALIGNED ? "tile%dx%d_bnd_any_%s" : "tile%dx%d_bnd_%s") : tile >= TILE_RING + RING_UNALIGNED ? "tile%dx%d_any_%s" : by_lines ? "tile%dx%d_dtl_lines_%s" : "tile%dx%d_dtl_%s",
                  bm, bn, ops[op]);
         return buf;
     }
@@ -853,14 +856,23 @@ static int gemm_common(void* c, int c_type, const void* a, const void* b, int ab
     // row's last one).  With a workspace the tile is the one that the same product takes with a column-major B, so that both
     // have the same bits; where that tile has no row-major form, B is re-ordered for it.  (Register-staged tiles are left out with
     // a workspace: they run a few slabs of K, for which the re-ordering launch costs more than they save.)
-    const bool nd_ok = b_layout == PTOAMD_B_ND && ebytes == 2 && !options().b_nd_in_loader && options().tile < 0 && (n % 8) == 0 &&
-                       aligned4(a) && aligned4(b) && (lda_b % 4) == 0 && (ldb_b % 4) == 0 && (k_bytes % 4) == 0 &&
-                       dma_offsets_fit(m, RING_MAX_STAGE_BYTES / 2 + 8, lda_b, ldb_b, std::max(k_bytes, 2 * (long)n));
+    const bool nd_fits = b_layout == PTOAMD_B_ND && ebytes == 2 && !options().b_nd_in_loader && options().tile < 0 &&
+                         dma_offsets_fit(m, RING_MAX_STAGE_BYTES / 2 + 8, lda_b, ldb_b, std::max(k_bytes, 2 * (long)n));
+    const bool nd_ok = nd_fits && (n % 8) == 0 && aligned4(a) && aligned4(b) && (lda_b % 4) == 0 && (ldb_b % 4) == 0 && (k_bytes % 4) == 0;
+    // Without a workspace, rows that start on other bytes or end inside a chunk: the form whose copies go through registers.  Two slabs of
+    // K stay with the register-staged tiles (bf16 1 x 1501 x 65 6.1 us, deep ring 7.3; 2000 x 5001 x 33 18.2 and 21.7), and three where one round
+    // of them covers C (600 x 1501 x 129 8.2 and 8.5; 4000 x 1501 x 129 17.9 and 14.3); from there on the deep ring was ahead at all of 144
+    // sizes: K 191 0.99 to 1.3 times, 513 1.5 to 2, 7274 (18 x 308) seven times.
+    const long tiles64 = (long)((m + 63) / 64) * ((n + 63) / 64);
+    const bool few_slabs = k_bytes <= 256 || (k_bytes <= 384 && tiles64 <= device_compute_units());
+    const bool nd_any = nd_fits && !nd_ok && b_in_kernel && (!few_slabs || options().ring >= 0);
     const DrainKind drain = atomic_add                 ? DRAIN_ATOMIC
                             : qwords == nullptr        ? (c_in != nullptr ? DRAIN_ACC_IN : DRAIN_PLAIN)
                             : q_per_column             ? DRAIN_COLUMN_WORDS
                                                        : DRAIN_WORD;
-    const int nd_tile = nd_ok ? pick_dma_tile(m, n, k_bytes, op, {b_via_ws ? dtl_k : whole_slabs ? DTL_256_ONLY : DTL_NONE, drain, false, b_via_ws ? STAGED_NONE : STAGED_ROW_MAJOR_B}) : -1;
+    const int nd_tile = nd_ok ? pick_dma_tile(m, n, k_bytes, op, {b_via_ws ? dtl_k : whole_slabs ? DTL_256_ONLY : DTL_NONE, drain, false, b_via_ws ? STAGED_NONE : STAGED_ROW_MAJOR_B})
+                        : nd_any ? pick_dma_tile(m, n, k_bytes, op, {DTL_NONE, drain, true, STAGED_NONE})
+                                 : -1;
     const bool nd_direct = nd_tile >= TILE_RING || (nd_tile == 4 && whole_slabs);
     const uint8_t* b_kmajor = reinterpret_cast<const uint8_t*>(b);
     long ldb_kmajor = ldb_b;

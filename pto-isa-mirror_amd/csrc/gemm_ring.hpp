@@ -34,8 +34,10 @@ struct TileGemmParams;
     X(7, 192, 128, 2, 2, 1, 128, 4, 0, 0, 0, 0, 0, 4, true)       \
     X(8, 256, 128, 2, 2, 1, 128, 3, 0, 0, 0, 0, 0, 4, true)
 constexpr int RING_SHAPES = 9, RING_SHAPES_SCALED = 7, RING_MAX_STAGE_BYTES = 1024, RING_SHAPE_128X128 = 6;
-// Added to the id of a shape with copying waves (3 and up) of the plain types: the form for rows that start on any byte.
-constexpr int RING_UNALIGNED = 16, RING_FIRST_UNALIGNED = 3;
+// Added to the id of a shape with copying waves (3 and up) of the plain types: the form for rows that start on any byte.  So has the
+// 32 x 32 shape, as four waves that multiply and four that copy.
+constexpr int RING_UNALIGNED = 16, RING_FIRST_UNALIGNED = 3, RING_NARROW_UNALIGNED = 1;
+constexpr bool ring_unaligned_shape(int shape) { return shape >= RING_FIRST_UNALIGNED || shape == RING_NARROW_UNALIGNED; }
 
 inline void ring_shape(int shape, int* bm, int* bn)
 {

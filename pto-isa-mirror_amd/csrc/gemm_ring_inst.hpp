@@ -61,14 +61,16 @@ static hipError_t launch_ring_shape(int shape, const TileGemmParams& p, hipStrea
 }
 
 // the form for rows at any alignment, shapes with copying waves only
-template <class Op>
+template <class Op, bool BND = false>
 static hipError_t launch_ring_unaligned(int shape, const TileGemmParams& p, hipStream_t stream)
 {
     switch (shape) {
 #define PTOAMD_RING_CASE(id, bm, bn, wm, wn, wk, sb, r, swm, swn, swk, ssb, sr, lw, pipe)                            \
     case id:                                                                                                        \
         if constexpr (pipe)                                                                                         \
-            return launch_ring<RingCfg<bm, bn, wm, wn, wk, sb, r, lw, pipe, Op, false, true>>(p, stream);           \
+            return launch_ring<RingCfg<bm, bn, wm, wn, wk, sb, r, lw, pipe, Op, BND, true>>(p, stream);             \
+        else if constexpr (id == RING_NARROW_UNALIGNED)                                                             \
+            return launch_ring<RingCfg<bm, bn, 1, 1, 4, sb, r, 4, true, Op, BND, true>>(p, stream);                 \
         break;
         PTOAMD_RING_SHAPES_ALL(PTOAMD_RING_CASE)
         PTOAMD_RING_SHAPES_PLAIN(PTOAMD_RING_CASE)
@@ -87,8 +89,9 @@ hipError_t PTOAMD_RING_FN(int shape, const TileGemmParams& p, hipStream_t stream
 #endif
     if (shape >= RING_UNALIGNED && shape != TILE_PREPARE_ALL) {
         if constexpr (!PTOAMD_RING_OP::SCALED)
-            if (!p.b_nd)
-                return launch_ring_unaligned<PTOAMD_RING_OP>(shape - RING_UNALIGNED, p, stream);
+            if (!p.b_nd || has_bnd)
+                return p.b_nd ? launch_ring_unaligned<PTOAMD_RING_OP, has_bnd>(shape - RING_UNALIGNED, p, stream)
+                              : launch_ring_unaligned<PTOAMD_RING_OP>(shape - RING_UNALIGNED, p, stream);
         return hipErrorInvalidValue;
     }
     if (shape != TILE_PREPARE_ALL) {
@@ -106,8 +109,10 @@ hipError_t PTOAMD_RING_FN(int shape, const TileGemmParams& p, hipStream_t stream
                 e = launch_ring_shape<PTOAMD_RING_OP, true>(s, none, stream);
         }
         if constexpr (!PTOAMD_RING_OP::SCALED) {
-            if (e == hipSuccess && s >= RING_FIRST_UNALIGNED)
+            if (e == hipSuccess && ring_unaligned_shape(s))
                 e = launch_ring_unaligned<PTOAMD_RING_OP>(s, none, stream);
+            if (e == hipSuccess && has_bnd && ring_unaligned_shape(s))
+                e = launch_ring_unaligned<PTOAMD_RING_OP, has_bnd>(s, none, stream);
         }
         if (e != hipSuccess)
             return e;

@@ -91,7 +91,8 @@ struct RingCfg {
     static_assert(PIECES % NW == 0 && (BM * SB) % 1024 == 0, "every wave issues the same number of 1 KiB copies, each of one operand");
     static_assert(!BND || (!Op::SCALED && FR == 1 && (NB & (NB - 1)) == 0), "the row-major form is for the 16-bit types");
     static_assert(!SKEW || (PIPE && !BND && !ANY && !Op::SCALED && R >= 4), "two stages have to have landed where one is multiplied");
-    static_assert(!ANY || (PIPE && !BND && !Op::SCALED), "the register copies are the copying waves' and know no scales");
+    static_assert(!ANY || (PIPE && !Op::SCALED), "the register copies are the copying waves' and know no scales");
+    static_assert(!ANY || !BND || A_PIECES % NW == 0, "which copies are B's is known at compile time");
     static_assert((ROWS * STAGE_SPS) % 64 == 0, "scale pieces are whole");
     static_assert(!CHUNKED || (SCB / 4 % SPS == 0 && (SBUFS - 1) * SPC >= R - 1 && BM * SCB % 1024 == 0 && BN * SCB % 1024 == 0 && ROWS <= CW * 64),
                   "a chunk of scales is whole stages; a 1 KiB copy of them is of one operand; a thread can hold a row's");
@@ -131,6 +132,19 @@ __device__ __forceinline__ uint4 ring_chunk_mask(int valid)
     return make_uint4(m[0], m[1], m[2], m[3]);
 }
 __device__ __forceinline__ uint4 ring_masked(uint4 v, uint4 m) { return make_uint4(v.x & m.x, v.y & m.y, v.z & m.z, v.w & m.w); }
+
+// the chunk without its first `bytes` bytes, an even number below 16 (from 16 on: anything)
+__device__ __forceinline__ uint4 ring_shift_down(uint4 v, uint32_t bytes)
+{
+    const uint64_t lo = (uint64_t)v.y << 32 | v.x, hi = (uint64_t)v.w << 32 | v.z;
+    const uint32_t bits = (bytes & 6) * 8;
+    uint64_t low = lo >> bits | hi << 1 << (63 - bits), high = hi >> bits;
+    if (bytes & 8) {
+        low = high;
+        high = 0;
+    }
+    return make_uint4((uint32_t)low, (uint32_t)(low >> 32), (uint32_t)high, (uint32_t)(high >> 32));
+}
 
 // Consecutive columns of an output row that one thread drains: 16 bytes of 16- and 32-bit outputs, 4 of one-byte outputs and, where a thread
 // would have more than four such pieces, 8 (int8 by a word: 256 x 128 tiles 0.91 to 0.97 of the time with 4, 128 x 128 0.93 to 0.97; on 128 x
@@ -380,10 +394,8 @@ __global__ void __launch_bounds__(Cfg::THREADS) gemm_tile_ring_kernel(const uint
     };
     // BND: a stage's B is KR rows of BN columns; row and byte offset (columns past N repeat the row's last chunk)
     auto nd_row = [&](int q) { return ((lw + q * NW - Cfg::A_PIECES) * 64 + lane) / Cfg::CB; };
-    auto nd_col = [&](int q) -> uint32_t {
-        const int chunk = (lane % Cfg::CB) ^ (swizzle_row_major<BN>(nd_row(q)) << 1);
-        return (uint32_t)min(n0 * 2 + chunk * 16, p.n * 2 - 16);
-    };
+    auto nd_chunk = [&](int q) { return (lane % Cfg::CB) ^ (swizzle_row_major<BN>(nd_row(q)) << 1); };
+    auto nd_col = [&](int q) -> uint32_t { return (uint32_t)min(n0 * 2 + nd_chunk(q) * 16, p.n * 2 - 16); };
     // SKEW: a stage of a row is whole 128-byte lines, so it starts `skew` chunks ahead of its own k.  Of the chunks of a stage's lines
     // that belong to this k stage and to the one before, each stands where its k has it: fragment reads find it at the same place
     // in either buffer, and their banks are those of rows that start on a line.
@@ -726,21 +738,35 @@ __global__ void __launch_bounds__(Cfg::THREADS) gemm_tile_ring_kernel(const uint
             uint4 held[G][NPW];
 #pragma unroll
             for (int q = 0; q < NPW; ++q) {
-                row[q] = row_offset(q);
-                chunk[q] = piece_chunk(q) * 16;
+                const bool rows_of_k = Cfg::BND && q * NW >= Cfg::A_PIECES;
+                row[q] = rows_of_k ? nd_col(q) : row_offset(q);
+                chunk[q] = rows_of_k ? 0 : piece_chunk(q) * 16;
             }
             auto load = [&](auto gc, int st) __attribute__((always_inline)) {
-                const uint32_t k0 = min(st, nst - 1) * SB;
+                const int stage = min(st, nst - 1);
+                const uint32_t k0 = stage * SB;
+                const int base_row = max(stage * Cfg::KR - 8, 0);
 #pragma unroll
                 for (int q = 0; q < NPW; ++q) {
+                    if (Cfg::BND && q * NW >= Cfg::A_PIECES) {  // (eight rows that K ends in: as in issue_operands)
+                        const int k = p.k_bytes / 2, r = stage * Cfg::KR + nd_row(q), src = (r | 7) < k ? r : k - 8 + (r & 7);
+                        held[decltype(gc)::value][q] = load_unaligned16(p.b + (long)base_row * p.ldb_bytes + ((uint32_t)((src - base_row) * p.ldb_bytes) + row[q]));
+                        continue;
+                    }
                     const uint32_t off = row[q] + min(k0 + chunk[q], (uint32_t)(p.k_bytes - 16));
                     held[decltype(gc)::value][q] = load_unaligned16((lw + q * NW < Cfg::A_PIECES ? p.a : p.b) + off);
                 }
             };
+            // BND: the chunk of a row that N ends in came as the 16 bytes that end there
+            const bool n_tail = Cfg::BND && n0 + BN > p.n && p.n % 8 != 0;
             auto store = [&](auto gc, int b) __attribute__((always_inline)) {
 #pragma unroll
-                for (int q = 0; q < NPW; ++q)
-                    *reinterpret_cast<uint4*>(smem + b * Cfg::STAGE + (lw + q * NW) * 1024 + lane * 16) = held[decltype(gc)::value][q];
+                for (int q = 0; q < NPW; ++q) {
+                    uint4 v = held[decltype(gc)::value][q];
+                    if (Cfg::BND && q * NW >= Cfg::A_PIECES && n_tail)
+                        v = ring_shift_down(v, (uint32_t)(n0 * 2 + nd_chunk(q) * 16) - row[q]);
+                    *reinterpret_cast<uint4*>(smem + b * Cfg::STAGE + (lw + q * NW) * 1024 + lane * 16) = v;
+                }
             };
             static_for<G>([&](auto gc) { load(gc, decltype(gc)::value); });
             static_for<R>([&](auto sc) {

@@ -46,7 +46,7 @@ def test_plain_types(pa, oracle, kind, shape):  # noqa: F811
             check_f32_drain(got, ref, np.abs(fa) @ np.abs(fb).T, k, f"{kind} {m}x{n}x{k} shape {shape}")
 
 
-@pytest.mark.parametrize("shape", range(3, 9))
+@pytest.mark.parametrize("shape", [1, 3, 4, 5, 6, 7, 8])
 @pytest.mark.parametrize("kind", ["bf16", "f16", "i8"])
 def test_rows_on_any_byte(pa, kind, shape):  # noqa: F811
     """Rows that start on any byte (16-bit types: on any element), from one chunk of K to more stages than ring and registers
@@ -76,6 +76,43 @@ def test_rows_on_any_byte(pa, kind, shape):  # noqa: F811
             out = pa.gemm_w8a8(a[:, :k].contiguous(), b[:, :k].contiguous(), sa, sb)
             assert pa.last_kernel() == f"tile{bm}x{bn}_any_i8", pa.last_kernel()
         assert torch.equal(out, (got.float() * sa[:, None] * sb[None, :]).to(torch.bfloat16))
+
+
+@pytest.mark.parametrize("shape", [1, 3, 4, 5, 6, 7, 8])
+@pytest.mark.parametrize("kind", ["bf16", "f16"])
+def test_row_major_b_rows_on_any_element(pa, kind, shape):  # noqa: F811
+    """B as [K][N], no workspace, rows that start on any element and end anywhere in a chunk of eight columns (one chunk of columns, a tile
+    and part of one, two tiles and one to seven columns), K from one chunk of eight rows to more stages than ring and registers hold,
+    ending anywhere in a chunk: exact products of small whole numbers, NaN around the operands."""
+    tdt, t = (torch.float16, pa.F16) if kind == "f16" else (torch.bfloat16, pa.BF16)
+    gen = torch.Generator(device="cuda").manual_seed(shape)
+    bm, bn, stage = SHAPES[shape][:3]
+    kr = stage // 2
+
+    def rows(count, length, pitch, start):  # whole numbers of -7 .. 7, all sums below 2^24; nothing behind the last row's values
+        flat = torch.full((start + (count - 1) * pitch + length,), float("nan"), device="cuda").to(tdt)
+        view = flat.as_strided((count, length), (pitch, 1), start)
+        view.copy_(torch.randint(-7, 8, (count, length), generator=gen, device="cuda"))
+        return view
+    for m, n, k in [(bm - 1, 9, 8), (1, bn - 1, 9), (bm, 8, kr + 3), (bm + 1, 2 * bn + 1, 2 * kr + 7), (bm, bn + 2, 4 * kr), (2, bn + 3, 4 * kr + 1), (bm - 1, 2 * bn + 4, 7 * kr + 2),
+                    (3, bn + 5, 7 * kr - 4), (bm + 2, bn + 6, 9 * kr + 13), (bm, 2 * bn + 7, 9 * kr + 6)]:
+        for wide, start in ((0, 0), (3, 1)):
+            a, b = rows(m, k, k + wide, start), rows(k, n, n + wide, start)
+            with tile_env(PTOAMD_RING=shape):
+                got = pa.gemm(a, b, t, pa.F32, pa.B_ND)
+                name = pa.last_kernel()
+            in_place = n % 8 == 0 and k % 2 == 0 and wide == 0
+            assert in_place or name == f"tile{bm}x{bn}_bnd_any_{kind}", (name, m, n, k)
+            assert torch.equal(got.double(), a.double() @ b.double()), (m, n, k, wide)
+
+
+def test_row_major_b_without_workspace_takes_the_form_for_any_row(pa):  # noqa: F811
+    for m, n, k in [(18, 308, 7274), (2, 1020, 4474), (55, 287, 3027), (300, 2049, 1025)]:
+        gen = torch.Generator(device="cuda").manual_seed(m)
+        a, b = (torch.randint(-7, 8, x, generator=gen, device="cuda").to(torch.bfloat16) for x in ((m, k), (k, n)))
+        got = pa.gemm(a, b, pa.BF16, pa.F32, pa.B_ND)
+        assert "_bnd_any_" in pa.last_kernel(), pa.last_kernel()
+        assert torch.equal(got.double(), a.double() @ b.double())
 
 
 @pytest.mark.parametrize("shape", [3, 4, 6, 7])
