@@ -22,6 +22,8 @@
 //              A stage takes about twice as long as by LDS-DMA.
 //              Measured, bf16, against the register-staged tile chosen by grid size: 64 x 4097 x 4095 28 us (63), 1000 x 2049 x 2047
 //              33 (57; 2048 x 2048 by LDS-DMA: 17), 2100 x 2049 x 2047 43 (61), 4000 x 1025 x 4097 73 (110)
+//              With a row-major B (BND as well) a chunk of B is eight columns of a k row; the chunk that N ends in is the 16 bytes that end
+//              there, shifted in registers.  bf16 18 x 308 x 7274 18.9 us (register-staged loader 134), 1111 x 3347 x 4028 54 (194)
 //   rows on 16 bytes off the 128-byte lines (SKEW, plain types, shapes with four stages): a copy's cost is the lines it touches, and
 //              a stage of such a row lies across two per 128 bytes.  Each row's copies are cut at its lines instead, up to 112 bytes
 //              ahead of the row's k, so a stage is multiplied when the next one has landed as well.  bf16 1237 x 4100 x 2056 with
