@@ -585,7 +585,7 @@ static hipError_t launch_tiles(int tile, int op, const TileGemmParams& p, hipStr
         TileGemmParams r = p;
         // a contiguous run of tiles shares an XCD's L2: whole columns of up to eight tiles, so that a panel of B is read once
         const int tiles_m = (p.m + bm - 1) / bm;
-        r.group_m = tiles_m <= 8 ? tiles_m : 4;
+        r.group_m = tiles_m <= 8 ? tiles_m : RING_GROUP;
         return launch_gemm_ring(tile - TILE_RING, op, r, stream);
     }
     // tile id 3: the 16x16x128 form of the block-scaled fp8 types' large tile (the other types have one form, under both

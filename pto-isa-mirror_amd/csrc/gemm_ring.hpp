@@ -5,6 +5,8 @@
 
 #include <algorithm>
 
+#include "ring_index.hpp"
+
 namespace ptoamd {
 
 struct TileGemmParams;

@@ -12,7 +12,7 @@ static hipError_t launch_ring(const TileGemmParams& p, hipStream_t stream)
     const hipError_t e = ensure_dynamic_lds<&gemm_tile_ring_kernel<Cfg>>(Cfg::LDS_BYTES);
     if (e != hipSuccess || p.m <= 0)  // m = 0: only make the kernel ready to launch on the current device
         return e;
-    const RingTiles tiles = ring_tiles(p, Cfg::BM, Cfg::BN);
+    const RingTiles tiles = ring_tiles(p.m, p.n, Cfg::BM, Cfg::BN, p.group_m);
     hipLaunchKernelGGL((gemm_tile_ring_kernel<Cfg>), dim3(tiles.grid), dim3(Cfg::THREADS), Cfg::LDS_BYTES, stream, p.a, p.b, (uint32_t)p.lda_bytes, (uint32_t)p.ldb_bytes, p.m, p.n, p.k_bytes, tiles.grid,
                        tiles.tiles_m, tiles.per_group, tiles.divisor.magic, tiles.divisor.shift, p);
     return hipGetLastError();

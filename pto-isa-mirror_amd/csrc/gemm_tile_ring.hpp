@@ -31,7 +31,10 @@
 //   K tail     copies never read past a row: a chunk that would is read as the 16 bytes that END at the row's end, and the
 //              last stage's fragments are masked in registers -- the same bytes of A and B, so k positions still agree
 #pragma once
+#include <cstddef>
+
 #include "gemm_tile_dtl.hpp"
+#include "ring_index.hpp"
 
 namespace ptoamd {
 
@@ -267,38 +270,6 @@ __device__ __forceinline__ void ring_store(const TileGemmParams& p, Elem (&v)[NE
     }
 }
 
-// n / d for 0 <= n < 2^31 as a product (division by an invariant integer through multiplication, Granlund and Montgomery 1994): with l = ceil(log2 d) and magic = ceil(2^(31 + l) / d), which is below 2^32, the error of
-// n * magic / 2^(31 + l) is below 1 / d.
-struct RingDivisor {
-    uint32_t magic, shift;
-    __host__ static RingDivisor of(uint32_t d)
-    {
-        uint32_t l = 0;
-        while ((1ull << l) < d)
-            ++l;
-        return {(uint32_t)(((1ull << (31 + l)) + d - 1) / d), 31 + l};
-    }
-    __device__ __forceinline__ int divide(int n) const { return (int)(((uint64_t)(uint32_t)n * magic) >> shift); }
-};
-// Workgroup -> tile, prepared by the host: `grid` tiles in tiles_m rows, walked in groups of rows; per_group tiles make a group of
-// RING_GROUP rows (the last one has fewer), or all tiles are one group of tiles_m rows (per_group = grid).  divisor: of per_group,
-// or of tiles_m.  Two divisions of run-time values in the kernel took 90 scalar instructions.
-constexpr int RING_GROUP = 4;
-struct RingTiles {
-    int grid, tiles_m, per_group;
-    RingDivisor divisor;
-};
-inline RingTiles ring_tiles(const TileGemmParams& p, int bm, int bn)
-{
-    RingTiles t;
-    const int tiles_n = (p.n + bn - 1) / bn;
-    t.tiles_m = (p.m + bm - 1) / bm;
-    t.grid = t.tiles_m * tiles_n;
-    const bool one_group = p.group_m >= t.tiles_m;
-    t.per_group = one_group ? t.grid : RING_GROUP * tiles_n;
-    t.divisor = RingDivisor::of(one_group ? t.tiles_m : t.per_group);
-    return t;
-}
 // Has arguments in scalar registers from here on: they arrive in one wait, where the compiler's own loads, each in front of its first
 // use, stand one after the other.
 template <class T>
@@ -323,7 +294,12 @@ struct RingArguments {
     uint32_t magic, shift;
     TileGemmParams rest;
 };
-static_assert(sizeof(RingArguments) == 56 + sizeof(TileGemmParams), "the parameters' offsets, each aligned by itself");
+// (in the kernel's order, each aligned by itself)
+static_assert(offsetof(RingArguments, a) == 0 && offsetof(RingArguments, b) == 8 && offsetof(RingArguments, lda_bytes) == 16 && offsetof(RingArguments, ldb_bytes) == 20 &&
+                  offsetof(RingArguments, m) == 24 && offsetof(RingArguments, n) == 28 && offsetof(RingArguments, k_bytes) == 32 && offsetof(RingArguments, grid) == 36 &&
+                  offsetof(RingArguments, tiles_m) == 40 && offsetof(RingArguments, per_group) == 44 && offsetof(RingArguments, magic) == 48 &&
+                  offsetof(RingArguments, shift) == 52 && offsetof(RingArguments, rest) == 56 && alignof(TileGemmParams) == 8,
+              "the parameters' offsets");
 template <class Cfg>
 __global__ void __launch_bounds__(Cfg::THREADS) gemm_tile_ring_kernel(const uint8_t* a, const uint8_t* b, const uint32_t lda_bytes, const uint32_t ldb_bytes, const int m, const int n, const int k_bytes,
                                                                      const int grid, const int tiles_m, const int per_group, const uint32_t magic, const uint32_t shift, const TileGemmParams)
@@ -343,8 +319,6 @@ __global__ void __launch_bounds__(Cfg::THREADS) gemm_tile_ring_kernel(const uint
     const int wk = wave / (Cfg::WM * Cfg::WN), wmn = wave % (Cfg::WM * Cfg::WN), wm = wmn % Cfg::WM, wn = wmn / Cfg::WM;
     const int l16 = lane & 15, lg = lane >> 4;
 
-    // ---- workgroup -> tile.  Workgroup ids go round-robin to the 8 XCDs; XCD x takes a contiguous run of tiles, walked in
-    // groups of group_m tile rows, so that what an L2 holds is a few panels of A and of B.
     const TileGemmParams& rest = reinterpret_cast<const RingArguments*>((const void*)__builtin_amdgcn_kernarg_segment_ptr())->rest;
     TileGemmParams p;
     p.a = a;
@@ -372,16 +346,8 @@ __global__ void __launch_bounds__(Cfg::THREADS) gemm_tile_ring_kernel(const uint
         p.atomic_add = rest.atomic_add;
         ring_arguments(p.c, p.c_in, p.bias, p.acc_out, p.row_scale, p.col_scale, p.ldc, p.relu, p.out_kind, p.qwords, p.q_per_column, p.atomic_add);
     };
-    const int xcd = blockIdx.x & 7;
-    const int lid = xcd * (grid >> 3) + min(xcd, grid & 7) + (blockIdx.x >> 3);
-    const int quotient = RingDivisor{magic, shift}.divide(lid);
-    int row = lid - quotient * tiles_m, column = quotient;
-    if (per_group != grid) {
-        const int in_group = lid - quotient * per_group, first = quotient * RING_GROUP, gsize = min(tiles_m - first, RING_GROUP);
-        column = gsize == 4 ? in_group >> 2 : gsize == 3 ? (int)(uint32_t)(((uint64_t)(uint32_t)in_group * 0xAAAAAAABu) >> 33) : in_group >> (gsize - 1);
-        row = first + in_group - column * gsize;
-    }
-    const int m0 = row * BM, n0 = column * BN;
+    const RingTile tile = RingTiles{grid, tiles_m, per_group, {magic, shift}}.tile(blockIdx.x);
+    const int m0 = tile.row * BM, n0 = tile.column * BN;
 
     // ---- TLOAD addressing: piece w + q * NW of a stage, lane -> (row, position) linear, fetching chunk position ^ swizzle
     const int nst = (p.k_bytes + SB - 1) / SB;

@@ -505,3 +505,21 @@ def test_every_count_of_stages(pa, kind, shape):  # noqa: F811
                     got = pa.gemm(a.to(torch.int8), b.to(torch.int8), pa.I8, pa.I32, pa.B_DN)
                 assert pa.last_kernel().startswith(f"tile{bm}x{bn}_"), pa.last_kernel()
             assert torch.equal(got, ref.float().to(got.dtype)), (kind, m, n, kb)
+
+
+@pytest.mark.parametrize("kind,shape", [("bf16", s) for s in range(9)] + [("fp8", s) for s in range(7)])
+def test_last_group_of_tile_rows(pa, kind, shape):  # noqa: F811
+    """One, two and three tile rows behind whole groups of four, several tile columns: exact, the sums being whole numbers."""
+    bm, bn = SHAPES[shape][:2]
+    gen = torch.Generator(device="cuda").manual_seed(shape)
+    lut = torch.tensor([0, 0x38, 0x40, 0x44], device="cuda", dtype=torch.uint8)  # 0, 1, 2, 3 in E4M3
+    for rest in (1, 2, 3):
+        m, n, k = (8 + rest) * bm - 3, 5 * bn - 7, 128
+        a, b = (torch.randint(-3, 4, (x, k), generator=gen, device="cuda") for x in (m, n))
+        with tile_env(PTOAMD_RING=shape):
+            if kind == "fp8":
+                got = pa.gemm_fp8(*(lut[x.abs()] | (0x80 * (x < 0)).to(torch.uint8) for x in (a, b)), pa.E4M3, pa.E4M3, pa.F32)
+            else:
+                got = pa.gemm(a.bfloat16(), b.bfloat16(), pa.BF16, pa.F32, pa.B_DN)
+            assert pa.last_kernel().startswith(f"tile{bm}x{bn}_"), pa.last_kernel()
+        assert torch.equal(got.double(), a.double() @ b.double().T), (m, n)
