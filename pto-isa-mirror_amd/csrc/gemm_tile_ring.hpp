@@ -610,28 +610,19 @@ __global__ void __launch_bounds__(Cfg::THREADS) gemm_tile_ring_kernel(const uint
         const int as = aset(set, i);
         Op::mma(acc[i][j], fa[as][i], fb[set][j], Op::SCALED ? (CHUNKED || has_scales ? xa[as][i] : 127u) : 0u, Op::SCALED ? (CHUNKED || has_scales ? xb[set][j] : 127u) : 0u);
     };
-    // k-step s of the last stage, which may reach past K
-    auto tail_step = [&](int set, int s) __attribute__((always_inline)) {
-        const int k0 = (nst - 1) * SB + wk * Cfg::KW + s * Cfg::KB;  // first K byte of the step
-        if (k0 >= p.k_bytes)
-            return;
-        if (k_tail) {
+    // k-step s of the last stage may reach past K: the first K byte of it, and its fragments masked
+    auto tail_start = [&](int s) { return (nst - 1) * SB + wk * Cfg::KW + s * Cfg::KB; };
+    auto mask_all = [&](int set, int s) __attribute__((always_inline)) {
 #pragma unroll
-            for (int f = 0; f < FR; ++f) {
-                const uint4 mask = ring_chunk_mask(p.k_bytes - (k0 + (4 * f + lg) * 16));
+        for (int f = 0; f < FR; ++f) {
+            const uint4 mask = ring_chunk_mask(p.k_bytes - (tail_start(s) + (4 * f + lg) * 16));
 #pragma unroll
-                for (int i = 0; i < MB; ++i)
-                    fa[aset(set, i)][i][f] = ring_masked(fa[aset(set, i)][i][f], mask);
-#pragma unroll
-                for (int j = 0; j < NB; ++j)
-                    fb[set][j][f] = ring_masked(fb[set][j][f], mask);
-            }
-        }
-#pragma unroll
-        for (int i = 0; i < MB; ++i)
+            for (int i = 0; i < MB; ++i)
+                fa[aset(set, i)][i][f] = ring_masked(fa[aset(set, i)][i][f], mask);
 #pragma unroll
             for (int j = 0; j < NB; ++j)
-                mma(set, i, j);
+                fb[set][j][f] = ring_masked(fb[set][j][f], mask);
+        }
     };
 
     // ---- the K loop
@@ -690,8 +681,17 @@ __global__ void __launch_bounds__(Cfg::THREADS) gemm_tile_ring_kernel(const uint
         step(nst - 1);
         if (computes)
             static_for<Cfg::KSTEPS>([&](auto sc) {
-                read_all(0, decltype(sc)::value, buf, rows, Skewed{});
-                tail_step(0, decltype(sc)::value);
+                constexpr int s = decltype(sc)::value;
+                read_all(0, s, buf, rows, Skewed{});
+                if (tail_start(s) >= p.k_bytes)
+                    return;
+                if (k_tail)
+                    mask_all(0, s);
+#pragma unroll
+                for (int i = 0; i < MB; ++i)
+#pragma unroll
+                    for (int j = 0; j < NB; ++j)
+                        mma(0, i, j);
             });
     } else {
         // Barrier st stands in front of or in the last k-step of stage st: every wave holds that k-step's fragments, so the stage's
@@ -800,46 +800,49 @@ __global__ void __launch_bounds__(Cfg::THREADS) gemm_tile_ring_kernel(const uint
             ring_wait_and_barrier<63>();
             read_all(0, 0, 0, rows, skew);
             int buf = 0, st = 0;
-            auto body = [&](auto parc, auto lastc) __attribute__((always_inline)) {
+            // One k-step on register set SET.  NEXT: under its matrix instructions the fragments of the next one are read, k-step rs of ring
+            // buffer rb.  BARRIER: that one is another stage's.
+            // The barrier waits for the wave's own reads, the last of which go out a row of matrix instructions before the k-step's end:
+            // it stands a row into the last k-step, so that two rows cover them (and nothing is moved across it: the compiler put
+            // all but one of that row's instructions behind it).  128 x 128 tiles 700 -> 680 clocks a stage, 256 x 128 1211 -> 1160, 192 x
+            // 128 970 -> 953, MXFP8 on 96 x 64 936 -> 880.
+            auto k_step = [&](auto setc, auto nextc, auto barrierc, int rs, int rb, const ScaleRows& rsc, const Skewed& rsk) __attribute__((always_inline)) {
+                constexpr int SET = decltype(setc)::value;
+                constexpr bool NEXT = decltype(nextc)::value, BARRIER = decltype(barrierc)::value;
+                constexpr int BAR = BARRIER && MB > 1 && NMMA >= 6 ? NB : 0;
+                static_for<NMMA>([&](auto xc) {
+                    constexpr int x = decltype(xc)::value, i = x / NB, j = x % NB;
+                    if constexpr (BARRIER && x == BAR) {
+                        __builtin_amdgcn_sched_barrier(0);
+                        ring_wait_and_barrier<63>();
+                    }
+                    mma(SET, i, j);
+                    constexpr int y = x - BAR, AL = NB < NMMA - BAR ? NB : NMMA - BAR - 1;
+                    if constexpr (NEXT && y >= 0 && (y < NB || y == AL || (j == NB - 1 && i < MB - 1))) {
+                        __builtin_amdgcn_sched_barrier(0);
+                        if constexpr (y < NB)
+                            read_b(SET ^ 1, y, rs, rb, rsc, rsk);
+                        if constexpr (y == 0)
+                            static_for<BAR / NB>([&](auto rc) { read_a(0, decltype(rc)::value, rs, rb, rsc, rsk); });
+                        if constexpr (y == AL)
+                            read_a(SET ^ 1, MB - 1, rs, rb, rsc, rsk);
+                        if constexpr (j == NB - 1 && i < MB - 1)
+                            read_a(0, i, rs, rb, rsc, rsk);
+                        __builtin_amdgcn_sched_barrier(0);
+                    }
+                });
+            };
+            auto body = [&](auto parc) __attribute__((always_inline)) {
                 constexpr int PAR = decltype(parc)::value;
-                constexpr bool LASTSTAGE = decltype(lastc)::value;
                 const int nbuf = buf + 1 == R ? 0 : buf + 1;
                 static_for<Cfg::KSTEPS>([&](auto sc) {
-                    constexpr int s = decltype(sc)::value, SET = (PAR + s) & 1;
-                    constexpr bool LASTSTEP = s + 1 == Cfg::KSTEPS;
-                    constexpr int rs = LASTSTEP ? 0 : s + 1;
-                    const int rb = LASTSTEP ? nbuf : buf;
-                    const ScaleRows& rsc = LASTSTEP ? next_rows : rows;
-                    const Skewed& rsk = LASTSTEP ? next_skew : skew;
-                    // The barrier waits for the wave's own reads, the last of which go out a row of matrix instructions before the k-step's end:
-                    // it stands a row into the last k-step, so that two rows cover them (and nothing is moved across it: the compiler put
-                    // all but one of that row's instructions behind it).  128 x 128 tiles 700 -> 680 clocks a stage, 256 x 128 1211 -> 1160, 192 x
-                    // 128 970 -> 953, MXFP8 on 96 x 64 936 -> 880.
-                    constexpr int BAR = LASTSTEP && MB > 1 && NMMA >= 6 ? NB : 0;
-                    static_for<NMMA>([&](auto xc) {
-                        constexpr int x = decltype(xc)::value, i = x / NB, j = x % NB;
-                        if constexpr (LASTSTEP && !LASTSTAGE && x == BAR) {
-                            __builtin_amdgcn_sched_barrier(0);
-                            ring_wait_and_barrier<63>();
-                        }
-                        mma(SET, i, j);
-                        constexpr int y = x - BAR, AL = NB < NMMA - BAR ? NB : NMMA - BAR - 1;
-                        if constexpr (!(LASTSTEP && LASTSTAGE) && y >= 0 && (y < NB || y == AL || (j == NB - 1 && i < MB - 1))) {
-                            __builtin_amdgcn_sched_barrier(0);
-                            if constexpr (y < NB)
-                                read_b(SET ^ 1, y, rs, rb, rsc, rsk);
-                            if constexpr (y == 0)
-                                static_for<BAR / NB>([&](auto rc) { read_a(0, decltype(rc)::value, rs, rb, rsc, rsk); });
-                            if constexpr (y == AL)
-                                read_a(SET ^ 1, MB - 1, rs, rb, rsc, rsk);
-                            if constexpr (j == NB - 1 && i < MB - 1)
-                                read_a(0, i, rs, rb, rsc, rsk);
-                            __builtin_amdgcn_sched_barrier(0);
-                        }
-                    });
+                    constexpr int s = decltype(sc)::value;
+                    constexpr integral_constant<int, (PAR + s) & 1> set{};
+                    if constexpr (s + 1 < Cfg::KSTEPS)
+                        k_step(set, std::true_type{}, std::false_type{}, s + 1, buf, rows, skew);
+                    else
+                        k_step(set, std::true_type{}, std::true_type{}, 0, nbuf, next_rows, next_skew);
                 });
-                if constexpr (LASTSTAGE)
-                    return;
                 buf = nbuf;
                 ++st;
                 rows = next_rows;
@@ -847,33 +850,33 @@ __global__ void __launch_bounds__(Cfg::THREADS) gemm_tile_ring_kernel(const uint
                 skew = next_skew;
                 next_skew = skewed(nbuf + 1 == R ? 0 : nbuf + 1);
             };
+            // The last stage: nothing behind it, and K may end in it.  One piece of code for both kinds of K, of the steps that the loop has: next to
+            // a copy for whole stages only and one that masks, read by read, the accumulators had registers of their own in either (128 x 128 tiles
+            // 200 for 128, rows on any byte 238 for 162, on 96 x 64 tiles 256 for 156), and rows on any byte, whose K hardly ever is whole
+            // stages, took longer: bf16 1 x 469 x 739 on 96 x 64 tiles 9.3 us before there were two, 9.6 with two, 8.95 now; 2198 x 3141 x 931 on
+            // 128 x 64 58.3, 60.2, 57.3.  All stages through the loop, one more barrier and the reads in it for nothing: whole stages 1 % longer.
             auto last = [&](auto parc) __attribute__((always_inline)) {
-                // (K of whole stages: as any other stage.  Larger wave tiles have no registers for a second copy of the loop's body: 256 x 128
-                // tiles kept 164 bytes of it in scratch memory and took 65 us instead of 55)
-                if constexpr (NMMA * FR <= 16) {
-                    if (!k_tail) {
-                        body(parc, std::true_type{});
-                        return;
-                    }
-                }
                 static_for<Cfg::KSTEPS>([&](auto sc) {
-                    constexpr int s = decltype(sc)::value, SET = (decltype(parc)::value + s) & 1;
-                    if constexpr (s > 0)
-                        read_all(SET, s, buf, rows, skew);
-                    tail_step(SET, s);
+                    constexpr int s = decltype(sc)::value;
+                    constexpr integral_constant<int, (decltype(parc)::value + s) & 1> set{};
+                    if (tail_start(s) >= p.k_bytes)
+                        return;
+                    if (k_tail)  // (masks always: whole stages 2.5 % longer)
+                        mask_all(set, s);
+                    k_step(set, integral_constant<bool, (s + 1 < Cfg::KSTEPS)>{}, std::false_type{}, s + 1, buf, rows, skew);
                 });
             };
             if constexpr (Cfg::KSTEPS % 2 == 0) {
                 while (st < nst - 1)
-                    body(integral_constant<int, 0>{}, std::false_type{});
+                    body(integral_constant<int, 0>{});
                 last(integral_constant<int, 0>{});
             } else {  // the register sets change places from stage to stage
                 while (st + 2 < nst) {
-                    body(integral_constant<int, 0>{}, std::false_type{});
-                    body(integral_constant<int, 1>{}, std::false_type{});
+                    body(integral_constant<int, 0>{});
+                    body(integral_constant<int, 1>{});
                 }
                 if (st + 1 < nst) {
-                    body(integral_constant<int, 0>{}, std::false_type{});
+                    body(integral_constant<int, 0>{});
                     last(integral_constant<int, 1>{});
                 } else {
                     last(integral_constant<int, 0>{});

@@ -99,3 +99,14 @@ def test_tiles_without_an_edge_carry_no_code_for_one(kernels):
         assert ("ELb0EEEv" in name) != ("ELb1EEEv" in name), name
         if "ELb1EEEv" in name:
             assert by_name[name.replace("ELb1EEEv", "ELb0EEEv")] <= count, name
+
+
+def test_pipelined_deep_ring_tiles_hold_their_accumulators_once(kernels):
+    """Deep-ring tiles of 64 x 64 to 128 x 128, copying waves beside multiplying ones: 16 to 64 accumulators a thread, two sets of
+    fragments and, in the waves that copy rows on any byte, the pieces under way, all within a third of a SIMD's 512 registers.  A second
+    set of accumulators for another copy of the K loop's code takes them past it.  (fp8 on 128 x 128 has fragments of twice the size.)"""
+    shapes = ["64ELi64E", "96ELi64E", "128ELi64E", "128ELi128E"]
+    ks = [k for k in kernels if "gemm_tile_ring_kernel" in k[".name"] and any(f"RingCfgILi{s}" in k[".name"] for s in shapes)]
+    assert len(ks) >= 30, len(ks)
+    over = {k[".name"]: k[".vgpr_count"] for k in ks if k[".vgpr_count"] > 168 and not ("OpFP8" in k[".name"] and "Li128ELi128E" in k[".name"])}
+    assert not over, over
