@@ -514,6 +514,31 @@ struct StagedStore {
     static_assert((32 * Cfg::WTN / 16) % 64 == 0, "a band is a whole number of 64-lane reads, down to one-byte outputs");
 };
 
+// C is not read again by this kernel: pieces of whole 64-byte sectors are stored non-temporally (plain stores end TSTORE 0.3 us
+// sooner, but their write-backs cost the next launch 1 us).  Where rows start off the sectors, two wave tiles share one at every seam:
+// streamed, its parts go to memory one by one, written plainly they meet in the L2s, which have it written back later.  Whether a result of
+// `bytes` is stored plainly there: where that is ahead with A and C in the caches, as a program has them that uses its activations' buffers again.
+// Time with plain stores over time with streamed ones, geometric means over some 900 sizes a column: launches on the same buffers | on four
+// sets in turn | on weights of 640 MB in turn, A and C the same | all of A, B and C in turn, 640 MB, which no cache holds:
+//   256 x 256 tiles      up to 127 of them, which leave half of the CUs idle, 0.99 | 1.02 | 1.02 | 1.14; from 128 on 0.82 | 0.84 | 0.81 | 0.98
+//   256 x 128            to 16 MiB 0.95 | 0.97 | 0.98 | 1.13; above 0.88 | 0.83 | 0.82 | 1.13
+//   128 x 128, by DMA    to 4 MiB 0.95 | 0.96 | 0.97 | 1.04; to 16 0.94 | 1.00 | 0.98 | 1.22; above 0.91 | 0.83 | 0.80 | 1.05
+//   register-staged      to 8 MiB 0.95 | 0.97 | 0.98 | 1.04; above 0.98 | 1.00 | 0.98 | 1.15, but few slabs of K 0.58 to 0.95 in the first column
+//   by a word, 16 bits   (bound by the conversions) to 4 MiB 0.98 | 0.99 | 0.99 | 1.00, above 1.00 | 1.02 | 1.02 | 1.09; 256 x 256 1.00 | 1.04 | 1.04 | 1.03
+//   by a word, one byte  (a wave's pieces are a sector long) 1.00 in all, 256 x 256 tiles as above, 4096 x 4104 x 1024 56.3 -> 53.2 us
+// Of the sizes that are stored plainly one in ten is 1 to 5 % behind in the first three columns.  256 x 256 tiles, us, streamed and plain: MXFP4
+// 2040 x 8100 x 8192 72.1 / 66.0, bf16 4096 x 4104 x 1024 51.9 / 46.3.
+template <int KIND, class Cfg>
+__device__ __forceinline__ bool plain_off_sectors(long bytes)
+{
+    constexpr long MIB = 1 << 20, TILE = Cfg::BM * Cfg::BN;
+    if (KIND == OUT_Q8 && TILE < 65536)
+        return false;
+    if (TILE >= 65536)
+        return KIND != OUT_QF16 && gridDim.x >= 128;
+    return KIND != OUT_QF16 || bytes < 4 * MIB;
+}
+
 // `stage` is the calling wave's private LDS region of StagedStore<Cfg>::WAVE_BYTES bytes.  The wave tile starts inside the matrix
 // (checked by the caller); its last rows may lie past row m - 1: they are computed on clamped row indices and not stored.  Its
 // last columns may lie past column n - 1: a row piece is then its whole 16-byte chunks and, from one lane per row, the elements of the
@@ -589,14 +614,7 @@ __device__ __forceinline__ void tstore_staged(const TileGemmParams& p, Acc (&acc
             rs_pre[i] = p.row_scale[min(row0 + i * BLK + l32, p.m - 1)];
         fetch_columns(cs_pre, p.col_scale);
     }
-    // C is not read again by this kernel: pieces of whole 64-byte sectors are stored non-temporally (plain stores end TSTORE 0.3 us
-    // sooner, but their write-backs cost the next launch 1 us).  Where rows start off the sectors, two wave tiles share one at every
-    // seam: streamed, its parts go to memory one by one, written plainly they meet in the L2.  4096 x n x 1024 on 256 x 256 tiles, us,
-    // streamed and plain: bf16 n 4096 27.6 / 28.4, 4128 46.6 / 45.9, 4104 51.9 / 46.3, 4100 52.6 / 46.3; f32 4128 51.6 / 50.2, 4104 58.6 /
-    // 50.7; one byte 4104 56.3 / 53.2; 128 x 128 tiles bf16 4100 45.7 / 42.8, f32 4100 55.3 / 50.0, but one byte 57.2 / 58.8 (a wave's
-    // pieces are a sector long there, and its drain is bound by the conversions); MXFP4 2040 x 8100 x 8192 72.1 / 66.0.
-    constexpr bool NARROW = ESZ == 1 && Cfg::BM * Cfg::BN < 65536;
-    const bool streamed = NARROW || ((reinterpret_cast<uintptr_t>(p.c) | (uintptr_t)p.ldc * ESZ) & 63) == 0;
+    const bool streamed = !plain_off_sectors<KIND, Cfg>((long)p.m * p.n * ESZ) || ((reinterpret_cast<uintptr_t>(p.c) | (uintptr_t)p.ldc * ESZ) & 63) == 0;
     constexpr int EPC = 16 / ESZ;  // elements of a chunk
     const int live = EDGE ? p.n - col0 : Cfg::WTN, whole = live / EPC, rest = live % EPC;
     static_assert(64 % CHUNKS == 0, "a lane stores the same chunk of several rows");

@@ -110,3 +110,37 @@ def test_rows_on_and_off_the_64_byte_sectors(pa, dtype, tile):  # noqa: F811
             pa.gemm(a.bfloat16(), b.bfloat16(), pa.BF16, pa.F32 if dtype == torch.float32 else pa.BF16, pa.B_DN, out=view[:, :n])
         assert torch.equal(view[:, :n], ref), (tile, pitch, lead)
         assert (view[:, n:] == 77).all() and (wide[:lead] == 77).all() and (wide[lead + m * pitch:] == 77).all(), (tile, pitch, lead)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.int32])
+def test_rows_off_the_sectors_on_either_side_of_half_a_grid(pa, dtype):  # noqa: F811
+    """127 tiles of 256 x 256, which stream them, and a row more, 128, which store them plainly."""
+    gen = torch.Generator(device="cuda").manual_seed(1)
+    n, k = 253, 64
+    for m in (127 * 256, 127 * 256 + 1):
+        a, b = (torch.randint(-3, 4, (x, k), generator=gen, device="cuda") for x in (m, n))
+        if dtype == torch.int32:
+            run = (a.to(torch.int8), b.to(torch.int8), pa.I8, pa.I32)
+        else:
+            run = (a.bfloat16(), b.bfloat16(), pa.BF16, pa.F32 if dtype == torch.float32 else pa.BF16)
+        flat = torch.full((m * n + 1000,), 77, device="cuda", dtype=dtype)
+        with tile_env(PTOAMD_TILE=4):
+            pa.gemm(*run, pa.B_DN, out=flat[:m * n].view(m, n))
+        assert torch.equal(flat[:m * n].view(m, n), (a.double() @ b.double().T).float().to(dtype)), m
+        assert (flat[m * n:] == 77).all()
+
+
+@pytest.mark.parametrize("tile", [1, 2, 4, 5, 6])
+def test_requantised_rows_off_the_sectors_at_the_size_where_their_store_changes(pa, tile):  # noqa: F811
+    """16-bit results by a word of 4 MiB less one row's and a row more."""
+    gen = torch.Generator(device="cuda").manual_seed(tile)
+    n, k = 1021, 64
+    word = torch.tensor([0x3C000000], dtype=torch.int64, device="cuda")  # * 2 ** -7
+    m0 = (4 << 20) // (2 * n)
+    for m in (m0, m0 + 1):
+        a, b = (torch.randint(-100, 100, (x, k), generator=gen, device="cuda", dtype=torch.int8) for x in (m, n))
+        with tile_env(PTOAMD_TILE=tile):
+            got = pa.gemm_requant(a, b, pa.I8, pa.F16, word, per_column=False)
+        with tile_env(PTOAMD_FORCE_GENERIC=1):
+            assert torch.equal(got, pa.gemm_requant(a, b, pa.I8, pa.F16, word, per_column=False)), (tile, m)
+        assert got.unique().numel() > 100
