@@ -5,7 +5,9 @@ tenth of the run time without failing any result check, so the library's own cod
 no kernel of the library may use scratch at all.
 """
 import os
+import re
 import struct
+import subprocess
 
 import msgpack
 import pytest
@@ -110,3 +112,28 @@ def test_pipelined_deep_ring_tiles_hold_their_accumulators_once(kernels):
     assert len(ks) >= 30, len(ks)
     over = {k[".name"]: k[".vgpr_count"] for k in ks if k[".vgpr_count"] > 168 and not ("OpFP8" in k[".name"] and "Li128ELi128E" in k[".name"])}
     assert not over, over
+
+
+def test_rows_of_c_can_leave_either_way(tmp_path):
+    """Tiles that store through LDS hold their 16-byte stores of C twice, non-temporal and plain, but for the result types that are never
+    stored plainly.  The compiler can make one of two branches that differ in this only, then of plain stores, and no result would tell."""
+    objdump = "/opt/rocm/llvm/bin/llvm-objdump"
+    if not (os.path.exists(LIB) and os.path.exists(objdump)):
+        pytest.skip("no library or no disassembler")
+    with open(LIB, "rb") as f:
+        blob = f.read()
+    seen = 0
+    for elf in _code_objects(blob):
+        names = [k[".name"] for k in _kernels(elf) if "gemm_tile_dtl_kernel" in k[".name"] or "16gemm_tile_kernel" in k[".name"]]
+        names = [n for n in names if "OpBF16" in n or "OpI8" in n]  # (the others are of the same templates)
+        if not names:
+            continue
+        (tmp_path / "code.elf").write_bytes(elf)
+        text = subprocess.run([objdump, "-d", "--no-show-raw-insn", "--disassemble-symbols=" + ",".join(names), str(tmp_path / "code.elf")],
+                              check=True, capture_output=True, text=True).stdout
+        for kernel in re.split(r"^[0-9a-f]+ <", text, flags=re.M)[1:]:
+            stores = [line for line in kernel.splitlines() if "_store_dwordx4" in line]
+            streamed = sum(" nt" in line for line in stores)
+            assert 0 < len(stores) - streamed <= streamed, (kernel.split(">")[0], streamed, len(stores))
+            seen += 1
+    assert seen >= 20, seen
