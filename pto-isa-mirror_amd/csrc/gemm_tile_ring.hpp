@@ -104,6 +104,25 @@ struct RingCfg {
     static_assert(LDS_BYTES <= 160 * 1024 && R >= 2 && R * NV + (CHUNKED ? ROWS * SCB / 1024 / NW + 1 : 0) < 64, "LDS capacity; vmcnt is a 6-bit count");
 };
 
+// The copies of a row-major B (BND): what lane `lane` of copy q of copying wave lw brings.  A stage is KR k rows of BN columns, a chunk
+// eight columns of a k row.
+template <class Cfg>
+struct RingRowCopies {
+    // the stage's row, and the chunk of it
+    __host__ __device__ static __forceinline__ int row(int lw, int q, int lane) { return ((lw + q * Cfg::NW - Cfg::A_PIECES) * 64 + lane) / Cfg::CB; }
+    __host__ __device__ static __forceinline__ int chunk(int row, int lane) { return (lane % Cfg::CB) ^ (swizzle_row_major<Cfg::BN>(row) << 1); }
+    // first byte fetched of a k row: of the chunk that N ends in, and of those past it, the 16 that end there
+    __host__ __device__ static __forceinline__ int byte(int n, int n0, int chunk)
+    {
+        const int at = n0 * 2 + chunk * 16, last = n * 2 - 16;
+        return at < last ? at : last;
+    }
+    // k row fetched for row r of the matrix: of eight rows that K ends in, and of those past them, the eight that end there, as in A's chunk of the
+    // same k.  base: the row that a stage's offsets are counted from.
+    __host__ __device__ static __forceinline__ int source(int k, int r) { return (r | 7) < k ? r : k - 8 + (r & 7); }
+    __host__ __device__ static __forceinline__ int base(int stage) { return stage * Cfg::KR > 8 ? stage * Cfg::KR - 8 : 0; }
+};
+
 // position of a row's 16-byte chunk is chunk ^ ring_swizzle(row)
 template <int SB>
 __device__ __forceinline__ int ring_swizzle(int row)
@@ -360,10 +379,10 @@ __global__ void __launch_bounds__(Cfg::THREADS) gemm_tile_ring_kernel(const uint
         const int r = piece_row(q);
         return lw + q * NW < Cfg::A_PIECES ? (uint32_t)(min(m0 + r, p.m - 1) * p.lda_bytes) : (uint32_t)(min(n0 + r - BM, p.n - 1) * p.ldb_bytes);
     };
-    // BND: a stage's B is KR rows of BN columns; row and byte offset (columns past N repeat the row's last chunk)
-    auto nd_row = [&](int q) { return ((lw + q * NW - Cfg::A_PIECES) * 64 + lane) / Cfg::CB; };
-    auto nd_chunk = [&](int q) { return (lane % Cfg::CB) ^ (swizzle_row_major<BN>(nd_row(q)) << 1); };
-    auto nd_col = [&](int q) -> uint32_t { return (uint32_t)min(n0 * 2 + nd_chunk(q) * 16, p.n * 2 - 16); };
+    using RowCopies = RingRowCopies<Cfg>;
+    auto nd_row = [&](int q) { return RowCopies::row(lw, q, lane); };
+    auto nd_chunk = [&](int q) { return RowCopies::chunk(nd_row(q), lane); };
+    auto nd_col = [&](int q) -> uint32_t { return (uint32_t)RowCopies::byte(p.n, n0, nd_chunk(q)); };
     // SKEW: a stage of a row is whole 128-byte lines, so it starts `skew` chunks ahead of its own k.  Of the chunks of a stage's lines
     // that belong to this k stage and to the one before, each stands where its k has it: fragment reads find it at the same place
     // in either buffer, and their banks are those of rows that start on a line.
@@ -465,9 +484,7 @@ __global__ void __launch_bounds__(Cfg::THREADS) gemm_tile_ring_kernel(const uint
             for (int q = 0; q < NPW; ++q) {
                 const int piece = lw + q * NW;
                 if (Cfg::BND && piece >= Cfg::A_PIECES) {
-                    // eight rows that K ends in are the eight that end there, as in A's chunk of the same k
-                    const int k = p.k_bytes / 2, row = st * Cfg::KR + nd_row(q), base_row = max(st * Cfg::KR - 8, 0);
-                    const int src = (row | 7) < k ? row : k - 8 + (row & 7);
+                    const int base_row = RowCopies::base(st), src = RowCopies::source(p.k_bytes / 2, st * Cfg::KR + nd_row(q));
                     lds_dma16_off(p.b + (long)base_row * p.ldb_bytes, (uint32_t)((src - base_row) * p.ldb_bytes) + nd_col(q), dst + piece * 1024);
                     continue;
                 }
@@ -713,11 +730,11 @@ __global__ void __launch_bounds__(Cfg::THREADS) gemm_tile_ring_kernel(const uint
             auto load = [&](auto gc, int st) __attribute__((always_inline)) {
                 const int stage = min(st, nst - 1);
                 const uint32_t k0 = stage * SB;
-                const int base_row = max(stage * Cfg::KR - 8, 0);
+                const int base_row = RowCopies::base(stage);
 #pragma unroll
                 for (int q = 0; q < NPW; ++q) {
-                    if (Cfg::BND && q * NW >= Cfg::A_PIECES) {  // (eight rows that K ends in: as in issue_operands)
-                        const int k = p.k_bytes / 2, r = stage * Cfg::KR + nd_row(q), src = (r | 7) < k ? r : k - 8 + (r & 7);
+                    if (Cfg::BND && q * NW >= Cfg::A_PIECES) {
+                        const int src = RowCopies::source(p.k_bytes / 2, stage * Cfg::KR + nd_row(q));
                         held[decltype(gc)::value][q] = load_unaligned16(p.b + (long)base_row * p.ldb_bytes + ((uint32_t)((src - base_row) * p.ldb_bytes) + row[q]));
                         continue;
                     }

@@ -39,7 +39,7 @@ __device__ __forceinline__ uint32_t lds_address(const void* generic_ptr)
 // piece ^ swizzle_row_major(row).  A half wave of the transposing read takes one piece of rows 0 .. 3 and 8 .. 11 (counted from
 // a multiple of 4): they lie in different banks from 32 columns on.
 template <int COLS>
-__device__ __forceinline__ int swizzle_row_major(int row)
+__host__ __device__ __forceinline__ int swizzle_row_major(int row)
 {
     const int b3 = (row >> 3) & 1;
     return COLS == 128 ? (row & 3) | (b3 << 2) : COLS == 64 ? ((row >> 1) & 1) | (b3 << 1) : COLS == 32 ? b3 : 0;

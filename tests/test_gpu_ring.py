@@ -523,3 +523,31 @@ def test_last_group_of_tile_rows(pa, kind, shape):  # noqa: F811
                 got = pa.gemm(a.bfloat16(), b.bfloat16(), pa.BF16, pa.F32, pa.B_DN)
             assert pa.last_kernel().startswith(f"tile{bm}x{bn}_"), pa.last_kernel()
         assert torch.equal(got.double(), a.double() @ b.double().T), (m, n)
+
+
+@pytest.mark.parametrize("shape", [1, 3, 4, 5, 6, 7, 8])
+def test_row_major_b_rows_on_any_element_through_every_drain(pa, shape):  # noqa: F811
+    """As above with a bias row and a 16-bit result, an accumulator input, a quantisation word for all columns and one per column, atomic
+    additions: exact, the sums being whole numbers; what is quantised as on the order-exact kernel."""
+    bm, bn, stage = SHAPES[shape][:3]
+    gen = torch.Generator(device="cuda").manual_seed(shape)
+    m, n, k = bm + 1, bn + 3, 2 * (stage // 2) + 5
+    a, b = (torch.randint(-3, 4, x, generator=gen, device="cuda").bfloat16() for x in ((m, k), (k, n)))
+    ref = a.double() @ b.double()
+    bias = torch.randint(-9, 10, (n,), generator=gen, device="cuda").float()
+    c_in = torch.randint(-9, 10, (m, n), generator=gen, device="cuda").float()
+    words = ((torch.randint(0, 2 ** 5, (n,), generator=gen, device="cuda") << 37) | (torch.arange(n, device="cuda") % 2 * (1 << 46))) | 0x3E000000
+    name = f"tile{bm}x{bn}_bnd_any_bf16"
+    with tile_env(PTOAMD_RING=shape):
+        got = pa.gemm(a, b, pa.BF16, pa.BF16, pa.B_ND, bias=bias)
+        assert pa.last_kernel() == name and torch.equal(got, (ref + bias.double()).float().bfloat16())
+        assert torch.equal(pa.gemm(a, b, pa.BF16, pa.F32, pa.B_ND, c_in=c_in).double(), ref + c_in.double())
+        c = c_in.clone()
+        pa.gemm_atomic_add(c, a, b, pa.BF16, pa.B_ND)
+        assert pa.last_kernel() == name and torch.equal(c.double(), ref + c_in.double())
+        quantised = [pa.gemm_requant(a, b, pa.BF16, t, w, per_column=w.numel() > 1, b_layout=pa.B_ND) for t in (pa.I8, pa.F16) for w in (words[:1].contiguous(), words)]
+        assert pa.last_kernel() == name
+    with tile_env(PTOAMD_FORCE_GENERIC=1):
+        exact = [pa.gemm_requant(a, b, pa.BF16, t, w, per_column=w.numel() > 1, b_layout=pa.B_ND) for t in (pa.I8, pa.F16) for w in (words[:1].contiguous(), words)]
+    for q, e in zip(quantised, exact):
+        assert torch.equal(q, e) and q.unique().numel() > 10
