@@ -127,8 +127,9 @@ int ptoamd_event_elapsed_ms(float* ms, void* start, void* stop);
  * bytes; for bf16 / f16 / int8 rows that start on other bytes the deep-ring tiles with copies through registers; for
  * bf16 / f16 / int8 rows that start on 4-byte boundaries with a K that is not a multiple of 4 bytes the two-slab DMA tiles
  * where K is longer than 128 bytes and the grid large enough (a few dozen 128 x 128 tiles of C), else, as for everything left
- * over and for a short K, the register-staged tiles; a row-major B of 16-bit elements is read in place where its rows allow it (ptoamd_gemm_ws below) and else
- * transposed on its way into LDS by the latter.  Rows of C need no alignment either.
+ * over and for a short K, the register-staged tiles; a row-major B of 16-bit elements, of 8 columns or more, is read in place beyond two or three times
+ * 128 bytes of K, whatever its rows start on, and else transposed on its way into LDS by the latter, as one of int8.  Rows of C need no
+ * alignment either.
  * The kernel follows from the whole shape, m included, and kernels add the k products of an output in different orders: a
  * row's f32 sums agree from one batch size to another to rounding, not bit for bit (int8 sums are exact).
  * PTOAMD_F32 and PTOAMD_HIF8 operands (hif8 x hif8 only, cpu/TMatmul.hpp:38) run on the order-exact kernel: one thread
@@ -152,11 +153,14 @@ int ptoamd_gemm_bias(void* c, int c_type, const void* a, const void* b, int ab_t
  * ptoamd_gemm_bias with a caller-owned workspace for a row-major B (PTOAMD_B_ND): where the fastest tiles need a column-major
  * B, it is re-ordered into the workspace ([N][K] with rows padded to 16 bytes, ptoamd_gemm_workspace_bytes(n, k, ab_type,
  * b_layout) bytes, 256-byte aligned) first.  The deep-ring tiles read a row-major B of 16-bit elements in place, with or
- * without a workspace, where n is a multiple of 8, k and both pitches are even and the operands lie on 4-byte addresses;
- * otherwise ptoamd_gemm transposes B inside the loader of the register-staged tiles, for every tile row of C.
+ * without a workspace, where n is a multiple of 8, k and both pitches are even and the operands lie on 4-byte addresses.
+ * Other rows of 16-bit elements, n from 8 up, they read in place without a workspace only, beyond two or three times 128 bytes of K (bf16
+ * 18 x 308 x 7274 18.9 us): a workspace has such a B re-ordered first.  For a shorter K, and for int8, ptoamd_gemm transposes B inside
+ * the loader of the register-staged tiles, for every tile row of C.
  * With a workspace the tile is the one that the column-major product takes (but for a K of a few slabs, where that may be a
- * register-staged one), and its sums have the same order; reading in place can be faster than the re-ordering that this asks
- * for, so pass a workspace where B is not readable in place, or for that order.
+ * register-staged one), and its sums have the same order; reading in place is faster than the re-ordering that this asks for but
+ * for many rows of C where B's start on any element (bf16, n 4097, k 4096: m 512 45 us in place and 50, m 2048 112 and 100), so pass a
+ * workspace for an int8 B, for some 2000 rows of C and more of that kind, or for that order.
  * workspace == NULL is ptoamd_gemm_bias.  No counterpart in
  * the reference (its TLOAD re-orders an ND panel into L1 per tile, cpu/TLoad.hpp:287-321).
  */

@@ -823,8 +823,8 @@ static int gemm_common(void* c, int c_type, const void* a, const void* b, int ab
     const uintptr_t emask = (uintptr_t)ebytes - 1;
     // The register-staged MFMA tiles take rows at any alignment and of any length from 16 bytes up (the row's last chunk
     // is masked), so only f32 / hif8 operands, rows shorter than 16 bytes and misaligned elements go to the order-exact
-    // kernel.  B row-major: with a workspace it is re-ordered there once and the fastest tiles run; without one the
-    // register-staged tiles transpose it on its way into LDS.  Nothing is allocated either way.
+    // kernel.  B row-major: 16-bit elements are read in place where that is possible; otherwise, with a workspace, it is re-ordered there once and
+    // the fastest tiles run, and without one the register-staged tiles transpose it on its way into LDS.  Nothing is allocated either way.
     const bool mfma_type = ab_type != PTOAMD_F32 && ab_type != PTOAMD_HIF8;
     const bool elems_ok = (reinterpret_cast<uintptr_t>(a) & emask) == 0 && (reinterpret_cast<uintptr_t>(b) & emask) == 0;
     const size_t ws_need = b_layout == PTOAMD_B_ND ? (size_t)n * (size_t)ws_row_bytes(k_bytes) : 0;
@@ -852,8 +852,8 @@ static int gemm_common(void* c, int c_type, const void* a, const void* b, int ab
     const bool ragged_k_form = op == TOP_BF16 || op == TOP_F16 || op == TOP_I8, whole_slabs = (k_bytes % 128) == 0;
     const DtlTiles dtl_k = whole_slabs || (ragged_k_form && k_bytes > 128) ? DTL_ALL : DTL_NONE;
     // A row-major B of 16-bit elements is read as it is by the deep-ring kernel and, over whole slabs, by the 256 x 256 tile,
-    // transposed on its way out of LDS (its rows have to be whole 16-byte chunks; a column chunk past N is fetched from the
-    // row's last one).  With a workspace the tile is the one that the same product takes with a column-major B, so that both
+    // transposed on its way out of LDS (where its rows are whole 16-byte chunks that start on dwords; a column chunk past N is fetched from
+    // the row's last one.  Other rows: nd_any below).  With a workspace the tile is the one that the same product takes with a column-major B, so that both
     // have the same bits; where that tile has no row-major form, B is re-ordered for it.  (Register-staged tiles are left out with
     // a workspace: they run a few slabs of K, for which the re-ordering launch costs more than they save.)
     const bool nd_fits = b_layout == PTOAMD_B_ND && ebytes == 2 && !options().b_nd_in_loader && options().tile < 0 &&

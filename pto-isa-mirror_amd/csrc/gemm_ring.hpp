@@ -83,7 +83,7 @@ inline bool ring_by_lines(int shape, const void* a, const void* b, int m, int n,
            rows_off_lines(a, b, m, n, k_bytes, lda_bytes, ldb_bytes, forms[shape].stage_bytes);
 }
 
-// shape: 0 .. RING_SHAPES - 1, RING_UNALIGNED + one of the later ones, or TILE_PREPARE_ALL
+// shape: 0 .. RING_SHAPES - 1, RING_UNALIGNED + one of those of ring_unaligned_shape(), or TILE_PREPARE_ALL
 hipError_t launch_gemm_ring_bf16(int shape, const TileGemmParams& p, hipStream_t stream);
 hipError_t launch_gemm_ring_f16(int shape, const TileGemmParams& p, hipStream_t stream);
 hipError_t launch_gemm_ring_i8(int shape, const TileGemmParams& p, hipStream_t stream);

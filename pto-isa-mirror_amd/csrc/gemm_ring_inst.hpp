@@ -60,7 +60,7 @@ static hipError_t launch_ring_shape(int shape, const TileGemmParams& p, hipStrea
     return hipErrorInvalidValue;
 }
 
-// the form for rows at any alignment, shapes with copying waves only
+// the form for rows at any alignment: shapes with copying waves, and 32 x 32 as four waves that multiply and four that copy
 template <class Op, bool BND = false>
 static hipError_t launch_ring_unaligned(int shape, const TileGemmParams& p, hipStream_t stream)
 {

@@ -520,14 +520,14 @@ struct StagedStore {
 // `bytes` is stored plainly there: where that is ahead with A and C in the caches, as a program has them that uses its activations' buffers again.
 // Time with plain stores over time with streamed ones, geometric means over some 900 sizes a column: launches on the same buffers | on four
 // sets in turn | on weights of 640 MB in turn, A and C the same | all of A, B and C in turn, 640 MB, which no cache holds:
-//   256 x 256 tiles      up to 127 of them, which leave half of the CUs idle, 0.99 | 1.02 | 1.02 | 1.14; from 128 on 0.82 | 0.84 | 0.81 | 0.98
-//   256 x 128            to 16 MiB 0.95 | 0.97 | 0.98 | 1.13; above 0.88 | 0.83 | 0.82 | 1.13
+//   256 x 256 tiles      48 to 127 of them, which leave half of the CUs idle, 1.00 | 1.05 | 1.03 | 1.23; from 128 on 0.82 | 0.84 | 0.82 | 0.98
+//   256 x 128            to 16 MiB 0.95 | 0.97 | 0.97 | 1.13; above 0.88 | 0.83 | 0.81 | 1.13
 //   128 x 128, by DMA    to 4 MiB 0.95 | 0.96 | 0.97 | 1.04; to 16 0.94 | 1.00 | 0.98 | 1.22; above 0.91 | 0.83 | 0.80 | 1.05
 //   register-staged      to 8 MiB 0.95 | 0.97 | 0.98 | 1.04; above 0.98 | 1.00 | 0.98 | 1.15, but few slabs of K 0.58 to 0.95 in the first column
-//   by a word, 16 bits   (bound by the conversions) to 4 MiB 0.98 | 0.99 | 0.99 | 1.00, above 1.00 | 1.02 | 1.02 | 1.09; 256 x 256 1.00 | 1.04 | 1.04 | 1.03
-//   by a word, one byte  (a wave's pieces are a sector long) 1.00 in all, 256 x 256 tiles as above, 4096 x 4104 x 1024 56.3 -> 53.2 us
-// Of the sizes that are stored plainly one in ten is 1 to 5 % behind in the first three columns.  256 x 256 tiles, us, streamed and plain: MXFP4
-// 2040 x 8100 x 8192 72.1 / 66.0, bf16 4096 x 4104 x 1024 51.9 / 46.3.
+//   by a word, 16 bits   (bound by the conversions) to 4 MiB 0.97 | 0.98 | 0.98 | 1.01, above 1.00 | 1.02 | 1.01 | 1.10; 256 x 256 from there on 0.99 | 1.11 | 1.11 | 1.08
+//   by a word, one byte  (a wave's pieces are a sector long) 1.00 in all; 256 x 256 0.98 | 1.00 | 0.99 | 1.01, and on a full grid, 4096 x 4104 x 1024, 56.3 -> 53.2 us
+// Of the sizes that the launcher has stored plainly 1, 8 and 5 in a hundred are more than 2 % behind in the first three columns, and one in three in the
+// last.  256 x 256 tiles, us, streamed and plain: MXFP4 2040 x 8100 x 8192 72.1 / 66.0, bf16 4096 x 4104 x 1024 51.9 / 46.3.
 template <int KIND, class Cfg>
 __device__ __forceinline__ bool plain_off_sectors(long bytes)
 {

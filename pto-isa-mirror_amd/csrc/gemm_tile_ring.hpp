@@ -99,6 +99,7 @@ struct RingCfg {
     static_assert(!ANY || (PIPE && !Op::SCALED), "the register copies are the copying waves' and know no scales");
     static_assert(!ANY || !BND || A_PIECES % NW == 0, "which copies are B's is known at compile time");
     static_assert((ROWS * STAGE_SPS) % 64 == 0, "scale pieces are whole");
+    static_assert(PIPE == (LW > 0), "where some waves only copy, all read the scales' arguments: the pipelined form");
     static_assert(!CHUNKED || (SCB / 4 % SPS == 0 && (SBUFS - 1) * SPC >= R - 1 && BM * SCB % 1024 == 0 && BN * SCB % 1024 == 0 && ROWS <= CW * 64),
                   "a chunk of scales is whole stages; a 1 KiB copy of them is of one operand; a thread can hold a row's");
     static_assert(LDS_BYTES <= 160 * 1024 && R >= 2 && R * NV + (CHUNKED ? ROWS * SCB / 1024 / NW + 1 : 0) < 64, "LDS capacity; vmcnt is a 6-bit count");
